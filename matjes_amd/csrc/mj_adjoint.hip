@@ -61,10 +61,8 @@ __device__ __forceinline__ v3 v_scale(double s, v3 a) { return mk3(s * a.x, s * 
 // (I - [a]x + a a^T)^T ... M(-a) g = (g + a x g + (a.g) a) / (1 + |a|^2)
 __device__ __forceinline__ v3 minv_t(v3 a, v3 g)
 {
-    v3 axg = cross3(a, g);
-    double ag = dot3(a, g);
-    double inv = 1.0 / (1.0 + dot3(a, a));
-    return mk3((g.x + axg.x + ag * a.x) * inv, (g.y + axg.y + ag * a.y) * inv, (g.z + axg.z + ag * a.z) * inv);
+    const v3 w = fma3(dot3(a, g), a, cross3_add(a, g, g));
+    return v_scale(mj_rcp(fma(a.z, a.z, fma(a.y, a.y, fma(a.x, a.x, 1.0)))), w);
 }
 
 __device__ __forceinline__ void adj_tile(const AdjArgs &a, const double *src, double *L, int x0, int y0, int z0)
@@ -206,9 +204,7 @@ __global__ void k_adj_sib1(const AdjArgs a)
     v3 zb = zeeman_t(a, s.gi);
     v3 B = mk3(-(acc.x + zb.x), -(acc.y + zb.y), -(acc.z + zb.z));
     v3 c = cross3(m, B);
-    v3 av = v_scale(a.f, mk3(B.x + a.alpha * c.x, B.y + a.alpha * c.y, B.z + a.alpha * c.z));
-    v3 mt = cayley(m, av);
-    st3(a.out0, s.gi, a.np, mk3(0.5 * (m.x + mt.x), 0.5 * (m.y + mt.y), 0.5 * (m.z + mt.z)));
+    st3(a.out0, s.gi, a.np, cayley_mid(m, v_scale(a.f, fma3(a.alpha, c, B))));
 }
 
 // forward stage 2: m' = cay(m, a2(p))
@@ -225,7 +221,7 @@ __global__ void k_adj_sib2(const AdjArgs a)
     v3 zb = zeeman_t(a, s.gi);
     v3 B = mk3(-(acc.x + zb.x), -(acc.y + zb.y), -(acc.z + zb.z));
     v3 c = cross3(p, B);
-    v3 av = v_scale(a.f, mk3(B.x + a.alpha * c.x, B.y + a.alpha * c.y, B.z + a.alpha * c.z));
+    v3 av = v_scale(a.f, fma3(a.alpha, c, B));
     st3(a.out0, s.gi, a.np, cayley(ld3(a.m, s.gi, a.np), av));
 }
 
@@ -252,9 +248,7 @@ __device__ __forceinline__ v3 adj_midpoint(const AdjArgs &a, const double *L0, i
     v3 zb = zeeman_t(a, gi);
     v3 B = mk3(-(acc.x + zb.x), -(acc.y + zb.y), -(acc.z + zb.z));
     v3 c = cross3(m, B);
-    v3 av = v_scale(a.f, mk3(B.x + a.alpha * c.x, B.y + a.alpha * c.y, B.z + a.alpha * c.z));
-    v3 mt = cayley(m, av);
-    return mk3(0.5 * (m.x + mt.x), 0.5 * (m.y + mt.y), 0.5 * (m.z + mt.z));
+    return cayley_mid(m, v_scale(a.f, fma3(a.alpha, c, B)));
 }
 
 // a whole forward step in one kernel: the tile plus twice the reach (S0) in
@@ -337,7 +331,7 @@ __global__ void k_adj_sibf(const AdjArgs a)
     v3 zb = zeeman_t(a, s.gi);
     v3 B = mk3(-(acc.x + zb.x), -(acc.y + zb.y), -(acc.z + zb.z));
     v3 c = cross3(p, B);
-    v3 av = v_scale(a.f, mk3(B.x + a.alpha * c.x, B.y + a.alpha * c.y, B.z + a.alpha * c.z));
+    v3 av = v_scale(a.f, fma3(a.alpha, c, B));
     st3(a.out0, s.gi, a.np, p);
     st3(a.out1, s.gi, a.np, cayley(m0, av));
 }
@@ -353,7 +347,7 @@ __device__ __forceinline__ void r1_site(const AdjArgs &a, const double *L, int T
         v3 zb = zeeman_t(a, s.gi);
         v3 B = mk3(-(acc.x + zb.x), -(acc.y + zb.y), -(acc.z + zb.z));
         v3 c = cross3(p, B);
-        v3 av = v_scale(a.f, mk3(B.x + a.alpha * c.x, B.y + a.alpha * c.y, B.z + a.alpha * c.z));
+        v3 av = v_scale(a.f, fma3(a.alpha, c, B));
         v3 m = ld3(a.m, s.gi, a.np), m1 = ld3(a.m1, s.gi, a.np);
         v3 gm = cayley(g, mk3(-av.x, -av.y, -av.z));
         v3 w = minv_t(av, g);
@@ -438,7 +432,7 @@ __global__ void k_adj_r2(const AdjArgs a)
         v3 zb = zeeman_t(a, s.gi);
         v3 B = mk3(-(acc.x + zb.x), -(acc.y + zb.y), -(acc.z + zb.z));
         v3 c = cross3(m, B);
-        v3 av = v_scale(a.f, mk3(B.x + a.alpha * c.x, B.y + a.alpha * c.y, B.z + a.alpha * c.z));
+        v3 av = v_scale(a.f, fma3(a.alpha, c, B));
         v3 mt = cayley(m, av);
         gm = v_add(gm, cayley(gmt, mk3(-av.x, -av.y, -av.z)));
         v3 w = minv_t(av, gmt);

@@ -1175,10 +1175,13 @@ static int run_steps(mj_ctx *c, int nsteps, int integ, double timestep, double a
     KArgs base;
     base_args(c, base);
     base.alpha = alpha;
-    base.den = 1.0 + alpha * alpha;
-    base.rden = 1.0 / base.den;
-    base.dt = stage_dt(ts);
-    base.sigma = sigma_of(base.dt);
+    const double rden = 1.0 / (1.0 + alpha * alpha);
+    auto set_dt = [&](KArgs &a, double dt) {
+        a.kt = dt / kHbar;
+        a.kdt = a.kt * rden;
+    };
+    set_dt(base, stage_dt(ts));
+    base.sigma = sigma_of(stage_dt(ts));
     base.seed = seed;
     const double escale = 1.0 / (double)c->n;
     double *bpart = c->epart + 2 * (size_t)c->epart_cap;
@@ -1236,11 +1239,11 @@ static int run_steps(mj_ctx *c, int nsteps, int integ, double timestep, double a
             // spindynamics.f90:282-318: every stage from the previous stage's state,
             // dt_i = Butcher(1, i+1) dt_{i-1} from timestep / N (get_dt_mode)
             const int N = nl;
-            double dt = a.dt / (double)N;   // a.dt: the step's timestep here (timestep_int / real(N_loop))
+            double dt = ts / (double)N;   // timestep_int / real(N_loop)
             for (int i = 1; i <= N; ++i) {
                 dt = rkT[1][i + 1] * dt;
                 KArgs s = a;
-                s.dt = dt;
+                set_dt(s, dt);
                 s.src = c->A;
                 MJ_TRY(prep_field(c, c->A, s));
                 s.dst = c->Bb;
@@ -1413,11 +1416,11 @@ static int run_steps(mj_ctx *c, int nsteps, int integ, double timestep, double a
         KArgs a = base;
         a.step = step0 + (uint64_t)j;
         if (adapt) {
-            a.dt = stage_dt(ts);
-            a.sigma = sigma_of(a.dt);
+            set_dt(a, stage_dt(ts));
+            a.sigma = sigma_of(stage_dt(ts));
             if (ad->ts_used) ad->ts_used[j] = ts;
         }
-        if (kT_steps) a.sigma = sigma_kt(a.dt, kT_steps[j]);
+        if (kT_steps) a.sigma = sigma_kt(stage_dt(ts), kT_steps[j]);
         if (noisy && noise_host) {
             MJ_HIP_CHECK(hipMemcpyAsync(c->Fb, noise_host + (size_t)j * 3 * c->n, sizeof(double) * 3 * c->n,
                                         hipMemcpyHostToDevice, c->stream));

@@ -46,7 +46,7 @@ struct BatchSys {
     int64_t hstride;
     double zb[3];
     double z9[9];         // the Zeeman block, for a per-site B map (bmode 2)
-    double alpha, den, rden;
+    double alpha, rden;   // rden = 1 / (1 + alpha^2)
     uint64_t seed;
 };
 
@@ -109,8 +109,7 @@ __device__ __forceinline__ KArgs sys_args(const KArgs &base, const BatchSys &S, 
         a.hstride = S.hstride;
     }
     a.alpha = S.alpha;
-    a.den = S.den;
-    a.rden = S.rden;
+    a.kdt = base.kt * S.rden;
     a.sigma = sigma;
     a.seed = S.seed;
     a.step = step;
@@ -184,22 +183,20 @@ __device__ __forceinline__ void batch_stage1(const KArgs &a0, const double *L0, 
     m0 = mk3(L0[c0], L0[T0 + c0], L0[2 * T0 + c0]);
     RtGeom::stencil(a0, L0, T0, c0, ax, ay, az);
     const v3 z = batch_zeeman(a0, true, gi);
-    const double hx = 0.0, hy = 0.0, hz = 0.0;
-    v3 B = mk3(-(ax + z.x) - 2.0 * hx, -(ay + z.y) - 2.0 * hy, -(az + z.z) - 2.0 * hz);
+    v3 B = mk3(-(ax + z.x), -(ay + z.y), -(az + z.z));
     if constexpr (INTEG == MJ_HEUN) {
         (void)bt;
-        X = llg_rhs(m0, B, a0.alpha, a0.den, a0.rden);
-        m1 = euler_step0(m0, X, a0.dt);
+        const MjUnit u = mj_unit(m0);
+        X = llg_torque(u.n, B, a0.alpha);
+        m1 = euler_step0(m0, u, X, a0.kdt);
     } else {
         B = mk3(B.x + bt.x, B.y + bt.y, B.z + bt.z);
         if constexpr (INTEG == MJ_SIB) {
-            const v3 av = sib_vec(m0, B, a0.alpha, a0.dt);
-            const v3 mt = cayley(m0, av);
-            m1 = mk3(0.5 * (m0.x + mt.x), 0.5 * (m0.y + mt.y), 0.5 * (m0.z + mt.z));
+            m1 = cayley_mid(m0, sib_vec(m0, B, a0.alpha, -0.5 * a0.kdt));
             X = mk3(0.0, 0.0, 0.0);
         } else {
-            X = dep_field(m0, B, a0.alpha, a0.den, a0.rden);
-            m1 = dep_rotate(m0, X, a0.dt);
+            X = dep_field(m0, B, a0.alpha);
+            m1 = dep_rotate(m0, X, a0.kdt);
         }
     }
 }
@@ -327,22 +324,20 @@ __device__ __forceinline__ void batch_fused_tile(const KArgs &a, const int *ofs0
         double ax = 0.0, ay = 0.0, az = 0.0;
         RtGeom::stencil(a, L1, T1, c1, ax, ay, az);
         const v3 z = batch_zeeman(a, true, gi);
-        const double hx = 0.0, hy = 0.0, hz = 0.0;
-        v3 B = mk3(-(ax + z.x) - 2.0 * hx, -(ay + z.y) - 2.0 * hy, -(az + z.z) - 2.0 * hz);
+        v3 B = mk3(-(ax + z.x), -(ay + z.y), -(az + z.z));
         v3 o;
         if constexpr (INTEG == MJ_HEUN) {
-            const v3 D2 = llg_rhs(m, B, a.alpha, a.den, a.rden);
-            const v3 dint = mk3(0.5 * D1.x + 0.5 * D2.x, 0.5 * D1.y + 0.5 * D2.y, 0.5 * D1.z + 0.5 * D2.z);
-            o = euler_step(m, dint, llg_rhs(m0, bt, a.alpha, a.den, a.rden), a.dt);
+            const MjUnit u = mj_unit(m);
+            const v3 dint = heun_dint(D1, llg_torque(u.n, B, a.alpha));
+            o = euler_step(m, u, dint, llg_torque(mj_unit(m0).n, bt, a.alpha), a.kdt);
         } else if constexpr (INTEG == MJ_SIB) {
             B = mk3(B.x + bt.x, B.y + bt.y, B.z + bt.z);
-            const v3 av = sib_vec(m, B, a.alpha, a.dt);
-            o = cayley(m0, av);
+            o = cayley(m0, sib_vec(m, B, a.alpha, -0.5 * a.kdt));
         } else {
             B = mk3(B.x + bt.x, B.y + bt.y, B.z + bt.z);
-            const v3 b2 = dep_field(m, B, a.alpha, a.den, a.rden);
+            const v3 b2 = dep_field(m, B, a.alpha);
             const v3 ba = mk3(0.5 * (D1.x + b2.x), 0.5 * (D1.y + b2.y), 0.5 * (D1.z + b2.z));
-            o = dep_rotate(m0, ba, a.dt);
+            o = dep_rotate(m0, ba, a.kdt);
         }
         a.dst[gi] = o.x;
         a.dst[gi + np] = o.y;
@@ -350,12 +345,11 @@ __device__ __forceinline__ void batch_fused_tile(const KArgs &a, const int *ofs0
     }
 }
 
-// one step of every system: base.src -> base.dst
-#ifndef MJ_FUSED_WAVES
-#define MJ_FUSED_WAVES 6
-#endif
+// one step of every system: base.src -> base.dst; compiled for at least 6
+// waves per SIMD (Heun) or 5 (SIB and Depondt, whose ring also draws the
+// thermal field: they spill at 6)
 template <int INTEG>
-__global__ void __launch_bounds__(MJ_BATCH_NTHR, MJ_FUSED_WAVES)
+__global__ void __launch_bounds__(MJ_BATCH_NTHR, INTEG == MJ_HEUN ? 6 : 5)
     k_batch_fused(const KArgs base, const BatchSys *__restrict__ sys, const int *__restrict__ blk2sys,
                   const double *__restrict__ sigma, const uint64_t *__restrict__ stepp, const int *__restrict__ ofs0)
 {
@@ -974,8 +968,7 @@ static int batch_finalize(mj_batch *b)
         for (int a = 0; a < 3; ++a) t.zb[a] = s.zb[a];
         for (int k = 0; k < 9; ++k) t.z9[k] = s.z9[k];
         t.alpha = s.alpha;
-        t.den = 1.0 + s.alpha * s.alpha;
-        t.rden = 1.0 / t.den;
+        t.rden = 1.0 / (1.0 + s.alpha * s.alpha);
         t.seed = s.seed;
         s.base = np;
         t.base = np;
@@ -1164,7 +1157,7 @@ static void batch_base(const mj_batch *b, KArgs &a, double timestep)
     a.ofs = b->d_ofs;
     a.cf = b->d_cf;
     a.bmap = b->bmap;
-    a.dt = batch_dt(b, timestep);
+    a.kt = batch_dt(b, timestep) / kHbarB;
 }
 
 // energies of the entering states per system, then the replica exchange of

@@ -1,11 +1,26 @@
 // Device-side helpers for the LLG hot path on gfx950.
 //
-// All per-site vector algebra is written out in the reference's operation
-// order and the library is compiled without floating-point contraction, so
-// LLG / euler / langevin reproduce src/solvers/propagator.f90:13-40,
-// src/solvers/solver.f90:157-178 and src/dynamics/BTeff_sd.f90:18-45 op for
-// op.  The stencil sum (where the reference's own order depends on its matrix
-// backend) uses explicit fma().
+// LLG / euler / langevin evaluate the formulas of
+// src/solvers/propagator.f90:13-40, src/solvers/solver.f90:157-178 and
+// src/dynamics/BTeff_sd.f90:18-45.  The library is compiled without
+// floating-point contraction; where products and sums are fused, fma() says
+// so, so that every kernel that runs a stage (compiled per Hamiltonian or
+// ahead of time, fused or one launch per stage, batched or not) rounds alike
+// and gives the same bits.
+//
+// What bounds the stage kernels is the issue of FP64 instructions (an LLG
+// evaluation and its euler step took about 140 besides the neighbour sum), so
+// the per-site algebra is arranged for few of them without giving up
+// accuracy: the constant factor dt / (hbar (1 + alpha^2)) is one operand, the
+// unit vector and the restored length are increments about 1 where the
+// length allows it (mj_unit, mj_restore), and a rotation is formed without
+// its axis and angle (dep_rotate).  Which branch a site takes depends on its
+// own values only.  Per step against the correctly rounded square roots and
+// quotients of the formulas as they stand: Heun, triangular 2048x2048 at 10 K
+// 143.6 -> 113.9 us, 1024x1024 44.7 -> 37.6 us; Depondt, square 768x640 at
+// 10 K 22.3 -> 16.9 us.  Against quadruple precision the states are 1.3 to 5
+// times closer (Heun, 1000 steps at 10 K: rms 1.0e-14, before 4.9e-14), since
+// the length is restored with one rounding.
 #pragma once
 #ifndef __HIPCC_RTC__
 #include <hip/hip_runtime.h>
@@ -15,19 +30,6 @@
 #include <stdint.h>
 
 #define MJ_HBAR 6.58211928e-1  // eV fs (src/fixed-parameters/constant.f90:25)
-#define MJ_RHBAR 0x1.84eeb74185935p+0  // RN(1/MJ_HBAR)
-
-// a / b for a divisor b known with its correctly rounded reciprocal r = RN(1/b):
-// q0 = RN(a r), e = a - b q0 (exact, fma), RN(q0 + e r) is the correctly rounded
-// quotient (Markstein, IBM J. Res. Dev. 34 (1990) 111) outside the
-// overflow/underflow range; three instructions instead of the general
-// division sequence, bit-identical to a / b.
-__device__ __forceinline__ double div_rn(double a, double b, double r)
-{
-    const double q0 = a * r;
-    const double e = fma(-b, q0, a);
-    return fma(e, r, q0);
-}
 
 struct v3 {
     double x, y, z;
@@ -45,8 +47,23 @@ __device__ __forceinline__ v3 mk3(double x, double y, double z)
 // cross_NM (src/vector_utils/vector.f90:451-465)
 __device__ __forceinline__ v3 cross3(v3 a, v3 b)
 {
-    return mk3(a.y * b.z - a.z * b.y, a.z * b.x - a.x * b.z, a.x * b.y - a.y * b.x);
+    return mk3(fma(a.y, b.z, -(a.z * b.y)), fma(a.z, b.x, -(a.x * b.z)), fma(a.x, b.y, -(a.y * b.x)));
 }
+
+// c + a x b
+__device__ __forceinline__ v3 cross3_add(v3 a, v3 b, v3 c)
+{
+    return mk3(fma(a.y, b.z, fma(-a.z, b.y, c.x)), fma(a.z, b.x, fma(-a.x, b.z, c.y)),
+               fma(a.x, b.y, fma(-a.y, b.x, c.z)));
+}
+
+// a + k b
+__device__ __forceinline__ v3 fma3(double k, v3 b, v3 a)
+{
+    return mk3(fma(k, b.x, a.x), fma(k, b.y, a.y), fma(k, b.z, a.z));
+}
+
+__device__ __forceinline__ double dot3(v3 a, v3 b) { return fma(a.z, b.z, fma(a.y, b.y, a.x * b.x)); }
 
 // Correctly rounded sqrt(x) and 1 / x for the per-site algebra: the
 // instruction sequences the compiler emits for sqrt and 1.0 / x in double
@@ -83,118 +100,169 @@ __device__ __forceinline__ double mj_rcp_rn(double x)
     return fma(f, r, r);
 }
 
-__device__ __forceinline__ double dot3(v3 a, v3 b) { return (a.x * b.x + a.y * b.y) + a.z * b.z; }
-__device__ __forceinline__ double norm3(v3 a) { return mj_sqrt_rn((a.x * a.x + a.y * a.y) + a.z * a.z); }
+__device__ __forceinline__ double norm3(v3 a) { return mj_sqrt_rn(dot3(a, a)); }
 
-// normalize with the 1e-8 guard (src/vector_utils/vector.f90:76-84); the three
-// quotients m_k / |m| share one correctly rounded reciprocal (div_rn)
-__device__ __forceinline__ v3 unit3(v3 m)
+// 1 / x to about an ulp, x in [2^-1000, 2^1000]: the hardware estimate and two
+// Newton steps (mj_rcp_rn without its last correction)
+__device__ __forceinline__ double mj_rcp(double x)
 {
-    double nr = norm3(m);
-    if (nr > 1.0e-8) {
-        const double r = mj_rcp_rn(nr);
-        return mk3(div_rn(m.x, nr, r), div_rn(m.y, nr, r), div_rn(m.z, nr, r));
+    double r = __builtin_amdgcn_rcp(x);
+    r = fma(r, fma(-x, r, 1.0), r);
+    return fma(r, fma(-x, r, 1.0), r);
+}
+
+// The unit vector n = m / |m| of normalize (src/vector_utils/vector.f90:76-84:
+// m itself where |m| <= 1e-8), with |m|^2 and 1 / |m|^2 for mj_restore.  A
+// spin that euler, Cayley or a rotation left at unit length has
+// |m|^2 = 1 + e with e of a few ulp: 1 / |m| = 1 - e/2 to 3 e^2 / 8, below
+// 2^-54 for |e| <= 2^-27; one instruction instead of a square root and a
+// division (28).  Where |m| <= 1e-8, r2 = infinity sends mj_restore to its
+// general branch.
+struct MjUnit {
+    v3 n;
+    double x, r2;
+};
+
+__device__ __forceinline__ MjUnit mj_unit(v3 m)
+{
+    MjUnit u;
+    u.x = dot3(m, m);
+    double r = fma(-0.5, u.x, 1.5);
+    u.r2 = r * r;
+    if (!(fabs(u.x - 1.0) <= 0x1p-27)) {
+        const bool ok = u.x > 1.0e-16;
+        r = ok ? mj_rcp_rn(mj_sqrt_rn(u.x)) : 1.0;
+        u.r2 = ok ? r * r : __builtin_inf();
     }
-    return m;
+    u.n = mk3(m.x * r, m.y * r, m.z * r);
+    return u;
 }
 
-// D = -m^ x (B + a m^ x B)/(1 + a^2)   (propagator.f90:32-40, BTeff_sd.f90:38-43)
-// den = 1 + a^2 and rden = RN(1/den)
-__device__ __forceinline__ v3 llg_rhs(v3 m, v3 B, double alpha, double den, double rden)
+// t |m| / |t| (the last line of euler, solver.f90:172-176; m where
+// |t| <= 1e-8), u = mj_unit(m).  With v = (|m|^2 - |t|^2) / |m|^2 the factor
+// is (1 - v)^(-1/2) = 1 + v f(v): t + t (v f) rounds once, where a product
+// with |m| and a division by |t| round twice beside the errors of both
+// lengths, and v = 0 (a spin at rest) returns t itself.  f of degree 6,
+// |v| <= 2^-6 (a turn of up to 7 degrees per stage), within 3e-17 in v f; 13
+// instructions instead of 51 (two square roots, a reciprocal and three
+// corrected quotients).
+__device__ __forceinline__ v3 mj_restore(v3 m, MjUnit u, v3 t)
 {
-    v3 mn = unit3(m);
-    v3 c = cross3(mn, B);
-    v3 l = mk3(B.x + alpha * c.x, B.y + alpha * c.y, B.z + alpha * c.z);
-    v3 o = cross3(mn, l);
-    return mk3(div_rn(-o.x, den, rden), div_rn(-o.y, den, rden), div_rn(-o.z, den, rden));
-}
-
-// the thermal increment DT*dt/hbar of euler (solver.f90:174), rounded as there
-__device__ __forceinline__ v3 thermal_increment(v3 dtf, double dt)
-{
-    return mk3(div_rn(dtf.x * dt, MJ_HBAR, MJ_RHBAR), div_rn(dtf.y * dt, MJ_HBAR, MJ_RHBAR),
-               div_rn(dtf.z * dt, MJ_HBAR, MJ_RHBAR));
-}
-
-// euler (solver.f90:172-176): t = (m + Dint*dt/hbar) + DT*dt/hbar; m' = t*|m|/|t|,
-// with q = DT*dt/hbar given
-__device__ __forceinline__ v3 euler_step_q(v3 m, v3 dint, v3 q, double dt)
-{
-    double mn = norm3(m);
-    v3 t = mk3((m.x + div_rn(dint.x * dt, MJ_HBAR, MJ_RHBAR)) + q.x, (m.y + div_rn(dint.y * dt, MJ_HBAR, MJ_RHBAR)) + q.y,
-               (m.z + div_rn(dint.z * dt, MJ_HBAR, MJ_RHBAR)) + q.z);
-    double tn = norm3(t);
-    if (tn > 1.0e-8) {
-        const double r = mj_rcp_rn(tn);
-        return mk3(div_rn(t.x * mn, tn, r), div_rn(t.y * mn, tn, r), div_rn(t.z * mn, tn, r));
+    const double y = dot3(t, t);
+    const double v = (u.x - y) * u.r2;
+    double f = 0.20955191976592094;
+    f = fma(f, v, 0.22566986332987313);
+    f = fma(f, v, 0.24609374032347447);
+    f = fma(f, v, 0.2734374897543061);
+    f = fma(f, v, 0.3125000000002953);
+    f = fma(f, v, 0.3750000000003127);
+    f = fma(f, v, 0.5);
+    v3 o = fma3(f * v, t, t);
+    if (!(fabs(v) <= 0x1p-6)) {
+        const double tn = mj_sqrt_rn(y);
+        const double s = mj_sqrt_rn(u.x) * mj_rcp_rn(tn);
+        o = tn > 1.0e-8 ? mk3(t.x * s, t.y * s, t.z * s) : m;
     }
-    return m;
+    return o;
 }
 
-__device__ __forceinline__ v3 euler_step(v3 m, v3 dint, v3 dtf, double dt)
+// D (1 + a^2) = -n x (B + a n x B), n = m / |m|   (propagator.f90:32-40,
+// BTeff_sd.f90:38-43); the division by 1 + a^2 is part of the stage's factor
+// k = dt / (hbar (1 + a^2))
+__device__ __forceinline__ v3 llg_torque(v3 n, v3 B, double alpha)
 {
-    return euler_step_q(m, dint, thermal_increment(dtf, dt), dt);
+    return cross3(fma3(alpha, cross3(n, B), B), n);
 }
 
-// euler without a thermal term (the reference adds Dmag_T_zero*dt/hbar = +0)
-__device__ __forceinline__ v3 euler_step0(v3 m, v3 dint, double dt)
+// euler (solver.f90:172-176): t = (m + Dint dt/hbar) + DT dt/hbar, m' = t |m| / |t|;
+// dint and dth torques (llg_torque), k = dt / (hbar (1 + a^2))
+__device__ __forceinline__ v3 euler_step(v3 m, MjUnit u, v3 dint, v3 dth, double k)
 {
-    double mn = norm3(m);
-    v3 t = mk3(m.x + div_rn(dint.x * dt, MJ_HBAR, MJ_RHBAR), m.y + div_rn(dint.y * dt, MJ_HBAR, MJ_RHBAR),
-               m.z + div_rn(dint.z * dt, MJ_HBAR, MJ_RHBAR));
-    double tn = norm3(t);
-    if (tn > 1.0e-8) {
-        const double r = mj_rcp_rn(tn);
-        return mk3(div_rn(t.x * mn, tn, r), div_rn(t.y * mn, tn, r), div_rn(t.z * mn, tn, r));
-    }
-    return m;
+    return mj_restore(m, u, fma3(k, dth, fma3(k, dint, m)));
 }
 
-// Implicit-midpoint (Cayley) solve (I + [a]x) x = m - a x m  (SIB, Mentink et al. 2010)
+__device__ __forceinline__ v3 euler_step0(v3 m, MjUnit u, v3 dint, double k)
+{
+    return mj_restore(m, u, fma3(k, dint, m));
+}
+
+// Dint = D1/2 + D2/2 of integration 2's second stage (get_Dmode_int)
+__device__ __forceinline__ v3 heun_dint(v3 d1, v3 d2)
+{
+    return mk3(0.5 * (d1.x + d2.x), 0.5 * (d1.y + d2.y), 0.5 * (d1.z + d2.z));
+}
+
+// Implicit-midpoint (Cayley) solve (I + [a]x) x = m - a x m  (SIB, Mentink et
+// al. 2010): x = m + 2 g w, w = u + u x a, u = m x a, g = 1 / (1 + |a|^2); the
+// midpoint (m + x) / 2 is m + g w
+__device__ __forceinline__ v3 cayley_inc(v3 m, v3 a, double &g)
+{
+    const v3 u = cross3(m, a);
+    g = mj_rcp(fma(a.z, a.z, fma(a.y, a.y, fma(a.x, a.x, 1.0))));
+    return cross3_add(u, a, u);
+}
+
 __device__ __forceinline__ v3 cayley(v3 m, v3 a)
 {
-    v3 axm = cross3(a, m);
-    v3 y = mk3(m.x - axm.x, m.y - axm.y, m.z - axm.z);
-    v3 axy = cross3(a, y);
-    double ay = dot3(a, y);
-    double aa = dot3(a, a);
-    double inv = mj_rcp_rn(1.0 + aa);
-    return mk3(((y.x - axy.x) + ay * a.x) * inv, ((y.y - axy.y) + ay * a.y) * inv,
-               ((y.z - axy.z) + ay * a.z) * inv);
+    double g;
+    const v3 w = cayley_inc(m, a, g);
+    return fma3(2.0 * g, w, m);
 }
 
-// a = (dt/2) Omega, Omega = -(B + alpha p x B)/((1+alpha^2) hbar)
-__device__ __forceinline__ v3 sib_vec(v3 p, v3 B, double alpha, double dt)
+__device__ __forceinline__ v3 cayley_mid(v3 m, v3 a)
 {
-    v3 c = cross3(p, B);
-    double f = -0.5 * dt / ((1.0 + alpha * alpha) * MJ_HBAR);
-    return mk3(f * (B.x + alpha * c.x), f * (B.y + alpha * c.y), f * (B.z + alpha * c.z));
+    double g;
+    const v3 w = cayley_inc(m, a, g);
+    return fma3(g, w, m);
 }
 
-// Depondt effective rotation field Bt = (B + alpha m^ x B)/(1+alpha^2)
-__device__ __forceinline__ v3 dep_field(v3 m, v3 B, double alpha, double den, double rden)
+// a = (dt/2) Omega, Omega = -(B + alpha p x B)/((1+alpha^2) hbar); f = -dt / (2 (1+alpha^2) hbar)
+__device__ __forceinline__ v3 sib_vec(v3 p, v3 B, double alpha, double f)
 {
-    v3 mn = unit3(m);
-    v3 c = cross3(mn, B);
-    return mk3(div_rn(B.x + alpha * c.x, den, rden), div_rn(B.y + alpha * c.y, den, rden),
-               div_rn(B.z + alpha * c.z, den, rden));
+    const v3 l = fma3(alpha, cross3(p, B), B);
+    return mk3(f * l.x, f * l.y, f * l.z);
 }
 
-// rotate m about b by |b| dt / hbar (Rodrigues), dm/dt = (1/hbar) b x m
-__device__ __forceinline__ v3 dep_rotate(v3 m, v3 b, double dt)
+// Depondt's rotation field times 1 + alpha^2: B + alpha n x B, n = m / |m|
+__device__ __forceinline__ v3 dep_field(v3 m, v3 B, double alpha) { return fma3(alpha, cross3(mj_unit(m).n, B), B); }
+
+// m rotated by the vector w = k b (k = dt / (hbar (1 + alpha^2)), b from
+// dep_field): Rodrigues without the axis and the angle,
+//   m' = m + S w x m + C w x (w x m), S = sin th / th, C = (1 - cos th) / th^2,
+// both polynomials in z = th^2 = |w|^2 for th <= 1/2 (within 5e-17 and 3e-18):
+// 39 instructions, where the normalised axis and a sincos with its range
+// reduction took about 200
+__device__ __forceinline__ v3 dep_rotate(v3 m, v3 b, double k)
 {
-    double bn = norm3(b);
-    if (!(bn > 0.0)) return m;
-    const double rb = mj_rcp_rn(bn);
-    v3 k = mk3(div_rn(b.x, bn, rb), div_rn(b.y, bn, rb), div_rn(b.z, bn, rb));
-    double th = div_rn(bn * dt, MJ_HBAR, MJ_RHBAR);
-    double st, ct;
-    sincos(th, &st, &ct);
-    v3 kxm = cross3(k, m);
-    double km = dot3(k, m);
-    double f = km * (1.0 - ct);
-    return mk3((m.x * ct + kxm.x * st) + k.x * f, (m.y * ct + kxm.y * st) + k.y * f,
-               (m.z * ct + kxm.z * st) + k.z * f);
+    const v3 w = mk3(k * b.x, k * b.y, k * b.z);
+    const double z = dot3(w, w);
+    double S = -2.4931934029233215e-08, C = -2.0790894217124703e-09;
+    S = fma(S, z, 2.7556981477681245e-06);
+    C = fma(C, z, 2.7557077887523167e-07);
+    S = fma(S, z, -0.00019841269403598734);
+    C = fma(C, z, -2.4801586988836374e-05);
+    S = fma(S, z, 0.00833333333307693);
+    C = fma(C, z, 0.0013888888888705666);
+    S = fma(S, z, -0.16666666666666116);
+    C = fma(C, z, -0.041666666666666276);
+    S = fma(S, z, 1.0);
+    C = fma(C, z, 0.5);
+    if (!(z <= 0.25)) {
+        const double th = sqrt(z);
+        double st, ct;
+        sincos(th, &st, &ct);
+        S = st / th;
+        C = (1.0 - ct) / z;
+    }
+    const v3 u = cross3(w, m);
+    return fma3(C, cross3(w, u), fma3(S, u, m));
+}
+
+// energy of a site: m.(H m) + b.(Z m) + m.H_fft = m.(a/2 + z), a the
+// neighbour sum, z = Z^T b + H_fft
+__device__ __forceinline__ double mj_site_energy(v3 m, v3 a, v3 z)
+{
+    return dot3(m, fma3(0.5, a, z));
 }
 
 // ---------------------------------------------------------------------------

@@ -52,7 +52,7 @@ struct KArgs {
     int dnx, dny;         // padded grid dims (x, y)
     int64_t hstride;
 
-    double alpha, den, rden, dt, sigma;   // den = 1 + alpha^2, rden = RN(1/den)
+    double alpha, kt, kdt, sigma;   // kt = dt / hbar of the stage, kdt = kt / (1 + alpha^2)
     uint64_t seed, step;
     const uint64_t *stepp;  // or null: the thermal-field step is *stepp + step (graph-replayed steps)
     const double *noise;  // injected thermal field (SoA) or null

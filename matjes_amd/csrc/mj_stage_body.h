@@ -171,7 +171,7 @@ struct SiteCtx {
 template <int MODE>
 __device__ __forceinline__ v3 thermal_term(const KArgs &a, const SiteCtx &s, v3 bt)
 {
-    if constexpr (MODE == MODE_HEUN2) return llg_rhs(s.pre_own, bt, a.alpha, a.den, a.rden);
+    if constexpr (MODE == MODE_HEUN2) return llg_torque(mj_unit(s.pre_own).n, bt, a.alpha);
     return bt;
 }
 
@@ -439,7 +439,7 @@ __device__ __forceinline__ void site_end(const KArgs &a, double *lds, const Site
     if (a.energy) {
         double e = 0.0;
         if (active)
-            e = m.x * ((0.5 * ax + zx) + hx) + m.y * ((0.5 * ay + zy) + hy) + m.z * ((0.5 * az + zz) + hz);
+            e = mj_site_energy(m, mk3(ax, ay, az), mk3(zx + hx, zy + hy, zz + hz));
         __syncthreads();
         double s = mj_block_sum(e, lds, nthr);
         if (threadIdx.x == 0) a.epart[part] = s;
@@ -464,39 +464,35 @@ __device__ __forceinline__ void site_end(const KArgs &a, double *lds, const Site
     }
     if constexpr (MODE == MODE_FIELD) {
     } else if constexpr (MODE == MODE_EULER) {
-        v3 D = llg_rhs(m, B, alpha, a.den, a.rden);
-        // Dint = 0 + 1 D (get_Dmode_int); the leading zero changes only the sign of an exact zero
-        v3 dint = D;
+        const MjUnit u = mj_unit(m);
+        // Dint = 1 D (get_Dmode_int)
+        const v3 D = llg_torque(u.n, B, alpha);
         v3 o;
-        if constexpr (NOISE) o = euler_step(m, dint, llg_rhs(m, site_thermal_final<MODE, G>(a, st), alpha, a.den, a.rden), a.dt);
-        else o = euler_step0(m, dint, a.dt);
+        if constexpr (NOISE) o = euler_step(m, u, D, llg_torque(u.n, site_thermal_final<MODE, G>(a, st), alpha), a.kdt);
+        else o = euler_step0(m, u, D, a.kdt);
         a.dst[gi] = o.x;
         a.dst[gi + np] = o.y;
         a.dst[gi + 2 * np] = o.z;
     } else if constexpr (MODE == MODE_RKS) {
         // stage i of integration 4 (spindynamics.f90:294-318 with get_Dmode_int,
-        // solver_order.f90:46-58): D_i = LLG(B(m), m); Dint = (0 + w_1 D_1) + ... + w_i D_i;
+        // solver_order.f90:46-58): D_i = LLG(B(m), m); Dint = w_1 D_1 + ... + w_i D_i;
         // m' = euler(m, Dint, 0, dt_i).  Unrolled over the at most 7 earlier stages
         // (constant indices keep the argument block in registers).
-        v3 D = llg_rhs(m, B, alpha, a.den, a.rden);
-        double dx = 0.0, dy = 0.0, dz = 0.0;
+        const MjUnit u = mj_unit(m);
+        const v3 D = llg_torque(u.n, B, alpha);
+        v3 dint = mk3(0.0, 0.0, 0.0);
 #pragma unroll
         for (int k = 0; k < 7; ++k) {
             if (k < a.nprev) {
                 const double *p = a.dprev[k];
-                dx = dx + a.wrk[k] * p[gi];
-                dy = dy + a.wrk[k] * p[gi + np];
-                dz = dz + a.wrk[k] * p[gi + 2 * np];
+                dint = fma3(a.wrk[k], mk3(p[gi], p[gi + np], p[gi + 2 * np]), dint);
             }
         }
         double wi = 0.0;
 #pragma unroll
         for (int k = 0; k < 8; ++k)
             if (k == a.nprev) wi = a.wrk[k];
-        dx = dx + wi * D.x;
-        dy = dy + wi * D.y;
-        dz = dz + wi * D.z;
-        v3 o = euler_step0(m, mk3(dx, dy, dz), a.dt);
+        const v3 o = euler_step0(m, u, fma3(wi, D, dint), a.kdt);
         if (a.dout) {
             a.dout[gi] = D.x;
             a.dout[gi + np] = D.y;
@@ -507,10 +503,9 @@ __device__ __forceinline__ void site_end(const KArgs &a, double *lds, const Site
         a.dst[gi + 2 * np] = o.z;
     } else if constexpr (MODE == MODE_HEUN1) {
         // stage 1 of integration 2: D1 = LLG(B(m0), m0); m1 = euler(m0, 1*D1 + 0*D2, 0, dt/2)
-        v3 D = llg_rhs(m, B, alpha, a.den, a.rden);
-        // Dint = 0 + 1 D (get_Dmode_int); the leading zero changes only the sign of an exact zero
-        v3 dint = D;
-        v3 o = euler_step0(m, dint, a.dt);
+        const MjUnit u = mj_unit(m);
+        const v3 D = llg_torque(u.n, B, alpha);
+        const v3 o = euler_step0(m, u, D, a.kdt);
         a.dst[gi] = o.x;
         a.dst[gi + np] = o.y;
         a.dst[gi + 2 * np] = o.z;
@@ -519,16 +514,14 @@ __device__ __forceinline__ void site_end(const KArgs &a, double *lds, const Site
         a.aux[gi + 2 * np] = D.z;
     } else if constexpr (MODE == MODE_HEUN2) {
         // stage 2: D2 = LLG(B(m1), m1); m2 = euler(m1, 0.5 D1 + 0.5 D2, DT(m0), dt/2)
-        v3 D2 = llg_rhs(m, B, alpha, a.den, a.rden);
-        const v3 D1 = pre_aux;
-        // Dint = (0 + D1/2) + D2/2 (get_Dmode_int) without the exact-zero start
-        v3 dint = mk3(0.5 * D1.x + 0.5 * D2.x, 0.5 * D1.y + 0.5 * D2.y, 0.5 * D1.z + 0.5 * D2.z);
+        const MjUnit u = mj_unit(m);
+        const v3 dint = heun_dint(pre_aux, llg_torque(u.n, B, alpha));
         v3 o;
         if constexpr (NOISE) {
             // Langevin term of the last stage on m0 (pre_own, site_thermal), spindynamics.f90:269-271,311
-            o = euler_step(m, dint, site_thermal_final<MODE, G>(a, st), a.dt);
+            o = euler_step(m, u, dint, site_thermal_final<MODE, G>(a, st), a.kdt);
         } else {
-            o = euler_step0(m, dint, a.dt);
+            o = euler_step0(m, u, dint, a.kdt);
         }
         a.dst[gi] = o.x;
         a.dst[gi + np] = o.y;
@@ -539,20 +532,19 @@ __device__ __forceinline__ void site_end(const KArgs &a, double *lds, const Site
             B = mk3(B.x + bt.x, B.y + bt.y, B.z + bt.z);
         }
         if constexpr (MODE == MODE_SIB1) {
-            v3 av = sib_vec(m, B, alpha, a.dt);
-            v3 mt = cayley(m, av);
-            a.dst[gi] = 0.5 * (m.x + mt.x);
-            a.dst[gi + np] = 0.5 * (m.y + mt.y);
-            a.dst[gi + 2 * np] = 0.5 * (m.z + mt.z);
+            const v3 p = cayley_mid(m, sib_vec(m, B, alpha, -0.5 * a.kdt));
+            a.dst[gi] = p.x;
+            a.dst[gi + np] = p.y;
+            a.dst[gi + 2 * np] = p.z;
         } else if constexpr (MODE == MODE_SIB2) {
-            v3 av = sib_vec(m, B, alpha, a.dt);   // m is the midpoint p here
-            v3 o = cayley(pre_own, av);
+            // m is the midpoint p here
+            const v3 o = cayley(pre_own, sib_vec(m, B, alpha, -0.5 * a.kdt));
             a.dst[gi] = o.x;
             a.dst[gi + np] = o.y;
             a.dst[gi + 2 * np] = o.z;
         } else if constexpr (MODE == MODE_DEP1) {
-            v3 b1 = dep_field(m, B, alpha, a.den, a.rden);
-            v3 mt = dep_rotate(m, b1, a.dt);
+            v3 b1 = dep_field(m, B, alpha);
+            v3 mt = dep_rotate(m, b1, a.kdt);
             a.dst[gi] = mt.x;
             a.dst[gi + np] = mt.y;
             a.dst[gi + 2 * np] = mt.z;
@@ -560,10 +552,10 @@ __device__ __forceinline__ void site_end(const KArgs &a, double *lds, const Site
             a.aux[gi + np] = b1.y;
             a.aux[gi + 2 * np] = b1.z;
         } else if constexpr (MODE == MODE_DEP2) {
-            v3 b2 = dep_field(m, B, alpha, a.den, a.rden);   // m is the predictor here
+            v3 b2 = dep_field(m, B, alpha);   // m is the predictor here
             const v3 b1 = pre_aux;
             v3 ba = mk3(0.5 * (b1.x + b2.x), 0.5 * (b1.y + b2.y), 0.5 * (b1.z + b2.z));
-            v3 o = dep_rotate(pre_own, ba, a.dt);
+            v3 o = dep_rotate(pre_own, ba, a.kdt);
             a.dst[gi] = o.x;
             a.dst[gi + np] = o.y;
             a.dst[gi + 2 * np] = o.z;
@@ -721,22 +713,23 @@ __device__ __forceinline__ bool fused_site(const KArgs &a, int gx, int gy, int g
     return true;
 }
 
-// stage 1 of integration 2 at one site from S0 (center c0): D1 and m1
-// (site_end, MODE_HEUN1), the energy term of m0 when wanted
+// stage 1 of integration 2 at one site from S0 (center c0): the unit vector
+// of m0, D1 and m1 (site_end, MODE_HEUN1), the energy term of m0 when wanted
 template <class F>
 __device__ __forceinline__ void fused_stage1(const KArgs &a, const double *L0, int c0, bool live, int64_t gi,
-                                             v3 &m0, v3 &D1, v3 &m1, double &e)
+                                             v3 &n0, v3 &D1, v3 &m1, double &e)
 {
     constexpr int T0 = F::kT0;
     double ax = 0.0, ay = 0.0, az = 0.0;
-    m0 = mk3(L0[c0], L0[T0 + c0], L0[2 * T0 + c0]);
+    const v3 m0 = mk3(L0[c0], L0[T0 + c0], L0[2 * T0 + c0]);
     F::stencil0(L0, c0, ax, ay, az);
     const v3 z = fused_zeeman<F>(a, live, gi);
-    const double hx = 0.0, hy = 0.0, hz = 0.0;
-    const v3 B = mk3(-(ax + z.x) - 2.0 * hx, -(ay + z.y) - 2.0 * hy, -(az + z.z) - 2.0 * hz);
-    e = m0.x * ((0.5 * ax + z.x) + hx) + m0.y * ((0.5 * ay + z.y) + hy) + m0.z * ((0.5 * az + z.z) + hz);
-    D1 = llg_rhs(m0, B, a.alpha, a.den, a.rden);
-    m1 = euler_step0(m0, D1, a.dt);   // Dint = 1 D1, as in stage 1 of the two-kernel path
+    const v3 B = mk3(-(ax + z.x), -(ay + z.y), -(az + z.z));
+    e = mj_site_energy(m0, mk3(ax, ay, az), z);
+    const MjUnit u = mj_unit(m0);
+    n0 = u.n;
+    D1 = llg_torque(u.n, B, a.alpha);
+    m1 = euler_step0(m0, u, D1, a.kdt);   // Dint = 1 D1, as in stage 1 of the two-kernel path
 }
 
 template <class F>
@@ -884,14 +877,12 @@ __device__ __forceinline__ void fused_heun_body(const KArgs &a, double *lds)
         v3 m1 = mk3(0.0, 0.0, 0.0);
         if (fused_site<F>(a, gx, y0 + lyj, gz, gw)) {
             const int c0 = (lz + 2 * RZ) * S0X * S0Y + (lyj + 2 * RY) * S0X + (lx + 2 * RX);
-            v3 m0;
+            v3 n0;
             double ee;
-            fused_stage1<F>(a, L0, c0, true, gw, m0, D1[j], m1, ee);
+            fused_stage1<F>(a, L0, c0, true, gw, n0, D1[j], m1, ee);
             if (active[j]) e[j] = ee;
-            if constexpr (NOISE) {
-                // Langevin term of the last stage on m0 (HEUN2: thermal_term, euler_step)
-                if (active[j]) q[j] = thermal_increment(llg_rhs(m0, th[j], a.alpha, a.den, a.rden), a.dt);
-            }
+            // Langevin term of the last stage on m0 (HEUN2: thermal_term)
+            if constexpr (NOISE) q[j] = llg_torque(n0, th[j], a.alpha);
         }
         L1[s1] = m1.x;
         L1[T1 + s1] = m1.y;
@@ -919,9 +910,9 @@ __device__ __forceinline__ void fused_heun_body(const KArgs &a, double *lds)
         v3 m1 = mk3(0.0, 0.0, 0.0);
         if (fused_site<F>(a, x0 - RX + sx, y0 - RY + sy, z0 - RZ + sz, gw)) {
             const int c0 = (sz + RZ) * S0X * S0Y + (sy + RY) * S0X + (sx + RX);
-            v3 m0, d;
+            v3 n0, d;
             double ee;
-            fused_stage1<F>(a, L0, c0, true, gw, m0, d, m1, ee);
+            fused_stage1<F>(a, L0, c0, true, gw, n0, d, m1, ee);
         }
         L1[s1] = m1.x;
         L1[T1 + s1] = m1.y;
@@ -957,18 +948,17 @@ __device__ __forceinline__ void fused_heun_body(const KArgs &a, double *lds)
             double ax = 0.0, ay = 0.0, az = 0.0;
             F::stencil1(L1, s1, ax, ay, az);
             const v3 z = fused_zeeman<F>(a, true, gia[j]);
-            const double hx = 0.0, hy = 0.0, hz = 0.0;
-            const v3 B = mk3(-(ax + z.x) - 2.0 * hx, -(ay + z.y) - 2.0 * hy, -(az + z.z) - 2.0 * hz);
+            const v3 B = mk3(-(ax + z.x), -(ay + z.y), -(az + z.z));
             if (a.fld_out) {   // the last stage's field, kept for the host
                 a.fld_out[gia[j]] = B.x;
                 a.fld_out[gia[j] + np] = B.y;
                 a.fld_out[gia[j] + 2 * np] = B.z;
             }
-            const v3 D2 = llg_rhs(m, B, a.alpha, a.den, a.rden);
-            const v3 dint = mk3(0.5 * D1[j].x + 0.5 * D2.x, 0.5 * D1[j].y + 0.5 * D2.y, 0.5 * D1[j].z + 0.5 * D2.z);
+            const MjUnit u = mj_unit(m);
+            const v3 dint = heun_dint(D1[j], llg_torque(u.n, B, a.alpha));
             v3 o;
-            if constexpr (NOISE) o = euler_step_q(m, dint, q[j], a.dt);
-            else o = euler_step0(m, dint, a.dt);
+            if constexpr (NOISE) o = euler_step(m, u, dint, q[j], a.kdt);
+            else o = euler_step0(m, u, dint, a.kdt);
             const int64_t g = gia[j];
             a.dst[g] = o.x;
             a.dst[g + np] = o.y;
@@ -1026,17 +1016,14 @@ __device__ __forceinline__ void fused_sib_stage1(const KArgs &a, const double *L
     m0 = mk3(L0[c0], L0[T0 + c0], L0[2 * T0 + c0]);
     F::stencil0(L0, c0, ax, ay, az);
     const v3 z = fused_zeeman<F>(a, true, gi);
-    const double hx = 0.0, hy = 0.0, hz = 0.0;
-    v3 B = mk3(-(ax + z.x) - 2.0 * hx, -(ay + z.y) - 2.0 * hy, -(az + z.z) - 2.0 * hz);
-    e = m0.x * ((0.5 * ax + z.x) + hx) + m0.y * ((0.5 * ay + z.y) + hy) + m0.z * ((0.5 * az + z.z) + hz);
+    v3 B = mk3(-(ax + z.x), -(ay + z.y), -(az + z.z));
+    e = mj_site_energy(m0, mk3(ax, ay, az), z);
     if constexpr (NOISE) B = mk3(B.x + bt.x, B.y + bt.y, B.z + bt.z);
     if constexpr (DEP) {
-        b1 = dep_field(m0, B, a.alpha, a.den, a.rden);
-        p = dep_rotate(m0, b1, a.dt);
+        b1 = dep_field(m0, B, a.alpha);
+        p = dep_rotate(m0, b1, a.kdt);
     } else {
-        const v3 av = sib_vec(m0, B, a.alpha, a.dt);
-        const v3 mt = cayley(m0, av);
-        p = mk3(0.5 * (m0.x + mt.x), 0.5 * (m0.y + mt.y), 0.5 * (m0.z + mt.z));
+        p = cayley_mid(m0, sib_vec(m0, B, a.alpha, -0.5 * a.kdt));
         b1 = mk3(0.0, 0.0, 0.0);
     }
 }
@@ -1169,8 +1156,7 @@ __device__ __forceinline__ void fused_sib_body(const KArgs &a, double *lds)
             double ax = 0.0, ay = 0.0, az = 0.0;
             F::stencil1(L1, s1, ax, ay, az);
             const v3 z = fused_zeeman<F>(a, true, gia[j]);
-            const double hx = 0.0, hy = 0.0, hz = 0.0;
-            v3 B = mk3(-(ax + z.x) - 2.0 * hx, -(ay + z.y) - 2.0 * hy, -(az + z.z) - 2.0 * hz);
+            v3 B = mk3(-(ax + z.x), -(ay + z.y), -(az + z.z));
             if (a.fld_out) {   // the last stage's field, kept for the host
                 a.fld_out[gia[j]] = B.x;
                 a.fld_out[gia[j] + np] = B.y;
@@ -1179,13 +1165,12 @@ __device__ __forceinline__ void fused_sib_body(const KArgs &a, double *lds)
             if constexpr (NOISE) B = mk3(B.x + th[j].x, B.y + th[j].y, B.z + th[j].z);
             v3 o;
             if constexpr (DEP) {
-                const v3 b2 = dep_field(p, B, a.alpha, a.den, a.rden);
+                const v3 b2 = dep_field(p, B, a.alpha);
                 const v3 b1 = b1s[j];
                 const v3 ba = mk3(0.5 * (b1.x + b2.x), 0.5 * (b1.y + b2.y), 0.5 * (b1.z + b2.z));
-                o = dep_rotate(m0s[j], ba, a.dt);
+                o = dep_rotate(m0s[j], ba, a.kdt);
             } else {
-                const v3 av = sib_vec(p, B, a.alpha, a.dt);
-                o = cayley(m0s[j], av);
+                o = cayley(m0s[j], sib_vec(p, B, a.alpha, -0.5 * a.kdt));
             }
             const int64_t g = gia[j];
             a.dst[g] = o.x;
