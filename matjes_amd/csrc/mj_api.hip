@@ -396,10 +396,13 @@ static void tile_shape(const mj_ctx *c, int &bx, int &by, int &bz)
         bz = c->bz;
         return;
     }
-    // 256-site tiles (32x8); on small lattices smaller ones (down to one
-    // wavefront) while there would be fewer than 512 workgroups
+    // 256-site tiles (32x8); below the lattices that get compiled kernels
+    // (mj_finalize) smaller ones, down to one wavefront, while there would be
+    // fewer than 512 workgroups.  The fused step is the faster for its smaller
+    // ring (64x64, Heun at 10 K: triangular 5.4 us per step against 6.2 with 8x8
+    // tiles, square 4.4 against 4.65; 256x256: 5.9 against 6.5 with 16x8)
     int nthr = 256;
-    while (nthr > 64 && c->n / nthr < 512) nthr >>= 1;
+    while (c->n < 4096 && nthr > 64 && c->n / nthr < 512) nthr >>= 1;
     bx = std::min(pow2ceil(c->dim[0]), std::max(8, nthr / 8));
     by = std::min(pow2ceil(c->dim[1]), std::max(1, nthr / bx));
     bz = std::min(pow2ceil(c->dim[2]), std::max(1, nthr / (bx * by)));
@@ -497,6 +500,10 @@ int mj_finalize(mj_ctx *c)
             MJ_HIP_CHECK(hipMemcpy(c->d_v, v.data(), sizeof(double) * v.size(), hipMemcpyHostToDevice));
         }
         c->n_iso = c->n_dm = c->n_gen = 0;
+        c->h_ofs3.clear();
+        c->h_cf.clear();
+        c->h_ord.clear();
+        c->h_blk.clear();
         c->rx = c->ry = c->rz = 0;
         c->use_jit = 0;
     } else {
@@ -529,8 +536,7 @@ int mj_finalize(mj_ctx *c)
             c->ry = std::max(c->ry, std::abs(o[1]));
             c->rz = std::max(c->rz, std::abs(o[2]));
         }
-        int sx = bx + 2 * c->rx, sy = by + 2 * c->ry;
-        std::vector<int> ofs_iso, ofs_dm, ofs_gen;
+        const int sx = bx + 2 * c->rx, sy = by + 2 * c->ry;
         std::vector<double> cf_iso, cf_dm, cf_gen;
         std::vector<int> o3_iso, o3_dm, o3_gen;
         for (size_t k = 0; k < offs.size(); ++k) {
@@ -539,35 +545,28 @@ int mj_finalize(mj_ctx *c)
             for (int t = 0; t < 9; ++t) mx = std::max(mx, fabs(q[t]));
             if (mx == 0.0) continue;
             double tol = 1.0e-14 * mx;
-            int lofs = offs[k][2] * sx * sy + offs[k][1] * sx + offs[k][0];
             bool diag_eq = fabs(q[0] - q[4]) <= tol && fabs(q[0] - q[8]) <= tol;
             bool offd0 = fabs(q[1]) <= tol && fabs(q[2]) <= tol && fabs(q[3]) <= tol && fabs(q[5]) <= tol &&
                          fabs(q[6]) <= tol && fabs(q[7]) <= tol;
             bool anti = fabs(q[1] + q[3]) <= tol && fabs(q[2] + q[6]) <= tol && fabs(q[5] + q[7]) <= tol;
             if (diag_eq && offd0 && q[0] == q[4] && q[0] == q[8]) {
-                ofs_iso.push_back(lofs);
                 o3_iso.insert(o3_iso.end(), offs[k].begin(), offs[k].end());
                 cf_iso.push_back(q[0]);
             } else if (diag_eq && anti && q[0] == q[4] && q[0] == q[8]) {
                 // C m = s m + w x m with w = (C_zy, C_xz, C_yx)
-                ofs_dm.push_back(lofs);
                 o3_dm.insert(o3_dm.end(), offs[k].begin(), offs[k].end());
                 cf_dm.push_back(q[0]);
                 cf_dm.push_back(0.5 * (q[7] - q[5]));
                 cf_dm.push_back(0.5 * (q[2] - q[6]));
                 cf_dm.push_back(0.5 * (q[3] - q[1]));
             } else {
-                ofs_gen.push_back(lofs);
                 o3_gen.insert(o3_gen.end(), offs[k].begin(), offs[k].end());
                 cf_gen.insert(cf_gen.end(), q.begin(), q.end());
             }
         }
-        c->n_iso = (int)ofs_iso.size();
-        c->n_dm = (int)ofs_dm.size();
-        c->n_gen = (int)ofs_gen.size();
-        std::vector<int> ofs(ofs_iso);
-        ofs.insert(ofs.end(), ofs_dm.begin(), ofs_dm.end());
-        ofs.insert(ofs.end(), ofs_gen.begin(), ofs_gen.end());
+        c->n_iso = (int)o3_iso.size() / 3;
+        c->n_dm = (int)o3_dm.size() / 3;
+        c->n_gen = (int)o3_gen.size() / 3;
         std::vector<double> cf(cf_iso);
         cf.insert(cf.end(), cf_dm.begin(), cf_dm.end());
         cf.insert(cf.end(), cf_gen.begin(), cf_gen.end());
@@ -575,22 +574,51 @@ int mj_finalize(mj_ctx *c)
         c->h_ofs3.insert(c->h_ofs3.end(), o3_dm.begin(), o3_dm.end());
         c->h_ofs3.insert(c->h_ofs3.end(), o3_gen.begin(), o3_gen.end());
         c->h_cf = cf;
+        // every kernel sums the entries by (dz, dy, dx), whatever their kind: the
+        // pairs of sites of the fused step (mj_jit.hip) then meet each neighbour
+        // they share once, row by row, and every form gives the same bits
+        const int nent = c->n_iso + c->n_dm + c->n_gen;
+        c->h_ord.resize(nent);
+        for (int k = 0; k < nent; ++k) c->h_ord[k] = k;
+        std::sort(c->h_ord.begin(), c->h_ord.end(), [&](int p, int q) {
+            const int *u = &c->h_ofs3[3 * p], *v = &c->h_ofs3[3 * q];
+            return std::make_tuple(u[2], u[1], u[0]) < std::make_tuple(v[2], v[1], v[0]);
+        });
+        c->h_blk.clear();
+        std::vector<int> ofs;
+        for (int k : c->h_ord) {
+            const int kind = k < c->n_iso ? 0 : k < c->n_iso + c->n_dm ? 1 : 2;
+            const double *p = &cf[kind == 0 ? k
+                                  : kind == 1 ? c->n_iso + 4 * (k - c->n_iso)
+                                              : c->n_iso + 4 * c->n_dm + 9 * (k - c->n_iso - c->n_dm)];
+            const double iso[9] = {p[0], 0.0, 0.0, 0.0, p[0], 0.0, 0.0, 0.0, p[0]};
+            if (kind == 0) {
+                c->h_blk.insert(c->h_blk.end(), iso, iso + 9);
+            } else if (kind == 1) {   // s m + w x m, p = (s, w)
+                const double dm[9] = {p[0], -p[3], p[2], p[3], p[0], -p[1], -p[2], p[1], p[0]};
+                c->h_blk.insert(c->h_blk.end(), dm, dm + 9);
+            } else {
+                c->h_blk.insert(c->h_blk.end(), p, p + 9);
+            }
+            const int *o = &c->h_ofs3[3 * k];
+            ofs.push_back(o[2] * sx * sy + o[1] * sx + o[0]);
+        }
         if (c->d_ofs) hipFree(c->d_ofs);
         if (c->d_cf) hipFree(c->d_cf);
         c->d_ofs = nullptr;
         c->d_cf = nullptr;
         MJ_HIP_CHECK(hipMalloc(&c->d_ofs, sizeof(int) * std::max<size_t>(1, ofs.size())));
-        MJ_HIP_CHECK(hipMalloc(&c->d_cf, sizeof(double) * std::max<size_t>(1, cf.size())));
+        MJ_HIP_CHECK(hipMalloc(&c->d_cf, sizeof(double) * std::max<size_t>(1, c->h_blk.size())));
         if (!ofs.empty()) {
             MJ_HIP_CHECK(hipMemcpy(c->d_ofs, ofs.data(), sizeof(int) * ofs.size(), hipMemcpyHostToDevice));
-            MJ_HIP_CHECK(hipMemcpy(c->d_cf, cf.data(), sizeof(double) * cf.size(), hipMemcpyHostToDevice));
+            MJ_HIP_CHECK(hipMemcpy(c->d_cf, c->h_blk.data(), sizeof(double) * c->h_blk.size(), hipMemcpyHostToDevice));
         }
         // per-Hamiltonian compiled kernels: MJ_JIT=0 off, 1 on, otherwise for lattices >= 64x64 sites
         const char *env = getenv("MJ_JIT");
         c->use_jit = env && env[0] == '0' ? 0 : (env && env[0] == '1') ? 1 : (c->n >= 4096 ? 1 : 0);
         if (c->use_jit) {
             int ntx = (c->dim[0] + bx - 1) / bx, nty = (c->dim[1] + by - 1) / by, ntz = (c->dim[2] + bz - 1) / bz;
-            MJ_TRY(mj_jit_prepare(c, ofs.data(), cf.data(), bx, by, bz, ntx * nty * ntz, ntx, nty));
+            MJ_TRY(mj_jit_prepare(c, bx, by, bz, ntx * nty * ntz, ntx, nty));
         }
     }
     // energy partial buffers
@@ -629,9 +657,7 @@ static void base_args(const mj_ctx *c, KArgs &a)
     a.ntz = (a.nz + a.bz - 1) / a.bz;
     a.nblocks = a.ntx * a.nty * a.ntz;
     a.np = c->np;
-    a.n_iso = c->n_iso;
-    a.n_dm = c->n_dm;
-    a.n_gen = c->n_gen;
+    a.n_ent = c->n_iso + c->n_dm + c->n_gen;
     a.ofs = c->d_ofs;
     a.cf = c->d_cf;
     a.use_stencil = c->mm_generic ? 0 : 1;
@@ -989,8 +1015,7 @@ struct Prof {
 
 static int launch(mj_ctx *c, int mode, bool noise, const KArgs &a)
 {
-    // integration 4 runs the ahead-of-time stage kernel (no per-Hamiltonian form)
-    if (c->use_jit && a.use_stencil && mode != MODE_RKS) return mj_jit_launch(c, mode, noise, a, c->stream);
+    if (c->use_jit && a.use_stencil) return mj_jit_launch(c, mode, noise, a, c->stream);
     return mj_launch_stage(mode, noise, a, c->stream);
 }
 
@@ -1349,9 +1374,9 @@ static int run_steps(mj_ctx *c, int nsteps, int integ, double timestep, double a
             if (c->use_jit && fused) {   // compile before capturing
                 MJ_TRY(mj_jit_resolve(c, fmode, noisy));
             } else if (c->use_jit) {
-                const int modes[4][2] = {{MODE_EULER, -1}, {MODE_HEUN1, MODE_HEUN2}, {MODE_SIB1, MODE_SIB2},
-                                         {MODE_DEP1, MODE_DEP2}};
-                const int row = integ == MJ_EULER ? 0 : integ == MJ_HEUN ? 1 : integ == MJ_SIB ? 2 : 3;
+                const int modes[5][2] = {{MODE_EULER, -1}, {MODE_HEUN1, MODE_HEUN2}, {MODE_SIB1, MODE_SIB2},
+                                         {MODE_DEP1, MODE_DEP2}, {MODE_RKS, -1}};
+                const int row = integ == MJ_EULER ? 0 : integ == MJ_HEUN ? 1 : integ == MJ_SIB ? 2 : integ == MJ_RK ? 4 : 3;
                 for (int q = 0; q < 2; ++q)
                     if (modes[row][q] >= 0)
                         MJ_TRY(mj_jit_resolve(c, modes[row][q], noisy && !(integ == MJ_HEUN && q == 0)));

@@ -38,7 +38,7 @@
 struct BatchSys {
     int nx, ny, nz, px, py, pz;
     int bx, by, bz, rx, ry, rz, sx, sy, sz, ntx, nty, ntz, nblocks, block0;
-    int n_iso, n_dm, n_gen, ofs_off, cf_off, bmode;
+    int n_ent, ofs_off, bmode;   // ofs_off: offsets and blocks of the entries
     int ofs0_off;         // the stencil's offsets in the fused step's S0 layout (tile + 2R)
     int64_t base;
     const double *hdip;   // dipolar systems: the padded grid of H_fft (null: none), its row / plane / component strides
@@ -91,10 +91,8 @@ __device__ __forceinline__ KArgs sys_args(const KArgs &base, const BatchSys &S, 
     a.dst = base.dst ? base.dst + S.base : nullptr;
     a.aux = base.aux ? base.aux + S.base : nullptr;
     a.ofs = base.ofs + S.ofs_off;
-    a.cf = base.cf + S.cf_off;
-    a.n_iso = S.n_iso;
-    a.n_dm = S.n_dm;
-    a.n_gen = S.n_gen;
+    a.cf = base.cf + 9 * S.ofs_off;
+    a.n_ent = S.n_ent;
     a.bmode = S.bmode;
     a.zb[0] = S.zb[0];
     a.zb[1] = S.zb[1];
@@ -328,8 +326,9 @@ __device__ __forceinline__ void batch_fused_tile(const KArgs &a, const int *ofs0
         v3 o;
         if constexpr (INTEG == MJ_HEUN) {
             const MjUnit u = mj_unit(m);
-            const v3 dint = heun_dint(D1, llg_torque(u.n, B, a.alpha));
-            o = euler_step(m, u, dint, llg_torque(mj_unit(m0).n, bt, a.alpha), a.kdt);
+            // Dint = D1/2 + D2/2 (get_Dmode_int)
+            const v3 d = D1 + llg_torque(u.n, B, a.alpha);
+            o = euler_step(m, u, d, 0.5 * a.kdt, llg_torque(mj_unit(m0).n, bt, a.alpha), a.kdt);
         } else if constexpr (INTEG == MJ_SIB) {
             B = mk3(B.x + bt.x, B.y + bt.y, B.z + bt.z);
             o = cayley(m0, sib_vec(m, B, a.alpha, -0.5 * a.kdt));
@@ -346,10 +345,10 @@ __device__ __forceinline__ void batch_fused_tile(const KArgs &a, const int *ofs0
 }
 
 // one step of every system: base.src -> base.dst; compiled for at least 6
-// waves per SIMD (Heun) or 5 (SIB and Depondt, whose ring also draws the
-// thermal field: they spill at 6)
+// waves per SIMD (Heun) or 4 (SIB and Depondt, whose ring also draws the
+// thermal field: they spill at 5)
 template <int INTEG>
-__global__ void __launch_bounds__(MJ_BATCH_NTHR, INTEG == MJ_HEUN ? 6 : 5)
+__global__ void __launch_bounds__(MJ_BATCH_NTHR, INTEG == MJ_HEUN ? 6 : 4)
     k_batch_fused(const KArgs base, const BatchSys *__restrict__ sys, const int *__restrict__ blk2sys,
                   const double *__restrict__ sigma, const uint64_t *__restrict__ stepp, const int *__restrict__ ofs0)
 {
@@ -611,8 +610,8 @@ __global__ void k_batch_soa2aos(const double *in, double *out, int64_t n, int64_
 struct HostSys {
     int dim[3], periodic[3];
     int64_t n, base;
-    int rx, ry, rz, n_iso, n_dm, n_gen, bmode;
-    std::vector<int> ofs3;
+    int rx, ry, rz, bmode;
+    std::vector<int> ofs3;   // the stencil in the order of the sum (mj_ctx::h_ord)
     std::vector<double> cf;
     double zb[3];
     double z9[9] = {0};
@@ -795,12 +794,9 @@ extern "C" int mj_batch_add(mj_batch *b, mj_ctx *c, double damping, double kT, u
     s.rx = c->rx;
     s.ry = c->ry;
     s.rz = c->rz;
-    s.n_iso = c->n_iso;
-    s.n_dm = c->n_dm;
-    s.n_gen = c->n_gen;
     s.bmode = c->bmode;
-    s.ofs3 = c->h_ofs3;
-    s.cf = c->h_cf;
+    for (int k : c->h_ord) s.ofs3.insert(s.ofs3.end(), &c->h_ofs3[3 * k], &c->h_ofs3[3 * k] + 3);
+    s.cf = c->h_blk;
     for (int a = 0; a < 3; ++a) s.zb[a] = c->zb[a];
     if (c->bmode == 2) {   // per-site B: the map (AoS on the context's host side) and the Zeeman block
         for (int k = 0; k < 9; ++k) s.z9[k] = c->zblk[k];
@@ -950,9 +946,7 @@ static int batch_finalize(mj_batch *b)
         t.block0 = nb;
         nb += t.nblocks;
         for (int k = 0; k < t.nblocks; ++k) blk2sys.push_back((int)q);
-        t.n_iso = s.n_iso;
-        t.n_dm = s.n_dm;
-        t.n_gen = s.n_gen;
+        t.n_ent = (int)s.ofs3.size() / 3;
         t.ofs_off = (int)ofs.size();
         for (size_t k = 0; k < s.ofs3.size() / 3; ++k)
             ofs.push_back(s.ofs3[3 * k + 2] * t.sx * t.sy + s.ofs3[3 * k + 1] * t.sx + s.ofs3[3 * k]);
@@ -962,7 +956,6 @@ static int batch_finalize(mj_batch *b)
         for (size_t k = 0; k < s.ofs3.size() / 3; ++k)
             ofs0.push_back(s.ofs3[3 * k + 2] * s0x * s0y + s.ofs3[3 * k + 1] * s0x + s.ofs3[3 * k]);
         shm_fused = std::max(shm_fused, (size_t)3 * ((size_t)s0x * s0y * s0z + (size_t)t.sx * t.sy * t.sz) * sizeof(double));
-        t.cf_off = (int)cf.size();
         cf.insert(cf.end(), s.cf.begin(), s.cf.end());
         t.bmode = s.bmode;
         for (int a = 0; a < 3; ++a) t.zb[a] = s.zb[a];

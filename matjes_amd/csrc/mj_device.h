@@ -35,6 +35,15 @@ struct v3 {
     double x, y, z;
 };
 
+__device__ __forceinline__ v3 operator+(v3 a, v3 b)
+{
+    v3 r;
+    r.x = a.x + b.x;
+    r.y = a.y + b.y;
+    r.z = a.z + b.z;
+    return r;
+}
+
 __device__ __forceinline__ v3 mk3(double x, double y, double z)
 {
     v3 r;
@@ -127,7 +136,7 @@ __device__ __forceinline__ MjUnit mj_unit(v3 m)
 {
     MjUnit u;
     u.x = dot3(m, m);
-    double r = fma(-0.5, u.x, 1.5);
+    double r = mj_fma_k(u.x, -0.5, 1.5);
     u.r2 = r * r;
     if (!(fabs(u.x - 1.0) <= 0x1p-27)) {
         const bool ok = u.x > 1.0e-16;
@@ -151,11 +160,11 @@ __device__ __forceinline__ v3 mj_restore(v3 m, MjUnit u, v3 t)
     const double y = dot3(t, t);
     const double v = (u.x - y) * u.r2;
     double f = 0.20955191976592094;
-    f = fma(f, v, 0.22566986332987313);
-    f = fma(f, v, 0.24609374032347447);
-    f = fma(f, v, 0.2734374897543061);
-    f = fma(f, v, 0.3125000000002953);
-    f = fma(f, v, 0.3750000000003127);
+    f = mj_fma_k(f, v, 0.22566986332987313);
+    f = mj_fma_k(f, v, 0.24609374032347447);
+    f = mj_fma_k(f, v, 0.2734374897543061);
+    f = mj_fma_k(f, v, 0.3125000000002953);
+    f = mj_fma_k(f, v, 0.3750000000003127);
     f = fma(f, v, 0.5);
     v3 o = fma3(f * v, t, t);
     if (!(fabs(v) <= 0x1p-6)) {
@@ -175,21 +184,15 @@ __device__ __forceinline__ v3 llg_torque(v3 n, v3 B, double alpha)
 }
 
 // euler (solver.f90:172-176): t = (m + Dint dt/hbar) + DT dt/hbar, m' = t |m| / |t|;
-// dint and dth torques (llg_torque), k = dt / (hbar (1 + a^2))
-__device__ __forceinline__ v3 euler_step(v3 m, MjUnit u, v3 dint, v3 dth, double k)
+// dint and dth torques (llg_torque), ki and k their factors: k = dt / (hbar (1 + a^2))
+__device__ __forceinline__ v3 euler_step(v3 m, MjUnit u, v3 dint, double ki, v3 dth, double k)
 {
-    return mj_restore(m, u, fma3(k, dth, fma3(k, dint, m)));
+    return mj_restore(m, u, fma3(k, dth, fma3(ki, dint, m)));
 }
 
 __device__ __forceinline__ v3 euler_step0(v3 m, MjUnit u, v3 dint, double k)
 {
     return mj_restore(m, u, fma3(k, dint, m));
-}
-
-// Dint = D1/2 + D2/2 of integration 2's second stage (get_Dmode_int)
-__device__ __forceinline__ v3 heun_dint(v3 d1, v3 d2)
-{
-    return mk3(0.5 * (d1.x + d2.x), 0.5 * (d1.y + d2.y), 0.5 * (d1.z + d2.z));
 }
 
 // Implicit-midpoint (Cayley) solve (I + [a]x) x = m - a x m  (SIB, Mentink et
@@ -237,14 +240,14 @@ __device__ __forceinline__ v3 dep_rotate(v3 m, v3 b, double k)
     const v3 w = mk3(k * b.x, k * b.y, k * b.z);
     const double z = dot3(w, w);
     double S = -2.4931934029233215e-08, C = -2.0790894217124703e-09;
-    S = fma(S, z, 2.7556981477681245e-06);
-    C = fma(C, z, 2.7557077887523167e-07);
-    S = fma(S, z, -0.00019841269403598734);
-    C = fma(C, z, -2.4801586988836374e-05);
-    S = fma(S, z, 0.00833333333307693);
-    C = fma(C, z, 0.0013888888888705666);
-    S = fma(S, z, -0.16666666666666116);
-    C = fma(C, z, -0.041666666666666276);
+    S = mj_fma_k(S, z, 2.7556981477681245e-06);
+    C = mj_fma_k(C, z, 2.7557077887523167e-07);
+    S = mj_fma_k(S, z, -0.00019841269403598734);
+    C = mj_fma_k(C, z, -2.4801586988836374e-05);
+    S = mj_fma_k(S, z, 0.00833333333307693);
+    C = mj_fma_k(C, z, 0.0013888888888705666);
+    S = mj_fma_k(S, z, -0.16666666666666116);
+    C = mj_fma_k(C, z, -0.041666666666666276);
     S = fma(S, z, 1.0);
     C = fma(C, z, 0.5);
     if (!(z <= 0.25)) {
@@ -269,15 +272,24 @@ __device__ __forceinline__ double mj_site_energy(v3 m, v3 a, v3 z)
 // Philox4x32-10 (Salmon, Moraes, Dror, Shaw, SC'11) and Box-Muller normals.
 // Key = seed, counter = (site, step lo, step hi, stream).
 // ---------------------------------------------------------------------------
+__host__ __device__ __forceinline__ uint32_t mj_xor3(uint32_t a, uint32_t b, uint32_t c)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    return __builtin_amdgcn_bitop3_b32(a, b, c, 0x96);   // one instruction
+#else
+    return a ^ b ^ c;
+#endif
+}
+
 __host__ __device__ __forceinline__ void philox4x32_10(uint32_t c[4], uint32_t k0, uint32_t k1)
 {
 #pragma unroll
     for (int r = 0; r < 10; ++r) {
         uint64_t p0 = (uint64_t)0xD2511F53u * c[0];
         uint64_t p1 = (uint64_t)0xCD9E8D57u * c[2];
-        uint32_t n0 = (uint32_t)(p1 >> 32) ^ c[1] ^ k0;
+        uint32_t n0 = mj_xor3((uint32_t)(p1 >> 32), c[1], k0);
         uint32_t n1 = (uint32_t)p1;
-        uint32_t n2 = (uint32_t)(p0 >> 32) ^ c[3] ^ k1;
+        uint32_t n2 = mj_xor3((uint32_t)(p0 >> 32), c[3], k1);
         uint32_t n3 = (uint32_t)p0;
         c[0] = n0;
         c[1] = n1;
@@ -296,8 +308,8 @@ __device__ __forceinline__ v3 normals3(uint64_t seed, uint64_t step, uint32_t si
 {
     uint32_t c[4] = {site, (uint32_t)step, (uint32_t)(step >> 32), 0u};
     philox4x32_10(c, (uint32_t)seed, (uint32_t)(seed >> 32));
-    const double r1 = mj_sqrt_pos(-2.0 * mj_ln_u32(c[0]));
-    const double r2 = mj_sqrt_pos(-2.0 * mj_ln_u32(c[2]));
+    const double r1 = mj_radius(mj_ln_u32(c[0]));
+    const double r2 = mj_radius(mj_ln_u32(c[2]));
     double s1, c1;
     mj_sincos2pi_u32(c[1], &s1, &c1);
     const double c2 = mj_cos2pi_u32(c[3]);

@@ -67,6 +67,8 @@ struct mj_ctx {
     int n_iso = 0, n_dm = 0, n_gen = 0;
     std::vector<int> h_ofs3;           // host copy of the classified stencil: offsets (3 each) and
     std::vector<double> h_cf;          // coefficients in the order iso | dm | gen
+    std::vector<int> h_ord;            // the entries in the order every kernel sums them, by (dz, dy, dx)
+    std::vector<double> h_blk;         // their 3x3 blocks in that order (KArgs::cf)
     int rx = 0, ry = 0, rz = 0;
     int bx = 0, by = 0, bz = 0;        // 0: auto
     int dirty = 1;
@@ -103,8 +105,7 @@ struct mj_ctx {
 int mj_finalize(mj_ctx *c);   // build device-side Hamiltonian if dirty
 
 // per-Hamiltonian stage kernels (mj_jit.hip)
-int mj_jit_prepare(mj_ctx *c, const int *ofs_lds, const double *cf, int bx, int by, int bz, int nblocks, int ntx,
-                   int nty);
+int mj_jit_prepare(mj_ctx *c, int bx, int by, int bz, int nblocks, int ntx, int nty);
 int mj_jit_launch(mj_ctx *c, int mode, bool noise, const KArgs &a, hipStream_t s);
 int mj_jit_resolve(mj_ctx *c, int mode, bool noise);
 int mj_jit_fused_ok(const mj_ctx *c);   // the fused integration-2 kernel was generated

@@ -15,6 +15,7 @@
 #include <string.h>
 
 #include <algorithm>
+#include <array>
 #include <map>
 #include <mutex>
 #include <sstream>
@@ -68,157 +69,123 @@ static int family_of(int mode)
     case MODE_SIB1:
     case MODE_SIB2:
     case MODE_SIBF: return 3;
+    case MODE_RKS: return 5;
     default: return 4;
     }
 }
 
-// the unrolled stencil sum over LDS components of stride TS: iso entries, then
-// DMI-like ones, then general blocks, each in the classified order (the same
-// sum for every tile geometry: only the LDS offsets differ)
-static void emit_stencil(std::ostringstream &g, const mj_ctx *c, const int *ofs_lds, const double *cf, int TS,
-                         int group = 0)
+// Entries between two scheduling barriers of an unrolled neighbour sum: without
+// barriers the LDS reads of the whole stencil are in flight at once, 87 VGPRs
+// to the one-site fused step of the 18-neighbour stencil instead of 63 and
+// more register moves (triangular 1024x1024, Heun: 4 to 12 entries equal within
+// 1%, none 1% slower)
+static const int kSumGroup = 12;
+
+// The unrolled neighbour sums of `ns` sites one above the other (1, or 2: the
+// site at c and the one a row of the region above it) over LDS components of
+// stride TS in a region of row length sx and plane size sxy: the neighbours by
+// (dz, dy, dx) as every kernel sums them, each read once and added to the sums
+// of the sites that have it.  A zero coefficient is left out: fma(0, m, a)
+// returns a for every finite m and nonzero a, and the sign of an exactly zero
+// sum is the only other difference (the on-site anisotropy block diag(0, 0, K)
+// and interfacial DMI, D_z = 0, are mostly zeros).
+static void emit_sum(std::ostringstream &g, const mj_ctx *c, const char *name, int ns, int sx, int sxy, int TS)
 {
-    // group > 0: a scheduling barrier after every `group` entries, so that the
-    // LDS reads of the whole stencil are not all in flight at once (registers)
-    auto fence = [&](int k) {
-        if (group > 0 && (k + 1) % group == 0) g << "    __builtin_amdgcn_sched_barrier(0);\n";
+    g << "  static __device__ __forceinline__ void " << name << "(const double *L, int c";
+    for (int q = 0; q < ns; ++q) g << ", double &ax" << q << ", double &ay" << q << ", double &az" << q;
+    g << ") {\n    const double *Lx = L + c, *Ly = L + " << TS << " + c, *Lz = L + " << 2 * TS << " + c;\n";
+    static const char *mm[3] = {"mx", "my", "mz"}, *acc[3] = {"ax", "ay", "az"};
+    struct Use {
+        int site, ent;
     };
-    // a zero coefficient is left out: fma(0, m, a) returns a for every finite
-    // m and nonzero a, and the sign of an exactly zero sum is the only other
-    // difference (the on-site anisotropy block diag(0, 0, K) and interfacial
-    // DMI, D_z = 0, are mostly zeros)
-    g << "    const double *Lx = L + c, *Ly = L + " << TS << " + c, *Lz = L + " << 2 * TS << " + c;\n";
-    const char *acc[3] = {"ax", "ay", "az"};
-    const char *mm[3] = {"mx", "my", "mz"};
-    // one 3x3 block: the products of the nonzero entries, row by row in the
-    // given column order
-    auto block = [&](int o, const double b[3][3], const int col[3][3]) {
-        bool any = false;
-        for (int r = 0; r < 3; ++r)
-            for (int q = 0; q < 3; ++q) any = any || b[r][col[r][q]] != 0.0;
-        if (!any) return;
-        g << "    { const double mx = Lx[" << o << "], my = Ly[" << o << "], mz = Lz[" << o << "];\n";
-        for (int r = 0; r < 3; ++r) {
-            g << "      ";
-            for (int q = 0; q < 3; ++q) {
-                const int cq = col[r][q];
-                if (b[r][cq] == 0.0) continue;
-                g << acc[r] << " = fma(";
-                hexd(g, b[r][cq]);
-                g << ", " << mm[cq] << ", " << acc[r] << "); ";
-            }
-            g << "\n";
+    std::map<std::array<int, 3>, std::vector<Use>> by;   // (dz, dy, dx) from site 0 -> the sites it is a neighbour of
+    for (size_t k = 0; k < c->h_ord.size(); ++k) {
+        const int *o = &c->h_ofs3[3 * c->h_ord[k]];
+        for (int q = 0; q < ns; ++q) by[{o[2], o[1] + q, o[0]}].push_back({q, (int)k});
+    }
+    int n = 0;
+    for (auto &kv : by) {
+        const int lofs = kv.first[0] * sxy + kv.first[1] * sx + kv.first[2];
+        g << "    { const double mx = Lx[" << lofs << "], my = Ly[" << lofs << "], mz = Lz[" << lofs << "];\n";
+        for (const Use &u : kv.second) {
+            const double *p = &c->h_blk[9 * u.ent];
+            for (int r = 0; r < 3; ++r)
+                for (int q = 0; q < 3; ++q) {
+                    if (p[3 * r + q] == 0.0) continue;
+                    g << "      " << acc[r] << u.site << " = fma(";
+                    hexd(g, p[3 * r + q]);
+                    g << ", " << mm[q] << ", " << acc[r] << u.site << ");\n";
+                }
         }
         g << "    }\n";
-    };
-    int k = 0;
-    const double *p = cf;
-    for (int i = 0; i < c->n_iso; ++i, ++k) {
-        if (p[0] != 0.0) {
-            g << "    { const double s = ";
-            hexd(g, p[0]);
-            g << "; ax = fma(s, Lx[" << ofs_lds[k] << "], ax); ay = fma(s, Ly[" << ofs_lds[k]
-              << "], ay); az = fma(s, Lz[" << ofs_lds[k] << "], az); }\n";
-        }
-        p += 1;
-        fence(k);
+        if (++n % kSumGroup == 0) g << "    __builtin_amdgcn_sched_barrier(0);\n";
     }
-    // J on the diagonal, the antisymmetric part from (p1, p2, p3): row x takes
-    // J mx, p2 mz, -p3 my; row y J my, p3 mx, -p1 mz; row z J mz, p1 my, -p2 mx
-    static const int dm_col[3][3] = {{0, 2, 1}, {1, 0, 2}, {2, 1, 0}};
-    for (int i = 0; i < c->n_dm; ++i, ++k) {
-        const double b[3][3] = {{p[0], -p[3], p[2]}, {p[3], p[0], -p[1]}, {-p[2], p[1], p[0]}};
-        block(ofs_lds[k], b, dm_col);
-        p += 4;
-        fence(k);
-    }
-    static const int gen_col[3][3] = {{0, 1, 2}, {0, 1, 2}, {0, 1, 2}};
-    for (int i = 0; i < c->n_gen; ++i, ++k) {
-        const double b[3][3] = {{p[0], p[1], p[2]}, {p[3], p[4], p[5]}, {p[6], p[7], p[8]}};
-        block(ofs_lds[k], b, gen_col);
-        p += 9;
-        fence(k);
-    }
+    g << "  }\n";
 }
 
-static int fuse_group()
-{
-    const char *e = getenv("MJ_FUSE_GROUP");
-    return e ? atoi(e) : 0;
-}
-
-// Geometry of the fused integration-2 kernel (fused_heun_body): the tile is the
-// stage kernels' tile (bx, by, bz), optionally several of them along y when
-// one plane deep (each then forms its own energy partial); regions S0 (reach
+// Geometry of the fused kernels (fused_body): the tile is the stage kernels'
+// tile (bx, by, bz), or two of them along y (one plane deep); regions S0 (reach
 // 2R) and S1 (reach R) in LDS.  Needs whole wavefronts per stage tile and at
-// most 64 KiB of LDS.
-static void prepare_fused(mj_ctx *c, JitState *j, std::ostringstream &g, const double *cf, int bx, int by, int bz,
-                          int ntx, int nty, int ntz)
+// most 64 KiB of LDS.  Three forms, by the number of double tiles: single
+// tiles while the double ones give a CU fewer than two workgroups (a launch of
+// a small lattice is the latency of one tile), double tiles with threads of
+// their own (a ring of 0.41 instead of 0.69 sites per site at reach 2), and
+// from six workgroups per CU on double tiles with two sites per thread, where
+// the CUs are full and the neighbours read once for both sites count.  Measured,
+// us per step, Heun at 10 K, single / double / pairs: triangular 384x384 8.45 /
+// 9.23 / 9.71, 512x512 10.5 / 9.6 / 10.2, 724x724 19.2 / 18.5 / 18.8, 1024x1024
+// 29.4 / 27.3 / 26.6, 1500x1500 62.3 / 56.9 / 54.9; square 384x384 6.2 / 7.0 /
+// 7.4, 512x512 7.6 / 7.4 / 7.9, 1024x1024 19.6 / 19.1 / 19.5, 1500x1500 39.3 /
+// 38.7 / 39.7 (SIB 42.4 / 39.5 / 39.4, Depondt 46.5 / 42.9 / 42.3).
+// MJ_FUSE_SPT=1 or 2 asks for single tiles or pairs, MJ_FUSE_SUB=2 for double
+// tiles.
+static void prepare_fused(mj_ctx *c, JitState *j, std::ostringstream &g, int bx, int by, int bz, int ntx, int nty,
+                          int ntz)
 {
     j->fuse_ok = 0;
     const int nb = bx * by * bz;
     if (nb % 64 != 0 || ntx <= 0) return;
     const int rx = c->rx, ry = c->ry, rz = c->rz;
-    // stage tiles per fused tile, each with threads of its own: one (measured
-    // on the 1024x1024 triangular workload: 45.7 us per step against 53.0
-    // with two, which halve the workgroups a CU holds at 150 VGPRs);
-    // MJ_FUSE_SUB for measurements
-    const char *se = getenv("MJ_FUSE_SUB");
-    int nsub0 = 1;
-    if (se && atoi(se) >= 1 && bz == 1 && atoi(se) * nb <= 1024) nsub0 = atoi(se);
-    // or two stage tiles sharing the threads, two sites per thread (one plane
-    // deep): S1 grows by 1.41 instead of 1.69 sites per tile site at reach 2,
-    // and the per-thread index and boundary work is shared; same workload:
-    // 41.4 us per step against 44.9 with one site and 46.3 with three (178
-    // VGPRs and 61 KiB of LDS: two workgroups per CU).  Only while that still
-    // gives every CU a workgroup: 512x512, 14.4 us against 15.6; 256x256 (128
-    // workgroups), 11.5 against 8.7.  MJ_FUSE_SPT=1 or 2 overrides
-    const char *sp = getenv("MJ_FUSE_SPT");
+    const char *sp = getenv("MJ_FUSE_SPT"), *su = getenv("MJ_FUSE_SUB");
     int cus = 0;
     if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->device) != hipSuccess) cus = 256;
-    const long nwg2 = (long)ntx * ((c->dim[1] + 2 * by - 1) / (2 * by)) * ((c->dim[2] + bz - 1) / bz);
-    int spt0 = (bz == 1 && !se && nwg2 >= cus) ? 2 : 1;
-    if (sp && bz == 1 && !se && (atoi(sp) == 1 || atoi(sp) == 2)) spt0 = atoi(sp);
-    if (spt0 > 1) nsub0 = spt0;
-    for (int nsub = nsub0; nsub >= 1; --nsub) {
-        const int spt = spt0 > 1 ? nsub : 1;
+    const bool pairs = bz == 1 && bx == 32 && by % 2 == 0;
+    const long nwg2 = (long)ntx * ((c->dim[1] + 2 * by - 1) / (2 * by)) * ntz;
+    int form = 0;   // 0: one stage tile; 1: two, threads of their own; 2: two, two sites per thread
+    if (bz == 1 && nwg2 >= 2L * cus) form = pairs && nwg2 >= 6L * cus ? 2 : 1;
+    if (sp) form = atoi(sp) == 2 && pairs ? 2 : 0;
+    if (su && atoi(su) == 2 && bz == 1) form = 1;
+    for (; form >= 0; --form) {
+        const int spt = form == 2 ? 2 : 1, nsub = form ? 2 : 1;
         const int BX = bx, BY = by * nsub, BZ = bz, nthr = BX * BY * BZ / spt;
         const int s0x = BX + 4 * rx, s0y = BY + 4 * ry, s0z = BZ + 4 * rz;
         const int s1x = BX + 2 * rx, s1y = BY + 2 * ry, s1z = BZ + 2 * rz;
         const int t0 = s0x * s0y * s0z, t1 = s1x * s1y * s1z;
         const bool dma = bx % 2 == 0 && c->dim[0] % 2 == 0 && nthr % 64 == 0;
         const int T0 = dma ? 2 * nthr * ((t0 / 2 + nthr - 1) / nthr) : t0;
-        const size_t shm = sizeof(double) * ((size_t)3 * T0 + (size_t)3 * t1 + BX * BY * BZ / 64 + 1);
-        if (shm > 65536) continue;
-        std::vector<int> l0, l1;
-        const size_t nofs = c->h_ofs3.size() / 3;
-        for (size_t k = 0; k < nofs; ++k) {
-            const int dx = c->h_ofs3[3 * k], dy = c->h_ofs3[3 * k + 1], dz = c->h_ofs3[3 * k + 2];
-            l0.push_back(dz * s0x * s0y + dy * s0x + dx);
-            l1.push_back(dz * s1x * s1y + dy * s1x + dx);
-        }
+        // S1 in S0's place while a thread holds its share of the ring in registers
+        const bool alias = t1 - BX * BY * BZ <= 2 * nthr;
+        const size_t shm = sizeof(double) * ((size_t)3 * T0 + (alias ? 0 : (size_t)3 * t1) + BX * BY * BZ / 64 + 1);
+        if (shm > 65536 || nthr > 1024) continue;
         const int ntyf = (c->dim[1] + BY - 1) / BY, ntzf = (c->dim[2] + BZ - 1) / BZ;
         g << "struct JitFused {\n";
         g << "  static constexpr int kBx = " << BX << ", kBy = " << BY << ", kBz = " << BZ << ", kRx = " << rx
           << ", kRy = " << ry << ", kRz = " << rz << ";\n";
+        g << "  static constexpr int kFill = " << (t0 + nthr - 1) / nthr << ";   // S0 sites per thread\n";
         g << "  static constexpr int kNx = " << c->dim[0] << ", kNy = " << c->dim[1] << ", kNz = " << c->dim[2] << ";\n";
         g << "  static constexpr int kS0x = " << s0x << ", kS0y = " << s0y << ", kS0z = " << s0z << ", kT0 = " << T0
           << ";\n";
-        g << "  static constexpr bool kDma = " << (dma ? "true" : "false") << ";\n";
+        g << "  static constexpr bool kDma = " << (dma ? "true" : "false") << ", kAlias = " << (alias ? "true" : "false")
+          << ";\n";
         g << "  static constexpr int kBmode = " << c->bmode << ";   // 0 no Zeeman, 1 uniform, 2 per site\n";
         g << "  static constexpr int kNtx = " << ntx << ", kNty = " << ntyf << ", kNblocks = " << ntx * ntyf * ntzf
           << ";\n";
-        g << "  static constexpr int kNthrBase = " << nb << ", kNsub = " << nsub << ", kSubAxis = 1, kNtyBase = " << nty
-          << ", kNtzBase = " << ntz << ";\n";
+        g << "  static constexpr int kNthrBase = " << nb << ", kNsub = " << nsub << ", kNtyBase = " << nty << ";\n";
         g << "  static constexpr int kSpt = " << spt << ", kNthr = " << nthr << ";   // sites per thread, threads\n";
-        g << "  static __device__ __forceinline__ void stencil0(const double *L, int c, double &ax, double &ay, "
-             "double &az) {\n";
-        emit_stencil(g, c, l0.data(), cf, T0, fuse_group());
-        g << "  }\n";
-        g << "  static __device__ __forceinline__ void stencil1(const double *L, int c, double &ax, double &ay, "
-             "double &az) {\n";
-        emit_stencil(g, c, l1.data(), cf, t1, fuse_group());
-        g << "  }\n};\n";
+        emit_sum(g, c, "stencil0", 1, s0x, s0x * s0y, T0);
+        emit_sum(g, c, spt == 2 ? "pair1" : "stencil1", spt, s1x, s1x * s1y, t1);
+        if (spt == 2) emit_sum(g, c, "pair0", 2, s0x, s0x * s0y, T0);
+        g << "};\n";
         j->fuse_ok = 1;
         j->fuse_nthr = nthr;
         j->fuse_nblocks = ntx * ntyf * ntzf;
@@ -229,8 +196,7 @@ static void prepare_fused(mj_ctx *c, JitState *j, std::ostringstream &g, const d
 
 int mj_jit_fused_ok(const mj_ctx *c) { return c->jit && ((const JitState *)c->jit)->fuse_ok; }
 
-int mj_jit_prepare(mj_ctx *c, const int *ofs_lds, const double *cf, int bx, int by, int bz, int nblocks, int ntx,
-                   int nty)
+int mj_jit_prepare(mj_ctx *c, int bx, int by, int bz, int nblocks, int ntx, int nty)
 {
     JitState *j = c->jit ? (JitState *)c->jit : new JitState();
     c->jit = j;
@@ -247,7 +213,7 @@ int mj_jit_prepare(mj_ctx *c, const int *ofs_lds, const double *cf, int bx, int 
     const int TS = dma ? 2 * nthr * ((T / 2 + nthr - 1) / nthr) : T;   // LDS component stride
     g << "struct JitGeom {\n";
     g << "  static constexpr int kNit = " << (T + bx * by * bz - 1) / (bx * by * bz) << ";\n";
-    g << "  static constexpr bool kDma = " << (dma ? "true" : "false") << ";\n";
+    g << "  static constexpr bool kDma = " << (dma ? "true" : "false") << ", kCfLds = false;\n";
     g << "  static constexpr int kT = " << TS << ";\n";
     g << "  static __device__ __forceinline__ int tstride(const KArgs &, int) { return " << TS << "; }\n";
     g << "  static constexpr int kBx = " << bx << ", kBy = " << by << ", kBz = " << bz << ", kRx = " << c->rx
@@ -263,10 +229,9 @@ int mj_jit_prepare(mj_ctx *c, const int *ofs_lds, const double *cf, int bx, int 
       << "); }\n";
     g << "  static __device__ __forceinline__ int part(const KArgs &) { return mj_xcd_remap(blockIdx.x, " << nblocks
       << "); }\n";
+    emit_sum(g, c, "sum", 1, sx, sx * sy, TS);
     g << "  static __device__ __forceinline__ void stencil(const KArgs &, const double *L, int, int c, double &ax, "
-         "double &ay, double &az) {\n";
-    emit_stencil(g, c, ofs_lds, cf, TS);
-    g << "  }\n};\n";
+         "double &ay, double &az) { sum(L, c, ax, ay, az); }\n};\n";
     j->nthr = nthr;
     size_t shm = (size_t)3 * TS * sizeof(double);
     if (shm < (size_t)j->nthr * sizeof(double)) shm = (size_t)j->nthr * sizeof(double);
@@ -276,7 +241,7 @@ int mj_jit_prepare(mj_ctx *c, const int *ofs_lds, const double *cf, int bx, int 
     j->pers_shm = (size_t)6 * TS * sizeof(double);
     for (auto &f : j->fnp) f = nullptr;
     for (auto &g2 : j->pers_grid) g2 = 0;
-    prepare_fused(c, j, g, cf, bx, by, bz, ntx, nty, ntx == 0 ? 0 : nblocks / (ntx * nty));
+    prepare_fused(c, j, g, bx, by, bz, ntx, nty, ntx == 0 ? 0 : nblocks / (ntx * nty));
     j->geom = g.str();
     return MJ_OK;
 }
@@ -341,8 +306,9 @@ static std::string family_source(const JitState *j, int fam)
 {
     std::ostringstream s;
     s << "#define MJ_JIT 1\n" << kJitRngH << "\n" << kJitDeviceH << "\n" << kJitKargsH << "\n" << kJitBodyH << "\n" << j->geom << "\n";
-    static const int fam_modes[5][3] = {{MODE_FIELD, -1, -1}, {MODE_EULER, -1, -1}, {MODE_HEUN1, MODE_HEUN2, MODE_HEUNF},
-                                        {MODE_SIB1, MODE_SIB2, MODE_SIBF}, {MODE_DEP1, MODE_DEP2, MODE_DEPF}};
+    static const int fam_modes[6][3] = {{MODE_FIELD, -1, -1}, {MODE_EULER, -1, -1}, {MODE_HEUN1, MODE_HEUN2, MODE_HEUNF},
+                                        {MODE_SIB1, MODE_SIB2, MODE_SIBF}, {MODE_DEP1, MODE_DEP2, MODE_DEPF},
+                                        {MODE_RKS, -1, -1}};
     // occupancy hint: minimum waves per SIMD (MJ_WAVES_PER_EU), which caps VGPRs
     const char *wpe = getenv("MJ_WAVES_PER_EU");
     std::string attr;
@@ -355,9 +321,7 @@ static std::string family_source(const JitState *j, int fam)
                 if (j->fuse_ok)
                     s << "extern \"C\" __global__ void __launch_bounds__(" << j->fuse_nthr << ")" << attr
                       << " mj_stage_" << mode << "_" << nz << "(const KArgs a) { extern __shared__ double lds[]; "
-                      << (mode == MODE_HEUNF ? "fused_heun_body<" : mode == MODE_SIBF ? "fused_sib_body<false, "
-                                                                                     : "fused_sib_body<true, ")
-                      << (nz ? "true" : "false") << ", JitFused>(a, lds); }\n";
+                      << "fused_body<" << mode << ", " << (nz ? "true" : "false") << ", JitFused>(a, lds); }\n";
                 continue;
             }
             s << "extern \"C\" __global__ void __launch_bounds__(" << j->nthr << ")" << attr << " mj_stage_" << mode << "_" << nz

@@ -27,9 +27,9 @@ struct KArgs {
     int ntx, nty, ntz, nblocks;
     int64_t np;  // SoA component stride
 
-    int n_iso, n_dm, n_gen;
-    const int *ofs;     // LDS-linear offsets per stencil entry
-    const double *cf;   // iso: s | dm: s,wx,wy,wz | gen: 9 (row-major)
+    int n_ent, cf_lds;  // cf_lds: the blocks are staged in LDS behind the tile (mj_launch_stage)
+    const int *ofs;     // LDS-linear offsets per stencil entry, by (dz, dy, dx)
+    const double *cf;   // per entry: its 3x3 block (row-major)
 
     int use_stencil;      // 1: field from LDS stencil, 0: MM field read from fld_in
     const double *fld_in; // MM accumulation sum_j Hs_ij m_j (SoA), generic path

@@ -9,7 +9,7 @@ template <int MODE, bool NOISE>
 __global__ void __launch_bounds__(1024) k_stage(const KArgs a)
 {
     extern __shared__ double lds[];
-    stage_body<MODE, NOISE, RtGeom>(a, lds);
+    stage_body<MODE, NOISE, AotGeom>(a, lds);
 }
 
 // energy partials -> E (one block) when no following kernel folds them
@@ -283,12 +283,16 @@ int mj_launch_term_energy(const TermArgs &t, int nblocks, hipStream_t s)
     return MJ_OK;
 }
 
-int mj_launch_stage(int mode, bool noise, const KArgs &a, hipStream_t s)
+int mj_launch_stage(int mode, bool noise, const KArgs &args, hipStream_t s)
 {
+    KArgs a = args;
     stage_fn f = pick(mode, noise);
     int nthr = a.bx * a.by * a.bz;
     size_t T = (size_t)a.sx * a.sy * a.sz;
     size_t shm = a.use_stencil ? 3 * T * sizeof(double) : 0;
+    const size_t blocks = (size_t)9 * a.n_ent * sizeof(double);
+    a.cf_lds = a.use_stencil && blocks <= 8192 && shm + blocks <= 65536;
+    if (a.cf_lds) shm += blocks;
     size_t need = (size_t)nthr * sizeof(double);
     if (shm < need) shm = need;  // block reduction scratch
     hipLaunchKernelGGL(f, dim3(a.nblocks), dim3(nthr), shm, s, a);

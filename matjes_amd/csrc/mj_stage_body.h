@@ -37,6 +37,15 @@ __device__ __forceinline__ int mj_xcd_remap(int bid, int nb)
     return (bid & 7) * (nb >> 3) + (bid >> 3);
 }
 
+// The neighbour sums, complete at this point of the program.  Without it the
+// compiler moves the sums' additions past the next branch of the site algebra
+// and keeps every neighbour's operands in registers across it: 160 VGPRs for
+// the two-site fused step of the 18-neighbour stencil, 116 with it.
+__device__ __forceinline__ void mj_settle(double &ax, double &ay, double &az)
+{
+    asm volatile("" : "+v"(ax), "+v"(ay), "+v"(az));
+}
+
 // Deterministic block reductions.  Full wavefronts: xor butterfly inside the
 // wave (every lane ends with the same value: each step adds the same two
 // operands in either order), then the per-wave values in wave order; one
@@ -89,6 +98,7 @@ __device__ __forceinline__ double mj_block_max(double v, double *red, int nthr)
 struct RtGeom {
     static constexpr int kNit = 0;         // trips of the tile fill: known only at run time
     static constexpr bool kDma = false;    // direct global -> LDS fill (compile-time geometry only)
+    static constexpr bool kCfLds = false;  // the stencil's blocks staged in LDS behind the tile
     // LDS stride between the x, y, z components of the tile (the tile size here)
     static __device__ __forceinline__ int tstride(const KArgs &, int T) { return T; }
     static __device__ __forceinline__ int bx(const KArgs &a) { return a.bx; }
@@ -110,32 +120,18 @@ struct RtGeom {
     static __device__ __forceinline__ void stencil(const KArgs &a, const double *L, int T, int c, double &ax,
                                                    double &ay, double &az)
     {
-        for (int k = 0; k < a.n_iso; ++k) {
-            const int j = c + a.ofs[k];
-            const double s = a.cf[k];
-            ax = fma(s, L[j], ax);
-            ay = fma(s, L[T + j], ay);
-            az = fma(s, L[2 * T + j], az);
-        }
-        const double *cd = a.cf + a.n_iso;
-        for (int k = 0; k < a.n_dm; ++k) {
-            const int j = c + a.ofs[a.n_iso + k];
-            const double s = cd[4 * k], wx = cd[4 * k + 1], wy = cd[4 * k + 2], wz = cd[4 * k + 3];
-            const double mx = L[j], my = L[T + j], mz = L[2 * T + j];
-            ax = fma(s, mx, ax);
-            ax = fma(wy, mz, ax);
-            ax = fma(-wz, my, ax);
-            ay = fma(s, my, ay);
-            ay = fma(wz, mx, ay);
-            ay = fma(-wx, mz, ay);
-            az = fma(s, mz, az);
-            az = fma(wx, my, az);
-            az = fma(-wy, mx, az);
-        }
-        const double *cg = cd + 4 * a.n_dm;
-        for (int k = 0; k < a.n_gen; ++k) {
-            const int j = c + a.ofs[a.n_iso + a.n_dm + k];
-            const double *q = cg + 9 * k;
+        sum(a.n_ent, a.ofs, a.cf, L, T, c, ax, ay, az);
+    }
+    // every entry as a full block (a zero coefficient adds an exact zero), in
+    // one loop without a test of its kind: the reads of several entries are in
+    // flight together
+    static __device__ __forceinline__ void sum(int n, const int *ofs, const double *cf, const double *L, int T, int c,
+                                               double &ax, double &ay, double &az)
+    {
+#pragma unroll 4
+        for (int k = 0; k < n; ++k) {
+            const int j = c + ofs[k];
+            const double *q = cf + 9 * k;
             const double mx = L[j], my = L[T + j], mz = L[2 * T + j];
             ax = fma(q[0], mx, ax);
             ax = fma(q[1], my, ax);
@@ -150,6 +146,28 @@ struct RtGeom {
     }
 };
 
+
+// The same for the ahead-of-time stage kernels, with the blocks staged in LDS
+// (where the host made room for them, KArgs::cf_lds): they run on lattices of a
+// few tiles, where a launch is the latency of one tile, and the blocks' way
+// through a cold scalar cache came after the tile's instead of with it (32x32,
+// Heun, us per step: square 11.5 -> 11.2, triangular 15.1 -> 15.3, integration 4
+// 26.5 -> 25.3 and 34.6 -> 33.6)
+struct AotGeom : RtGeom {
+    static constexpr bool kCfLds = true;
+    static __device__ __forceinline__ void stencil(const KArgs &a, const double *L, int T, int c, double &ax,
+                                                   double &ay, double &az)
+    {
+        if (a.cf_lds) sum(a.n_ent, a.ofs, L + 3 * T, L, T, c, ax, ay, az);
+        else sum(a.n_ent, a.ofs, a.cf, L, T, c, ax, ay, az);
+    }
+    // issued before the tile's loads
+    static __device__ __forceinline__ void stage(const KArgs &a, double *L, int T)
+    {
+        if (a.cf_lds)
+            for (int t = threadIdx.x; t < 9 * a.n_ent; t += blockDim.x) L[3 * T + t] = a.cf[t];
+    }
+};
 
 // The thread's own site in a tile, and the own-site operands of the epilogue
 // (issued early: their latency overlaps the tile fill or the stencil).
@@ -380,6 +398,7 @@ __device__ __forceinline__ void site_end(const KArgs &a, double *lds, const Site
         const int c = (lz + RZ) * SX * SY + (ly + RY) * SX + (lx + RX);
         m = mk3(lds[c], lds[T + c], lds[2 * T + c]);
         G::stencil(a, lds, T, c, ax, ay, az);
+        mj_settle(ax, ay, az);
     } else {
         m = active ? mk3(a.src[gi], a.src[gi + np], a.src[gi + 2 * np]) : mk3(0.0, 0.0, 0.0);
         if (active) {
@@ -468,7 +487,7 @@ __device__ __forceinline__ void site_end(const KArgs &a, double *lds, const Site
         // Dint = 1 D (get_Dmode_int)
         const v3 D = llg_torque(u.n, B, alpha);
         v3 o;
-        if constexpr (NOISE) o = euler_step(m, u, D, llg_torque(u.n, site_thermal_final<MODE, G>(a, st), alpha), a.kdt);
+        if constexpr (NOISE) o = euler_step(m, u, D, a.kdt, llg_torque(u.n, site_thermal_final<MODE, G>(a, st), alpha), a.kdt);
         else o = euler_step0(m, u, D, a.kdt);
         a.dst[gi] = o.x;
         a.dst[gi + np] = o.y;
@@ -515,13 +534,14 @@ __device__ __forceinline__ void site_end(const KArgs &a, double *lds, const Site
     } else if constexpr (MODE == MODE_HEUN2) {
         // stage 2: D2 = LLG(B(m1), m1); m2 = euler(m1, 0.5 D1 + 0.5 D2, DT(m0), dt/2)
         const MjUnit u = mj_unit(m);
-        const v3 dint = heun_dint(pre_aux, llg_torque(u.n, B, alpha));
+        // Dint = D1/2 + D2/2 (get_Dmode_int)
+        const v3 d = pre_aux + llg_torque(u.n, B, alpha);
         v3 o;
         if constexpr (NOISE) {
             // Langevin term of the last stage on m0 (pre_own, site_thermal), spindynamics.f90:269-271,311
-            o = euler_step(m, u, dint, site_thermal_final<MODE, G>(a, st), a.kdt);
+            o = euler_step(m, u, d, 0.5 * a.kdt, site_thermal_final<MODE, G>(a, st), a.kdt);
         } else {
-            o = euler_step0(m, u, dint, a.kdt);
+            o = euler_step0(m, u, d, 0.5 * a.kdt);
         }
         a.dst[gi] = o.x;
         a.dst[gi + np] = o.y;
@@ -590,6 +610,10 @@ __device__ __forceinline__ void stage_body(const KArgs &a, double *lds)
                                 (int64_t)(x0 - RX) + (int64_t)NX * ((int64_t)(y0 - RY) + (int64_t)NY * (z0 - RZ)));
     }
     SiteCtx st = site_begin<MODE, NOISE, G>(a, x0, y0, z0, nstep);
+    if constexpr (G::kCfLds) {
+        if (a.use_stencil)
+            G::stage(a, lds, (G::bx(a) + 2 * G::rx(a)) * (G::by(a) + 2 * G::ry(a)) * (G::bz(a) + 2 * G::rz(a)));
+    }
     if (direct) {
         site_thermal<MODE, NOISE>(a, st);
         __builtin_amdgcn_s_waitcnt(0);   // this wave's tile loads are in LDS
@@ -664,23 +688,42 @@ __device__ __forceinline__ void stage_body_persistent(const KArgs &a, double *ld
 }
 
 // ---------------------------------------------------------------------------
-// Both stages of the reference's integration 2 in one kernel (compile-time
+// Both stages of integration 2, SIB or Depondt in one kernel (compile-time
 // geometry F, mj_jit.hip).  Regions of a tile (BX x BY x BZ sites, reach R):
 //   S0 = the tile plus 2R on every side: m0, staged in LDS;
-//   S1 = the tile plus R: stage 1 (HEUN1) runs on every S1 site from S0 and
-//        its m1 goes to a second LDS region;
-// then stage 2 (HEUN2) runs on the tile from S1 and writes m2.  S1 sites
-// outside the tile repeat stage 1 of the neighbouring tiles with the same
-// arithmetic, and every operation is the two-kernel path's, so m2 equals that
-// path's bit for bit while HBM sees m0 in and m2 out (48 B per site-step
-// instead of 144).  A thread takes kSpt sites, one in each sub-tile of
-// BY/kSpt rows, so that the tile (and with it the share of S1 outside it)
-// grows without more threads per workgroup.  Energy partials of m0 are
-// formed per tile of the two-kernel path (the sub-tiles of BY_BASE rows,
-// whole wavefronts, in that path's lane order);
-// workgroup 0 of the next launch folds them in that path's order (a fold by
-// the last workgroup to finish would need agent-scope fences in every
-// workgroup, and those write back the whole L2 on this multi-XCD part).
+//   S1 = the tile plus R: stage 1 runs on every S1 site from S0 (the tile's own
+//        sites and the ring around them) and its result goes to LDS, in S0's
+//        place once every thread is done with S0;
+// then stage 2 runs on the tile from S1 and writes m' out of place (other tiles
+// still read m0 around this one).  S1 sites outside the tile repeat stage 1 of
+// the neighbouring tiles with the same arithmetic, and every operation is the
+// two-kernel path's, so m' equals that path's bit for bit while HBM sees m0 in
+// and m' out, 48 B per site-step.
+//   integration 2: stage 1 is HEUN1 (m1, the own sites keep D1 and the Langevin
+//     torque on m0), stage 2 HEUN2;
+//   SIB: stage 1 the midpoint p = m + g w(m, a1), stage 2 m' = cay(m, a2(p));
+//   Depondt: stage 1 rotates m about its field b1 into the predictor (the own
+//     sites keep b1), stage 2 rotates m about (b1 + b2)/2.
+// SIB and Depondt add the same thermal field (Philox of the site and step) in
+// both stages, so their ring draws it too.
+//
+// What bounds it is FP64 issue (84% of the cycles at 2048x2048) and the LDS
+// reads of the neighbour sums, 19 entries x 24 B per evaluation of the
+// triangular workload.  A thread takes kSpt = 1 site, or 2 sites one above the
+// other (tiles 32 wide, two wavefront halves per pair of rows), whose sums then
+// read each neighbour they share once (24 entries instead of 38); S1 in S0's
+// place leaves room for twice the workgroups per CU, the ring before the own
+// sites and the settled sums for their registers (106 VGPRs, 160 before); no
+// site of a tile is tested for lying off the lattice, which also keeps the
+// code in a few long blocks.  Heun, triangular at 10 K with the energy every
+// step: 1024x1024 37.1 -> 28.3 us per step, 2048x2048 (no energy) 112.6 -> 87.
+//
+// Energy partials of m0 are formed per tile of the two-kernel path (by rows of
+// BY / kNsub, whole wavefronts, in that path's lane order; a pair's two rows
+// are one wavefront there, and adding them first is that path's first
+// butterfly); workgroup 0 of the next launch folds them in that path's order
+// (a fold by the last workgroup to finish would need agent-scope fences in
+// every workgroup, and those write back the whole L2 on this multi-XCD part).
 // ---------------------------------------------------------------------------
 // Zeeman of the fused kernel: the field mode is a compile-time constant of the
 // geometry (no branch between the stencil's LDS reads and their sums)
@@ -702,38 +745,35 @@ __device__ __forceinline__ v3 fused_zeeman(const KArgs &a, bool live, int64_t gi
     return mk3(zx, zy, zz);
 }
 
+// coordinate g of a region position wrapped on a periodic axis of N sites;
+// false off an open edge.  A tile of B sites and its halo of 2R reach past the
+// lattice by less than one period unless N < B + 2R (then the remainder).
+template <int N, int B, int R>
+__device__ __forceinline__ bool fused_wrap(int &g, int periodic)
+{
+    if constexpr (N >= B + 2 * R) {
+        const bool in = g >= 0 && g < N;
+        g += g < 0 ? N : g >= N ? -N : 0;
+        return in || periodic;
+    } else {
+        return mj_wrap_idx(g, N, periodic);
+    }
+}
+
 // global site of a region position (lattice coordinates g*), wrapped on
 // periodic axes; false off an open edge
 template <class F>
 __device__ __forceinline__ bool fused_site(const KArgs &a, int gx, int gy, int gz, int64_t &gi)
 {
-    if (!mj_wrap_idx(gx, F::kNx, a.px) || !mj_wrap_idx(gy, F::kNy, a.py) || !mj_wrap_idx(gz, F::kNz, a.pz))
-        return false;
+    const bool in = fused_wrap<F::kNx, F::kBx, F::kRx>(gx, a.px) & fused_wrap<F::kNy, F::kBy, F::kRy>(gy, a.py) &
+                    fused_wrap<F::kNz, F::kBz, F::kRz>(gz, a.pz);
     gi = (int64_t)gx + (int64_t)F::kNx * ((int64_t)gy + (int64_t)F::kNy * gz);
-    return true;
-}
-
-// stage 1 of integration 2 at one site from S0 (center c0): the unit vector
-// of m0, D1 and m1 (site_end, MODE_HEUN1), the energy term of m0 when wanted
-template <class F>
-__device__ __forceinline__ void fused_stage1(const KArgs &a, const double *L0, int c0, bool live, int64_t gi,
-                                             v3 &n0, v3 &D1, v3 &m1, double &e)
-{
-    constexpr int T0 = F::kT0;
-    double ax = 0.0, ay = 0.0, az = 0.0;
-    const v3 m0 = mk3(L0[c0], L0[T0 + c0], L0[2 * T0 + c0]);
-    F::stencil0(L0, c0, ax, ay, az);
-    const v3 z = fused_zeeman<F>(a, live, gi);
-    const v3 B = mk3(-(ax + z.x), -(ay + z.y), -(az + z.z));
-    e = mj_site_energy(m0, mk3(ax, ay, az), z);
-    const MjUnit u = mj_unit(m0);
-    n0 = u.n;
-    D1 = llg_torque(u.n, B, a.alpha);
-    m1 = euler_step0(m0, u, D1, a.kdt);   // Dint = 1 D1, as in stage 1 of the two-kernel path
+    return in;
 }
 
 template <class F>
-__device__ __forceinline__ void fused_s0_fill(const KArgs &a, double *L0, int x0, int y0, int z0, bool direct)
+__device__ __forceinline__ void fused_s0_fill(const KArgs &a, double *L0, int x0, int y0, int z0, bool direct,
+                                              v3 v[F::kFill])
 {
     constexpr int SX = F::kS0x, SY = F::kS0y, SZ = F::kS0z, T0 = F::kT0, NTHR = F::kNthr;
     constexpr int RX2 = 2 * F::kRx, RY2 = 2 * F::kRy, RZ2 = 2 * F::kRz;
@@ -766,21 +806,35 @@ __device__ __forceinline__ void fused_s0_fill(const KArgs &a, double *L0, int x0
       }
     }
     (void)direct;
-    for (int t = threadIdx.x; t < SX * SY * SZ; t += NTHR) {
+    // boundary tiles, and lattices whose rows do not pair up: into registers, to
+    // be stored by fused_s0_store after the thermal field is drawn
+#pragma unroll
+    for (int it = 0; it < F::kFill; ++it) {
+        const int t = min((int)threadIdx.x + it * NTHR, SX * SY * SZ - 1);
         const int lx = t % SX;
         const int r = t / SX;
         const int ly = r % SY;
         const int lz = r / SY;
         int64_t g = 0;
-        double vx = 0.0, vy = 0.0, vz = 0.0;
-        if (fused_site<F>(a, x0 + lx - RX2, y0 + ly - RY2, z0 + lz - RZ2, g)) {
-            vx = a.src[g];
-            vy = a.src[g + np];
-            vz = a.src[g + 2 * np];
+        const bool in = fused_site<F>(a, x0 + lx - RX2, y0 + ly - RY2, z0 + lz - RZ2, g);
+        const double *p = a.src + (in ? g : 0);
+        const double vx = p[0], vy = p[np], vz = p[2 * np];
+        v[it] = in ? mk3(vx, vy, vz) : mk3(0.0, 0.0, 0.0);
+    }
+}
+
+template <class F>
+__device__ __forceinline__ void fused_s0_store(double *L0, const v3 v[F::kFill])
+{
+    constexpr int T = F::kS0x * F::kS0y * F::kS0z, T0 = F::kT0;
+#pragma unroll
+    for (int it = 0; it < F::kFill; ++it) {
+        const int t = (int)threadIdx.x + it * F::kNthr;
+        if (t < T) {
+            L0[t] = v[it].x;
+            L0[T0 + t] = v[it].y;
+            L0[2 * T0 + t] = v[it].z;
         }
-        L0[t] = vx;
-        L0[T0 + t] = vy;
-        L0[2 * T0 + t] = vz;
     }
 }
 
@@ -811,192 +865,92 @@ __device__ __forceinline__ void fused_ring_pos(int k, int &sx, int &sy, int &sz)
     }
 }
 
-template <bool NOISE, class F>
-__device__ __forceinline__ void fused_heun_body(const KArgs &a, double *lds)
+// What an own site carries from stage 1 to stage 2: Heun's D1 and the Langevin
+// torque on m0; SIB's and Depondt's m0, thermal field and (Depondt) b1
+template <int MODE>
+struct FusedKeep {
+    v3 p, q, r;
+};
+
+// field of the neighbour sum s
+__device__ __forceinline__ v3 fused_field(v3 s, v3 z) { return mk3(-(s.x + z.x), -(s.y + z.y), -(s.z + z.z)); }
+
+// stage 1 at a site with state m0 and neighbour sum s: the stage's result, the
+// energy term of m0, what stage 2 needs of it (th: the site's thermal field)
+template <int MODE, bool NOISE, class F>
+__device__ __forceinline__ v3 fused_stage1(const KArgs &a, v3 m0, v3 s, int64_t gi, v3 th, FusedKeep<MODE> &k, double &e)
 {
-    constexpr int BX = F::kBx, BY = F::kBy, BZ = F::kBz, RX = F::kRx, RY = F::kRy, RZ = F::kRz;
-    constexpr int SPT = F::kSpt, NTHR = F::kNthr, NB = F::kNthrBase, NBW = NB / 64;
-    constexpr int BYS = BY / SPT;                 // rows of one sub-tile of the thread's sites
-    constexpr int S0X = F::kS0x, S0Y = F::kS0y, T0 = F::kT0;
-    constexpr int S1X = BX + 2 * RX, S1Y = BY + 2 * RY, S1Z = BZ + 2 * RZ, T1 = S1X * S1Y * S1Z;
-    constexpr int NRING = T1 - BX * BY * BZ;
-    static_assert(NB % 64 == 0 && NTHR * SPT == BX * BY * BZ, "whole wavefronts, every tile site once");
-    static_assert(SPT == 1 || (SPT == F::kNsub && NTHR == NB && BZ == 1), "one site per energy sub-tile");
-    double *L0 = lds;                 // S0: 3 x T0
-    double *L1 = lds + 3 * T0;        // S1: 3 x T1
-    double *red = L1 + 3 * T1;        // per-wave sums (BX BY BZ / 64)
-    const int64_t np = a.np;
-
-    const int bid = mj_xcd_remap(blockIdx.x, F::kNblocks);
-    const int tx = bid % F::kNtx, tr = bid / F::kNtx, ty = tr % F::kNty, tz = tr / F::kNty;
-    const int x0 = tx * BX, y0 = ty * BY, z0 = tz * BZ;
-    uint64_t nstep = 0;
-    if constexpr (NOISE) nstep = a.stepp ? *a.stepp + a.step : a.step;
-    const bool direct = F::kDma && (((unsigned long long)a.src) & 15ull) == 0 && x0 - 2 * RX >= 0 &&
-                        x0 + BX + 2 * RX <= F::kNx && y0 - 2 * RY >= 0 && y0 + BY + 2 * RY <= F::kNy &&
-                        z0 - 2 * RZ >= 0 && z0 + BZ + 2 * RZ <= F::kNz;
-    fused_s0_fill<F>(a, L0, x0, y0, z0, direct);
-
-    // the thread's own sites: row ly + j BYS of the tile for j < SPT
-    const int lx = threadIdx.x % BX, ly = (threadIdx.x / BX) % BYS, lz = threadIdx.x / (BX * BYS);
-    const int gx = x0 + lx, gz = z0 + lz;
-    bool active[SPT];
-    int64_t gia[SPT];
-#pragma unroll
-    for (int j = 0; j < SPT; ++j) {
-        const int gy = y0 + ly + j * BYS;
-        active[j] = gx < F::kNx && gy < F::kNy && gz < F::kNz;
-        gia[j] = active[j] ? (int64_t)gx + (int64_t)F::kNx * ((int64_t)gy + (int64_t)F::kNy * gz) : 0;
+    const v3 z = fused_zeeman<F>(a, true, gi);
+    v3 B = fused_field(s, z);
+    e = mj_site_energy(m0, s, z);
+    if constexpr (MODE == MODE_HEUNF) {
+        const MjUnit u = mj_unit(m0);
+        k.p = llg_torque(u.n, B, a.alpha);
+        // Langevin term of the last stage on m0 (HEUN2: thermal_term)
+        if constexpr (NOISE) k.q = llg_torque(u.n, th, a.alpha);
+        return euler_step0(m0, u, k.p, a.kdt);   // Dint = 1 D1
     }
-    // the Philox thermal field of the own sites while the tile lands
-    v3 th[SPT];
-#pragma unroll
-    for (int j = 0; j < SPT; ++j) {
-        th[j] = mk3(0.0, 0.0, 0.0);
-        if constexpr (NOISE) {
-            if (active[j]) {
-                const v3 g = normals3(a.seed, nstep, (uint32_t)gia[j]);
-                th[j] = mk3(a.sigma * g.x, a.sigma * g.y, a.sigma * g.z);
-            }
-        }
+    if constexpr (NOISE) B = mk3(B.x + th.x, B.y + th.y, B.z + th.z);
+    k.p = m0;
+    k.q = th;
+    if constexpr (MODE == MODE_DEPF) {
+        k.r = dep_field(m0, B, a.alpha);
+        return dep_rotate(m0, k.r, a.kdt);
     }
-    if (direct) __builtin_amdgcn_s_waitcnt(0);
-    __syncthreads();
-
-    // pass A: stage 1 at the own positions (wrapped where the tile passes a periodic edge)
-    v3 D1[SPT], q[SPT];
-    double e[SPT];
-#pragma unroll
-    for (int j = 0; j < SPT; ++j) {
-        const int lyj = ly + j * BYS;
-        D1[j] = mk3(0.0, 0.0, 0.0);
-        q[j] = mk3(0.0, 0.0, 0.0);
-        e[j] = 0.0;
-        const int s1 = (lz + RZ) * S1X * S1Y + (lyj + RY) * S1X + (lx + RX);
-        int64_t gw = 0;
-        v3 m1 = mk3(0.0, 0.0, 0.0);
-        if (fused_site<F>(a, gx, y0 + lyj, gz, gw)) {
-            const int c0 = (lz + 2 * RZ) * S0X * S0Y + (lyj + 2 * RY) * S0X + (lx + 2 * RX);
-            v3 n0;
-            double ee;
-            fused_stage1<F>(a, L0, c0, true, gw, n0, D1[j], m1, ee);
-            if (active[j]) e[j] = ee;
-            // Langevin term of the last stage on m0 (HEUN2: thermal_term)
-            if constexpr (NOISE) q[j] = llg_torque(n0, th[j], a.alpha);
-        }
-        L1[s1] = m1.x;
-        L1[T1 + s1] = m1.y;
-        L1[2 * T1 + s1] = m1.z;
-    }
-    // energy partials of m0, one per sub-tile of NB sites (mj_block_reduce's
-    // order: the sub-tile's wavefronts in lane order, then in wave order)
-    if (a.energy) {
-#pragma unroll
-        for (int j = 0; j < SPT; ++j) {
-            double v = e[j];
-#pragma unroll
-            for (int o = 32; o > 0; o >>= 1) v = v + __shfl_xor(v, o, 64);
-            if ((threadIdx.x & 63) == 0) red[j * (NTHR / 64) + (threadIdx.x >> 6)] = v;
-        }
-    }
-    // pass B: stage 1 on the ring of S1 (kept apart from pass A in the
-    // schedule: overlapping them doubles the live registers)
-    __builtin_amdgcn_sched_barrier(0);
-    for (int k = threadIdx.x; k < NRING; k += NTHR) {
-        int sx, sy, sz;
-        fused_ring_pos<F>(k, sx, sy, sz);
-        const int s1 = sz * S1X * S1Y + sy * S1X + sx;
-        int64_t gw = 0;
-        v3 m1 = mk3(0.0, 0.0, 0.0);
-        if (fused_site<F>(a, x0 - RX + sx, y0 - RY + sy, z0 - RZ + sz, gw)) {
-            const int c0 = (sz + RZ) * S0X * S0Y + (sy + RY) * S0X + (sx + RX);
-            v3 n0, d;
-            double ee;
-            fused_stage1<F>(a, L0, c0, true, gw, n0, d, m1, ee);
-        }
-        L1[s1] = m1.x;
-        L1[T1 + s1] = m1.y;
-        L1[2 * T1 + s1] = m1.z;
-    }
-    __syncthreads();
-    // sub-tile h (the two-kernel path's tile (tx, ty * NSUB + h, tz)): its
-    // waves' sums are red[h NBW ...]; one thread per sub-tile adds them in order
-    const int hsub = SPT == 1 ? (int)threadIdx.x / NB : (int)threadIdx.x;
-    if (a.energy && (SPT == 1 ? (threadIdx.x % NB) == 0 : hsub < SPT)) {
-        int sub_ty, sub_tz;
-        if constexpr (F::kSubAxis == 1) {
-            sub_ty = ty * F::kNsub + hsub;
-            sub_tz = tz;
-        } else {
-            sub_ty = ty;
-            sub_tz = tz * F::kNsub + hsub;
-        }
-        if (sub_ty < F::kNtyBase && sub_tz < F::kNtzBase) {
-            double r = red[hsub * NBW];
-            for (int w = 1; w < NBW; ++w) r = r + red[hsub * NBW + w];
-            a.epart[tx + F::kNtx * (sub_ty + F::kNtyBase * sub_tz)] = r;
-        }
-    }
-
-    // stage 2 at the own sites from S1
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int j = 0; j < SPT; ++j) {
-        if (active[j]) {
-            const int s1 = (lz + RZ) * S1X * S1Y + (ly + j * BYS + RY) * S1X + (lx + RX);
-            const v3 m = mk3(L1[s1], L1[T1 + s1], L1[2 * T1 + s1]);
-            double ax = 0.0, ay = 0.0, az = 0.0;
-            F::stencil1(L1, s1, ax, ay, az);
-            const v3 z = fused_zeeman<F>(a, true, gia[j]);
-            const v3 B = mk3(-(ax + z.x), -(ay + z.y), -(az + z.z));
-            if (a.fld_out) {   // the last stage's field, kept for the host
-                a.fld_out[gia[j]] = B.x;
-                a.fld_out[gia[j] + np] = B.y;
-                a.fld_out[gia[j] + 2 * np] = B.z;
-            }
-            const MjUnit u = mj_unit(m);
-            const v3 dint = heun_dint(D1[j], llg_torque(u.n, B, a.alpha));
-            v3 o;
-            if constexpr (NOISE) o = euler_step(m, u, dint, q[j], a.kdt);
-            else o = euler_step0(m, u, dint, a.kdt);
-            const int64_t g = gia[j];
-            a.dst[g] = o.x;
-            a.dst[g + np] = o.y;
-            a.dst[g + 2 * np] = o.z;
-        }
-    }
-
-    // workgroup 0 folds the previous launch's partials (the energy of the state
-    // entering the previous step) as the stage-2 kernel's block 0 folds them:
-    // strided sums over its first NB threads, then their wavefronts in order
-    if (a.ered_in && blockIdx.x == 0) {
-        __syncthreads();
-        double v = 0.0;
-        if (threadIdx.x < NB)
-            for (int i = threadIdx.x; i < a.n_ered; i += NB) v += a.ered_in[i];
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) v = v + __shfl_xor(v, o, 64);
-        if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
-        __syncthreads();
-        if (threadIdx.x == 0) {
-            double r = red[0];
-            for (int w = 1; w < NBW; ++w) r = r + red[w];
-            *a.e_out = r * a.e_scale;
-        }
-    }
+    return cayley_mid(m0, sib_vec(m0, B, a.alpha, -0.5 * a.kdt));
 }
 
-// Both stages of SIB (integration 5) or of Depondt (integration 6) in one
-// kernel, the same regions as fused_heun_body.  SIB: stage 1 (SIB1, the
-// midpoint p = (m + cay(m, a1(m)))/2) runs on every S1 site from S0 and its p
-// goes to LDS; stage 2 (SIB2, m' = cay(m, a2(p))) runs on the tile from S1.
-// Depondt: stage 1 (DEP1) rotates m about its field b1 into the predictor,
-// which goes to LDS (the own sites keep b1); stage 2 (DEP2) rotates m about
-// (b1 + b2)/2, b2 the predictor's field.  Both stages add the same thermal
-// field (Philox of the site and step), so the S1 ring draws it too.  Every
-// operation is the two-kernel path's, so m' equals it bit for bit.
-template <bool NOISE, class F>
-__device__ __forceinline__ v3 fused_sib_thermal(const KArgs &a, uint64_t nstep, int64_t gi)
+// stage 2 at an own site from the stage-1 state m and its neighbour sum s
+template <int MODE, bool NOISE, class F>
+__device__ __forceinline__ void fused_stage2(const KArgs &a, v3 m, v3 s, int64_t gi, const FusedKeep<MODE> &k)
+{
+    const int64_t np = a.np;
+    v3 B = fused_field(s, fused_zeeman<F>(a, true, gi));
+    if (a.fld_out) {   // the last stage's field, kept for the host
+        a.fld_out[gi] = B.x;
+        a.fld_out[gi + np] = B.y;
+        a.fld_out[gi + 2 * np] = B.z;
+    }
+    v3 o;
+    if constexpr (MODE == MODE_HEUNF) {
+        const MjUnit u = mj_unit(m);
+        const v3 d = k.p + llg_torque(u.n, B, a.alpha);   // Dint = D1/2 + D2/2
+        if constexpr (NOISE) o = euler_step(m, u, d, 0.5 * a.kdt, k.q, a.kdt);
+        else o = euler_step0(m, u, d, 0.5 * a.kdt);
+    } else {
+        if constexpr (NOISE) B = mk3(B.x + k.q.x, B.y + k.q.y, B.z + k.q.z);
+        if constexpr (MODE == MODE_DEPF) {
+            const v3 b2 = dep_field(m, B, a.alpha);
+            o = dep_rotate(k.p, mk3(0.5 * (k.r.x + b2.x), 0.5 * (k.r.y + b2.y), 0.5 * (k.r.z + b2.z)), a.kdt);
+        } else {
+            o = cayley(k.p, sib_vec(m, B, a.alpha, -0.5 * a.kdt));
+        }
+    }
+    a.dst[gi] = o.x;
+    a.dst[gi + np] = o.y;
+    a.dst[gi + 2 * np] = o.z;
+}
+
+// the neighbour sums of a thread's sites (one, or two one above the other)
+// centred at c in LDS: REG 0 the S0 layout, 1 the S1 layout
+template <int REG, class F>
+__device__ __forceinline__ void fused_sums(const double *L, int c, v3 s[F::kSpt])
+{
+#pragma unroll
+    for (int j = 0; j < F::kSpt; ++j) s[j] = mk3(0.0, 0.0, 0.0);
+    if constexpr (F::kSpt == 2) {
+        if constexpr (REG == 0) F::pair0(L, c, s[0].x, s[0].y, s[0].z, s[1].x, s[1].y, s[1].z);
+        else F::pair1(L, c, s[0].x, s[0].y, s[0].z, s[1].x, s[1].y, s[1].z);
+        mj_settle(s[1].x, s[1].y, s[1].z);
+    } else {
+        if constexpr (REG == 0) F::stencil0(L, c, s[0].x, s[0].y, s[0].z);
+        else F::stencil1(L, c, s[0].x, s[0].y, s[0].z);
+    }
+    mj_settle(s[0].x, s[0].y, s[0].z);
+}
+
+template <bool NOISE>
+__device__ __forceinline__ v3 fused_thermal(const KArgs &a, uint64_t nstep, int64_t gi)
 {
     if constexpr (NOISE) {
         const v3 g = normals3(a.seed, nstep, (uint32_t)gi);
@@ -1005,45 +959,23 @@ __device__ __forceinline__ v3 fused_sib_thermal(const KArgs &a, uint64_t nstep, 
     return mk3(0.0, 0.0, 0.0);
 }
 
-// stage 1 at one site from S0: SIB's midpoint or Depondt's predictor p (and
-// its field b1), the energy term of m0
-template <bool DEP, bool NOISE, class F>
-__device__ __forceinline__ void fused_sib_stage1(const KArgs &a, const double *L0, int c0, int64_t gi, v3 bt, v3 &m0,
-                                                 v3 &p, v3 &b1, double &e)
-{
-    constexpr int T0 = F::kT0;
-    double ax = 0.0, ay = 0.0, az = 0.0;
-    m0 = mk3(L0[c0], L0[T0 + c0], L0[2 * T0 + c0]);
-    F::stencil0(L0, c0, ax, ay, az);
-    const v3 z = fused_zeeman<F>(a, true, gi);
-    v3 B = mk3(-(ax + z.x), -(ay + z.y), -(az + z.z));
-    e = mj_site_energy(m0, mk3(ax, ay, az), z);
-    if constexpr (NOISE) B = mk3(B.x + bt.x, B.y + bt.y, B.z + bt.z);
-    if constexpr (DEP) {
-        b1 = dep_field(m0, B, a.alpha);
-        p = dep_rotate(m0, b1, a.kdt);
-    } else {
-        p = cayley_mid(m0, sib_vec(m0, B, a.alpha, -0.5 * a.kdt));
-        b1 = mk3(0.0, 0.0, 0.0);
-    }
-}
-
-template <bool DEP, bool NOISE, class F>
-__device__ __forceinline__ void fused_sib_body(const KArgs &a, double *lds)
+template <int MODE, bool NOISE, class F>
+__device__ __forceinline__ void fused_body(const KArgs &a, double *lds)
 {
     constexpr int BX = F::kBx, BY = F::kBy, BZ = F::kBz, RX = F::kRx, RY = F::kRy, RZ = F::kRz;
     constexpr int SPT = F::kSpt, NTHR = F::kNthr, NB = F::kNthrBase, NBW = NB / 64;
-    constexpr int BYS = BY / SPT;
-    constexpr int S0X = F::kS0x, S0Y = F::kS0y;
+    constexpr int BYT = BY / SPT;                 // rows of threads
+    constexpr int S0X = F::kS0x, S0Y = F::kS0y, T0 = F::kT0;
     constexpr int S1X = BX + 2 * RX, S1Y = BY + 2 * RY, S1Z = BZ + 2 * RZ, T1 = S1X * S1Y * S1Z;
     constexpr int NRING = T1 - BX * BY * BZ;
+    constexpr int NRT = (NRING + NTHR - 1) / NTHR;   // ring sites per thread
+    constexpr bool ALIAS = F::kAlias;                // S1 in S0's place
     static_assert(NB % 64 == 0 && NTHR * SPT == BX * BY * BZ, "whole wavefronts, every tile site once");
-    static_assert(SPT == 1 || (SPT == F::kNsub && NTHR == NB && BZ == 1), "one site per energy sub-tile");
-    constexpr int T0 = F::kT0;
-    double *L0 = lds;
-    double *L1 = lds + 3 * T0;
-    double *red = L1 + 3 * T1;
-    const int64_t np = a.np;
+    static_assert(SPT == 1 || (SPT == 2 && BX == 32 && BZ == 1 && BYT % F::kNsub == 0 && NTHR >= NB),
+                  "a pair's rows are one wavefront of the two-kernel path");
+    double *L0 = lds;                                  // S0: 3 x T0
+    double *L1 = ALIAS ? lds : lds + 3 * T0;           // S1: 3 x T1
+    double *red = lds + 3 * T0 + (ALIAS ? 0 : 3 * T1);   // per-wave sums (BX BY BZ / 64)
 
     const int bid = mj_xcd_remap(blockIdx.x, F::kNblocks);
     const int tx = bid % F::kNtx, tr = bid / F::kNtx, ty = tr % F::kNty, tz = tr / F::kNty;
@@ -1053,133 +985,157 @@ __device__ __forceinline__ void fused_sib_body(const KArgs &a, double *lds)
     const bool direct = F::kDma && (((unsigned long long)a.src) & 15ull) == 0 && x0 - 2 * RX >= 0 &&
                         x0 + BX + 2 * RX <= F::kNx && y0 - 2 * RY >= 0 && y0 + BY + 2 * RY <= F::kNy &&
                         z0 - 2 * RZ >= 0 && z0 + BZ + 2 * RZ <= F::kNz;
-    fused_s0_fill<F>(a, L0, x0, y0, z0, direct);
+    v3 fill[F::kFill];
+    fused_s0_fill<F>(a, L0, x0, y0, z0, direct, fill);
 
-    const int lx = threadIdx.x % BX, ly = (threadIdx.x / BX) % BYS, lz = threadIdx.x / (BX * BYS);
+    // S1 inside the lattice: every site of it is one of the lattice's
+    const bool inside = x0 - RX >= 0 && x0 + BX + RX <= F::kNx && y0 - RY >= 0 && y0 + BY + RY <= F::kNy &&
+                        z0 - RZ >= 0 && z0 + BZ + RZ <= F::kNz;
+    // index of the site at lattice coordinates (x, y, z): wrapped on periodic
+    // axes, 0 off an open edge.  Stage 1 runs there all the same: S0 is zero
+    // around an open edge, and a zero spin stays zero in every stage.
+    auto index = [&](int x, int y, int z) -> int64_t {
+        if (inside) return (int64_t)x + (int64_t)F::kNx * ((int64_t)y + (int64_t)F::kNy * z);
+        int64_t g = 0;
+        return fused_site<F>(a, x, y, z, g) ? g : 0;
+    };
+
+    // the thread's own sites (rows SPT ly + j); active: inside the lattice
+    const int lx = threadIdx.x % BX, ly = (threadIdx.x / BX) % BYT * SPT, lz = threadIdx.x / (BX * BYT);
     const int gx = x0 + lx, gz = z0 + lz;
     bool active[SPT];
-    int64_t gia[SPT];
+    int64_t gi[SPT];
     v3 th[SPT];
 #pragma unroll
     for (int j = 0; j < SPT; ++j) {
-        const int gy = y0 + ly + j * BYS;
-        active[j] = gx < F::kNx && gy < F::kNy && gz < F::kNz;
-        gia[j] = active[j] ? (int64_t)gx + (int64_t)F::kNx * ((int64_t)gy + (int64_t)F::kNy * gz) : 0;
-        th[j] = mk3(0.0, 0.0, 0.0);
+        const int gy = y0 + ly + j;
+        active[j] = inside || (gx < F::kNx && gy < F::kNy && gz < F::kNz);
+        gi[j] = index(gx, gy, gz);
+        // the Philox thermal field while the tile lands, one site after the other
+        th[j] = fused_thermal<NOISE>(a, nstep, gi[j]);
+        if constexpr (NOISE) mj_settle(th[j].x, th[j].y, th[j].z);
+        __builtin_amdgcn_sched_barrier(0);
     }
     if (direct) __builtin_amdgcn_s_waitcnt(0);
+    else fused_s0_store<F>(L0, fill);
     __syncthreads();
 
-    // stage 1 at the own positions; the own sites keep m0, the thermal field
-    // and (Depondt) the predictor's field b1
-    v3 m0s[SPT], b1s[SPT];
-    double e[SPT];
-#pragma unroll
-    for (int j = 0; j < SPT; ++j) {
-        const int lyj = ly + j * BYS;
-        m0s[j] = mk3(0.0, 0.0, 0.0);
-        b1s[j] = mk3(0.0, 0.0, 0.0);
-        e[j] = 0.0;
-        const int s1 = (lz + RZ) * S1X * S1Y + (lyj + RY) * S1X + (lx + RX);
-        int64_t gw = 0;
-        v3 p = mk3(0.0, 0.0, 0.0);
-        if (fused_site<F>(a, gx, y0 + lyj, gz, gw)) {
-            const int c0 = (lz + 2 * RZ) * S0X * S0Y + (lyj + 2 * RY) * S0X + (lx + 2 * RX);
-            const v3 bt = fused_sib_thermal<NOISE, F>(a, nstep, gw);
-            double ee;
-            v3 m0, b1;
-            fused_sib_stage1<DEP, NOISE, F>(a, L0, c0, gw, bt, m0, p, b1, ee);
-            if (active[j]) {
-                e[j] = ee;
-                m0s[j] = m0;
-                b1s[j] = b1;
-                th[j] = bt;
-            }
-        }
-        L1[s1] = p.x;
-        L1[T1 + s1] = p.y;
-        L1[2 * T1 + s1] = p.z;
-    }
-    if (a.energy) {
-#pragma unroll
-        for (int j = 0; j < SPT; ++j) {
-            double v = e[j];
-#pragma unroll
-            for (int o = 32; o > 0; o >>= 1) v = v + __shfl_xor(v, o, 64);
-            if ((threadIdx.x & 63) == 0) red[j * (NTHR / 64) + (threadIdx.x >> 6)] = v;
-        }
-    }
-    // stage 1 on the ring of S1
-    __builtin_amdgcn_sched_barrier(0);
-    for (int k = threadIdx.x; k < NRING; k += NTHR) {
+    // stage 1 on the ring of S1, before the own sites: they have more to keep
+    // (kept apart in the schedule: overlapping the two doubles the live registers)
+    auto ring = [&](int k, int &c1) -> v3 {
         int sx, sy, sz;
         fused_ring_pos<F>(k, sx, sy, sz);
-        const int s1 = sz * S1X * S1Y + sy * S1X + sx;
-        int64_t gw = 0;
-        v3 p = mk3(0.0, 0.0, 0.0);
-        if (fused_site<F>(a, x0 - RX + sx, y0 - RY + sy, z0 - RZ + sz, gw)) {
-            const int c0 = (sz + RZ) * S0X * S0Y + (sy + RY) * S0X + (sx + RX);
-            const v3 bt = fused_sib_thermal<NOISE, F>(a, nstep, gw);
-            v3 m0, b1;
-            double ee;
-            fused_sib_stage1<DEP, NOISE, F>(a, L0, c0, gw, bt, m0, p, b1, ee);
+        c1 = sz * S1X * S1Y + sy * S1X + sx;
+        const int c0 = (sz + RZ) * S0X * S0Y + (sy + RY) * S0X + (sx + RX);
+        const int64_t gw = index(x0 - RX + sx, y0 - RY + sy, z0 - RZ + sz);
+        v3 bt = mk3(0.0, 0.0, 0.0);
+        if constexpr (MODE != MODE_HEUNF) bt = fused_thermal<NOISE>(a, nstep, gw);
+        v3 s = mk3(0.0, 0.0, 0.0);
+        F::stencil0(L0, c0, s.x, s.y, s.z);
+        mj_settle(s.x, s.y, s.z);
+        FusedKeep<MODE> drop;
+        double ee;
+        const v3 m = fused_stage1<MODE, NOISE && MODE != MODE_HEUNF, F>(
+            a, mk3(L0[c0], L0[T0 + c0], L0[2 * T0 + c0]), s, gw, bt, drop, ee);
+        return m;
+    };
+    v3 mr[ALIAS && NRT > 0 ? NRT : 1];
+    int cr[ALIAS && NRT > 0 ? NRT : 1];
+    if constexpr (ALIAS) {
+#pragma unroll
+        for (int r = 0; r < NRT; ++r) {
+            const int k = threadIdx.x + r * NTHR;
+            cr[r] = -1;
+            if (k < NRING) mr[r] = ring(k, cr[r]);
         }
-        L1[s1] = p.x;
-        L1[T1 + s1] = p.y;
-        L1[2 * T1 + s1] = p.z;
+    } else {
+        for (int k = threadIdx.x; k < NRING; k += NTHR) {
+            int c1;
+            const v3 m = ring(k, c1);
+            L1[c1] = m.x;
+            L1[T1 + c1] = m.y;
+            L1[2 * T1 + c1] = m.z;
+        }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+
+    // stage 1 at the own positions
+    FusedKeep<MODE> keep[SPT];
+    v3 m1[SPT];
+    double e = 0.0;
+    {
+        const int c0 = (lz + 2 * RZ) * S0X * S0Y + (ly + 2 * RY) * S0X + (lx + 2 * RX);
+        v3 s[SPT];
+        fused_sums<0, F>(L0, c0, s);
+#pragma unroll
+        for (int j = 0; j < SPT; ++j) {
+            const int c = c0 + j * S0X;
+            const v3 m0 = mk3(L0[c], L0[T0 + c], L0[2 * T0 + c]);
+            double ej;
+            m1[j] = fused_stage1<MODE, NOISE, F>(a, m0, s[j], gi[j], th[j], keep[j], ej);
+            if (!active[j]) ej = 0.0;
+            e = j == 0 ? ej : e + ej;
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+    // energy partials of m0 (mj_block_reduce's order: wavefronts in lane order,
+    // then in wave order); red[q]: wavefront q of the two-kernel path's tiles
+    if (a.energy) {
+        constexpr int W = 64 / SPT;
+        double v = e;
+#pragma unroll
+        for (int o = W / 2; o > 0; o >>= 1) v = v + __shfl_xor(v, o, 64);
+        if (threadIdx.x % W == 0) red[threadIdx.x / W] = v;
+    }
+    const int s1 = (lz + RZ) * S1X * S1Y + (ly + RY) * S1X + (lx + RX);
+    if constexpr (ALIAS) {
+        __syncthreads();   // S0 is done with
+#pragma unroll
+        for (int r = 0; r < NRT; ++r) {
+            if (cr[r] >= 0) {
+                L1[cr[r]] = mr[r].x;
+                L1[T1 + cr[r]] = mr[r].y;
+                L1[2 * T1 + cr[r]] = mr[r].z;
+            }
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < SPT; ++j) {
+        const int c = s1 + j * S1X;
+        L1[c] = m1[j].x;
+        L1[T1 + c] = m1[j].y;
+        L1[2 * T1 + c] = m1[j].z;
     }
     __syncthreads();
-    const int hsub = SPT == 1 ? (int)threadIdx.x / NB : (int)threadIdx.x;
-    if (a.energy && (SPT == 1 ? (threadIdx.x % NB) == 0 : hsub < SPT)) {
-        int sub_ty, sub_tz;
-        if constexpr (F::kSubAxis == 1) {
-            sub_ty = ty * F::kNsub + hsub;
-            sub_tz = tz;
-        } else {
-            sub_ty = ty;
-            sub_tz = tz * F::kNsub + hsub;
-        }
-        if (sub_ty < F::kNtyBase && sub_tz < F::kNtzBase) {
-            double r = red[hsub * NBW];
-            for (int w = 1; w < NBW; ++w) r = r + red[hsub * NBW + w];
-            a.epart[tx + F::kNtx * (sub_ty + F::kNtyBase * sub_tz)] = r;
+    // tile h of the two-kernel path (tx, ty * NSUB + h, tz): its wavefronts'
+    // sums are red[h NBW ...]; one thread per tile adds them in order
+    if (a.energy && (int)threadIdx.x < F::kNsub) {
+        const int h = threadIdx.x, sub_ty = ty * F::kNsub + h;
+        if (sub_ty < F::kNtyBase) {
+            double r = red[h * NBW];
+            for (int w = 1; w < NBW; ++w) r = r + red[h * NBW + w];
+            a.epart[tx + F::kNtx * (sub_ty + F::kNtyBase * tz)] = r;
         }
     }
 
     // stage 2 at the own sites from S1
     __builtin_amdgcn_sched_barrier(0);
+    {
+        v3 s[SPT];
+        fused_sums<1, F>(L1, s1, s);
 #pragma unroll
-    for (int j = 0; j < SPT; ++j) {
-        if (active[j]) {
-            const int s1 = (lz + RZ) * S1X * S1Y + (ly + j * BYS + RY) * S1X + (lx + RX);
-            const v3 p = mk3(L1[s1], L1[T1 + s1], L1[2 * T1 + s1]);
-            double ax = 0.0, ay = 0.0, az = 0.0;
-            F::stencil1(L1, s1, ax, ay, az);
-            const v3 z = fused_zeeman<F>(a, true, gia[j]);
-            v3 B = mk3(-(ax + z.x), -(ay + z.y), -(az + z.z));
-            if (a.fld_out) {   // the last stage's field, kept for the host
-                a.fld_out[gia[j]] = B.x;
-                a.fld_out[gia[j] + np] = B.y;
-                a.fld_out[gia[j] + 2 * np] = B.z;
+        for (int j = 0; j < SPT; ++j) {
+            if (active[j]) {
+                const int c = s1 + j * S1X;
+                fused_stage2<MODE, NOISE, F>(a, mk3(L1[c], L1[T1 + c], L1[2 * T1 + c]), s[j], gi[j], keep[j]);
             }
-            if constexpr (NOISE) B = mk3(B.x + th[j].x, B.y + th[j].y, B.z + th[j].z);
-            v3 o;
-            if constexpr (DEP) {
-                const v3 b2 = dep_field(p, B, a.alpha);
-                const v3 b1 = b1s[j];
-                const v3 ba = mk3(0.5 * (b1.x + b2.x), 0.5 * (b1.y + b2.y), 0.5 * (b1.z + b2.z));
-                o = dep_rotate(m0s[j], ba, a.kdt);
-            } else {
-                o = cayley(m0s[j], sib_vec(p, B, a.alpha, -0.5 * a.kdt));
-            }
-            const int64_t g = gia[j];
-            a.dst[g] = o.x;
-            a.dst[g + np] = o.y;
-            a.dst[g + 2 * np] = o.z;
+            __builtin_amdgcn_sched_barrier(0);
         }
     }
 
-    // workgroup 0 folds the previous launch's partials (fused_heun_body's fold)
+    // workgroup 0 folds the previous launch's partials (the energy of the state
+    // entering the previous step) as the stage-2 kernel's block 0 folds them:
+    // strided sums over its first NB threads, then their wavefronts in order
     if (a.ered_in && blockIdx.x == 0) {
         __syncthreads();
         double v = 0.0;

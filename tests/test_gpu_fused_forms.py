@@ -1,0 +1,60 @@
+"""The forms of the fused step (single tiles, double tiles, double tiles with two
+sites per thread) against the two stage kernels, bit for bit, where they can go
+wrong: lattices smaller than a tile and its halo, one site past whole tiles, one
+row short of them, open edges, odd rows (no paired loads), several planes, a
+per-site field, every reach of the stencil from 1 to 3."""
+import os
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+CASES = {
+    "tri_whole": dict(w="tri", size=[96, 64, 1]),
+    "tri_past": dict(w="tri", size=[97, 65, 1]),
+    "tri_short": dict(w="tri", size=[95, 47, 1]),
+    "tri_open": dict(w="tri", size=[70, 61, 1], periodic=[False, False, False]),
+    "tri_narrow": dict(w="tri", size=[33, 130, 1]),
+    "tri_flat": dict(w="tri", size=[300, 14, 1]),
+    "sq_map_mixed": dict(w="sq", size=[66, 79, 1], periodic=[True, False, False], bmap_sigma=0.3),
+    "sq_reach3": dict(w="sq", size=[64, 66, 1], J=[1e-3, -0.2e-3, 0.1e-3, 0.05e-3, -0.04e-3, 0.03e-3]),
+    "planes": dict(w="film", size=[34, 40, 5]),
+}
+
+
+def _run(c, env, integ, T, n):
+    from matjes_amd import llg
+    env = dict({"MJ_FUSE": "1", "MJ_JIT": "1"}, **env)
+    old = {k: os.environ.get(k) for k in ("MJ_FUSE", "MJ_JIT", "MJ_FUSE_SPT", "MJ_FUSE_SUB")}
+    for k in old:
+        os.environ.pop(k, None)
+    os.environ.update(env)
+    try:
+        with llg.Hamiltonian(c["lat"].dim_lat, c["lat"].periodic, tile=(32, 8, 1)) as h:
+            h.load_terms(c["H"], form="stencil")
+            h.set_state(c["m0"])
+            h.keep_last_field(True)
+            E = h.steps(n, integ, 0.5, 0.05, kT=T * 0.000086173324, seed=3, energies=True)
+            return h.get_state(), E, h.last_field()
+    finally:
+        for k, v in old.items():
+            if v is None:
+                os.environ.pop(k, None)
+            else:
+                os.environ[k] = v
+
+
+@pytest.mark.parametrize("integ,T", [(2, 0.0), (2, 10.0), (5, 10.0), (6, 10.0)])
+@pytest.mark.parametrize("name", sorted(CASES))
+def test_forms_equal_the_stage_kernels(name, integ, T):
+    from matjes_amd import workloads
+    s = dict(CASES[name])
+    base = {"tri": workloads.TRIANGULAR_J3DKB, "sq": workloads.SQUARE_JDKB,
+            "film": dict(workloads.FILM_DIP, dipolar=False)}[s.pop("w")]
+    c = workloads.build_case(dict(base, seed=11, **s))
+    ref = _run(c, {"MJ_FUSE": "0"}, integ, T, 5)
+    for env in ({"MJ_FUSE_SPT": "1"}, {"MJ_FUSE_SUB": "2"}, {"MJ_FUSE_SPT": "2"}):
+        got = _run(c, env, integ, T, 5)
+        for a, b in zip(ref, got):
+            assert np.array_equal(a, b), (name, env)
