@@ -26,6 +26,7 @@
 // only the temperature assignment moves, the states stay in place.  The step
 // counter lives in device memory, so the captured graph is replayed as is.
 #include <math.h>
+#include <stdlib.h>
 #include <string.h>
 
 #include <algorithm>
@@ -34,21 +35,7 @@
 #include "mj_device.h"
 #include "mj_internal.h"
 #include "mj_stage_body.h"
-
-struct BatchSys {
-    int nx, ny, nz, px, py, pz;
-    int bx, by, bz, rx, ry, rz, sx, sy, sz, ntx, nty, ntz, nblocks, block0;
-    int n_ent, ofs_off, bmode;   // ofs_off: offsets and blocks of the entries
-    int ofs0_off;         // the stencil's offsets in the fused step's S0 layout (tile + 2R)
-    int64_t base;
-    const double *hdip;   // dipolar systems: the padded grid of H_fft (null: none), its row / plane / component strides
-    int dnx, dny;
-    int64_t hstride;
-    double zb[3];
-    double z9[9];         // the Zeeman block, for a per-site B map (bmode 2)
-    double alpha, rden;   // rden = 1 / (1 + alpha^2)
-    uint64_t seed;
-};
+#include "mj_batch_args.h"
 
 struct BatchGeom : RtGeom {
     static __device__ __forceinline__ int block(const KArgs &a) { return a.vbid; }
@@ -56,63 +43,6 @@ struct BatchGeom : RtGeom {
 };
 
 #define MJ_BATCH_NTHR 256
-
-// the arguments of tile gb (a tile of system S) from the batch-wide ones:
-// the system's geometry, stencil, Zeeman term, damping and Philox stream, its
-// slice of the state buffers, its thermal amplitude and the absolute step;
-// DIP: the batch holds dipolar systems (their H_fft grids)
-template <bool DIP = false>
-__device__ __forceinline__ KArgs sys_args(const KArgs &base, const BatchSys &S, int gb, double sigma, uint64_t step)
-{
-    KArgs a = base;
-    a.nx = S.nx;
-    a.ny = S.ny;
-    a.nz = S.nz;
-    a.px = S.px;
-    a.py = S.py;
-    a.pz = S.pz;
-    a.bx = S.bx;
-    a.by = S.by;
-    a.bz = S.bz;
-    a.rx = S.rx;
-    a.ry = S.ry;
-    a.rz = S.rz;
-    a.sx = S.sx;
-    a.sy = S.sy;
-    a.sz = S.sz;
-    a.ntx = S.ntx;
-    a.nty = S.nty;
-    a.ntz = S.ntz;
-    a.nblocks = S.nblocks;
-    a.vbid = gb - S.block0;
-    a.vbase = S.block0;
-    a.src = base.src + S.base;
-    a.own = base.own ? base.own + S.base : nullptr;
-    a.dst = base.dst ? base.dst + S.base : nullptr;
-    a.aux = base.aux ? base.aux + S.base : nullptr;
-    a.ofs = base.ofs + S.ofs_off;
-    a.cf = base.cf + 9 * S.ofs_off;
-    a.n_ent = S.n_ent;
-    a.bmode = S.bmode;
-    a.zb[0] = S.zb[0];
-    a.zb[1] = S.zb[1];
-    a.zb[2] = S.zb[2];
-    a.bmap = base.bmap ? base.bmap + S.base : nullptr;
-#pragma unroll
-    for (int k = 0; k < 9; ++k) a.z[k] = S.z9[k];
-    if constexpr (DIP) {
-        a.hdip = S.hdip;
-        a.dnx = S.dnx;
-        a.dny = S.dny;
-        a.hstride = S.hstride;
-    }
-    a.alpha = S.alpha;
-    a.kdt = base.kt * S.rden;
-    a.sigma = sigma;
-    a.seed = S.seed;
-    a.step = step;
-    return a;
-}
 
 #ifndef MJ_STAGE_WAVES
 #define MJ_STAGE_WAVES 6
@@ -623,6 +553,17 @@ struct HostSys {
     mj_ctx *dipc = nullptr;   // dipolar term: a context holding the batch's own copy of the transform (owned)
 };
 
+// systems that share a stencil's offsets and a tile: their fused step's kernels
+// (per integration, compiled on first use), their blocks and coefficient classes
+struct BatchGroup {
+    std::vector<int> ofs3, cls, blocks;
+    int bx, by, rx, ry, rz, ncls = 0;
+    int *d_list = nullptr;       // their blocks (null: all of the batch's)
+    double *d_vals = nullptr;    // the classes' values, ncls per system of the batch
+    hipFunction_t fn[3] = {};    // Heun, SIB, Depondt
+    size_t shm = 0;
+};
+
 struct mj_batch {
     int device = 0;
     hipStream_t stream = nullptr;
@@ -653,6 +594,7 @@ struct mj_batch {
     int fused_ok = 0;
     size_t shm_fused = 0;
     int *d_ofs0 = nullptr;
+    std::vector<BatchGroup> groups;   // the compiled fused step (empty: the ahead-of-time one)
     GridBar *d_bar = nullptr;
     int pgrid = 0, pgrid_fused = 0;
     int ran_persist = 0;   // a persistent segment ran since the barrier was last checked
@@ -701,6 +643,11 @@ static void free_dev(mj_batch *b)
                   b->d_step, b->d_beta, b->d_sigl, b->d_rep_of_temp, b->d_temp_of_rep, b->d_acc, b->d_att,
                   b->bmap, b->d_bar, b->d_ofs0};
     for (void *p : ps) bfree(p);
+    for (auto &g : b->groups) {
+        bfree(g.d_list);
+        bfree(g.d_vals);
+    }
+    b->groups.clear();
     b->A = b->Bb = b->Db = b->epart = b->E = b->sigma = b->bmap = nullptr;
     b->d_bar = nullptr;
     b->d_ofs0 = nullptr;
@@ -903,6 +850,125 @@ static void auto_tile(const HostSys &s, int &bx, int &by)
     }
 }
 
+static int blaunch_err(const char *what)
+{
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) {
+        mj_set_error(std::string(what) + ": " + hipGetErrorString(e));
+        return MJ_EHIP;
+    }
+    return MJ_OK;
+}
+
+// Groups of systems for the compiled fused step.  A batch of more than 4
+// groups (one launch each per step), or of coefficients in more than 32
+// classes, keeps the ahead-of-time kernel; so does a batch below the size from
+// which a lattice gets compiled kernels (MJ_JIT=0 never, 1 always).
+static int batch_groups(mj_batch *b, const std::vector<BatchSys> &tab, const std::vector<int> &blk2sys)
+{
+    const char *env = getenv("MJ_JIT");
+    int64_t sites = 0;
+    for (auto &s : b->sys) sites += s.n;
+    if ((env && env[0] == '0') || b->has_dip || !b->fused_ok || (!(env && env[0] == '1') && sites < 4096)) return MJ_OK;
+    std::vector<BatchGroup> gr;
+    std::vector<int> of(b->sys.size());
+    for (size_t q = 0; q < b->sys.size(); ++q) {
+        const HostSys &s = b->sys[q];
+        size_t k = 0;
+        while (k < gr.size() && !(gr[k].ofs3 == s.ofs3 && gr[k].bx == tab[q].bx && gr[k].by == tab[q].by)) ++k;
+        if (k == gr.size()) {
+            if (k == 4) return MJ_OK;
+            gr.emplace_back();
+            gr[k].ofs3 = s.ofs3;
+            gr[k].bx = tab[q].bx;
+            gr[k].by = tab[q].by;
+            gr[k].rx = s.rx;
+            gr[k].ry = s.ry;
+            gr[k].rz = s.rz;
+        }
+        of[q] = (int)k;
+    }
+    for (size_t k = 0; k < gr.size(); ++k) {
+        BatchGroup &g = gr[k];
+        std::vector<int> first;   // a place of each class
+        auto matches = [&](int p, int c, double sign) {
+            for (size_t q = 0; q < b->sys.size(); ++q)
+                if (of[q] == (int)k && b->sys[q].cf[p] != sign * b->sys[q].cf[c]) return false;
+            return true;
+        };
+        auto zero = [&](int p) {
+            for (size_t q = 0; q < b->sys.size(); ++q)
+                if (of[q] == (int)k && b->sys[q].cf[p] != 0.0) return false;
+            return true;
+        };
+        g.cls.assign(3 * g.ofs3.size(), 0);
+        for (size_t p = 0; p < g.cls.size(); ++p) {
+            if (zero((int)p)) continue;
+            size_t c = 0;
+            int sign = 0;
+            for (; c < first.size() && !sign; c += sign ? 0 : 1)
+                sign = matches((int)p, first[c], 1.0) ? 1 : matches((int)p, first[c], -1.0) ? -1 : 0;
+            if (!sign) {
+                first.push_back((int)p);
+                c = first.size() - 1;
+                sign = 1;
+            }
+            g.cls[p] = sign * (int)(c + 1);
+        }
+        if (first.size() > 32) return MJ_OK;
+        g.ncls = (int)std::max<size_t>(first.size(), 1);
+        std::vector<double> v(g.ncls * b->sys.size(), 0.0);
+        for (size_t q = 0; q < b->sys.size(); ++q)
+            if (of[q] == (int)k)
+                for (size_t c = 0; c < first.size(); ++c) v[q * g.ncls + c] = b->sys[q].cf[first[c]];
+        if (hipMalloc(&g.d_vals, sizeof(double) * v.size()) != hipSuccess) BFAIL(MJ_ENOMEM, "mj_batch: device allocation failed");
+        b->groups.push_back(g);   // owned from here (free_dev)
+        MJ_HIP_CHECK(hipMemcpy(g.d_vals, v.data(), sizeof(double) * v.size(), hipMemcpyHostToDevice));
+    }
+    for (size_t q = 0; q < blk2sys.size(); ++q) b->groups[of[blk2sys[q]]].blocks.push_back((int)q);
+    if (b->groups.size() > 1)
+        for (auto &g : b->groups) {
+            MJ_HIP_CHECK(hipMalloc(&g.d_list, sizeof(int) * g.blocks.size()));
+            MJ_HIP_CHECK(hipMemcpy(g.d_list, g.blocks.data(), sizeof(int) * g.blocks.size(), hipMemcpyHostToDevice));
+        }
+    return MJ_OK;
+}
+
+static int fused_slot(int integ) { return integ == MJ_SIB ? 1 : integ == MJ_DEPONDT ? 2 : 0; }
+
+// compile the groups' kernels of the batch's integration (before a capture)
+static int batch_resolve(mj_batch *b)
+{
+    for (auto &g : b->groups) {
+        hipFunction_t &fn = g.fn[fused_slot(b->integ)];
+        const int mode = b->integ == MJ_SIB ? MODE_SIBF : b->integ == MJ_DEPONDT ? MODE_DEPF : MODE_HEUNF;
+        if (!fn) BTRY(mj_jit_batch_fused(g.ofs3, g.cls, g.ncls, g.bx, g.by, g.rx, g.ry, g.rz, mode, &fn, &g.shm));
+    }
+    return MJ_OK;
+}
+
+// the fused step of every system, a.src -> a.dst: one launch per group, or the ahead-of-time kernel
+static int launch_fused(mj_batch *b, const KArgs &a)
+{
+    const int slot = fused_slot(b->integ);
+    bool compiled = !b->groups.empty();
+    for (auto &g : b->groups) compiled = compiled && g.fn[slot];
+    if (!compiled) {
+        auto *k = slot == 1 ? k_batch_fused<MJ_SIB> : slot == 2 ? k_batch_fused<MJ_DEPONDT> : k_batch_fused<MJ_HEUN>;
+        hipLaunchKernelGGL(k, dim3(b->nblocks), dim3(MJ_BATCH_NTHR), b->shm_fused, b->stream, a, b->d_sys, b->d_blk2sys,
+                           b->sigma, b->d_step, b->d_ofs0);
+        return blaunch_err("batched fused step");
+    }
+    for (auto &g : b->groups) {
+        KArgs arg = a;
+        int n = (int)g.blocks.size();
+        void *params[] = {&arg, &b->d_sys, &b->d_blk2sys, &b->sigma, &b->d_step, &g.d_list, &n, &g.d_vals};
+        MJ_HIP_CHECK(hipModuleLaunchKernel(g.fn[slot], (unsigned)n, 1, 1, MJ_BATCH_NTHR, 1, 1, (unsigned)g.shm, b->stream,
+                                           params, nullptr));
+    }
+    return MJ_OK;
+}
+
 // (re)build the device tables and arrays; the states come from HostSys::m0
 static int batch_finalize(mj_batch *b)
 {
@@ -1071,6 +1137,7 @@ static int batch_finalize(mj_batch *b)
         MJ_HIP_CHECK(hipMemcpy(b->d_acc, kept ? b->k_acc.data() : z.data(), sizeof(uint64_t) * R, hipMemcpyHostToDevice));
         MJ_HIP_CHECK(hipMemcpy(b->d_att, kept ? b->k_att.data() : z.data(), sizeof(uint64_t) * R, hipMemcpyHostToDevice));
     }
+    BTRY(batch_groups(b, tab, blk2sys));
     b->g_timestep = -1.0;
     b->dirty = 0;
     return MJ_OK;
@@ -1116,16 +1183,6 @@ static int set_timestep(mj_batch *b, double timestep)
     }
     b->g_timestep = timestep;
     b->g_integ = b->integ;
-    return MJ_OK;
-}
-
-static int blaunch_err(const char *what)
-{
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) {
-        mj_set_error(std::string(what) + ": " + hipGetErrorString(e));
-        return MJ_EHIP;
-    }
     return MJ_OK;
 }
 
@@ -1343,16 +1400,7 @@ static int enqueue_segment(mj_batch *b, double timestep, int len)
                 BTRY(blaunch_err("batched energy pass"));
                 BTRY(enqueue_exchange(b, (uint64_t)j));
             }
-            if (b->integ == MJ_SIB)
-                hipLaunchKernelGGL(k_batch_fused<MJ_SIB>, dim3(b->nblocks), dim3(MJ_BATCH_NTHR), b->shm_fused,
-                                   b->stream, a, b->d_sys, b->d_blk2sys, b->sigma, b->d_step, b->d_ofs0);
-            else if (b->integ == MJ_DEPONDT)
-                hipLaunchKernelGGL(k_batch_fused<MJ_DEPONDT>, dim3(b->nblocks), dim3(MJ_BATCH_NTHR), b->shm_fused,
-                                   b->stream, a, b->d_sys, b->d_blk2sys, b->sigma, b->d_step, b->d_ofs0);
-            else
-                hipLaunchKernelGGL(k_batch_fused<MJ_HEUN>, dim3(b->nblocks), dim3(MJ_BATCH_NTHR), b->shm_fused,
-                                   b->stream, a, b->d_sys, b->d_blk2sys, b->sigma, b->d_step, b->d_ofs0);
-            BTRY(blaunch_err("batched fused step"));
+            BTRY(launch_fused(b, a));
         }
         hipLaunchKernelGGL(k_bump, dim3(1), dim3(64), 0, b->stream, b->d_step, (uint64_t)len);
         return blaunch_err("step counter");
@@ -1384,6 +1432,7 @@ static int batch_run(mj_batch *b, int nsteps, double timestep)
         // dipolar systems: every step eager (the transforms are not captured)
         if (!b->has_dip && b->h_step % (uint64_t)seg == 0 && nsteps >= seg) {
             if (!b->gexec) {
+                if (mode == MJ_BATCH_FUSED) BTRY(batch_resolve(b));
                 MJ_HIP_CHECK(hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal));
                 int rc = enqueue_segment(b, timestep, seg);
                 hipGraph_t g = nullptr;

@@ -110,6 +110,9 @@ int mj_jit_launch(mj_ctx *c, int mode, bool noise, const KArgs &a, hipStream_t s
 int mj_jit_resolve(mj_ctx *c, int mode, bool noise);
 int mj_jit_fused_ok(const mj_ctx *c);   // the fused integration-2 kernel was generated
 void mj_jit_destroy(mj_ctx *c);
+// the fused step of a batch's systems of one stencil and tile (fn null: its tile does not fit in LDS)
+int mj_jit_batch_fused(const std::vector<int> &ofs3, const std::vector<int> &cls, int ncls, int bx, int by, int rx,
+                       int ry, int rz, int mode, hipFunction_t *fn, size_t *shm);
 
 void mj_adj_destroy(mj_ctx *c);   // mj_adjoint.hip
 void mj_mc_destroy(mj_ctx *c);    // mj_mc.hip

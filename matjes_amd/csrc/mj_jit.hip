@@ -83,15 +83,18 @@ static const int kSumGroup = 12;
 
 // The unrolled neighbour sums of `ns` sites one above the other (1, or 2: the
 // site at c and the one a row of the region above it) over LDS components of
-// stride TS in a region of row length sx and plane size sxy: the neighbours by
-// (dz, dy, dx) as every kernel sums them, each read once and added to the sums
-// of the sites that have it.  A zero coefficient is left out: fma(0, m, a)
-// returns a for every finite m and nonzero a, and the sign of an exactly zero
-// sum is the only other difference (the on-site anisotropy block diag(0, 0, K)
-// and interfacial DMI, D_z = 0, are mostly zeros).
-static void emit_sum(std::ostringstream &g, const mj_ctx *c, const char *name, int ns, int sx, int sxy, int TS)
+// stride TS in a region of row length sx and plane size sxy: the neighbours
+// (ofs3, 3 per entry) by (dz, dy, dx) as every kernel sums them, each read once
+// and added to the sums of the sites that have it.  coef(entry, 3 row + column)
+// is the coefficient's expression, empty for a zero one, which is left out:
+// fma(0, m, a) returns a for every finite m and nonzero a, and the sign of an
+// exactly zero sum is the only other difference (the on-site anisotropy block
+// diag(0, 0, K) and interfacial DMI, D_z = 0, are mostly zeros).
+template <class Coef>
+static void emit_sum(std::ostringstream &g, const std::vector<int> &ofs3, const char *name, int ns, int sx, int sxy,
+                     int TS, Coef coef)
 {
-    g << "  static __device__ __forceinline__ void " << name << "(const double *L, int c";
+    g << "  static __device__ __forceinline__ void " << name << "(const KArgs &a, const double *L, int c";
     for (int q = 0; q < ns; ++q) g << ", double &ax" << q << ", double &ay" << q << ", double &az" << q;
     g << ") {\n    const double *Lx = L + c, *Ly = L + " << TS << " + c, *Lz = L + " << 2 * TS << " + c;\n";
     static const char *mm[3] = {"mx", "my", "mz"}, *acc[3] = {"ax", "ay", "az"};
@@ -99,28 +102,64 @@ static void emit_sum(std::ostringstream &g, const mj_ctx *c, const char *name, i
         int site, ent;
     };
     std::map<std::array<int, 3>, std::vector<Use>> by;   // (dz, dy, dx) from site 0 -> the sites it is a neighbour of
-    for (size_t k = 0; k < c->h_ord.size(); ++k) {
-        const int *o = &c->h_ofs3[3 * c->h_ord[k]];
+    for (size_t k = 0; k < ofs3.size() / 3; ++k) {
+        const int *o = &ofs3[3 * k];
         for (int q = 0; q < ns; ++q) by[{o[2], o[1] + q, o[0]}].push_back({q, (int)k});
     }
     int n = 0;
     for (auto &kv : by) {
         const int lofs = kv.first[0] * sxy + kv.first[1] * sx + kv.first[2];
         g << "    { const double mx = Lx[" << lofs << "], my = Ly[" << lofs << "], mz = Lz[" << lofs << "];\n";
-        for (const Use &u : kv.second) {
-            const double *p = &c->h_blk[9 * u.ent];
+        for (const Use &u : kv.second)
             for (int r = 0; r < 3; ++r)
                 for (int q = 0; q < 3; ++q) {
-                    if (p[3 * r + q] == 0.0) continue;
-                    g << "      " << acc[r] << u.site << " = fma(";
-                    hexd(g, p[3 * r + q]);
-                    g << ", " << mm[q] << ", " << acc[r] << u.site << ");\n";
+                    const std::string v = coef(u.ent, 3 * r + q);
+                    if (v.empty()) continue;
+                    g << "      " << acc[r] << u.site << " = fma(" << v << ", " << mm[q] << ", " << acc[r] << u.site
+                      << ");\n";
                 }
-        }
         g << "    }\n";
         if (++n % kSumGroup == 0) g << "    __builtin_amdgcn_sched_barrier(0);\n";
     }
     g << "  }\n";
+}
+
+// offsets of a context's stencil in the order of the sum, and its coefficients as literals
+static std::vector<int> sum_offsets(const mj_ctx *c)
+{
+    std::vector<int> o;
+    for (int k : c->h_ord) o.insert(o.end(), &c->h_ofs3[3 * k], &c->h_ofs3[3 * k] + 3);
+    return o;
+}
+static auto literal_coef(const mj_ctx *c)
+{
+    return [c](int ent, int q) -> std::string {
+        const double v = c->h_blk[9 * ent + q];
+        if (v == 0.0) return std::string();
+        std::ostringstream o;
+        hexd(o, v);
+        return o.str();
+    };
+}
+
+// the regions of a fused tile: its constants (JitFused, BatchFused) and LDS bytes
+static size_t emit_fused_tile(std::ostringstream &g, int BX, int BY, int BZ, int rx, int ry, int rz, int nthr, int spt,
+                              int nsub, int nb, bool dma, int &T0, bool &alias)
+{
+    const int s0x = BX + 4 * rx, s0y = BY + 4 * ry, s0z = BZ + 4 * rz;
+    const int t0 = s0x * s0y * s0z, t1 = (BX + 2 * rx) * (BY + 2 * ry) * (BZ + 2 * rz);
+    T0 = dma ? 2 * nthr * ((t0 / 2 + nthr - 1) / nthr) : t0;
+    // S1 in S0's place while a thread holds its share of the ring in registers
+    alias = t1 - BX * BY * BZ <= 2 * nthr;
+    g << "  static constexpr int kBx = " << BX << ", kBy = " << BY << ", kBz = " << BZ << ", kRx = " << rx
+      << ", kRy = " << ry << ", kRz = " << rz << ";\n";
+    g << "  static constexpr int kFill = " << (t0 + nthr - 1) / nthr << ";   // S0 sites per thread\n";
+    g << "  static constexpr int kS0x = " << s0x << ", kS0y = " << s0y << ", kS0z = " << s0z << ", kT0 = " << T0 << ";\n";
+    g << "  static constexpr bool kDma = " << (dma ? "true" : "false") << ", kAlias = " << (alias ? "true" : "false")
+      << ";\n";
+    g << "  static constexpr int kNthrBase = " << nb << ", kNsub = " << nsub << ";\n";
+    g << "  static constexpr int kSpt = " << spt << ", kNthr = " << nthr << ";   // sites per thread, threads\n";
+    return sizeof(double) * ((size_t)3 * T0 + (alias ? 0 : (size_t)3 * t1) + BX * BY * BZ / 64 + 1);
 }
 
 // Geometry of the fused kernels (fused_body): the tile is the stage kernels'
@@ -158,33 +197,31 @@ static void prepare_fused(mj_ctx *c, JitState *j, std::ostringstream &g, int bx,
     for (; form >= 0; --form) {
         const int spt = form == 2 ? 2 : 1, nsub = form ? 2 : 1;
         const int BX = bx, BY = by * nsub, BZ = bz, nthr = BX * BY * BZ / spt;
-        const int s0x = BX + 4 * rx, s0y = BY + 4 * ry, s0z = BZ + 4 * rz;
-        const int s1x = BX + 2 * rx, s1y = BY + 2 * ry, s1z = BZ + 2 * rz;
-        const int t0 = s0x * s0y * s0z, t1 = s1x * s1y * s1z;
+        const int s0x = BX + 4 * rx, s0y = BY + 4 * ry, s1x = BX + 2 * rx, s1y = BY + 2 * ry;
         const bool dma = bx % 2 == 0 && c->dim[0] % 2 == 0 && nthr % 64 == 0;
-        const int T0 = dma ? 2 * nthr * ((t0 / 2 + nthr - 1) / nthr) : t0;
-        // S1 in S0's place while a thread holds its share of the ring in registers
-        const bool alias = t1 - BX * BY * BZ <= 2 * nthr;
-        const size_t shm = sizeof(double) * ((size_t)3 * T0 + (alias ? 0 : (size_t)3 * t1) + BX * BY * BZ / 64 + 1);
+        std::ostringstream t;
+        int T0 = 0;
+        bool alias = false;
+        const size_t shm = emit_fused_tile(t, BX, BY, BZ, rx, ry, rz, nthr, spt, nsub, nb, dma, T0, alias);
         if (shm > 65536 || nthr > 1024) continue;
         const int ntyf = (c->dim[1] + BY - 1) / BY, ntzf = (c->dim[2] + BZ - 1) / BZ;
-        g << "struct JitFused {\n";
-        g << "  static constexpr int kBx = " << BX << ", kBy = " << BY << ", kBz = " << BZ << ", kRx = " << rx
-          << ", kRy = " << ry << ", kRz = " << rz << ";\n";
-        g << "  static constexpr int kFill = " << (t0 + nthr - 1) / nthr << ";   // S0 sites per thread\n";
-        g << "  static constexpr int kNx = " << c->dim[0] << ", kNy = " << c->dim[1] << ", kNz = " << c->dim[2] << ";\n";
-        g << "  static constexpr int kS0x = " << s0x << ", kS0y = " << s0y << ", kS0z = " << s0z << ", kT0 = " << T0
-          << ";\n";
-        g << "  static constexpr bool kDma = " << (dma ? "true" : "false") << ", kAlias = " << (alias ? "true" : "false")
-          << ";\n";
-        g << "  static constexpr int kBmode = " << c->bmode << ";   // 0 no Zeeman, 1 uniform, 2 per site\n";
-        g << "  static constexpr int kNtx = " << ntx << ", kNty = " << ntyf << ", kNblocks = " << ntx * ntyf * ntzf
-          << ";\n";
-        g << "  static constexpr int kNthrBase = " << nb << ", kNsub = " << nsub << ", kNtyBase = " << nty << ";\n";
-        g << "  static constexpr int kSpt = " << spt << ", kNthr = " << nthr << ";   // sites per thread, threads\n";
-        emit_sum(g, c, "stencil0", 1, s0x, s0x * s0y, T0);
-        emit_sum(g, c, spt == 2 ? "pair1" : "stencil1", spt, s1x, s1x * s1y, t1);
-        if (spt == 2) emit_sum(g, c, "pair0", 2, s0x, s0x * s0y, T0);
+        g << "struct JitFused {\n" << t.str();
+        g << "  static constexpr bool kEnergy = true;\n";
+        auto cst = [&](const char *n, const char *ty, long v) {
+            g << "  static __device__ __forceinline__ constexpr " << ty << " " << n << "(const KArgs &) { return " << v
+              << "; }\n";
+        };
+        cst("nx", "int", c->dim[0]), cst("ny", "int", c->dim[1]), cst("nz", "int", c->dim[2]);
+        cst("ntx", "int", ntx), cst("nty", "int", ntyf), cst("nty_base", "int", nty);
+        cst("bmode", "int", c->bmode), cst("dma", "bool", dma);   // bmode: 0 no Zeeman, 1 uniform, 2 per site
+        g << "  static __device__ __forceinline__ int block(const KArgs &) { return mj_xcd_remap(blockIdx.x, "
+          << ntx * ntyf * ntzf << "); }\n";
+        const auto ofs3 = sum_offsets(c);
+        const auto cf = literal_coef(c);
+        const int t1 = s1x * s1y * (BZ + 2 * rz);
+        emit_sum(g, ofs3, "stencil0", 1, s0x, s0x * s0y, T0, cf);
+        emit_sum(g, ofs3, spt == 2 ? "pair1" : "stencil1", spt, s1x, s1x * s1y, t1, cf);
+        if (spt == 2) emit_sum(g, ofs3, "pair0", 2, s0x, s0x * s0y, T0, cf);
         g << "};\n";
         j->fuse_ok = 1;
         j->fuse_nthr = nthr;
@@ -229,9 +266,9 @@ int mj_jit_prepare(mj_ctx *c, int bx, int by, int bz, int nblocks, int ntx, int 
       << "); }\n";
     g << "  static __device__ __forceinline__ int part(const KArgs &) { return mj_xcd_remap(blockIdx.x, " << nblocks
       << "); }\n";
-    emit_sum(g, c, "sum", 1, sx, sx * sy, TS);
-    g << "  static __device__ __forceinline__ void stencil(const KArgs &, const double *L, int, int c, double &ax, "
-         "double &ay, double &az) { sum(L, c, ax, ay, az); }\n};\n";
+    emit_sum(g, sum_offsets(c), "sum", 1, sx, sx * sy, TS, literal_coef(c));
+    g << "  static __device__ __forceinline__ void stencil(const KArgs &a, const double *L, int, int c, double &ax, "
+         "double &ay, double &az) { sum(a, L, c, ax, ay, az); }\n};\n";
     j->nthr = nthr;
     size_t shm = (size_t)3 * TS * sizeof(double);
     if (shm < (size_t)j->nthr * sizeof(double)) shm = (size_t)j->nthr * sizeof(double);
@@ -260,9 +297,9 @@ std::string mj_jit_source(const mj_ctx *c, int fam)
     return c->jit ? family_source((const JitState *)c->jit, fam) : std::string();
 }
 
-static int compile_family(JitState *j, int fam, hipModule_t *out)
+// the module of a source text: compiled once per process
+static int compile_source(const std::string &src, hipModule_t *out)
 {
-    std::string src = family_source(j, fam);
     std::lock_guard<std::mutex> lk(g_jit_mu);
     auto it = g_mod_cache.find(src);
     if (it != g_mod_cache.end()) {
@@ -302,10 +339,76 @@ static int compile_family(JitState *j, int fam, hipModule_t *out)
     return MJ_OK;
 }
 
+static int compile_family(JitState *j, int fam, hipModule_t *out) { return compile_source(family_source(j, fam), out); }
+
+static std::string device_headers()
+{
+    std::ostringstream s;
+    s << "#define MJ_JIT 1\n" << kJitRngH << "\n" << kJitDeviceH << "\n" << kJitKargsH << "\n" << kJitBodyH << "\n";
+    return s.str();
+}
+
+// The fused step of the systems of a batch that share a stencil's offsets and a
+// tile (bx x by, 256 sites): tile, regions and neighbour sums compile-time, the
+// lattices' sizes, Zeeman terms and coefficients read from the batch's tables.
+// cls[9 entry + q]: 0 a coefficient that is zero in every such system, +-k the
+// k-th value of a system's `ncls` (or its negative): the values stay in scalar
+// registers, an operand of the fused products.
+// FP64 issue bounds it, as the single lattice's step.  24 replicas of 256^2
+// (18 neighbours, T > 0) and 12 more lattices of 32 to 400 a side, 2.2 M sites:
+// 50 us a step, the ahead-of-time kernel (k_batch_fused: offsets and full 3x3
+// blocks read in a loop, wrapped coordinates per staged site) 81 us.
+int mj_jit_batch_fused(const std::vector<int> &ofs3, const std::vector<int> &cls, int ncls, int bx, int by, int rx,
+                       int ry, int rz, int mode, hipFunction_t *fn, size_t *shm)
+{
+    std::ostringstream g;
+    int T0 = 0;
+    bool alias = false;
+    const int s0x = bx + 4 * rx, s0y = by + 4 * ry, s1x = bx + 2 * rx, s1y = by + 2 * ry;
+    g << "struct BatchFused {\n";
+    *shm = emit_fused_tile(g, bx, by, 1, rx, ry, rz, bx * by, 1, 1, bx * by, true, T0, alias);
+    if (*shm > 65536) {
+        *fn = nullptr;
+        return MJ_OK;
+    }
+    g << "  static constexpr bool kEnergy = false;\n";
+    auto arg = [&](const char *n, const char *ty, const char *v) {
+        g << "  static __device__ __forceinline__ " << ty << " " << n << "(const KArgs &a) { return " << v << "; }\n";
+    };
+    arg("nx", "int", "a.nx"), arg("ny", "int", "a.ny"), arg("nz", "int", "a.nz");
+    arg("ntx", "int", "a.ntx"), arg("nty", "int", "a.nty"), arg("nty_base", "int", "a.nty");
+    arg("bmode", "int", "a.bmode"), arg("dma", "bool", "((a.nx | a.np) & 1) == 0"), arg("block", "int", "a.vbid");
+    auto cf = [&](int ent, int q) -> std::string {
+        const int k = cls[9 * ent + q];
+        return k == 0 ? std::string() : std::string(k < 0 ? "-" : "") + "a.cf[" + std::to_string(abs(k) - 1) + "]";
+    };
+    emit_sum(g, ofs3, "stencil0", 1, s0x, s0x * s0y, T0, cf);
+    emit_sum(g, ofs3, "stencil1", 1, s1x, s1x * s1y, s1x * s1y * (1 + 2 * rz), cf);
+    g << "};\n";
+    std::ostringstream s;
+    s << device_headers() << kJitBatchH << "\n" << g.str();
+    s << "extern \"C\" __global__ void __launch_bounds__(" << bx * by
+      << ") mj_batch_fused(const KArgs base, const BatchSys *__restrict__ sys, const int *__restrict__ blk2sys, "
+         "const double *__restrict__ sigma, const uint64_t *__restrict__ stepp, const int *__restrict__ list, int nlist, "
+         "const double *__restrict__ vals) {\n  extern __shared__ double lds[];\n"
+         "  const int b = mj_xcd_remap(blockIdx.x, nlist);\n  const int gb = list ? list[b] : b;\n"
+         "  const int s = blk2sys[gb];\n  KArgs a = sys_args(base, sys[s], gb, sigma[s], *stepp + base.step);\n"
+         "  a.cf = vals + (int64_t)s * " << ncls << ";\n  fused_body<" << mode << ", true, BatchFused>(a, lds);\n}\n";
+    hipModule_t mod;
+    const int rc = compile_source(s.str(), &mod);
+    if (rc != MJ_OK) return rc;
+    const hipError_t e = hipModuleGetFunction(fn, mod, "mj_batch_fused");
+    if (e != hipSuccess) {
+        mj_set_error(std::string("hipModuleGetFunction mj_batch_fused: ") + hipGetErrorString(e));
+        return MJ_EHIP;
+    }
+    return MJ_OK;
+}
+
 static std::string family_source(const JitState *j, int fam)
 {
     std::ostringstream s;
-    s << "#define MJ_JIT 1\n" << kJitRngH << "\n" << kJitDeviceH << "\n" << kJitKargsH << "\n" << kJitBodyH << "\n" << j->geom << "\n";
+    s << device_headers() << j->geom << "\n";
     static const int fam_modes[6][3] = {{MODE_FIELD, -1, -1}, {MODE_EULER, -1, -1}, {MODE_HEUN1, MODE_HEUN2, MODE_HEUNF},
                                         {MODE_SIB1, MODE_SIB2, MODE_SIBF}, {MODE_DEP1, MODE_DEP2, MODE_DEPF},
                                         {MODE_RKS, -1, -1}};

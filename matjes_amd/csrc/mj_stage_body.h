@@ -688,8 +688,9 @@ __device__ __forceinline__ void stage_body_persistent(const KArgs &a, double *ld
 }
 
 // ---------------------------------------------------------------------------
-// Both stages of integration 2, SIB or Depondt in one kernel (compile-time
-// geometry F, mj_jit.hip).  Regions of a tile (BX x BY x BZ sites, reach R):
+// Both stages of integration 2, SIB or Depondt in one kernel (geometry F of
+// mj_jit.hip: compile-time tile and stencil; the lattice's sizes and the
+// coefficients compile-time for one Hamiltonian, run-time for a batch).  Regions of a tile (BX x BY x BZ sites, reach R):
 //   S0 = the tile plus 2R on every side: m0, staged in LDS;
 //   S1 = the tile plus R: stage 1 runs on every S1 site from S0 (the tile's own
 //        sites and the ring around them) and its result goes to LDS, in S0's
@@ -725,17 +726,18 @@ __device__ __forceinline__ void stage_body_persistent(const KArgs &a, double *ld
 // (a fold by the last workgroup to finish would need agent-scope fences in
 // every workgroup, and those write back the whole L2 on this multi-XCD part).
 // ---------------------------------------------------------------------------
-// Zeeman of the fused kernel: the field mode is a compile-time constant of the
-// geometry (no branch between the stencil's LDS reads and their sums)
+// Zeeman of the fused kernel: the field mode is a compile-time constant of a
+// per-Hamiltonian geometry (no branch between the stencil's LDS reads and their sums)
 template <class F>
 __device__ __forceinline__ v3 fused_zeeman(const KArgs &a, bool live, int64_t gi)
 {
     double zx = 0.0, zy = 0.0, zz = 0.0;
-    if constexpr (F::kBmode == 1) {
+    const int bmode = F::bmode(a);
+    if (bmode == 1) {
         zx = a.zb[0];
         zy = a.zb[1];
         zz = a.zb[2];
-    } else if (F::kBmode == 2 && live) {
+    } else if (bmode == 2 && live) {
         const int64_t np = a.np;
         const double bxv = a.bmap[gi], byv = a.bmap[gi + np], bzv = a.bmap[gi + 2 * np];
         zx = (bxv * a.z[0] + byv * a.z[3]) + bzv * a.z[6];
@@ -745,19 +747,15 @@ __device__ __forceinline__ v3 fused_zeeman(const KArgs &a, bool live, int64_t gi
     return mk3(zx, zy, zz);
 }
 
-// coordinate g of a region position wrapped on a periodic axis of N sites;
-// false off an open edge.  A tile of B sites and its halo of 2R reach past the
-// lattice by less than one period unless N < B + 2R (then the remainder).
-template <int N, int B, int R>
-__device__ __forceinline__ bool fused_wrap(int &g, int periodic)
+// coordinate g of a region position wrapped on a periodic axis of n sites;
+// false off an open edge.  A tile of b sites and its halo of 2r reach past the
+// lattice by less than one period unless n < b + 2r (then the remainder).
+__device__ __forceinline__ bool fused_wrap(int &g, int n, int b, int r, int periodic)
 {
-    if constexpr (N >= B + 2 * R) {
-        const bool in = g >= 0 && g < N;
-        g += g < 0 ? N : g >= N ? -N : 0;
-        return in || periodic;
-    } else {
-        return mj_wrap_idx(g, N, periodic);
-    }
+    if (n < b + 2 * r) return mj_wrap_idx(g, n, periodic);
+    const bool in = g >= 0 && g < n;
+    g += g < 0 ? n : g >= n ? -n : 0;
+    return in || periodic;
 }
 
 // global site of a region position (lattice coordinates g*), wrapped on
@@ -765,9 +763,9 @@ __device__ __forceinline__ bool fused_wrap(int &g, int periodic)
 template <class F>
 __device__ __forceinline__ bool fused_site(const KArgs &a, int gx, int gy, int gz, int64_t &gi)
 {
-    const bool in = fused_wrap<F::kNx, F::kBx, F::kRx>(gx, a.px) & fused_wrap<F::kNy, F::kBy, F::kRy>(gy, a.py) &
-                    fused_wrap<F::kNz, F::kBz, F::kRz>(gz, a.pz);
-    gi = (int64_t)gx + (int64_t)F::kNx * ((int64_t)gy + (int64_t)F::kNy * gz);
+    const bool in = fused_wrap(gx, F::nx(a), F::kBx, F::kRx, a.px) & fused_wrap(gy, F::ny(a), F::kBy, F::kRy, a.py) &
+                    fused_wrap(gz, F::nz(a), F::kBz, F::kRz, a.pz);
+    gi = (int64_t)gx + (int64_t)F::nx(a) * ((int64_t)gy + (int64_t)F::ny(a) * gz);
     return in;
 }
 
@@ -784,7 +782,7 @@ __device__ __forceinline__ void fused_s0_fill(const KArgs &a, double *L0, int x0
         constexpr int P = SX * SY * SZ / 2;
         static_assert(T0 >= 2 * NTHR * ((P + NTHR - 1) / NTHR), "S0 stride must hold whole trips");
         const int64_t base =
-            (int64_t)(x0 - RX2) + (int64_t)F::kNx * ((int64_t)(y0 - RY2) + (int64_t)F::kNy * (z0 - RZ2));
+            (int64_t)(x0 - RX2) + (int64_t)F::nx(a) * ((int64_t)(y0 - RY2) + (int64_t)F::ny(a) * (z0 - RZ2));
         const int wave = (int)threadIdx.x >> 6;
 #pragma unroll
         for (int p0 = 0; p0 < P; p0 += NTHR) {
@@ -794,7 +792,7 @@ __device__ __forceinline__ void fused_s0_fill(const KArgs &a, double *L0, int x0
             const int r = t / SX;
             const int ly = r % SY;
             const int lz = r / SY;
-            const int64_t g = base + lx + (int64_t)F::kNx * ((int64_t)ly + (int64_t)F::kNy * lz);
+            const int64_t g = base + lx + (int64_t)F::nx(a) * ((int64_t)ly + (int64_t)F::ny(a) * lz);
             const int wfirst = __builtin_amdgcn_readfirstlane(p0 + 64 * wave);
 #pragma unroll
             for (int c = 0; c < 3; ++c)
@@ -934,17 +932,17 @@ __device__ __forceinline__ void fused_stage2(const KArgs &a, v3 m, v3 s, int64_t
 // the neighbour sums of a thread's sites (one, or two one above the other)
 // centred at c in LDS: REG 0 the S0 layout, 1 the S1 layout
 template <int REG, class F>
-__device__ __forceinline__ void fused_sums(const double *L, int c, v3 s[F::kSpt])
+__device__ __forceinline__ void fused_sums(const KArgs &a, const double *L, int c, v3 s[F::kSpt])
 {
 #pragma unroll
     for (int j = 0; j < F::kSpt; ++j) s[j] = mk3(0.0, 0.0, 0.0);
     if constexpr (F::kSpt == 2) {
-        if constexpr (REG == 0) F::pair0(L, c, s[0].x, s[0].y, s[0].z, s[1].x, s[1].y, s[1].z);
-        else F::pair1(L, c, s[0].x, s[0].y, s[0].z, s[1].x, s[1].y, s[1].z);
+        if constexpr (REG == 0) F::pair0(a, L, c, s[0].x, s[0].y, s[0].z, s[1].x, s[1].y, s[1].z);
+        else F::pair1(a, L, c, s[0].x, s[0].y, s[0].z, s[1].x, s[1].y, s[1].z);
         mj_settle(s[1].x, s[1].y, s[1].z);
     } else {
-        if constexpr (REG == 0) F::stencil0(L, c, s[0].x, s[0].y, s[0].z);
-        else F::stencil1(L, c, s[0].x, s[0].y, s[0].z);
+        if constexpr (REG == 0) F::stencil0(a, L, c, s[0].x, s[0].y, s[0].z);
+        else F::stencil1(a, L, c, s[0].x, s[0].y, s[0].z);
     }
     mj_settle(s[0].x, s[0].y, s[0].z);
 }
@@ -977,25 +975,25 @@ __device__ __forceinline__ void fused_body(const KArgs &a, double *lds)
     double *L1 = ALIAS ? lds : lds + 3 * T0;           // S1: 3 x T1
     double *red = lds + 3 * T0 + (ALIAS ? 0 : 3 * T1);   // per-wave sums (BX BY BZ / 64)
 
-    const int bid = mj_xcd_remap(blockIdx.x, F::kNblocks);
-    const int tx = bid % F::kNtx, tr = bid / F::kNtx, ty = tr % F::kNty, tz = tr / F::kNty;
+    const int bid = F::block(a);
+    const int tx = bid % F::ntx(a), tr = bid / F::ntx(a), ty = tr % F::nty(a), tz = tr / F::nty(a);
     const int x0 = tx * BX, y0 = ty * BY, z0 = tz * BZ;
     uint64_t nstep = 0;
     if constexpr (NOISE) nstep = a.stepp ? *a.stepp + a.step : a.step;
-    const bool direct = F::kDma && (((unsigned long long)a.src) & 15ull) == 0 && x0 - 2 * RX >= 0 &&
-                        x0 + BX + 2 * RX <= F::kNx && y0 - 2 * RY >= 0 && y0 + BY + 2 * RY <= F::kNy &&
-                        z0 - 2 * RZ >= 0 && z0 + BZ + 2 * RZ <= F::kNz;
+    const bool direct = F::dma(a) && (((unsigned long long)a.src) & 15ull) == 0 && x0 - 2 * RX >= 0 &&
+                        x0 + BX + 2 * RX <= F::nx(a) && y0 - 2 * RY >= 0 && y0 + BY + 2 * RY <= F::ny(a) &&
+                        z0 - 2 * RZ >= 0 && z0 + BZ + 2 * RZ <= F::nz(a);
     v3 fill[F::kFill];
     fused_s0_fill<F>(a, L0, x0, y0, z0, direct, fill);
 
     // S1 inside the lattice: every site of it is one of the lattice's
-    const bool inside = x0 - RX >= 0 && x0 + BX + RX <= F::kNx && y0 - RY >= 0 && y0 + BY + RY <= F::kNy &&
-                        z0 - RZ >= 0 && z0 + BZ + RZ <= F::kNz;
+    const bool inside = x0 - RX >= 0 && x0 + BX + RX <= F::nx(a) && y0 - RY >= 0 && y0 + BY + RY <= F::ny(a) &&
+                        z0 - RZ >= 0 && z0 + BZ + RZ <= F::nz(a);
     // index of the site at lattice coordinates (x, y, z): wrapped on periodic
     // axes, 0 off an open edge.  Stage 1 runs there all the same: S0 is zero
     // around an open edge, and a zero spin stays zero in every stage.
     auto index = [&](int x, int y, int z) -> int64_t {
-        if (inside) return (int64_t)x + (int64_t)F::kNx * ((int64_t)y + (int64_t)F::kNy * z);
+        if (inside) return (int64_t)x + (int64_t)F::nx(a) * ((int64_t)y + (int64_t)F::ny(a) * z);
         int64_t g = 0;
         return fused_site<F>(a, x, y, z, g) ? g : 0;
     };
@@ -1009,7 +1007,7 @@ __device__ __forceinline__ void fused_body(const KArgs &a, double *lds)
 #pragma unroll
     for (int j = 0; j < SPT; ++j) {
         const int gy = y0 + ly + j;
-        active[j] = inside || (gx < F::kNx && gy < F::kNy && gz < F::kNz);
+        active[j] = inside || (gx < F::nx(a) && gy < F::ny(a) && gz < F::nz(a));
         gi[j] = index(gx, gy, gz);
         // the Philox thermal field while the tile lands, one site after the other
         th[j] = fused_thermal<NOISE>(a, nstep, gi[j]);
@@ -1031,7 +1029,7 @@ __device__ __forceinline__ void fused_body(const KArgs &a, double *lds)
         v3 bt = mk3(0.0, 0.0, 0.0);
         if constexpr (MODE != MODE_HEUNF) bt = fused_thermal<NOISE>(a, nstep, gw);
         v3 s = mk3(0.0, 0.0, 0.0);
-        F::stencil0(L0, c0, s.x, s.y, s.z);
+        F::stencil0(a, L0, c0, s.x, s.y, s.z);
         mj_settle(s.x, s.y, s.z);
         FusedKeep<MODE> drop;
         double ee;
@@ -1066,7 +1064,7 @@ __device__ __forceinline__ void fused_body(const KArgs &a, double *lds)
     {
         const int c0 = (lz + 2 * RZ) * S0X * S0Y + (ly + 2 * RY) * S0X + (lx + 2 * RX);
         v3 s[SPT];
-        fused_sums<0, F>(L0, c0, s);
+        fused_sums<0, F>(a, L0, c0, s);
 #pragma unroll
         for (int j = 0; j < SPT; ++j) {
             const int c = c0 + j * S0X;
@@ -1080,7 +1078,7 @@ __device__ __forceinline__ void fused_body(const KArgs &a, double *lds)
     }
     // energy partials of m0 (mj_block_reduce's order: wavefronts in lane order,
     // then in wave order); red[q]: wavefront q of the two-kernel path's tiles
-    if (a.energy) {
+    if (F::kEnergy && a.energy) {
         constexpr int W = 64 / SPT;
         double v = e;
 #pragma unroll
@@ -1109,12 +1107,12 @@ __device__ __forceinline__ void fused_body(const KArgs &a, double *lds)
     __syncthreads();
     // tile h of the two-kernel path (tx, ty * NSUB + h, tz): its wavefronts'
     // sums are red[h NBW ...]; one thread per tile adds them in order
-    if (a.energy && (int)threadIdx.x < F::kNsub) {
+    if (F::kEnergy && a.energy && (int)threadIdx.x < F::kNsub) {
         const int h = threadIdx.x, sub_ty = ty * F::kNsub + h;
-        if (sub_ty < F::kNtyBase) {
+        if (sub_ty < F::nty_base(a)) {
             double r = red[h * NBW];
             for (int w = 1; w < NBW; ++w) r = r + red[h * NBW + w];
-            a.epart[tx + F::kNtx * (sub_ty + F::kNtyBase * tz)] = r;
+            a.epart[tx + F::ntx(a) * (sub_ty + F::nty_base(a) * tz)] = r;
         }
     }
 
@@ -1122,7 +1120,7 @@ __device__ __forceinline__ void fused_body(const KArgs &a, double *lds)
     __builtin_amdgcn_sched_barrier(0);
     {
         v3 s[SPT];
-        fused_sums<1, F>(L1, s1, s);
+        fused_sums<1, F>(a, L1, s1, s);
 #pragma unroll
         for (int j = 0; j < SPT; ++j) {
             if (active[j]) {
@@ -1136,7 +1134,7 @@ __device__ __forceinline__ void fused_body(const KArgs &a, double *lds)
     // workgroup 0 folds the previous launch's partials (the energy of the state
     // entering the previous step) as the stage-2 kernel's block 0 folds them:
     // strided sums over its first NB threads, then their wavefronts in order
-    if (a.ered_in && blockIdx.x == 0) {
+    if (F::kEnergy && a.ered_in && blockIdx.x == 0) {
         __syncthreads();
         double v = 0.0;
         if (threadIdx.x < NB)
