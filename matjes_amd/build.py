@@ -19,7 +19,8 @@ FDIR = os.path.join(PKG, "fortran")
 HIP_SOURCES = ["mj_api.hip", "mj_kernels.hip", "mj_fft.hip", "mj_jit.hip", "mj_adjoint.hip", "mj_batch.hip", "mj_mc.hip", "mj_noalloc.hip"]
 # device sources embedded as text for the per-Hamiltonian kernels compiled at set-up
 JIT_EMBED = [("kJitRngH", "mj_rngmath.h"), ("kJitDeviceH", "mj_device.h"), ("kJitKargsH", "mj_kargs.h"), ("kJitBodyH", "mj_stage_body.h"),
-             ("kJitBatchH", "mj_batch_args.h")]
+             ("kJitBatchH", "mj_batch_args.h"),
+             ("kJitMcH", "mj_mc_body.h")]
 
 
 def gen_jit_embed():

@@ -110,6 +110,10 @@ int mj_jit_launch(mj_ctx *c, int mode, bool noise, const KArgs &a, hipStream_t s
 int mj_jit_resolve(mj_ctx *c, int mode, bool noise);
 int mj_jit_fused_ok(const mj_ctx *c);   // the fused integration-2 kernel was generated
 void mj_jit_destroy(mj_ctx *c);
+// Monte Carlo kernels of a stencil without its on-site entry (offsets o3, full blocks cf9, class shifts csh) on the
+// context's lattice coloured (x + ca y + cb z) mod p
+int mj_jit_mc(const mj_ctx *c, const std::vector<int> &o3, const std::vector<double> &cf9, const std::vector<int> &csh,
+              int p, int ca, int cb, hipFunction_t *pass, hipFunction_t *energy);
 // the fused step of a batch's systems of one stencil and tile (fn null: its tile does not fit in LDS)
 int mj_jit_batch_fused(const std::vector<int> &ofs3, const std::vector<int> &cls, int ncls, int bx, int by, int rx,
                        int ry, int rz, int mode, hipFunction_t *fn, size_t *shm);

@@ -405,6 +405,116 @@ int mj_jit_batch_fused(const std::vector<int> &ofs3, const std::vector<int> &cls
     return MJ_OK;
 }
 
+// Monte Carlo passes and replica energies: the neighbours' slots from the
+// lattice's constants, the spins of 18 neighbours in flight together (the
+// proposal is computed under the first ones), coefficients as literals, terms
+// in the order and with the operations of mc_pair_field_cm (zero ones left out).
+// Latency bounds a pass (two wavefronts per SIMD at 131072 sites): 18 neighbours
+// in three trips through a table of slots took 18.2 us per class of 1024^2 (8
+// classes) and 13.9 us for 8 replicas of 256^2, one trip with the addresses from
+// constants 8.1 and 6.6; replica energies 34.6 -> 22.  Blocks of 64 and 128
+// threads: 8 and 2 % slower at 1024^2, equal at 256^2.
+int mj_jit_mc(const mj_ctx *c, const std::vector<int> &o3, const std::vector<double> &cf9, const std::vector<int> &csh,
+              int p, int ca, int cb, hipFunction_t *pass, hipFunction_t *energy)
+{
+    constexpr int kGroup = 18;
+    const int nx = c->dim[0], ny = c->dim[1], nz = c->dim[2], W = (nx + p - 1) / p, ne = (int)csh.size();
+    const int64_t RW = (int64_t)ny * nz * W;
+    std::ostringstream g;
+    g << "struct McGeom {\n  static constexpr int kNx = " << nx << ", kNy = " << ny << ", kRows = " << ny * nz
+      << ", kW = " << W << ", kP = " << p << ";\n";
+    g << "  static __device__ __forceinline__ int first(int k, int y, int z) {\n    int x0 = (k - " << ca << " * y - " << cb
+      << " * z) % " << p << ";\n    return x0 < 0 ? x0 + " << p << " : x0;\n  }\n";
+    g << "  template <class Mid> static __device__ __forceinline__ v3 field(const McArgs &a, const double *cm, int k, int x0, "
+         "int jj, int x, int y, int z, Mid mid) {\n    double ax = 0.0, ay = 0.0, az = 0.0;\n";
+    // column of the neighbour at dx, row offset of the one at (dy, dz); open edges: false
+    std::map<int, int> dxs;
+    std::map<std::array<int, 2>, int> rows;
+    for (int e = 0; e < ne; ++e) {
+        dxs.insert({o3[3 * e], (int)dxs.size()});
+        rows.insert({{o3[3 * e + 1], o3[3 * e + 2]}, (int)rows.size()});
+    }
+    for (auto &kv : dxs) {
+        const int dx = kv.first, i = kv.second;
+        const int q0 = (dx % p + p) % p, f = (dx - q0) / p;   // dx = f p + q0
+        g << "    int j" << i << " = jj + " << f << " + (x0 + " << q0 << " >= " << p << " ? 1 : 0);\n";
+        g << "    const int u" << i << " = x + " << dx << "; const bool cx" << i << " = " << (c->periodic[0] ? "true" : "")
+          << (c->periodic[0] ? "" : "u" + std::to_string(i) + " >= 0 && u" + std::to_string(i) + " < " + std::to_string(nx))
+          << ";\n";
+        if (c->periodic[0])
+            g << "    j" << i << " += u" << i << " < 0 ? " << W << " : u" << i << " >= " << nx << " ? " << -W << " : 0;\n";
+    }
+    for (auto &kv : rows) {
+        const int i = kv.second;
+        auto axis = [&](const char *v, int d, int n, int per) {
+            const std::string w = std::string(v) + std::to_string(i);
+            g << "    int " << w << " = " << v << " + " << d << "; const bool c" << w << " = ";
+            if (d == 0) g << "true;\n";
+            else if (!per) g << w << " >= 0 && " << w << " < " << n << ";\n";
+            else if (abs(d) <= n) g << "true; " << w << " += " << w << " < 0 ? " << n << " : " << w << " >= " << n << " ? " << -n << " : 0;\n";
+            else g << "true; " << w << " = ((" << w << " % " << n << ") + " << n << ") % " << n << ";\n";
+        };
+        axis("y", kv.first[0], ny, c->periodic[1]);
+        axis("z", kv.first[1], nz, c->periodic[2]);
+        g << "    const int r" << i << " = (y" << i << " + " << ny << " * z" << i << ") * " << W << "; const bool cr" << i
+          << " = cy" << i << " && cz" << i << ";\n";
+    }
+    auto has = [&](int e, int col) { return cf9[9 * e + col] != 0.0 || cf9[9 * e + 3 + col] != 0.0 || cf9[9 * e + 6 + col] != 0.0; };
+    static const char *mm[3] = {"mx", "my", "mz"}, *acc[3] = {"ax", "ay", "az"};
+    for (int e0 = 0; e0 < ne; e0 += kGroup) {
+        const int e1 = std::min(ne, e0 + kGroup);
+        for (int e = e0; e < e1; ++e) {
+            const int *o = &o3[3 * e];
+            const int i = dxs[o[0]], r = rows[{o[1], o[2]}];
+            const bool open = (!c->periodic[0] && o[0]) || (!c->periodic[1] && o[1]) || (!c->periodic[2] && o[2]);
+            g << "    const int k" << e << " = k + " << csh[e] << " >= " << p << " ? k + " << csh[e] - p << " : k + " << csh[e]
+              << ";\n    const double *q" << e << " = cm + (int64_t)k" << e << " * " << RW << "; const bool ok" << e << " = ";
+            if (open) g << "cx" << i << " && cr" << r << ";\n";
+            else g << "true;\n";
+            g << "    const unsigned s" << e << " = ok" << e << " ? 8u * (unsigned)(r" << r << " + j" << i << ") : 0u;\n";
+            for (int d = 0; d < 3; ++d)
+                if (has(e, d)) {
+                    g << "    double " << mm[d] << e << " = *(const double *)((const char *)(q" << e << " + " << d
+                      << " * a.cs) + s" << e << ");\n";
+                }
+        }
+        g << "    __builtin_amdgcn_sched_barrier(0);\n";
+        if (e0 == 0) g << "    mid();\n";
+        for (int e = e0; e < e1; ++e) {
+            const int *o = &o3[3 * e];
+            const bool open = (!c->periodic[0] && o[0]) || (!c->periodic[1] && o[1]) || (!c->periodic[2] && o[2]);
+            for (int d = 0; d < 3 && open; ++d)
+                if (has(e, d)) g << "    " << mm[d] << e << " = ok" << e << " ? " << mm[d] << e << " : 0.0;\n";
+            for (int r = 0; r < 3; ++r)
+                for (int d = 0; d < 3; ++d) {
+                    const double v = cf9[9 * e + 3 * r + d];
+                    if (v == 0.0) continue;
+                    g << "    " << acc[r] << " = fma(";
+                    hexd(g, v);
+                    g << ", " << mm[d] << e << ", " << acc[r] << ");\n";
+                }
+        }
+    }
+    if (ne == 0) g << "    mid();\n";
+    g << "    return mk3(ax, ay, az);\n  }\n};\n";
+    std::ostringstream s;
+    s << device_headers() << kJitMcH << "\n" << g.str();
+    s << "extern \"C\" __global__ void __launch_bounds__(kMcThreads) mj_mc_pass(const McArgs a) { "
+         "mc_pass_body<McGeom>(a); }\n";
+    s << "extern \"C\" __global__ void __launch_bounds__(kMcThreads) mj_mc_energy(const McArgs a, double *part) { "
+         "mc_energy_body<McGeom>(a, part); }\n";
+    hipModule_t mod;
+    const int rc = compile_source(s.str(), &mod);
+    if (rc != MJ_OK) return rc;
+    hipError_t e = hipModuleGetFunction(pass, mod, "mj_mc_pass");
+    if (e == hipSuccess) e = hipModuleGetFunction(energy, mod, "mj_mc_energy");
+    if (e != hipSuccess) {
+        mj_set_error(std::string("hipModuleGetFunction: ") + hipGetErrorString(e));
+        return MJ_EHIP;
+    }
+    return MJ_OK;
+}
+
 static std::string family_source(const JitState *j, int fam)
 {
     std::ostringstream s;

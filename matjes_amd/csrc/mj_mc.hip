@@ -33,6 +33,7 @@
 #include "mj_device.h"
 #include "mj_internal.h"
 #include "mj_stage_body.h"
+#include "mj_mc_body.h"
 
 #define MJ_FAIL(code, msg)        \
     do {                          \
@@ -46,55 +47,6 @@
     } while (0)
 
 namespace {
-
-constexpr uint32_t kMcStream = 0x4D430000u;   // counter word 3 of the Monte Carlo draws
-constexpr int kMcThreads = 256;
-
-struct McState {
-    double cone, cos_cone, acc, nb, rate;
-};
-
-struct McArgs {
-    double *m;              // state, SoA
-    int64_t np;
-    int nx, ny, nz, px, py, pz;
-    int p, ca, cb, color;
-    int64_t nthreads;
-    int n_iso, n_dm, n_gen;
-    const int *o3;          // offsets (3 each), classes iso | dm | gen, no d = 0
-    const double *cf;       // iso: s; dm: s, w; gen: 9
-    double c0[9];           // on-site C_0 = A_0 + A_0^T
-    int bmode;
-    double zb[3], z[9];
-    const double *bmap;
-    double kT;
-    uint64_t seed, sweep;
-    int sampler;
-    McState *st;
-    double *acc_part;
-    // replicas (parallel tempering): blockIdx.y is the replica; its state, counters,
-    // partials and temperature are at these strides (kT_rep null: one temperature)
-    int64_t rep_cm, rep_part;
-    const double *kT_rep;
-    // colour-major copy of the state used by the passes: slot of site (x, y, z) =
-    // class * R * W + (y + ny z) * W + x / p, R = ny nz rows, W = ceil(nx / p)
-    double *cm;
-    const double *cbmap;    // per-site field map in the same order (or null)
-    int64_t cs;             // component stride of cm (p R W)
-    int W;
-    const int *csh;         // per stencil entry: class shift (dx + a dy + b dz) mod p
-    const double *cf9;      // every stencil entry as a full 3x3 block (passes)
-    // rows at least the stencil reach from the y and z boundaries take the
-    // neighbour slots from a table: slot + tab[x0 * ne + e] (+-W across x)
-    int fast, ne;
-    const int *tab;
-    int ylo, yhi, zlo, zhi;
-    // single-site energies
-    int64_t nsites;
-    const int64_t *sites;
-    const double *spins;    // AoS 3 per site, or null for the current spin
-    double *e_out;
-};
 
 __device__ __forceinline__ bool mc_nb(const McArgs &a, int x, int y, int z, const int *o, int64_t &j)
 {
@@ -247,74 +199,6 @@ __device__ __forceinline__ v3 mc_pair_field_cm(const McArgs &a, const double *cm
     return mk3(ax, ay, az);
 }
 
-__device__ __forceinline__ v3 mc_zeeman(const McArgs &a, const double *bmap, int64_t stride, int64_t i)
-{
-    if (a.bmode == 1) return mk3(a.zb[0], a.zb[1], a.zb[2]);
-    if (a.bmode == 2) {
-        const double bx = bmap[i], by = bmap[i + stride], bz = bmap[i + 2 * stride];
-        return mk3((bx * a.z[0] + by * a.z[3]) + bz * a.z[6], (bx * a.z[1] + by * a.z[4]) + bz * a.z[7],
-                   (bx * a.z[2] + by * a.z[5]) + bz * a.z[8]);
-    }
-    return mk3(0.0, 0.0, 0.0);
-}
-
-// energy of site i with spin s: s.(h + z) + s^T C_0 s / 2
-__device__ __forceinline__ double mc_site_energy(const McArgs &a, v3 s, v3 h)
-{
-    const double *c = a.c0;
-    const double qx = (c[0] * s.x + c[1] * s.y) + c[2] * s.z;
-    const double qy = (c[3] * s.x + c[4] * s.y) + c[5] * s.z;
-    const double qz = (c[6] * s.x + c[7] * s.y) + c[8] * s.z;
-    return dot3(s, h) + 0.5 * dot3(s, mk3(qx, qy, qz));
-}
-
-// sphereft: uniform in the cap of half-angle `cone` around s (cc = cos cone)
-__device__ __forceinline__ v3 mc_sphere(v3 s, double cc, double u1, double u2)
-{
-    const double ct = u1 + cc * (1.0 - u1);
-    const double st = sqrt(1.0 - ct * ct);
-    double sp, cp;
-    mj_sincos2pi(u2, &sp, &cp);
-    const double cti = s.z;
-    const double rr = s.x * s.x + s.y * s.y;
-    const double sti = sqrt(rr);
-    double cpi = 1.0, spi = 0.0;
-    if (!(rr < 0.00001)) {
-        cpi = s.x / sqrt(rr);
-        spi = s.y / sqrt(rr);
-    }
-    const double t = st * sp * cti + ct * sti;
-    const double ny = st * cp * cpi + t * spi;
-    const double nx = -(st * cp * spi) + t * cpi;
-    const double nz = -(st * sp * sti) + ct * cti;
-    const double ss = sqrt((nx * nx + ny * ny) + nz * nz);
-    return mk3(nx / ss, ny / ss, nz / ss);
-}
-
-// acceptance counters after a sweep (s accepted of n_done), and the cone for the
-// next sweep's n_next proposals (cone_update n_next times at the running rate)
-__device__ __forceinline__ void mc_fold_state(McState *st, double s, double n_done, double n_next, int adapt)
-{
-    const double acc = st->acc + s, nb = st->nb + n_done;
-    st->acc = acc;
-    st->nb = nb;
-    if (nb > 0.0) st->rate = acc / nb;
-    if (adapt && n_next > 0.0) {
-        const double pi = 3.14159265358979323846264338327950288;   // constant.f90:32
-        const double rate = st->rate;
-        double cone = st->cone;
-        if (rate > 0.5 && cone < pi) {
-            const double k = fmin(ceil((pi - cone) / 1.0e-4), n_next);
-            cone = cone + k * 1.0e-4;
-        } else if (rate < 0.5 && cone > 0.01) {
-            const double k = fmin(ceil((cone - 0.01) / 1.0e-4), n_next);
-            cone = cone - k * 1.0e-4;
-        }
-        st->cone = cone;
-        st->cos_cone = cos(cone);
-    }
-}
-
 constexpr int kMcTab = 2048;   // neighbour-slot table entries held in LDS
 
 // pair field of an interior row: neighbour slots from the table, x wrapped by +-W
@@ -392,27 +276,12 @@ __global__ void __launch_bounds__(kMcThreads) k_mc_pass(const McArgs a)
             const int64_t i = (int64_t)x + (int64_t)a.nx * row;
             const int64_t slot = (int64_t)a.color * a.ny * a.nz * a.W + t;
             const v3 s = mk3(cm[slot], cm[slot + a.cs], cm[slot + 2 * a.cs]);
-            uint32_t c[4] = {(uint32_t)i, (uint32_t)a.sweep, (uint32_t)(a.sweep >> 32), kMcStream + (uint32_t)rep};
-            philox4x32_10(c, (uint32_t)a.seed, (uint32_t)(a.seed >> 32));
-            const double two_m32 = 2.3283064365386962890625e-10;
-            v3 sn;
-            if (a.sampler == MJ_MC_ISING)
-                sn = mk3(-s.x, -s.y, -s.z);
-            else
-                sn = mc_sphere(s, st->cos_cone, (double)c[0] * two_m32, (double)c[1] * two_m32);
+            uint32_t c[4];
+            const v3 sn = mc_propose(a, rep, i, s, st->cos_cone, c);
             const bool interior = a.fast && y >= a.ylo && y < a.ny - a.yhi && z >= a.zlo && z < a.nz - a.zhi;
             const v3 pf = interior ? mc_pair_field_tab(a, cm, tab, x0, x, slot)
                                    : mc_pair_field_cm(a, cm, a.color, x0, jj, y, z, slot);
-            const v3 zf = mc_zeeman(a, a.cbmap, a.cs, slot);
-            const v3 h = mk3(pf.x + zf.x, pf.y + zf.y, pf.z + zf.z);
-            const double e_old = mc_site_energy(a, s, h);
-            const double e_new = mc_site_energy(a, sn, h);
-            const double de = e_new - e_old;
-            bool acc = de < 0.0;
-            if (!acc && kT > 0.0) {
-                const double tmp = fmax(-de / kT, -200.0);
-                acc = c[2] == 0u || mj_log01((double)c[2] * two_m32) < tmp;
-            }
+            const bool acc = mc_accept(a, s, sn, pf, slot, kT, c[2]);
             if (acc) {
                 cm[slot] = sn.x;
                 cm[slot + a.cs] = sn.y;
@@ -427,15 +296,20 @@ __global__ void __launch_bounds__(kMcThreads) k_mc_pass(const McArgs a)
 
 // acceptance counts of a sweep (the partials of its passes) and the cone of the next sweep
 // (one block per replica: state st[blockIdx.x], partials part + blockIdx.x * rep_part)
-__global__ void __launch_bounds__(kMcThreads) k_mc_fold(McState *st, const double *part, int nparts, int64_t rep_part,
-                                                        double n_done, double n_next, int adapt)
+__global__ void __launch_bounds__(kMcThreads) k_mc_fold(const McState *st_in, McState *st, const double *part,
+                                                        int nparts, int64_t rep_part, double n_done, double n_next,
+                                                        int adapt)
 {
     __shared__ double red[kMcThreads];
     const double *pp = part + blockIdx.x * rep_part;
     double v = 0.0;
     for (int b = threadIdx.x; b < nparts; b += blockDim.x) v += pp[b];
     const double tot = mj_block_sum(v, red, blockDim.x);
-    if (threadIdx.x == 0) mc_fold_state(st + blockIdx.x, tot, n_done, n_next, adapt);
+    if (threadIdx.x == 0) {
+        McState v1 = st_in[blockIdx.x];
+        mc_fold_state(&v1, tot, n_done, n_next, adapt);
+        st[blockIdx.x] = v1;
+    }
 }
 
 // site order <-> colour-major order of a 3-component SoA field
@@ -561,7 +435,7 @@ __global__ void k_mc_rep_samples(const double *E4, const int *image, int nrep, d
     }
 }
 
-// sum of the spins: per-block partials (3 per block), then one block
+// sum of the spins: per-block partials (3 per block), then one block per component
 __global__ void __launch_bounds__(kMcThreads) k_mc_msum(const double *m, int64_t n, int64_t np, double *part)
 {
     __shared__ double red[kMcThreads];
@@ -577,18 +451,21 @@ __global__ void __launch_bounds__(kMcThreads) k_mc_msum(const double *m, int64_t
 __global__ void __launch_bounds__(kMcThreads) k_mc_msum_final(const double *part, int nparts, double *out)
 {
     __shared__ double red[kMcThreads];
-    for (int c = 0; c < 3; ++c) {
-        double v = 0.0;
-        for (int i = threadIdx.x; i < nparts; i += blockDim.x) v += part[3 * i + c];
-        const double s = mj_block_sum(v, red, blockDim.x);
-        if (threadIdx.x == 0) out[c] = s;
-    }
+    const int c = blockIdx.x;
+    double v = 0.0;
+    for (int i = threadIdx.x; i < nparts; i += blockDim.x) v += part[3 * i + c];
+    const double s = mj_block_sum(v, red, blockDim.x);
+    if (threadIdx.x == 0) out[c] = s;
 }
 
 // ---------------------------------------------------------------------------
 // host side
 // ---------------------------------------------------------------------------
+static_assert(kMcIsing == MJ_MC_ISING, "sampler codes");
+
 struct McCtx {
+    hipFunction_t fn_pass = nullptr, fn_energy = nullptr;   // compiled for this stencil and lattice (null: ahead-of-time)
+    int resolved = 0;
     // stencil without the on-site entry, and the colouring it admits
     std::vector<int> o3;
     std::vector<double> cf;
@@ -856,8 +733,103 @@ static int mc_prepare(mj_ctx *c, const char *who)
     }
     mc->key_cf = c->h_cf;
     mc->key_o3 = c->h_ofs3;
+    mc->fn_pass = mc->fn_energy = nullptr;
+    mc->resolved = 0;
     return MJ_OK;
 }
+
+static int launch_check(const char *what)
+{
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) MJ_FAIL(MJ_EHIP, std::string(what) + ": " + hipGetErrorString(e));
+    return MJ_OK;
+}
+
+// The compiled kernels of passes over `sites` sites: from the size at which a
+// lattice gets compiled kernels (MJ_JIT=0 never, 1 always), where a class's
+// offsets and the slots fit 31 bits
+static int mc_resolve(mj_ctx *c, McCtx *mc, int64_t sites)
+{
+    const char *env = getenv("MJ_JIT");
+    const int64_t W = ceil_div(c->dim[0], mc->p), cs = (int64_t)mc->p * c->dim[1] * c->dim[2] * W;
+    const bool want = !(env && env[0] == '0') && ((env && env[0] == '1') || sites >= 4096) && cs < (1 << 28) &&
+                      (!c->periodic[0] || c->dim[0] % mc->p == 0);
+    if (!want) {
+        mc->fn_pass = mc->fn_energy = nullptr;
+        mc->resolved = 0;
+        return MJ_OK;
+    }
+    if (mc->resolved) return MJ_OK;
+    MJ_TRY(mj_jit_mc(c, mc->o3, mc->cf9, mc->csh, mc->p, mc->ca, mc->cb, &mc->fn_pass, &mc->fn_energy));
+    mc->resolved = 1;
+    return MJ_OK;
+}
+
+static int launch_kernel(hipFunction_t f, int64_t blocks, int nrep, hipStream_t st, McArgs &a, double *part)
+{
+    void *params[] = {&a, &part};
+    MJ_HIP_CHECK(hipModuleLaunchKernel(f, (unsigned)blocks, (unsigned)nrep, 1, kMcThreads, 1, 1, 0, st, params,
+                                       nullptr));
+    return MJ_OK;
+}
+
+// Sweeps of a call, one launch per colour class.  Ahead-of-time passes leave p
+// partials a block, folded into the state (counters, cone) by a launch after the
+// sweep; the compiled ones add up one, in two buffers taken in turn, and fold the
+// sweep before in their first pass, so that only the call's last sweep needs a
+// launch for it (k_mc_fold: 6.4 us of the 86 us of a sweep of 1024^2 in 8 classes).
+struct McSweeps {
+    mj_ctx *c;
+    McCtx *mc;
+    McState *st;          // nrep states, then nrep of the other buffer
+    double *part;         // rep_part per replica
+    int64_t nblocks;
+    int nrep, adapt;
+
+    McState *state(int s) const { return st + (s % 2) * nrep; }
+    double *parts(int s) const { return part + (s % 2) * nblocks; }
+
+    int begin(McArgs &a) const
+    {
+        a.st = st;
+        if (mc->fn_pass) return MJ_OK;
+        hipLaunchKernelGGL(k_mc_fold, dim3(nrep), dim3(kMcThreads), 0, c->stream, (const McState *)st, st,
+                           (const double *)part, 0, a.rep_part, 0.0, (double)c->n, adapt);
+        return launch_check("fold launch");
+    }
+
+    int sweep(McArgs &a, int s, bool last) const
+    {
+        const double nsite = (double)c->n;
+        for (int k = 0; k < mc->p; ++k) {
+            a.color = k;
+            if (mc->fn_pass) {
+                a.first = k == 0;
+                a.st_in = state(s);
+                a.st = state(s + 1);
+                a.acc_part = parts(s);
+                a.fold_part = parts(s + 1);
+                a.fold_n = s == 0 ? 0 : (int)nblocks;
+                a.n_done = s == 0 ? 0.0 : nsite;
+                a.n_next = nsite;
+                a.adapt = adapt;
+                MJ_TRY(launch_kernel(mc->fn_pass, nblocks, nrep, c->stream, a, nullptr));
+            } else {
+                a.tab = mc->fast ? mc->d_tab + (size_t)k * mc->p * a.ne : nullptr;
+                a.acc_part = part + (size_t)k * nblocks;
+                hipLaunchKernelGGL(k_mc_pass, dim3((unsigned)nblocks, (unsigned)nrep), dim3(kMcThreads), 0, c->stream, a);
+                MJ_TRY(launch_check("Monte Carlo pass launch"));
+            }
+        }
+        if (mc->fn_pass && !last) return MJ_OK;
+        const McState *in = mc->fn_pass ? state(s + 1) : st;
+        const double *p0 = mc->fn_pass ? parts(s) : part;
+        const int64_t n = mc->fn_pass ? nblocks : mc->p * nblocks;
+        hipLaunchKernelGGL(k_mc_fold, dim3(nrep), dim3(kMcThreads), 0, c->stream, in, st, p0, (int)n, a.rep_part, nsite,
+                           last ? 0.0 : nsite, adapt);
+        return launch_check("fold launch");
+    }
+};
 
 static void mc_args(const mj_ctx *c, const McCtx *mc, McArgs &a)
 {
@@ -903,13 +875,6 @@ static int ensure_part(McCtx *mc, int64_t n)
     mc->d_part = nullptr;
     MJ_HIP_CHECK(hipMalloc(&mc->d_part, sizeof(double) * (size_t)n));
     mc->part_cap = n;
-    return MJ_OK;
-}
-
-static int launch_check(const char *what)
-{
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) MJ_FAIL(MJ_EHIP, std::string(what) + ": " + hipGetErrorString(e));
     return MJ_OK;
 }
 
@@ -1037,6 +1002,7 @@ extern "C" int mj_mc_sweeps(mj_ctx *c, int nsweeps, int sampler, double kT, uint
     MJ_TRY(mc_prepare(c, "mj_mc_sweeps"));
     McCtx *mc = mc_of(c);
     if (nsweeps == 0) return MJ_OK;
+    MJ_TRY(mc_resolve(c, mc, c->n));
     const int adapt = sampler == MJ_MC_SPHERE ? 1 : 0;
     const int p = mc->p;
     McArgs a;
@@ -1046,8 +1012,9 @@ extern "C" int mj_mc_sweeps(mj_ctx *c, int nsweeps, int sampler, double kT, uint
     if (nblocks > INT32_MAX) MJ_FAIL(MJ_ENOTSUP, "mj_mc_sweeps: lattice too large");
     const int64_t msum_blocks = std::min<int64_t>(ceil_div(c->n, kMcThreads), 4096);
     if ((int64_t)p * nblocks > INT32_MAX) MJ_FAIL(MJ_ENOTSUP, "mj_mc_sweeps: lattice too large");
-    MJ_TRY(ensure_part(mc, (int64_t)p * nblocks + 3 * msum_blocks));
-    double *msum_part = mc->d_part + (size_t)p * nblocks;
+    const int64_t nparts = std::max(p, 2) * nblocks;
+    MJ_TRY(ensure_part(mc, nparts + 3 * msum_blocks));
+    double *msum_part = mc->d_part + nparts;
     if (nsamp > 0 && mc->samples_cap < 4 * nsamp) {
         if (mc->d_samples) hipFree(mc->d_samples);
         mc->d_samples = nullptr;
@@ -1081,34 +1048,19 @@ extern "C" int mj_mc_sweeps(mj_ctx *c, int nsweeps, int sampler, double kT, uint
                            (const double *)c->d_bmap, c->np, (double *)a.cbmap, a.cs, 1);
         MJ_TRY(launch_check("layout launch"));
     }
-    McState *st = mc->d_st;
-    const double nsite = (double)c->n;
-    // cone of the first sweep
-    hipLaunchKernelGGL(k_mc_fold, dim3(1), dim3(kMcThreads), 0, c->stream, st, (const double *)mc->d_part, 0,
-                       (int64_t)0, 0.0, nsite, adapt);
-    MJ_TRY(launch_check("fold launch"));
-    a.st = st;
+    const McSweeps sw = {c, mc, mc->d_st, mc->d_part, nblocks, 1, adapt};
+    MJ_TRY(sw.begin(a));
     int64_t js = 0;
     for (int s = 0; s < nsweeps; ++s) {
         a.sweep = sweep0 + (uint64_t)s;
-        for (int k = 0; k < p; ++k) {
-            a.color = k;
-            a.tab = mc->fast ? mc->d_tab + (size_t)k * p * a.ne : nullptr;
-            a.acc_part = mc->d_part + (size_t)k * nblocks;
-            hipLaunchKernelGGL(k_mc_pass, dim3((unsigned)nblocks), dim3(kMcThreads), 0, c->stream, a);
-            MJ_TRY(launch_check("Monte Carlo pass launch"));
-        }
-        const double n_next = s == nsweeps - 1 ? 0.0 : nsite;
-        hipLaunchKernelGGL(k_mc_fold, dim3(1), dim3(kMcThreads), 0, c->stream, st, (const double *)mc->d_part,
-                           (int)(p * nblocks), (int64_t)0, nsite, n_next, adapt);
-        MJ_TRY(launch_check("fold launch"));
+        MJ_TRY(sw.sweep(a, s, s == nsweeps - 1));
         if (measure_every > 0 && (s + 1) % measure_every == 0 && js < nsamp) {
             MJ_TRY(to_sites());
             MJ_TRY(mj_energy_into(c, mc->d_samples + js));
             hipLaunchKernelGGL(k_mc_msum, dim3((unsigned)msum_blocks), dim3(kMcThreads), 0, c->stream,
                                (const double *)c->A, c->n, c->np, msum_part);
             MJ_TRY(launch_check("spin sum launch"));
-            hipLaunchKernelGGL(k_mc_msum_final, dim3(1), dim3(kMcThreads), 0, c->stream, (const double *)msum_part,
+            hipLaunchKernelGGL(k_mc_msum_final, dim3(3), dim3(kMcThreads), 0, c->stream, (const double *)msum_part,
                                (int)msum_blocks, mc->d_samples + nsamp + 3 * js);
             MJ_TRY(launch_check("spin sum launch"));
             ++js;
@@ -1160,7 +1112,7 @@ extern "C" int mj_mc_pt_setup(mj_ctx *c, int nrep, const double *kT_ladder, doub
     mc_args(c, mc, a);
     const size_t rep_bytes = sizeof(double) * 3 * (size_t)a.cs;
     MJ_HIP_CHECK(hipMalloc(&mc->d_rcm, rep_bytes * nrep));
-    MJ_HIP_CHECK(hipMalloc(&mc->d_rst, sizeof(McState) * nrep));
+    MJ_HIP_CHECK(hipMalloc(&mc->d_rst, sizeof(McState) * 2 * nrep));
     MJ_HIP_CHECK(hipMalloc(&mc->d_rkT, sizeof(double) * nrep));
     MJ_HIP_CHECK(hipMalloc(&mc->d_ladder, sizeof(double) * nrep));
     MJ_HIP_CHECK(hipMalloc(&mc->d_image, sizeof(int) * nrep));
@@ -1210,6 +1162,7 @@ extern "C" int mj_mc_pt_sweeps(mj_ctx *c, int nsweeps, int sampler, uint64_t see
     if (nsamp > 0 && !E_samples && !M_samples) MJ_FAIL(MJ_EINVAL, "mj_mc_pt_sweeps: no sample array");
     if (nsweeps == 0) return MJ_OK;
     const int nrep = mc->nrep, p = mc->p;
+    MJ_TRY(mc_resolve(c, mc, c->n * nrep));
     const int adapt = sampler == MJ_MC_SPHERE ? 1 : 0;
     McArgs a;
     mc_args(c, mc, a);
@@ -1218,8 +1171,8 @@ extern "C" int mj_mc_pt_sweeps(mj_ctx *c, int nsweeps, int sampler, uint64_t see
     const int64_t eblocks = ceil_div((int64_t)p * c->dim[1] * c->dim[2] * a.W, kMcThreads);
     if (nblocks > INT32_MAX || eblocks > INT32_MAX || nrep > 65535)
         MJ_FAIL(MJ_ENOTSUP, "mj_mc_pt_sweeps: lattice or replica count too large");
-    const int64_t rep_part = (int64_t)p * nblocks;
-    const int64_t need = std::max<int64_t>(rep_part, 4 * eblocks) * nrep;
+    const int64_t rep_part = std::max(p, 2) * nblocks;
+    const int64_t need = (rep_part + 4 * eblocks) * nrep;
     if (mc->rpart_cap < need) {
         if (mc->d_rpart) hipFree(mc->d_rpart);
         mc->d_rpart = nullptr;
@@ -1252,34 +1205,27 @@ extern "C" int mj_mc_pt_sweeps(mj_ctx *c, int nsweeps, int sampler, uint64_t see
     a.nthreads = nthreads;
     a.seed = seed;
     a.sampler = sampler;
-    const double nsite = (double)c->n;
-    hipLaunchKernelGGL(k_mc_fold, dim3(nrep), dim3(kMcThreads), 0, c->stream, mc->d_rst, (const double *)mc->d_rpart,
-                       0, rep_part, 0.0, nsite, adapt);
-    MJ_TRY(launch_check("fold launch"));
+    const McSweeps sw = {c, mc, mc->d_rst, mc->d_rpart, nblocks, nrep, adapt};
+    MJ_TRY(sw.begin(a));
+    double *epart = mc->d_rpart + rep_part * nrep;
     auto energies = [&]() -> int {
         McArgs e = a;
         e.tab = mc->d_tab;
-        hipLaunchKernelGGL(k_mc_rep_energy, dim3((unsigned)eblocks, nrep), dim3(kMcThreads), 0, c->stream, e,
-                           mc->d_rpart);
-        MJ_TRY(launch_check("replica energy launch"));
-        hipLaunchKernelGGL(k_mc_rep_reduce, dim3(nrep), dim3(kMcThreads), 0, c->stream, (const double *)mc->d_rpart,
+        if (mc->fn_energy) {
+            MJ_TRY(launch_kernel(mc->fn_energy, eblocks, nrep, c->stream, e, epart));
+        } else {
+            hipLaunchKernelGGL(k_mc_rep_energy, dim3((unsigned)eblocks, nrep), dim3(kMcThreads), 0, c->stream, e,
+                               epart);
+            MJ_TRY(launch_check("replica energy launch"));
+        }
+        hipLaunchKernelGGL(k_mc_rep_reduce, dim3(nrep), dim3(kMcThreads), 0, c->stream, (const double *)epart,
                            (int)eblocks, mc->d_E4);
         return launch_check("replica energy launch");
     };
     int64_t js = 0;
     for (int s = 0; s < nsweeps; ++s) {
         a.sweep = sweep0 + (uint64_t)s;
-        for (int k = 0; k < p; ++k) {
-            a.color = k;
-            a.tab = mc->fast ? mc->d_tab + (size_t)k * p * a.ne : nullptr;
-            a.acc_part = mc->d_rpart + (size_t)k * nblocks;
-            hipLaunchKernelGGL(k_mc_pass, dim3((unsigned)nblocks, nrep), dim3(kMcThreads), 0, c->stream, a);
-            MJ_TRY(launch_check("Monte Carlo pass launch"));
-        }
-        const double n_next = s == nsweeps - 1 ? 0.0 : nsite;
-        hipLaunchKernelGGL(k_mc_fold, dim3(nrep), dim3(kMcThreads), 0, c->stream, mc->d_rst,
-                           (const double *)mc->d_rpart, (int)rep_part, rep_part, nsite, n_next, adapt);
-        MJ_TRY(launch_check("fold launch"));
+        MJ_TRY(sw.sweep(a, s, s == nsweeps - 1));
         const bool ex = exchange_every > 0 && (s + 1) % exchange_every == 0;
         const bool me = measure_every > 0 && (s + 1) % measure_every == 0 && js < nsamp;
         if (ex || me) MJ_TRY(energies());
