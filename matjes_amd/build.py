@@ -20,7 +20,8 @@ HIP_SOURCES = ["mj_api.hip", "mj_kernels.hip", "mj_fft.hip", "mj_jit.hip", "mj_a
 # device sources embedded as text for the per-Hamiltonian kernels compiled at set-up
 JIT_EMBED = [("kJitRngH", "mj_rngmath.h"), ("kJitDeviceH", "mj_device.h"), ("kJitKargsH", "mj_kargs.h"), ("kJitBodyH", "mj_stage_body.h"),
              ("kJitBatchH", "mj_batch_args.h"),
-             ("kJitMcH", "mj_mc_body.h")]
+             ("kJitMcH", "mj_mc_body.h"),
+             ("kJitAdjH", "mj_adj_body.h")]
 
 
 def gen_jit_embed():

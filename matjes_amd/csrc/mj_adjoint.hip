@@ -27,445 +27,51 @@
 
 #include "mj_device.h"
 #include "mj_internal.h"
-#include "mj_stage_body.h"   // mj_block_sum
+#include "mj_stage_body.h"   // mj_block_sum, fused_wrap
+#include "mj_adj_body.h"
 
-struct AdjArgs {
-    int nx, ny, nz, px, py, pz, bx, by, bz, rx, ry, rz, sx, sy, sz, ntx, nty, nblocks;
-    int64_t np;
-    int nofs;
-    const int *ofs;     // LDS offsets of the total stencil
-    const int *ofs0;    // the same in the fused step's S0 layout (tile + 2 reach)
-    const double *cf;   // 9 per offset (row-major C_d)
-    int nparam;
-    const int *pstart;  // unit stencils: entries [pstart[k], pstart[k+1]) of pofs/pcf
-    const int *pofs;
-    const double *pcf;
-    double z[9];
-    const double *bmap; // b_i (SoA)
-    double alpha, f;
-    // state
-    const double *x;    // stencil state of the kernel (SoA)
-    const double *x2;   // second stencil state (fused R3 + R1: the midpoint of the earlier step)
-    const double *m;    // own-site state m_n
-    const double *m1;   // own-site state m_{n+1}
-    const double *gin;  // own-site input gradient
-    const double *gacc_in, *gpd_in;
-    double *out0, *out1, *out2;
-    double *ghmap;
-    double *ppart;      // [nblocks][nparam + 3]
-};
+#define MJ_ADJ_MAXP kAdjMaxParam
 
-__device__ __forceinline__ v3 v_add(v3 a, v3 b) { return mk3(a.x + b.x, a.y + b.y, a.z + b.z); }
-__device__ __forceinline__ v3 v_scale(double s, v3 a) { return mk3(s * a.x, s * a.y, s * a.z); }
-
-// (I - [a]x + a a^T)^T ... M(-a) g = (g + a x g + (a.g) a) / (1 + |a|^2)
-__device__ __forceinline__ v3 minv_t(v3 a, v3 g)
-{
-    const v3 w = fma3(dot3(a, g), a, cross3_add(a, g, g));
-    return v_scale(mj_rcp(fma(a.z, a.z, fma(a.y, a.y, fma(a.x, a.x, 1.0)))), w);
-}
-
-__device__ __forceinline__ void adj_tile(const AdjArgs &a, const double *src, double *L, int x0, int y0, int z0)
-{
-    const int T = a.sx * a.sy * a.sz;
-    const int nthr = a.bx * a.by * a.bz;
-    for (int t = threadIdx.x; t < T; t += nthr) {
-        int lx = t % a.sx, r = t / a.sx, ly = r % a.sy, lz = r / a.sy;
-        int gx = x0 + lx - a.rx, gy = y0 + ly - a.ry, gz = z0 + lz - a.rz;
-        double vx = 0.0, vy = 0.0, vz = 0.0;
-        bool ok = true;
-        int g3[3] = {gx, gy, gz};
-        const int n3[3] = {a.nx, a.ny, a.nz}, p3[3] = {a.px, a.py, a.pz};
-        for (int d = 0; d < 3; ++d) {
-            if (g3[d] < 0 || g3[d] >= n3[d]) {
-                if (!p3[d]) ok = false;
-                g3[d] = ((g3[d] % n3[d]) + n3[d]) % n3[d];
-            }
-        }
-        if (ok) {
-            int64_t g = (int64_t)g3[0] + (int64_t)a.nx * ((int64_t)g3[1] + (int64_t)a.ny * g3[2]);
-            vx = src[g];
-            vy = src[g + a.np];
-            vz = src[g + 2 * a.np];
-        }
-        L[t] = vx;
-        L[T + t] = vy;
-        L[2 * T + t] = vz;
-    }
-}
-
-__device__ __forceinline__ v3 apply_blocks(const double *L, int T, int c, int n, const int *ofs, const double *cf)
-{
-    double ax = 0.0, ay = 0.0, az = 0.0;
-    for (int k = 0; k < n; ++k) {
-        const int j = c + ofs[k];
-        const double *q = cf + 9 * k;
-        const double mx = L[j], my = L[T + j], mz = L[2 * T + j];
-        ax = fma(q[0], mx, ax);
-        ax = fma(q[1], my, ax);
-        ax = fma(q[2], mz, ax);
-        ay = fma(q[3], mx, ay);
-        ay = fma(q[4], my, ay);
-        ay = fma(q[5], mz, ay);
-        az = fma(q[6], mx, az);
-        az = fma(q[7], my, az);
-        az = fma(q[8], mz, az);
-    }
-    return mk3(ax, ay, az);
-}
-
-struct Site {
-    int x0, y0, z0, c;
-    bool active;
-    int64_t gi;
-};
-
-__device__ __forceinline__ Site adj_site(const AdjArgs &a)
-{
-    Site s;
-    int bid = blockIdx.x;
-    int tx = bid % a.ntx, tr = bid / a.ntx, ty = tr % a.nty, tz = tr / a.nty;
-    s.x0 = tx * a.bx;
-    s.y0 = ty * a.by;
-    s.z0 = tz * a.bz;
-    int lx = threadIdx.x % a.bx, ly = (threadIdx.x / a.bx) % a.by, lz = threadIdx.x / (a.bx * a.by);
-    int gx = s.x0 + lx, gy = s.y0 + ly, gz = s.z0 + lz;
-    s.active = gx < a.nx && gy < a.ny && gz < a.nz;
-    s.gi = s.active ? (int64_t)gx + (int64_t)a.nx * ((int64_t)gy + (int64_t)a.ny * gz) : 0;
-    s.c = (lz + a.rz) * a.sx * a.sy + (ly + a.ry) * a.sx + (lx + a.rx);
-    return s;
-}
-
-__device__ __forceinline__ v3 ld3(const double *p, int64_t i, int64_t np) { return mk3(p[i], p[i + np], p[i + 2 * np]); }
-__device__ __forceinline__ void st3(double *p, int64_t i, int64_t np, v3 v)
-{
-    p[i] = v.x;
-    p[i + np] = v.y;
-    p[i + 2 * np] = v.z;
-}
-
-__device__ __forceinline__ v3 zeeman_t(const AdjArgs &a, int64_t gi)   // Z^T b_i
-{
-    v3 b = ld3(a.bmap, gi, a.np);
-    return mk3((b.x * a.z[0] + b.y * a.z[3]) + b.z * a.z[6], (b.x * a.z[1] + b.y * a.z[4]) + b.z * a.z[7],
-               (b.x * a.z[2] + b.y * a.z[5]) + b.z * a.z[8]);
-}
-
-__device__ __forceinline__ v3 zeeman_vjp(const AdjArgs &a, v3 g)   // -Z g
-{
-    return mk3(-((a.z[0] * g.x + a.z[1] * g.y) + a.z[2] * g.z), -((a.z[3] * g.x + a.z[4] * g.y) + a.z[5] * g.z),
-               -((a.z[6] * g.x + a.z[7] * g.y) + a.z[8] * g.z));
-}
-
-// per-block deterministic sums of nparam + 3 values, accumulated into
-// ppart[block][*]: every value's wavefront butterflies, one barrier, then
-// thread q adds value q's wave sums in wave order (mj_block_sum's order for
-// each value, without a barrier pair per value)
-__device__ __forceinline__ void adj_reduce(const AdjArgs &a, double *red, const double *vals, int nv)
-{
-    const int nthr = a.bx * a.by * a.bz;
-    __syncthreads();
-    if ((nthr & 63) != 0) {
-        for (int q = 0; q < nv; ++q) {
-            const double t = mj_block_sum(vals[q], red, nthr);
-            if (threadIdx.x == 0) a.ppart[(size_t)blockIdx.x * nv + q] += t;
-        }
-        return;
-    }
-    const int nw = nthr >> 6;
-    for (int q = 0; q < nv; ++q) {
-        double v = vals[q];
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) v = v + __shfl_xor(v, o, 64);
-        if ((threadIdx.x & 63) == 0) red[q * nw + (threadIdx.x >> 6)] = v;
-    }
-    __syncthreads();
-    if ((int)threadIdx.x < nv) {
-        const int q = threadIdx.x;
-        double r = red[q * nw];
-        for (int w = 1; w < nw; ++w) r = r + red[q * nw + w];
-        a.ppart[(size_t)blockIdx.x * nv + q] += r;
-    }
-}
-
-#define MJ_ADJ_MAXP 13
-
-// forward stage 1: p = (m + cay(m, a1(m)))/2
 __global__ void k_adj_sib1(const AdjArgs a)
 {
     extern __shared__ double L[];
-    Site s = adj_site(a);
-    adj_tile(a, a.x, L, s.x0, s.y0, s.z0);
-    __syncthreads();
-    if (!s.active) return;
-    const int T = a.sx * a.sy * a.sz;
-    v3 m = mk3(L[s.c], L[T + s.c], L[2 * T + s.c]);
-    v3 acc = apply_blocks(L, T, s.c, a.nofs, a.ofs, a.cf);
-    v3 zb = zeeman_t(a, s.gi);
-    v3 B = mk3(-(acc.x + zb.x), -(acc.y + zb.y), -(acc.z + zb.z));
-    v3 c = cross3(m, B);
-    st3(a.out0, s.gi, a.np, cayley_mid(m, v_scale(a.f, fma3(a.alpha, c, B))));
+    adj_sib1_body<AdjRt>(a, L);
 }
 
-// forward stage 2: m' = cay(m, a2(p))
 __global__ void k_adj_sib2(const AdjArgs a)
 {
     extern __shared__ double L[];
-    Site s = adj_site(a);
-    adj_tile(a, a.x, L, s.x0, s.y0, s.z0);
-    __syncthreads();
-    if (!s.active) return;
-    const int T = a.sx * a.sy * a.sz;
-    v3 p = mk3(L[s.c], L[T + s.c], L[2 * T + s.c]);
-    v3 acc = apply_blocks(L, T, s.c, a.nofs, a.ofs, a.cf);
-    v3 zb = zeeman_t(a, s.gi);
-    v3 B = mk3(-(acc.x + zb.x), -(acc.y + zb.y), -(acc.z + zb.z));
-    v3 c = cross3(p, B);
-    v3 av = v_scale(a.f, fma3(a.alpha, c, B));
-    st3(a.out0, s.gi, a.np, cayley(ld3(a.m, s.gi, a.np), av));
+    adj_sib2_body<AdjRt>(a, L);
 }
 
-// lattice site of a region position (wrapped on periodic axes; false off an open edge)
-__device__ __forceinline__ bool adj_site_of(const AdjArgs &a, int gx, int gy, int gz, int64_t &g)
-{
-    int g3[3] = {gx, gy, gz};
-    const int n3[3] = {a.nx, a.ny, a.nz}, p3[3] = {a.px, a.py, a.pz};
-    for (int d = 0; d < 3; ++d) {
-        if (g3[d] < 0 || g3[d] >= n3[d]) {
-            if (!p3[d]) return false;
-            g3[d] = ((g3[d] % n3[d]) + n3[d]) % n3[d];
-        }
-    }
-    g = (int64_t)g3[0] + (int64_t)a.nx * ((int64_t)g3[1] + (int64_t)a.ny * g3[2]);
-    return true;
-}
-
-// the midpoint p of SIB's first stage at one site from the S0 tile
-__device__ __forceinline__ v3 adj_midpoint(const AdjArgs &a, const double *L0, int T0, int c0, int64_t gi, v3 &m)
-{
-    m = mk3(L0[c0], L0[T0 + c0], L0[2 * T0 + c0]);
-    v3 acc = apply_blocks(L0, T0, c0, a.nofs, a.ofs0, a.cf);
-    v3 zb = zeeman_t(a, gi);
-    v3 B = mk3(-(acc.x + zb.x), -(acc.y + zb.y), -(acc.z + zb.z));
-    v3 c = cross3(m, B);
-    return cayley_mid(m, v_scale(a.f, fma3(a.alpha, c, B)));
-}
-
-// a whole forward step in one kernel: the tile plus twice the reach (S0) in
-// LDS, the midpoint on the tile plus the reach (S1: the tile's own sites and
-// a ring repeating the neighbouring tiles' first stage with the same
-// operations), the second stage on the tile.  out0 = the midpoint p (kept for
-// the reverse sweep), out1 = m'; bit for bit k_adj_sib1 then k_adj_sib2.
 __global__ void k_adj_sibf(const AdjArgs a)
 {
     extern __shared__ double L[];
-    const int s0x = a.bx + 4 * a.rx, s0y = a.by + 4 * a.ry, s0z = a.bz + 4 * a.rz, T0 = s0x * s0y * s0z;
-    const int T1 = a.sx * a.sy * a.sz;
-    const int nthr = a.bx * a.by * a.bz;
-    double *L0 = L;
-    double *L1 = L + 3 * T0;
-    Site s = adj_site(a);
-    for (int t = threadIdx.x; t < T0; t += nthr) {
-        const int lx = t % s0x, r = t / s0x, ly = r % s0y, lz = r / s0y;
-        int64_t g = 0;
-        double vx = 0.0, vy = 0.0, vz = 0.0;
-        if (adj_site_of(a, s.x0 + lx - 2 * a.rx, s.y0 + ly - 2 * a.ry, s.z0 + lz - 2 * a.rz, g)) {
-            vx = a.x[g];
-            vy = a.x[g + a.np];
-            vz = a.x[g + 2 * a.np];
-        }
-        L0[t] = vx;
-        L0[T0 + t] = vy;
-        L0[2 * T0 + t] = vz;
-    }
-    __syncthreads();
-    const int lx = threadIdx.x % a.bx, ly = (threadIdx.x / a.bx) % a.by, lz = threadIdx.x / (a.bx * a.by);
-    v3 m0 = mk3(0.0, 0.0, 0.0);
-    {
-        int64_t gw = 0;
-        v3 p = mk3(0.0, 0.0, 0.0);
-        if (adj_site_of(a, s.x0 + lx, s.y0 + ly, s.z0 + lz, gw)) {
-            const int c0 = (lz + 2 * a.rz) * s0x * s0y + (ly + 2 * a.ry) * s0x + (lx + 2 * a.rx);
-            p = adj_midpoint(a, L0, T0, c0, gw, m0);
-        }
-        L1[s.c] = p.x;
-        L1[T1 + s.c] = p.y;
-        L1[2 * T1 + s.c] = p.z;
-    }
-    // the ring of S1: z slabs, then y slabs of the tile's planes, then x slabs of its rows
-    const int nzs = 2 * a.rz * a.sx * a.sy, nys = 2 * a.ry * a.bz * a.sx;
-    for (int k = threadIdx.x; k < T1 - nthr; k += nthr) {
-        int sx, sy, sz;
-        if (k < nzs) {
-            const int plane = k / (a.sx * a.sy), rem = k % (a.sx * a.sy);
-            sz = plane < a.rz ? plane : plane + a.bz;
-            sy = rem / a.sx;
-            sx = rem % a.sx;
-        } else if (k < nzs + nys) {
-            const int q = k - nzs, row = q / a.sx, yy = row % (2 * a.ry);
-            sz = a.rz + row / (2 * a.ry);
-            sy = yy < a.ry ? yy : yy + a.by;
-            sx = q % a.sx;
-        } else {
-            const int q = k - nzs - nys, col = q % (2 * a.rx), row = q / (2 * a.rx);
-            sy = a.ry + row % a.by;
-            sz = a.rz + row / a.by;
-            sx = col < a.rx ? col : col + a.bx;
-        }
-        const int c1 = sz * a.sx * a.sy + sy * a.sx + sx;
-        int64_t gw = 0;
-        v3 p = mk3(0.0, 0.0, 0.0);
-        if (adj_site_of(a, s.x0 - a.rx + sx, s.y0 - a.ry + sy, s.z0 - a.rz + sz, gw)) {
-            const int c0 = (sz + a.rz) * s0x * s0y + (sy + a.ry) * s0x + (sx + a.rx);
-            v3 mm;
-            p = adj_midpoint(a, L0, T0, c0, gw, mm);
-        }
-        L1[c1] = p.x;
-        L1[T1 + c1] = p.y;
-        L1[2 * T1 + c1] = p.z;
-    }
-    __syncthreads();
-    if (!s.active) return;
-    v3 p = mk3(L1[s.c], L1[T1 + s.c], L1[2 * T1 + s.c]);
-    v3 acc = apply_blocks(L1, T1, s.c, a.nofs, a.ofs, a.cf);
-    v3 zb = zeeman_t(a, s.gi);
-    v3 B = mk3(-(acc.x + zb.x), -(acc.y + zb.y), -(acc.z + zb.z));
-    v3 c = cross3(p, B);
-    v3 av = v_scale(a.f, fma3(a.alpha, c, B));
-    st3(a.out0, s.gi, a.np, p);
-    st3(a.out1, s.gi, a.np, cayley(m0, av));
-}
-
-// R1: reverse of the stage-2 site math.  x = p (stencil), m, m1 = m', gin = g'.
-// out0 = gB2, out1 = gacc (cay(g', -a2)), out2 = gp_direct
-// R1 site algebra: the midpoint tile p is in L, g = dL/dm' at the own site
-__device__ __forceinline__ void r1_site(const AdjArgs &a, const double *L, int T, const Site &s, v3 g, double *vals)
-{
-    {
-        v3 p = mk3(L[s.c], L[T + s.c], L[2 * T + s.c]);
-        v3 acc = apply_blocks(L, T, s.c, a.nofs, a.ofs, a.cf);
-        v3 zb = zeeman_t(a, s.gi);
-        v3 B = mk3(-(acc.x + zb.x), -(acc.y + zb.y), -(acc.z + zb.z));
-        v3 c = cross3(p, B);
-        v3 av = v_scale(a.f, fma3(a.alpha, c, B));
-        v3 m = ld3(a.m, s.gi, a.np), m1 = ld3(a.m1, s.gi, a.np);
-        v3 gm = cayley(g, mk3(-av.x, -av.y, -av.z));
-        v3 w = minv_t(av, g);
-        v3 ga = cross3(w, v_add(m1, m));
-        v3 gB = v_scale(a.f, v_add(ga, v_scale(a.alpha, cross3(ga, p))));
-        v3 gp = v_scale(a.f * a.alpha, cross3(B, ga));
-        st3(a.out0, s.gi, a.np, gB);
-        st3(a.out1, s.gi, a.np, gm);
-        st3(a.out2, s.gi, a.np, gp);
-        for (int k = 0; k < a.nparam; ++k) {
-            v3 u = apply_blocks(L, T, s.c, a.pstart[k + 1] - a.pstart[k], a.pofs + a.pstart[k], a.pcf + 9 * a.pstart[k]);
-            vals[k] = -dot3(gB, u);
-        }
-        v3 gb = zeeman_vjp(a, gB);
-        vals[a.nparam] = gb.x;
-        vals[a.nparam + 1] = gb.y;
-        vals[a.nparam + 2] = gb.z;
-        st3(a.ghmap, s.gi, a.np, v_add(ld3(a.ghmap, s.gi, a.np), gb));
-    }
+    adj_sibf_body<AdjRt>(a, L);
 }
 
 __global__ void k_adj_r1(const AdjArgs a)
 {
     extern __shared__ double L[];
-    const int T = a.sx * a.sy * a.sz;
-    double *red = L + 3 * T;
-    Site s = adj_site(a);
-    adj_tile(a, a.x, L, s.x0, s.y0, s.z0);
-    __syncthreads();
-    double vals[MJ_ADJ_MAXP + 3];
-    for (int q = 0; q < a.nparam + 3; ++q) vals[q] = 0.0;
-    if (s.active) r1_site(a, L, T, s, ld3(a.gin, s.gi, a.np), vals);
-    adj_reduce(a, red, vals, a.nparam + 3);
+    adj_r1_body<AdjRt>(a, L);
 }
 
-// R3 of step q fused with R1 of step q-1: lambda_q = gacc - C * gB1 at the own
-// site (tile of gB1 in x), then the stage-2 reverse of step q-1 with
-// g = lambda_q (tile of its midpoint in x2); lambda_q never goes to memory
 __global__ void k_adj_r3r1(const AdjArgs a)
 {
     extern __shared__ double L[];
-    const int T = a.sx * a.sy * a.sz;
-    double *LP = L + 3 * T;
-    double *red = L + 6 * T;
-    Site s = adj_site(a);
-    adj_tile(a, a.x, L, s.x0, s.y0, s.z0);
-    adj_tile(a, a.x2, LP, s.x0, s.y0, s.z0);
-    __syncthreads();
-    double vals[MJ_ADJ_MAXP + 3];
-    for (int q = 0; q < a.nparam + 3; ++q) vals[q] = 0.0;
-    if (s.active) {
-        const v3 t = apply_blocks(L, T, s.c, a.nofs, a.ofs, a.cf);
-        const v3 g = ld3(a.gacc_in, s.gi, a.np);
-        r1_site(a, LP, T, s, mk3(g.x - t.x, g.y - t.y, g.z - t.z), vals);
-    }
-    adj_reduce(a, red, vals, a.nparam + 3);
+    adj_r3r1_body<AdjRt>(a, L);
 }
 
-// R2: transpose of the stage-2 field (stencil over gB2 in x) + reverse of the
-// stage-1 site math (needs the stencil of m: second tile).
-// gin = gB2 is x; m stencil read from a.m; gacc_in, gpd_in own.
-// out0 = gB1, out1 = gacc2
 __global__ void k_adj_r2(const AdjArgs a)
 {
     extern __shared__ double L[];
-    const int T = a.sx * a.sy * a.sz;
-    double *LM = L + 3 * T;
-    double *red = L + 6 * T;
-    Site s = adj_site(a);
-    adj_tile(a, a.x, L, s.x0, s.y0, s.z0);
-    adj_tile(a, a.m, LM, s.x0, s.y0, s.z0);
-    __syncthreads();
-    double vals[MJ_ADJ_MAXP + 3];
-    for (int q = 0; q < a.nparam + 3; ++q) vals[q] = 0.0;
-    if (s.active) {
-        v3 tgb = apply_blocks(L, T, s.c, a.nofs, a.ofs, a.cf);
-        v3 gp = mk3(a.gpd_in[s.gi] - tgb.x, a.gpd_in[s.gi + a.np] - tgb.y, a.gpd_in[s.gi + 2 * a.np] - tgb.z);
-        v3 gmt = v_scale(0.5, gp);
-        v3 gm = v_add(ld3(a.gacc_in, s.gi, a.np), gmt);
-        v3 m = mk3(LM[s.c], LM[T + s.c], LM[2 * T + s.c]);
-        v3 acc = apply_blocks(LM, T, s.c, a.nofs, a.ofs, a.cf);
-        v3 zb = zeeman_t(a, s.gi);
-        v3 B = mk3(-(acc.x + zb.x), -(acc.y + zb.y), -(acc.z + zb.z));
-        v3 c = cross3(m, B);
-        v3 av = v_scale(a.f, fma3(a.alpha, c, B));
-        v3 mt = cayley(m, av);
-        gm = v_add(gm, cayley(gmt, mk3(-av.x, -av.y, -av.z)));
-        v3 w = minv_t(av, gmt);
-        v3 ga = cross3(w, v_add(mt, m));
-        v3 gB = v_scale(a.f, v_add(ga, v_scale(a.alpha, cross3(ga, m))));
-        gm = v_add(gm, v_scale(a.f * a.alpha, cross3(B, ga)));
-        st3(a.out0, s.gi, a.np, gB);
-        st3(a.out1, s.gi, a.np, gm);
-        for (int k = 0; k < a.nparam; ++k) {
-            v3 u = apply_blocks(LM, T, s.c, a.pstart[k + 1] - a.pstart[k], a.pofs + a.pstart[k], a.pcf + 9 * a.pstart[k]);
-            vals[k] = -dot3(gB, u);
-        }
-        v3 gb = zeeman_vjp(a, gB);
-        vals[a.nparam] = gb.x;
-        vals[a.nparam + 1] = gb.y;
-        vals[a.nparam + 2] = gb.z;
-        st3(a.ghmap, s.gi, a.np, v_add(ld3(a.ghmap, s.gi, a.np), gb));
-    }
-    adj_reduce(a, red, vals, a.nparam + 3);
+    adj_r2_body<AdjRt>(a, L);
 }
 
-// R3: lambda_n = gacc2 - C * gB1   (x = gB1)
 __global__ void k_adj_r3(const AdjArgs a)
 {
     extern __shared__ double L[];
-    const int T = a.sx * a.sy * a.sz;
-    Site s = adj_site(a);
-    adj_tile(a, a.x, L, s.x0, s.y0, s.z0);
-    __syncthreads();
-    if (!s.active) return;
-    v3 t = apply_blocks(L, T, s.c, a.nofs, a.ofs, a.cf);
-    v3 g = ld3(a.gacc_in, s.gi, a.np);
-    st3(a.out0, s.gi, a.np, mk3(g.x - t.x, g.y - t.y, g.z - t.z));
+    adj_r3_body<AdjRt>(a, L);
 }
 
 __global__ void k_adj_bmap(const double *bext, const double *h_aos, double *bmap, int64_t n, int64_t np)
@@ -497,6 +103,8 @@ struct AdjState {
     int *d_ofs0 = nullptr;           // the total stencil in the fused step's S0 layout (null: two kernels per step)
     size_t shm_fused = 0;
     double *d_cf = nullptr, *d_pcf = nullptr;
+    double *d_cls = nullptr;         // compiled kernels: the total stencil's distinct values
+    hipFunction_t fn[MJ_ADJ_KERNELS] = {};   // (null: ahead-of-time)
     double *d_bext = nullptr, *d_bmap = nullptr;
     double *ckpt = nullptr;          // ncp * 3np
     double *segm = nullptr, *segp = nullptr;   // (ckpt + 1) * 3np and ckpt * 3np
@@ -525,8 +133,8 @@ static void adj_free(AdjState *s)
     int *ip[] = {s->d_ofs, s->d_pstart, s->d_pofs, s->d_ofs0};
     for (int *p : ip)
         if (p) hipFree(p);
-    double *dp[] = {s->d_cf, s->d_pcf, s->d_bext, s->d_bmap, s->ckpt, s->segm, s->segp, s->g, s->gB, s->gacc,
-                    s->gpd, s->ghmap, s->ppart};
+    double *dp[] = {s->d_cf, s->d_pcf, s->d_cls, s->d_bext, s->d_bmap, s->ckpt, s->segm, s->segp,
+                    s->g, s->gB, s->gacc, s->gpd, s->ghmap, s->ppart};
     for (double *p : dp)
         if (p) hipFree(p);
 }
@@ -612,9 +220,6 @@ static void adj_args(const mj_ctx *c, const AdjState *s, AdjArgs &a)
     a.rx = s->rx;
     a.ry = s->ry;
     a.rz = s->rz;
-    a.sx = a.bx + 2 * a.rx;
-    a.sy = a.by + 2 * a.ry;
-    a.sz = a.bz + 2 * a.rz;
     a.ntx = (a.nx + a.bx - 1) / a.bx;
     a.nty = (a.ny + a.by - 1) / a.by;
     a.nblocks = a.ntx * a.nty * ((a.nz + a.bz - 1) / a.bz);
@@ -623,6 +228,7 @@ static void adj_args(const mj_ctx *c, const AdjState *s, AdjArgs &a)
     a.ofs = s->d_ofs;
     a.ofs0 = s->d_ofs0;
     a.cf = s->d_cf;
+    a.cls = s->d_cls;
     a.nparam = s->nparam;
     a.pstart = s->d_pstart;
     a.pofs = s->d_pofs;
@@ -633,16 +239,26 @@ static void adj_args(const mj_ctx *c, const AdjState *s, AdjArgs &a)
     a.f = -0.5 * s->dt / ((1.0 + s->alpha * s->alpha) * MJ_HBAR);
 }
 
-static int adj_launch(void (*k)(const AdjArgs), const AdjArgs &a, int ntiles, hipStream_t st)
+static int adj_launch(const AdjState *s, int kind, const AdjArgs &a, int ntiles, hipStream_t st)
 {
-    const int T = a.sx * a.sy * a.sz;
+    const int T = (a.bx + 2 * a.rx) * (a.by + 2 * a.ry) * (a.bz + 2 * a.rz);
     const int nthr = a.bx * a.by * a.bz;
     size_t shm = sizeof(double) * ((size_t)3 * T * ntiles + nthr);
-    if (shm > 65536) {
+    if (kind != MJ_ADJ_SIBF && shm > 65536) {
         mj_set_error("adjoint: the stencil reach needs more LDS than a workgroup has");
         return MJ_ENOTSUP;
     }
-    hipLaunchKernelGGL(k, dim3(a.nblocks), dim3(nthr), shm, st, a);
+    if (kind == MJ_ADJ_SIBF) shm = s->shm_fused;
+    if (s->fn[kind]) {
+        AdjArgs arg = a;
+        void *params[] = {&arg};
+        MJ_HIP_CHECK(hipModuleLaunchKernel(s->fn[kind], (unsigned)a.nblocks, 1, 1, (unsigned)nthr, 1, 1, (unsigned)shm, st,
+                                           params, nullptr));
+        return MJ_OK;
+    }
+    void (*const aot[MJ_ADJ_KERNELS])(const AdjArgs) = {k_adj_sib1, k_adj_sib2, k_adj_sibf, k_adj_r1,
+                                                        k_adj_r2,   k_adj_r3r1, k_adj_r3};
+    hipLaunchKernelGGL(aot[kind], dim3(a.nblocks), dim3(nthr), shm, st, a);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) {
         mj_set_error(std::string("adjoint kernel launch: ") + hipGetErrorString(e));
@@ -668,6 +284,65 @@ static int adj_alloc(double **p, size_t n)
     return MJ_OK;
 }
 
+// The kernels compiled for the parameter set (mj_jit_adjoint), from the size at
+// which a lattice gets compiled kernels (MJ_JIT=0 never, 1 always).  The values
+// of the total stencil change with theta, its structure does not: places with
+// the same unit coefficients in every parameter (up to one sign) hold the same
+// value, places with none hold zero.  More than 64 values, or places whose sums
+// round differently, keep the ahead-of-time kernels.
+static int adj_compile(mj_ctx *c, AdjState *s, const std::vector<std::array<int, 3>> &offs,
+                       const std::vector<std::array<double, 9>> &C,
+                       const std::vector<std::vector<std::array<int, 3>>> &poffs,
+                       const std::vector<std::vector<std::array<double, 9>>> &pC)
+{
+    for (auto &f : s->fn) f = nullptr;
+    const char *env = getenv("MJ_JIT");
+    if ((env && env[0] == '0') || (!(env && env[0] == '1') && c->n < 4096)) return MJ_OK;
+    AdjStencil st;
+    std::vector<std::vector<double>> keys;
+    std::vector<double> vals;
+    for (size_t e = 0; e < offs.size(); ++e) {
+        st.o3.insert(st.o3.end(), offs[e].begin(), offs[e].end());
+        for (int q = 0; q < 9; ++q) {
+            std::vector<double> key(s->nparam, 0.0);
+            for (int k = 0; k < s->nparam; ++k)
+                for (size_t j = 0; j < poffs[k].size(); ++j)
+                    if (poffs[k][j] == offs[e]) key[k] = pC[k][j][q];
+            double lead = 0.0;
+            for (double v : key)
+                if (lead == 0.0) lead = v;
+            if (lead == 0.0) {
+                if (C[e][q] != 0.0) return MJ_OK;
+                st.cls.push_back(0);
+                continue;
+            }
+            const double sign = lead < 0.0 ? -1.0 : 1.0;
+            for (double &v : key) v = sign * v + 0.0;
+            size_t i = std::find(keys.begin(), keys.end(), key) - keys.begin();
+            if (i == keys.size()) {
+                keys.push_back(key);
+                vals.push_back(sign * C[e][q]);
+            }
+            if (vals[i] != sign * C[e][q]) return MJ_OK;
+            st.cls.push_back((int)sign * (int)(i + 1));
+        }
+    }
+    if (vals.size() > 64) return MJ_OK;
+    for (int k = 0; k < s->nparam; ++k) {
+        st.po3.emplace_back();
+        st.pblk.emplace_back();
+        for (size_t j = 0; j < poffs[k].size(); ++j) {
+            st.po3[k].insert(st.po3[k].end(), poffs[k][j].begin(), poffs[k][j].end());
+            st.pblk[k].insert(st.pblk[k].end(), pC[k][j].begin(), pC[k][j].end());
+        }
+    }
+    const int b[3] = {s->bx, s->by, s->bz}, r[3] = {s->rx, s->ry, s->rz};
+    ATRY(adj_alloc(&s->d_cls, vals.size()));
+    if (!vals.empty())
+        MJ_HIP_CHECK(hipMemcpy(s->d_cls, vals.data(), sizeof(double) * vals.size(), hipMemcpyHostToDevice));
+    return mj_jit_adjoint(c, st, b, r, s->d_ofs0 != nullptr, s->fn);
+}
+
 // one forward SIB step from x_in to x_out (SoA), storing the midpoint in pbuf:
 // one fused kernel when its tiles fit, else the two stage kernels
 static int adj_step(mj_ctx *c, AdjState *s, const double *xin, double *pbuf, double *xout)
@@ -678,19 +353,13 @@ static int adj_step(mj_ctx *c, AdjState *s, const double *xin, double *pbuf, dou
     a.out0 = pbuf;
     if (s->d_ofs0) {
         a.out1 = xout;
-        hipLaunchKernelGGL(k_adj_sibf, dim3(a.nblocks), dim3(a.bx * a.by * a.bz), s->shm_fused, c->stream, a);
-        hipError_t e = hipGetLastError();
-        if (e != hipSuccess) {
-            mj_set_error(std::string("adjoint fused step launch: ") + hipGetErrorString(e));
-            return MJ_EHIP;
-        }
-        return MJ_OK;
+        return adj_launch(s, MJ_ADJ_SIBF, a, 1, c->stream);
     }
-    ATRY(adj_launch(k_adj_sib1, a, 1, c->stream));
+    ATRY(adj_launch(s, MJ_ADJ_SIB1, a, 1, c->stream));
     a.x = pbuf;
     a.m = xin;
     a.out0 = xout;
-    return adj_launch(k_adj_sib2, a, 1, c->stream);
+    return adj_launch(s, MJ_ADJ_SIB2, a, 1, c->stream);
 }
 
 // `len` steps of one segment: segm[q] -> (segp[q], segm[q+1]); a full segment
@@ -822,6 +491,7 @@ extern "C" int mj_adjoint_forward(mj_ctx *c, const double *theta, const double *
         MJ_HIP_CHECK(hipMemcpy(s->d_pofs, hpofs.data(), sizeof(int) * hpofs.size(), hipMemcpyHostToDevice));
         MJ_HIP_CHECK(hipMemcpy(s->d_pcf, hpcf.data(), sizeof(double) * hpcf.size(), hipMemcpyHostToDevice));
     }
+    ATRY(adj_compile(c, s, offs, C, poffs, pC));
     // buffers
     const size_t n3 = 3 * (size_t)c->np;
     s->ncp = (nsteps + ckpt_every - 1) / ckpt_every;
@@ -873,7 +543,7 @@ static int adj_segment_rev(mj_ctx *c, AdjState *s, int len)
             a.out0 = gB2;
             a.out1 = s->gacc;
             a.out2 = s->gpd;
-            ATRY(adj_launch(k_adj_r1, a, 1, c->stream));
+            ATRY(adj_launch(s, MJ_ADJ_R1, a, 1, c->stream));
         }
         for (int q = n - 1; q >= 0; --q) {
             AdjArgs b = a0;          // R2: transpose of the stage-2 field + stage-1 site math
@@ -883,7 +553,7 @@ static int adj_segment_rev(mj_ctx *c, AdjState *s, int len)
             b.gpd_in = s->gpd;
             b.out0 = gB1;
             b.out1 = s->gacc;        // own-site read-then-write
-            ATRY(adj_launch(k_adj_r2, b, 2, c->stream));
+            ATRY(adj_launch(s, MJ_ADJ_R2, b, 2, c->stream));
             if (q > 0) {             // R3 of step q + R1 of step q-1
                 AdjArgs f = a0;
                 f.x = gB1;
@@ -894,7 +564,7 @@ static int adj_segment_rev(mj_ctx *c, AdjState *s, int len)
                 f.out0 = gB2;
                 f.out1 = s->gacc;    // own-site read-then-write
                 f.out2 = s->gpd;
-                ATRY(adj_launch(k_adj_r3r1, f, 2, c->stream));
+                ATRY(adj_launch(s, MJ_ADJ_R3R1, f, 2, c->stream));
             } else {                 // R3 of the segment's first step: lambda to memory
                 AdjArgs r = a0;
                 r.ppart = nullptr;
@@ -902,7 +572,7 @@ static int adj_segment_rev(mj_ctx *c, AdjState *s, int len)
                 r.x = gB1;
                 r.gacc_in = s->gacc;
                 r.out0 = s->g;
-                ATRY(adj_launch(k_adj_r3, r, 1, c->stream));
+                ATRY(adj_launch(s, MJ_ADJ_R3, r, 1, c->stream));
             }
         }
         return MJ_OK;

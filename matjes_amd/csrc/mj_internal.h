@@ -110,6 +110,16 @@ int mj_jit_launch(mj_ctx *c, int mode, bool noise, const KArgs &a, hipStream_t s
 int mj_jit_resolve(mj_ctx *c, int mode, bool noise);
 int mj_jit_fused_ok(const mj_ctx *c);   // the fused integration-2 kernel was generated
 void mj_jit_destroy(mj_ctx *c);
+// kernels of the differentiable SIB trajectory for a parameter set's stencil: offsets (3 per entry) and value
+// classes (9 per entry: 0 zero, +-k the k-th value or its negative), the parameters' unit stencils (offsets, blocks)
+enum { MJ_ADJ_SIB1, MJ_ADJ_SIB2, MJ_ADJ_SIBF, MJ_ADJ_R1, MJ_ADJ_R2, MJ_ADJ_R3R1, MJ_ADJ_R3, MJ_ADJ_KERNELS };
+struct AdjStencil {
+    std::vector<int> o3, cls;
+    std::vector<std::vector<int>> po3;
+    std::vector<std::vector<double>> pblk;
+};
+int mj_jit_adjoint(const mj_ctx *c, const AdjStencil &st, const int b[3], const int r[3], bool fused,
+                   hipFunction_t fn[MJ_ADJ_KERNELS]);
 // Monte Carlo kernels of a stencil without its on-site entry (offsets o3, full blocks cf9, class shifts csh) on the
 // context's lattice coloured (x + ca y + cb z) mod p
 int mj_jit_mc(const mj_ctx *c, const std::vector<int> &o3, const std::vector<double> &cf9, const std::vector<int> &csh,

@@ -405,6 +405,94 @@ int mj_jit_batch_fused(const std::vector<int> &ofs3, const std::vector<int> &cls
     return MJ_OK;
 }
 
+// The differentiable SIB trajectory's kernels for a parameter set: lattice, tile
+// and stencils compile-time, the values (they change with the parameters) from
+// scalar registers; terms in the order of apply_blocks, structural zeros left
+// out.  Latency bounds them on the lattices they are used for (one wavefront a
+// workgroup at 128^2): the halo's wraps and the table of offsets went, all of a
+// workgroup's loads are in flight before its first store to LDS.  128^2, 4
+// neighbours, 3 parameters: forward step 7.9 -> 4.2 us, R2 11.1 -> 4.8, R3 with
+// R1 11.2 -> 4.9.
+int mj_jit_adjoint(const mj_ctx *c, const AdjStencil &st, const int b[3], const int r[3], bool fused,
+                   hipFunction_t fn[MJ_ADJ_KERNELS])
+{
+    std::ostringstream g;
+    const int nthr = b[0] * b[1] * b[2];
+    int s1[3], s0[3];
+    for (int d = 0; d < 3; ++d) {
+        s1[d] = b[d] + 2 * r[d];
+        s0[d] = b[d] + 4 * r[d];
+    }
+    const int t1 = s1[0] * s1[1] * s1[2], t0 = s0[0] * s0[1] * s0[2], np = (int)st.po3.size();
+    g << "struct AdjJit {\n  static constexpr bool kConst = true;\n  static constexpr int kTrips = "
+      << (t1 + nthr - 1) / nthr << ", kTrips0 = " << (t0 + nthr - 1) / nthr << ", kMaxVals = " << np + 3 << ";\n";
+    auto cst = [&](const char *n, int v) {
+        g << "  static __device__ __forceinline__ constexpr int " << n << "(const AdjArgs &) { return " << v << "; }\n";
+    };
+    cst("nx", c->dim[0]), cst("ny", c->dim[1]), cst("nz", c->dim[2]), cst("bx", b[0]), cst("by", b[1]), cst("bz", b[2]);
+    cst("rx", r[0]), cst("ry", r[1]), cst("rz", r[2]), cst("nparam", np);
+    cst("ntx", (c->dim[0] + b[0] - 1) / b[0]), cst("nty", (c->dim[1] + b[1] - 1) / b[1]);
+    // sum over entries (offsets o3, coefficient expressions) into name(x, y, z)
+    auto emit = [&](const char *v, const std::vector<int> &o3, const int sz[3], auto coef) {
+        static const char *mm[3] = {"mx", "my", "mz"}, *ac[3] = {"ax", "ay", "az"};
+        g << "    { double ax = 0.0, ay = 0.0, az = 0.0;\n";
+        for (size_t e = 0; e < o3.size() / 3; ++e) {
+            const int l = (o3[3 * e + 2] * sz[1] + o3[3 * e + 1]) * sz[0] + o3[3 * e];
+            g << "    { const double mx = L[c + " << l << "], my = L[T + c + " << l << "], mz = L[2 * T + c + " << l << "];\n";
+            for (int q = 0; q < 9; ++q) {
+                const std::string w = coef(e, q);
+                if (!w.empty())
+                    g << "      " << ac[q / 3] << " = fma(" << w << ", " << mm[q % 3] << ", " << ac[q / 3] << ");\n";
+            }
+            g << "    }\n";
+        }
+        g << "    " << v << " }\n";
+    };
+    auto cls = [&](size_t e, int q) -> std::string {
+        const int k = st.cls[9 * e + q];
+        return k == 0 ? std::string() : std::string(k < 0 ? "-" : "") + "a.cls[" + std::to_string(abs(k) - 1) + "]";
+    };
+    for (int h = 0; h < 2; ++h) {
+        g << "  static __device__ __forceinline__ v3 " << (h ? "sum0" : "sum")
+          << "(const AdjArgs &a, const double *L, int T, int c) {\n";
+        emit("return mk3(ax, ay, az);", st.o3, h ? s0 : s1, cls);
+        g << "  }\n";
+    }
+    g << "  static __device__ __forceinline__ void units(const AdjArgs &a, const double *L, int T, int c, v3 gB, double *vals) "
+         "{\n";
+    for (int k = 0; k < np; ++k) {
+        const std::string v = "vals[" + std::to_string(k) + "] = -dot3(gB, mk3(ax, ay, az));";
+        emit(v.c_str(), st.po3[k], s1, [&](size_t e, int q) -> std::string {
+            const double w = st.pblk[k][9 * e + q];
+            if (w == 0.0) return std::string();
+            std::ostringstream o;
+            hexd(o, w);
+            return o.str();
+        });
+    }
+    g << "  }\n};\n";
+    std::ostringstream s;
+    s << device_headers() << kJitAdjH << "\n" << g.str();
+    static const char *names[MJ_ADJ_KERNELS] = {"sib1", "sib2", "sibf", "r1", "r2", "r3r1", "r3"};
+    auto want = [&](int k) { return k == MJ_ADJ_SIBF ? fused : k == MJ_ADJ_SIB1 || k == MJ_ADJ_SIB2 ? !fused : true; };
+    for (int k = 0; k < MJ_ADJ_KERNELS; ++k)
+        if (want(k))
+            s << "extern \"C\" __global__ void __launch_bounds__(" << nthr << ") mj_adj_" << names[k]
+              << "(const AdjArgs a) { extern __shared__ double lds[]; adj_" << names[k] << "_body<AdjJit>(a, lds); }\n";
+    hipModule_t mod;
+    const int rc = compile_source(s.str(), &mod);
+    if (rc != MJ_OK) return rc;
+    for (int k = 0; k < MJ_ADJ_KERNELS; ++k) {
+        if (!want(k)) continue;
+        const hipError_t e = hipModuleGetFunction(&fn[k], mod, (std::string("mj_adj_") + names[k]).c_str());
+        if (e != hipSuccess) {
+            mj_set_error(std::string("hipModuleGetFunction: ") + hipGetErrorString(e));
+            return MJ_EHIP;
+        }
+    }
+    return MJ_OK;
+}
+
 // Monte Carlo passes and replica energies: the neighbours' slots from the
 // lattice's constants, the spins of 18 neighbours in flight together (the
 // proposal is computed under the first ones), coefficients as literals, terms
