@@ -388,7 +388,7 @@ static int pow2ceil(int v)
 }
 
 // effective tile for the current lattice
-static void tile_shape(const mj_ctx *c, int &bx, int &by, int &bz)
+static void tile_shape(const mj_ctx *c, int rz, int &bx, int &by, int &bz)
 {
     if (c->bx && c->by && c->bz) {
         bx = c->bx;
@@ -401,6 +401,18 @@ static void tile_shape(const mj_ctx *c, int &bx, int &by, int &bz)
     // fewer than 512 workgroups.  The fused step is the faster for its smaller
     // ring (64x64, Heun at 10 K: triangular 5.4 us per step against 6.2 with 8x8
     // tiles, square 4.4 against 4.65; 256x256: 5.9 against 6.5 with 16x8)
+    // Bonds across the planes: 16x4x4 (two planes: 16x8x2), whose ring is half of
+    // 32x8x1's (392 sites against 764 at reach 1), so that the fused step's regions
+    // fit in LDS (Heun at 10 K, 7 entries: 256x256x8 17.5 us per step against 25.8,
+    // 64x64x16 6.4 against 10.8, 96x96x2 5.8 against 10.1; 32x4x2 and 32x2x4 do not
+    // fit either).  With a dipolar term, a launch per stage: 256x256x16 2153 us
+    // for 8 steps against 2276.
+    if (c->n >= 4096 && rz > 0) {
+        bx = std::min(pow2ceil(c->dim[0]), 16);
+        bz = std::min(pow2ceil(c->dim[2]), 4);
+        by = std::min(pow2ceil(c->dim[1]), 256 / (bx * bz));
+        if (bx * by * bz >= 64) return;
+    }
     int nthr = 256;
     while (c->n < 4096 && nthr > 64 && c->n / nthr < 512) nthr >>= 1;
     bx = std::min(pow2ceil(c->dim[0]), std::max(8, nthr / 8));
@@ -529,13 +541,13 @@ int mj_finalize(mj_ctx *c)
                 for (int b = 0; b < 3; ++b) g[3 * a + b] += A[3 * b + a];
         }
         int bx, by, bz;
-        tile_shape(c, bx, by, bz);
         c->rx = c->ry = c->rz = 0;
         for (auto &o : offs) {
             c->rx = std::max(c->rx, std::abs(o[0]));
             c->ry = std::max(c->ry, std::abs(o[1]));
             c->rz = std::max(c->rz, std::abs(o[2]));
         }
+        tile_shape(c, c->rz, bx, by, bz);
         const int sx = bx + 2 * c->rx, sy = by + 2 * c->ry;
         std::vector<double> cf_iso, cf_dm, cf_gen;
         std::vector<int> o3_iso, o3_dm, o3_gen;
@@ -623,7 +635,7 @@ int mj_finalize(mj_ctx *c)
     }
     // energy partial buffers
     int bx, by, bz;
-    tile_shape(c, bx, by, bz);
+    tile_shape(c, c->rz, bx, by, bz);
     int nb = ((c->dim[0] + bx - 1) / bx) * ((c->dim[1] + by - 1) / by) * ((c->dim[2] + bz - 1) / bz);
     if (c->epart_cap < nb) {
         if (c->epart) hipFree(c->epart);
@@ -645,7 +657,7 @@ static void base_args(const mj_ctx *c, KArgs &a)
     a.px = c->periodic[0];
     a.py = c->periodic[1];
     a.pz = c->periodic[2];
-    tile_shape(c, a.bx, a.by, a.bz);
+    tile_shape(c, c->rz, a.bx, a.by, a.bz);
     a.rx = c->rx;
     a.ry = c->ry;
     a.rz = c->rz;

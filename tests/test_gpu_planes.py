@@ -1,0 +1,47 @@
+"""Lattices of several planes coupled to each other on their default tiles (16x4x4,
+16x8x2, fewer where an axis is short) against one launch per stage on 32x8x1,
+bit for bit: planes that do not fill a tile, one axis shorter than a tile, open
+and periodic across the planes."""
+import os
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+CASES = {
+    "whole": dict(size=[32, 32, 8]),
+    "past": dict(size=[33, 37, 5]),
+    "two": dict(size=[65, 34, 2]),
+    "three_open": dict(size=[47, 40, 3], periodic=[False, False, False]),
+    "periodic_z": dict(size=[24, 18, 10], periodic=[True, True, True]),
+    "narrow": dict(size=[6, 130, 6]),
+    "flat": dict(size=[200, 3, 8]),
+}
+
+
+def _run(c, tile, fuse, integ, T):
+    from matjes_amd import llg
+    env = {"MJ_FUSE": fuse, "MJ_JIT": "1"}
+    old = {k: os.environ.get(k) for k in env}
+    os.environ.update(env)
+    try:
+        with llg.Hamiltonian(c["lat"].dim_lat, c["lat"].periodic, tile=tile) as h:
+            h.load_terms(c["H"], form="stencil")
+            h.set_state(c["m0"])
+            h.steps(6, integ, 0.5, 0.05, kT=T * 0.000086173324, seed=3)
+            return h.get_state()
+    finally:
+        for k, v in old.items():
+            if v is None:
+                os.environ.pop(k, None)
+            else:
+                os.environ[k] = v
+
+
+@pytest.mark.parametrize("integ,T", [(2, 10.0), (5, 10.0), (6, 0.0)])
+@pytest.mark.parametrize("name", sorted(CASES))
+def test_default_tile_equals_the_stage_kernels(name, integ, T):
+    from matjes_amd import workloads
+    c = workloads.build_case(dict(workloads.FILM_DIP, dipolar=False, D=0.3e-3, mediator_dz=-0.5, seed=2, **CASES[name]))
+    assert np.array_equal(_run(c, None, "1", integ, T), _run(c, (32, 8, 1), "0", integ, T))
