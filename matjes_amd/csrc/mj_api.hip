@@ -91,7 +91,7 @@ extern "C" int mj_create(mj_ctx **out, int device, const int dim_lat[3], const i
     if (hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) != hipSuccess ||
         hipMalloc(&c->A, bytes) != hipSuccess || hipMalloc(&c->Bb, bytes) != hipSuccess ||
         hipMalloc(&c->Db, bytes) != hipSuccess || hipMalloc(&c->Fb, bytes) != hipSuccess ||
-        hipMalloc(&c->Nb, bytes) != hipSuccess) {
+        hipMalloc(&c->Nb, bytes) != hipSuccess || mj_stage_alloc(c->host, 3 * c->n) != MJ_OK) {
         mj_destroy(&c);
         MJ_FAIL(MJ_ENOMEM, "mj_create: device allocation failed");
     }
@@ -116,6 +116,7 @@ extern "C" int mj_destroy(mj_ctx **pc)
     drop_graph(c);
     if (c->d_step) hipFree(c->d_step);
     if (c->estage) hipFree(c->estage);
+    mj_stage_free(c->host);
     double *bufs[] = {c->A, c->Bb, c->Db, c->Fb, c->Nb, c->epart, c->evals, c->d_cf, c->d_bmap, c->d_v, c->d_maps};
     for (double *p : bufs)
         if (p) hipFree(p);
@@ -714,9 +715,13 @@ extern "C" int mj_set_state(mj_ctx *c, const double *m, int64_t n3)
 {
     if (!c || !m || n3 != 3 * c->n) MJ_FAIL(MJ_EINVAL, "mj_set_state: size must be 3*Ncell");
     MJ_TRY(set_dev(c));
-    MJ_HIP_CHECK(hipMemcpyAsync(c->Nb, m, sizeof(double) * n3, hipMemcpyHostToDevice, c->stream));
-    MJ_TRY(mj_launch_aos2soa(c->Nb, c->A, c->n, c->np, c->stream));
-    MJ_HIP_CHECK(hipStreamSynchronize(c->stream));
+    if (n3 <= c->host.half) {
+        MJ_TRY(mj_upload(c->host, m, c->A, c->n, c->np, c->stream));
+    } else {
+        MJ_HIP_CHECK(hipMemcpyAsync(c->Nb, m, sizeof(double) * n3, hipMemcpyHostToDevice, c->stream));
+        MJ_TRY(mj_launch_aos2soa(c->Nb, c->A, c->n, c->np, c->stream));
+        MJ_HIP_CHECK(hipStreamSynchronize(c->stream));
+    }
     c->state_set = 1;
     c->field_valid = 0;
     return MJ_OK;
@@ -738,10 +743,7 @@ extern "C" int mj_get_state(mj_ctx *c, double *m, int64_t n3)
     if (!c || !m || n3 != 3 * c->n) MJ_FAIL(MJ_EINVAL, "mj_get_state: size must be 3*Ncell");
     if (!c->state_set) MJ_FAIL(MJ_ESTATE, "mj_get_state: no state set");
     MJ_TRY(set_dev(c));
-    MJ_TRY(mj_launch_soa2aos(c->A, c->Nb, c->n, c->np, 1.0e-50, c->stream));
-    MJ_HIP_CHECK(hipMemcpyAsync(m, c->Nb, sizeof(double) * n3, hipMemcpyDeviceToHost, c->stream));
-    MJ_HIP_CHECK(hipStreamSynchronize(c->stream));
-    return MJ_OK;
+    return mj_download(c->host, c->A, c->n, c->np, 1.0e-50, m, c->stream);
 }
 
 extern "C" int mj_get_state_device(mj_ctx *c, double *m, int64_t n3)
@@ -766,10 +768,7 @@ extern "C" int mj_eff_field(mj_ctx *c, double *B, int64_t n3)
     MJ_TRY(prep_field(c, c->A, a));
     a.fld_out = c->Bb;
     MJ_TRY(launch(c, MODE_FIELD, false, a));
-    MJ_TRY(mj_launch_soa2aos(c->Bb, c->Nb, c->n, c->np, 0.0, c->stream));
-    MJ_HIP_CHECK(hipMemcpyAsync(B, c->Nb, sizeof(double) * n3, hipMemcpyDeviceToHost, c->stream));
-    MJ_HIP_CHECK(hipStreamSynchronize(c->stream));
-    return MJ_OK;
+    return mj_download(c->host, c->Bb, c->n, c->np, 0.0, B, c->stream);
 }
 
 extern "C" int mj_keep_last_field(mj_ctx *c, int on)
@@ -786,10 +785,7 @@ extern "C" int mj_last_field(mj_ctx *c, double *B, int64_t n3)
     if (!c->field_valid)
         MJ_FAIL(MJ_ESTATE, "mj_last_field: no step has run since mj_keep_last_field(ctx, 1) or mj_set_state");
     MJ_TRY(set_dev(c));
-    MJ_TRY(mj_launch_soa2aos(c->Lf, c->Nb, c->n, c->np, 0.0, c->stream));
-    MJ_HIP_CHECK(hipMemcpyAsync(B, c->Nb, sizeof(double) * n3, hipMemcpyDeviceToHost, c->stream));
-    MJ_HIP_CHECK(hipStreamSynchronize(c->stream));
-    return MJ_OK;
+    return mj_download(c->host, c->Lf, c->n, c->np, 0.0, B, c->stream);
 }
 
 static int energy_async(mj_ctx *c, double *dst_dev, double scale)
@@ -812,10 +808,9 @@ extern "C" int mj_energy(mj_ctx *c, double *E)
     if (!c->state_set) MJ_FAIL(MJ_ESTATE, "mj_energy: no state set");
     MJ_TRY(set_dev(c));
     MJ_TRY(mj_finalize(c));
-    MJ_TRY(ensure_evals(c, 1));
-    MJ_TRY(energy_async(c, c->evals, 1.0));
-    MJ_HIP_CHECK(hipMemcpyAsync(E, c->evals, sizeof(double), hipMemcpyDeviceToHost, c->stream));
+    MJ_TRY(energy_async(c, c->host.buf, 1.0));   // reduced straight into pinned memory
     MJ_HIP_CHECK(hipStreamSynchronize(c->stream));
+    *E = c->host.buf[0];
     return MJ_OK;
 }
 
@@ -1491,12 +1486,8 @@ static int run_steps(mj_ctx *c, int nsteps, int integ, double timestep, double a
                               base.bx * base.by * base.bz, c->stream));
     if (prof && prof->block && prof->b1) MJ_HIP_CHECK(hipEventRecord(prof->b1, c->stream));
     if (adapt) *ad->ts_io = ts;
-    if (energies && dr) {
-        MJ_HIP_CHECK(hipMemcpyAsync(energies, c->evals, sizeof(double) * nsteps, hipMemcpyDeviceToHost, c->stream));
-    } else if (energies) {
-        MJ_TRY(energy_async(c, c->evals + (nsteps - 1), escale));
-        MJ_HIP_CHECK(hipMemcpyAsync(energies, c->evals, sizeof(double) * nsteps, hipMemcpyDeviceToHost, c->stream));
-    }
+    if (energies && !dr) MJ_TRY(energy_async(c, c->evals + (nsteps - 1), escale));
+    if (energies) MJ_TRY(mj_download_flat(c->host, c->evals, nsteps, energies, c->stream));
     MJ_HIP_CHECK(hipStreamSynchronize(c->stream));
     return MJ_OK;
 }

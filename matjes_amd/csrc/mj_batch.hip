@@ -525,15 +525,6 @@ __global__ void k_bump(uint64_t *stepp, uint64_t n)
     if (threadIdx.x == 0 && blockIdx.x == 0) *stepp += n;
 }
 
-__global__ void k_batch_soa2aos(const double *in, double *out, int64_t n, int64_t np)
-{
-    int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    out[3 * i] = in[i];
-    out[3 * i + 1] = in[i + np];
-    out[3 * i + 2] = in[i + 2 * np];
-}
-
 // ---------------------------------------------------------------------------
 // host side
 // ---------------------------------------------------------------------------
@@ -565,6 +556,7 @@ struct BatchGroup {
 };
 
 struct mj_batch {
+    MjHostStage host;   // made by the first read of a state or of the energies
     int device = 0;
     hipStream_t stream = nullptr;
     std::vector<HostSys> sys;
@@ -718,6 +710,7 @@ extern "C" int mj_batch_destroy(mj_batch **pb)
             delete s.dipc;
             s.dipc = nullptr;
         }
+    mj_stage_free(b->host);
     (void)hipStreamDestroy(b->stream);
     delete b;
     *pb = nullptr;
@@ -1533,6 +1526,14 @@ extern "C" int mj_batch_profile(mj_batch *b, int nsteps, int integrator, double 
     return check_barrier(b);
 }
 
+// pinned staging for the largest system
+static int batch_stage(mj_batch *b)
+{
+    int64_t most = 0;
+    for (auto &q : b->sys) most = std::max(most, 3 * q.n);
+    return mj_stage_alloc(b->host, most);
+}
+
 extern "C" int mj_batch_get_state(mj_batch *b, int sys, double *m, int64_t n3)
 {
     if (!b || !m) BFAIL(MJ_EINVAL, "mj_batch_get_state: null argument");
@@ -1545,15 +1546,8 @@ extern "C" int mj_batch_get_state(mj_batch *b, int sys, double *m, int64_t n3)
         return MJ_OK;
     }
     MJ_HIP_CHECK(hipSetDevice(b->device));
-    double *tmp = nullptr;
-    MJ_HIP_CHECK(hipMalloc(&tmp, sizeof(double) * 3 * s.n));
-    hipLaunchKernelGGL(k_batch_soa2aos, dim3((unsigned)((s.n + 255) / 256)), dim3(256), 0, b->stream, b->A + s.base,
-                       tmp, s.n, b->np);
-    hipError_t e = hipMemcpyAsync(m, tmp, sizeof(double) * 3 * s.n, hipMemcpyDeviceToHost, b->stream);
-    hipError_t e2 = hipStreamSynchronize(b->stream);
-    (void)hipFree(tmp);
-    if (e != hipSuccess || e2 != hipSuccess) BFAIL(MJ_EHIP, "mj_batch_get_state: copy failed");
-    return MJ_OK;
+    BTRY(batch_stage(b));
+    return mj_download(b->host, b->A + s.base, s.n, b->np, 0.0, m, b->stream);
 }
 
 // energy per site of every system's current state (the single-system mj_energy)
@@ -1572,10 +1566,9 @@ extern "C" int mj_batch_energies(mj_batch *b, double *E)
     BTRY(blaunch_err("batched energy pass"));
     hipLaunchKernelGGL(k_batch_esum, dim3((unsigned)b->sys.size()), dim3(256), 0, b->stream, b->epart, b->d_sys, b->E);
     BTRY(blaunch_err("batched energy sum"));
-    std::vector<double> t(b->sys.size());
-    MJ_HIP_CHECK(hipMemcpyAsync(t.data(), b->E, sizeof(double) * t.size(), hipMemcpyDeviceToHost, b->stream));
-    MJ_HIP_CHECK(hipStreamSynchronize(b->stream));
-    for (size_t q = 0; q < t.size(); ++q) E[q] = t[q] / (double)b->sys[q].n;
+    BTRY(batch_stage(b));
+    BTRY(mj_download_flat(b->host, b->E, (int64_t)b->sys.size(), E, b->stream));
+    for (size_t q = 0; q < b->sys.size(); ++q) E[q] /= (double)b->sys[q].n;
     return MJ_OK;
 }
 

@@ -23,7 +23,25 @@ void mj_set_error(const std::string &msg);
 
 struct DipolarFFT;  // mj_fft.hip
 
+// Pinned memory between a caller's arrays and the device, kept with its object:
+// the kernels that lay a field out read and write it themselves.
+struct MjHostStage {
+    double *buf = nullptr;
+    int64_t half = 0;                  // doubles of a chunk, whole sites
+    int chunks = 0;                    // 1 (the object's fields fit in one) or 2
+    hipEvent_t ev[2] = {nullptr, nullptr};
+};
+int mj_stage_alloc(MjHostStage &h, int64_t n3);
+void mj_stage_free(MjHostStage &h);
+// n sites of a field (SoA, stride np) to / from the caller's AoS array (up: 3 n <= half); |x| < eps goes out as 0.
+// Both end synchronised.
+int mj_download(MjHostStage &h, const double *soa, int64_t n, int64_t np, double eps, double *host, hipStream_t s);
+int mj_upload(MjHostStage &h, const double *host, double *soa, int64_t n, int64_t np, hipStream_t s);
+// count doubles as they are
+int mj_download_flat(MjHostStage &h, const double *dev, int64_t count, double *host, hipStream_t s);
+
 struct mj_ctx {
+    MjHostStage host;
     int device = 0;
     int dim[3] = {1, 1, 1};
     int periodic[3] = {0, 0, 0};

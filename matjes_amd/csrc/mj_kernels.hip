@@ -1,6 +1,11 @@
 // Ahead-of-time kernels of the LLG hot path: the fused stage kernel with
 // runtime geometry (used for small lattices and whenever no per-Hamiltonian
 // kernel is compiled), plus the small helper kernels.
+#include <string.h>
+
+#include <algorithm>
+#include <string>
+
 #include "mj_device.h"
 #include "mj_internal.h"
 #include "mj_stage_body.h"
@@ -119,6 +124,27 @@ __global__ void k_soa2aos(const double *in, double *out, int64_t n, int64_t np, 
     out[3 * i] = fabs(x) < eps ? 0.0 : x;
     out[3 * i + 1] = fabs(y) < eps ? 0.0 : y;
     out[3 * i + 2] = fabs(z) < eps ? 0.0 : z;
+}
+
+// m doubles of an AoS array (from site s0 on) in pinned host memory, one thread
+// a double so that whole lines cross the link: SITES 0 the array is flat
+template <bool SITES>
+__global__ void k_to_host(const double *in, double *out, int64_t s0, int m, int64_t np, double eps)
+{
+    const int t = (int)(blockIdx.x * blockDim.x + threadIdx.x);
+    if (t >= m) return;
+    if constexpr (SITES) {
+        const double x = in[s0 + t / 3 + (t % 3) * np];
+        out[t] = fabs(x) < eps ? 0.0 : x;
+    } else {
+        out[t] = in[s0 + t];
+    }
+}
+
+__global__ void k_from_host(const double *in, double *out, int m, int64_t np)
+{
+    const int t = (int)(blockIdx.x * blockDim.x + threadIdx.x);
+    if (t < m) out[t / 3 + (t % 3) * np] = in[t];
 }
 
 __global__ void k_normals(uint64_t seed, uint64_t step, int64_t n, double *out)
@@ -361,6 +387,78 @@ int mj_launch_soa2aos(const double *in, double *out, int64_t n, int64_t np, doub
 {
     hipLaunchKernelGGL(k_soa2aos, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, in, out, n, np, eps);
     return hipGetLastError() == hipSuccess ? MJ_OK : MJ_EHIP;
+}
+
+int mj_stage_alloc(MjHostStage &h, int64_t n3)
+{
+    if (h.buf && (h.chunks == 2 || n3 <= h.half)) return MJ_OK;
+    mj_stage_free(h);
+    const int64_t cap = 3 * 21824;   // 512 KiB
+    h.half = std::min<int64_t>(std::max<int64_t>(n3, 192), cap);
+    h.chunks = n3 > cap ? 2 : 1;
+    hipError_t e = hipHostMalloc(&h.buf, sizeof(double) * (size_t)(h.half * h.chunks), hipHostMallocDefault);
+    for (int k = 0; k < 2 && e == hipSuccess; ++k) e = hipEventCreateWithFlags(&h.ev[k], hipEventDisableTiming);
+    if (e == hipSuccess) return MJ_OK;
+    mj_stage_free(h);
+    mj_set_error(std::string("pinned staging memory: ") + hipGetErrorString(e));
+    return MJ_ENOMEM;
+}
+
+void mj_stage_free(MjHostStage &h)
+{
+    if (h.buf) (void)hipHostFree(h.buf);
+    for (auto &e : h.ev) {
+        if (e) (void)hipEventDestroy(e);
+        e = nullptr;
+    }
+    h.buf = nullptr;
+}
+
+// chunks of `half` doubles; with more than one, the host copies a chunk while
+// the next crosses the link.  A copy to pageable memory goes through the
+// runtime's own staging, one part after the other: 32^2 sites 31 us, 256^2 106,
+// 1024^2 1438; here 15, 73 and 861.
+template <bool SITES>
+static int download(MjHostStage &h, const double *dev, int64_t total, int64_t np, double eps, double *host, hipStream_t s)
+{
+    const int64_t step = h.half, n = (total + step - 1) / step;
+    for (int64_t k = 0; k <= n; ++k) {
+        if (k < n) {
+            const int m = (int)std::min(step, total - k * step);
+            hipLaunchKernelGGL(k_to_host<SITES>, dim3((m + 255) / 256), dim3(256), 0, s, dev,
+                               h.buf + (h.chunks == 2 ? k % 2 : 0) * step, SITES ? k * step / 3 : k * step, m, np, eps);
+            if (hipGetLastError() != hipSuccess) return MJ_EHIP;
+            MJ_HIP_CHECK(hipEventRecord(h.ev[k % 2], s));
+        }
+        const int64_t q = h.chunks == 2 ? k - 1 : k;   // one buffer: its chunk at once
+        if (q < 0 || q >= n) continue;
+        MJ_HIP_CHECK(hipEventSynchronize(h.ev[q % 2]));
+        memcpy(host + q * step, h.buf + (h.chunks == 2 ? q % 2 : 0) * step,
+               sizeof(double) * (size_t)std::min(step, total - q * step));
+    }
+    return MJ_OK;
+}
+
+int mj_download(MjHostStage &h, const double *soa, int64_t n, int64_t np, double eps, double *host, hipStream_t s)
+{
+    return download<true>(h, soa, 3 * n, np, eps, host, s);
+}
+
+int mj_download_flat(MjHostStage &h, const double *dev, int64_t count, double *host, hipStream_t s)
+{
+    return download<false>(h, dev, count, 0, 0.0, host, s);
+}
+
+// A field of one chunk; longer ones are better copied by the runtime (256^2
+// sites: 92 us in chunks, 81 by hipMemcpyAsync and a kernel; 128^2: 24.5 and 32.7).
+int mj_upload(MjHostStage &h, const double *host, double *soa, int64_t n, int64_t np, hipStream_t s)
+{
+    const int m = (int)(3 * n);
+    memcpy(h.buf, host, sizeof(double) * (size_t)m);
+    hipLaunchKernelGGL(k_from_host, dim3((m + 255) / 256), dim3(256), 0, s, h.buf, soa, m, np);
+    if (hipGetLastError() != hipSuccess) return MJ_EHIP;
+    MJ_HIP_CHECK(hipStreamSynchronize(s));
+    return MJ_OK;
 }
 
 int mj_launch_normals(uint64_t seed, uint64_t step, int64_t n, double *out, hipStream_t s)

@@ -312,10 +312,13 @@ __global__ void __launch_bounds__(kMcThreads) k_mc_fold(const McState *st_in, Mc
     }
 }
 
-// site order <-> colour-major order of a 3-component SoA field
+// site order <-> colour-major order of a 3-component SoA field (of the replica
+// at `rung` where image is given)
 __global__ void __launch_bounds__(kMcThreads) k_mc_layout(const McArgs a, const double *src, int64_t sstride,
-                                                          double *dst, int64_t dstride, int to_cm)
+                                                          double *dst, int64_t dstride, int to_cm,
+                                                          const int *image = nullptr, int rung = 0)
 {
+    if (image) src += (int64_t)image[rung] * 3 * sstride;
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     const int64_t n = (int64_t)a.nx * a.ny * a.nz;
     if (i >= n) return;
@@ -1068,12 +1071,8 @@ extern "C" int mj_mc_sweeps(mj_ctx *c, int nsweeps, int sampler, double kT, uint
     }
     MJ_TRY(to_sites());
     if (nsamp > 0) {
-        if (E_samples)
-            MJ_HIP_CHECK(hipMemcpyAsync(E_samples, mc->d_samples, sizeof(double) * nsamp, hipMemcpyDeviceToHost,
-                                        c->stream));
-        if (M_samples)
-            MJ_HIP_CHECK(hipMemcpyAsync(M_samples, mc->d_samples + nsamp, sizeof(double) * 3 * nsamp,
-                                        hipMemcpyDeviceToHost, c->stream));
+        if (E_samples) MJ_TRY(mj_download_flat(c->host, mc->d_samples, nsamp, E_samples, c->stream));
+        if (M_samples) MJ_TRY(mj_download_flat(c->host, mc->d_samples + nsamp, 3 * nsamp, M_samples, c->stream));
     }
     MJ_HIP_CHECK(hipStreamSynchronize(c->stream));
     return MJ_OK;
@@ -1244,12 +1243,9 @@ extern "C" int mj_mc_pt_sweeps(mj_ctx *c, int nsweeps, int sampler, uint64_t see
         }
     }
     if (nsamp > 0) {
-        if (E_samples)
-            MJ_HIP_CHECK(hipMemcpyAsync(E_samples, mc->d_rsamples, sizeof(double) * nsamp * nrep,
-                                        hipMemcpyDeviceToHost, c->stream));
+        if (E_samples) MJ_TRY(mj_download_flat(c->host, mc->d_rsamples, nsamp * nrep, E_samples, c->stream));
         if (M_samples)
-            MJ_HIP_CHECK(hipMemcpyAsync(M_samples, mc->d_rsamples + nsamp * nrep, sizeof(double) * 3 * nsamp * nrep,
-                                        hipMemcpyDeviceToHost, c->stream));
+            MJ_TRY(mj_download_flat(c->host, mc->d_rsamples + nsamp * nrep, 3 * nsamp * nrep, M_samples, c->stream));
     }
     MJ_HIP_CHECK(hipStreamSynchronize(c->stream));
     return MJ_OK;
@@ -1284,7 +1280,6 @@ extern "C" int mj_mc_pt_state(mj_ctx *c, int *image_of_rung, double *swaps_accep
     return MJ_OK;
 }
 
-int mj_launch_soa2aos(const double *in, double *out, int64_t n, int64_t np, double eps, hipStream_t s);
 
 extern "C" int mj_mc_pt_get_state(mj_ctx *c, int rung, double *m, int64_t n3)
 {
@@ -1293,16 +1288,10 @@ extern "C" int mj_mc_pt_get_state(mj_ctx *c, int rung, double *m, int64_t n3)
     if (!mc || mc->nrep < 1) MJ_FAIL(MJ_ESTATE, "mj_mc_pt_get_state: no replicas");
     if (rung < 0 || rung >= mc->nrep) MJ_FAIL(MJ_EINVAL, "mj_mc_pt_get_state: no such rung");
     MJ_HIP_CHECK(hipSetDevice(c->device));
-    MJ_HIP_CHECK(hipStreamSynchronize(c->stream));
-    int r = 0;
-    MJ_HIP_CHECK(hipMemcpy(&r, mc->d_image + rung, sizeof(int), hipMemcpyDeviceToHost));
     McArgs a;
     mc_args(c, mc, a);
     hipLaunchKernelGGL(k_mc_layout, dim3((unsigned)ceil_div(c->n, kMcThreads)), dim3(kMcThreads), 0, c->stream, a,
-                       (const double *)(mc->d_rcm + (size_t)r * 3 * a.cs), a.cs, c->Bb, c->np, 0);
+                       (const double *)mc->d_rcm, a.cs, c->Bb, c->np, 0, (const int *)mc->d_image, rung);
     MJ_TRY(launch_check("layout launch"));
-    MJ_TRY(mj_launch_soa2aos(c->Bb, c->Nb, c->n, c->np, 1.0e-50, c->stream));
-    MJ_HIP_CHECK(hipMemcpyAsync(m, c->Nb, sizeof(double) * n3, hipMemcpyDeviceToHost, c->stream));
-    MJ_HIP_CHECK(hipStreamSynchronize(c->stream));
-    return MJ_OK;
+    return mj_download(c->host, c->Bb, c->n, c->np, 1.0e-50, m, c->stream);
 }
