@@ -144,21 +144,24 @@ static auto literal_coef(const mj_ctx *c)
 
 // the regions of a fused tile: its constants (JitFused, BatchFused) and LDS bytes
 static size_t emit_fused_tile(std::ostringstream &g, int BX, int BY, int BZ, int rx, int ry, int rz, int nthr, int spt,
-                              int nsub, int nb, bool dma, int &T0, bool &alias)
+                              int nsub, int nb, int wide, bool dma, int &T0, bool &alias)
 {
     const int s0x = BX + 4 * rx, s0y = BY + 4 * ry, s0z = BZ + 4 * rz;
     const int t0 = s0x * s0y * s0z, t1 = (BX + 2 * rx) * (BY + 2 * ry) * (BZ + 2 * rz);
-    T0 = dma ? 2 * nthr * ((t0 / 2 + nthr - 1) / nthr) : t0;
+    const int all = nthr + wide, rthr = wide ? wide : nthr;
+    T0 = dma ? 2 * all * ((t0 / 2 + all - 1) / all) : t0;
     // S1 in S0's place while a thread holds its share of the ring in registers
-    alias = t1 - BX * BY * BZ <= 2 * nthr;
+    alias = t1 - BX * BY * BZ <= 2 * rthr;
     g << "  static constexpr int kBx = " << BX << ", kBy = " << BY << ", kBz = " << BZ << ", kRx = " << rx
       << ", kRy = " << ry << ", kRz = " << rz << ";\n";
-    g << "  static constexpr int kFill = " << (t0 + nthr - 1) / nthr << ";   // S0 sites per thread\n";
+    g << "  static constexpr int kFill = " << (t0 + all - 1) / all << ";   // S0 sites per thread\n";
     g << "  static constexpr int kS0x = " << s0x << ", kS0y = " << s0y << ", kS0z = " << s0z << ", kT0 = " << T0 << ";\n";
     g << "  static constexpr bool kDma = " << (dma ? "true" : "false") << ", kAlias = " << (alias ? "true" : "false")
       << ";\n";
     g << "  static constexpr int kNthrBase = " << nb << ", kNsub = " << nsub << ";\n";
-    g << "  static constexpr int kSpt = " << spt << ", kNthr = " << nthr << ";   // sites per thread, threads\n";
+    g << "  static constexpr int kSpt = " << spt << ", kNthr = " << nthr
+      << ";   // sites per thread, their threads\n  static constexpr int kWide = " << wide << ", kAll = " << all
+      << ";   // threads of the ring's own, all\n";
     return sizeof(double) * ((size_t)3 * T0 + (alias ? 0 : (size_t)3 * t1) + BX * BY * BZ / 64 + 1);
 }
 
@@ -176,8 +179,13 @@ static size_t emit_fused_tile(std::ostringstream &g, int BX, int BY, int BZ, int
 // 29.4 / 27.3 / 26.6, 1500x1500 62.3 / 56.9 / 54.9; square 384x384 6.2 / 7.0 /
 // 7.4, 512x512 7.6 / 7.4 / 7.9, 1024x1024 19.6 / 19.1 / 19.5, 1500x1500 39.3 /
 // 38.7 / 39.7 (SIB 42.4 / 39.5 / 39.4, Depondt 46.5 / 42.9 / 42.3).
+// Up to one single tile per CU the ring has wavefronts of its own: a launch is
+// one tile's latency, and the first stage then runs once instead of twice in
+// turn (us per step, Heun at 10 K: triangular 64x64 5.34 -> 4.90, 256x256 5.88 ->
+// 5.44, square 64x64 4.24 -> 4.03, 64x64x16 6.2 -> 5.4; beyond, 384x384 8.45 ->
+// 8.03 but Depondt 9.2 -> 10.2, square 6.2 -> 6.4, 128x128x16 11.8 -> 12.2).
 // MJ_FUSE_SPT=1 or 2 asks for single tiles or pairs, MJ_FUSE_SUB=2 for double
-// tiles.
+// tiles, MJ_FUSE_WIDE=0 or 1 against or for the ring's own wavefronts.
 static void prepare_fused(mj_ctx *c, JitState *j, std::ostringstream &g, int bx, int by, int bz, int ntx, int nty,
                           int ntz)
 {
@@ -202,8 +210,12 @@ static void prepare_fused(mj_ctx *c, JitState *j, std::ostringstream &g, int bx,
         std::ostringstream t;
         int T0 = 0;
         bool alias = false;
-        const size_t shm = emit_fused_tile(t, BX, BY, BZ, rx, ry, rz, nthr, spt, nsub, nb, dma, T0, alias);
-        if (shm > 65536 || nthr > 1024) continue;
+        const int nring = (BX + 2 * rx) * (BY + 2 * ry) * (BZ + 2 * rz) - BX * BY * BZ;
+        const char *we = getenv("MJ_FUSE_WIDE");
+        const bool few = we ? we[0] == '1' : (long)ntx * nty * ntz <= cus;
+        const int wide = form == 0 && few ? std::min((nring + 63) / 64 * 64, 1024 - nthr) : 0;
+        const size_t shm = emit_fused_tile(t, BX, BY, BZ, rx, ry, rz, nthr, spt, nsub, nb, wide, dma, T0, alias);
+        if (shm > 65536 || nthr + wide > 1024) continue;
         const int ntyf = (c->dim[1] + BY - 1) / BY, ntzf = (c->dim[2] + BZ - 1) / BZ;
         g << "struct JitFused {\n" << t.str();
         g << "  static constexpr bool kEnergy = true;\n";
@@ -224,7 +236,7 @@ static void prepare_fused(mj_ctx *c, JitState *j, std::ostringstream &g, int bx,
         if (spt == 2) emit_sum(g, ofs3, "pair0", 2, s0x, s0x * s0y, T0, cf);
         g << "};\n";
         j->fuse_ok = 1;
-        j->fuse_nthr = nthr;
+        j->fuse_nthr = nthr + wide;
         j->fuse_nblocks = ntx * ntyf * ntzf;
         j->fuse_shm = shm;
         return;
@@ -366,7 +378,7 @@ int mj_jit_batch_fused(const std::vector<int> &ofs3, const std::vector<int> &cls
     bool alias = false;
     const int s0x = bx + 4 * rx, s0y = by + 4 * ry, s1x = bx + 2 * rx, s1y = by + 2 * ry;
     g << "struct BatchFused {\n";
-    *shm = emit_fused_tile(g, bx, by, 1, rx, ry, rz, bx * by, 1, 1, bx * by, true, T0, alias);
+    *shm = emit_fused_tile(g, bx, by, 1, rx, ry, rz, bx * by, 1, 1, bx * by, 0, true, T0, alias);
     if (*shm > 65536) {
         *fn = nullptr;
         return MJ_OK;

@@ -773,7 +773,7 @@ template <class F>
 __device__ __forceinline__ void fused_s0_fill(const KArgs &a, double *L0, int x0, int y0, int z0, bool direct,
                                               v3 v[F::kFill])
 {
-    constexpr int SX = F::kS0x, SY = F::kS0y, SZ = F::kS0z, T0 = F::kT0, NTHR = F::kNthr;
+    constexpr int SX = F::kS0x, SY = F::kS0y, SZ = F::kS0z, T0 = F::kT0, NTHR = F::kAll;
     constexpr int RX2 = 2 * F::kRx, RY2 = 2 * F::kRy, RZ2 = 2 * F::kRz;
     const int64_t np = a.np;
     if constexpr (F::kDma) {
@@ -827,7 +827,7 @@ __device__ __forceinline__ void fused_s0_store(double *L0, const v3 v[F::kFill])
     constexpr int T = F::kS0x * F::kS0y * F::kS0z, T0 = F::kT0;
 #pragma unroll
     for (int it = 0; it < F::kFill; ++it) {
-        const int t = (int)threadIdx.x + it * F::kNthr;
+        const int t = (int)threadIdx.x + it * F::kAll;
         if (t < T) {
             L0[t] = v[it].x;
             L0[T0 + t] = v[it].y;
@@ -966,7 +966,9 @@ __device__ __forceinline__ void fused_body(const KArgs &a, double *lds)
     constexpr int S0X = F::kS0x, S0Y = F::kS0y, T0 = F::kT0;
     constexpr int S1X = BX + 2 * RX, S1Y = BY + 2 * RY, S1Z = BZ + 2 * RZ, T1 = S1X * S1Y * S1Z;
     constexpr int NRING = T1 - BX * BY * BZ;
-    constexpr int NRT = (NRING + NTHR - 1) / NTHR;   // ring sites per thread
+    // threads of the ring's own (after those of the tile), or the tile's threads
+    constexpr int WIDE = F::kWide, RTHR = WIDE ? WIDE : NTHR;
+    constexpr int NRT = (NRING + RTHR - 1) / RTHR;   // ring sites per thread
     constexpr bool ALIAS = F::kAlias;                // S1 in S0's place
     static_assert(NB % 64 == 0 && NTHR * SPT == BX * BY * BZ, "whole wavefronts, every tile site once");
     static_assert(SPT == 1 || (SPT == 2 && BX == 32 && BZ == 1 && BYT % F::kNsub == 0 && NTHR >= NB),
@@ -998,6 +1000,8 @@ __device__ __forceinline__ void fused_body(const KArgs &a, double *lds)
         return fused_site<F>(a, x, y, z, g) ? g : 0;
     };
 
+    const bool own = WIDE == 0 || (int)threadIdx.x < NTHR;   // whole wavefronts
+    const int rid = WIDE == 0 ? (int)threadIdx.x : own ? NRING : (int)threadIdx.x - NTHR;
     // the thread's own sites (rows SPT ly + j); active: inside the lattice
     const int lx = threadIdx.x % BX, ly = (threadIdx.x / BX) % BYT * SPT, lz = threadIdx.x / (BX * BYT);
     const int gx = x0 + lx, gz = z0 + lz;
@@ -1006,6 +1010,9 @@ __device__ __forceinline__ void fused_body(const KArgs &a, double *lds)
     v3 th[SPT];
 #pragma unroll
     for (int j = 0; j < SPT; ++j) {
+        active[j] = false;
+        gi[j] = 0;
+        if (!own) continue;
         const int gy = y0 + ly + j;
         active[j] = inside || (gx < F::nx(a) && gy < F::ny(a) && gz < F::nz(a));
         gi[j] = index(gx, gy, gz);
@@ -1042,12 +1049,12 @@ __device__ __forceinline__ void fused_body(const KArgs &a, double *lds)
     if constexpr (ALIAS) {
 #pragma unroll
         for (int r = 0; r < NRT; ++r) {
-            const int k = threadIdx.x + r * NTHR;
+            const int k = rid + r * RTHR;
             cr[r] = -1;
             if (k < NRING) mr[r] = ring(k, cr[r]);
         }
     } else {
-        for (int k = threadIdx.x; k < NRING; k += NTHR) {
+        for (int k = rid; k < NRING; k += RTHR) {
             int c1;
             const v3 m = ring(k, c1);
             L1[c1] = m.x;
@@ -1061,7 +1068,7 @@ __device__ __forceinline__ void fused_body(const KArgs &a, double *lds)
     FusedKeep<MODE> keep[SPT];
     v3 m1[SPT];
     double e = 0.0;
-    {
+    if (own) {
         const int c0 = (lz + 2 * RZ) * S0X * S0Y + (ly + 2 * RY) * S0X + (lx + 2 * RX);
         v3 s[SPT];
         fused_sums<0, F>(a, L0, c0, s);
@@ -1083,7 +1090,7 @@ __device__ __forceinline__ void fused_body(const KArgs &a, double *lds)
         double v = e;
 #pragma unroll
         for (int o = W / 2; o > 0; o >>= 1) v = v + __shfl_xor(v, o, 64);
-        if (threadIdx.x % W == 0) red[threadIdx.x / W] = v;
+        if (own && threadIdx.x % W == 0) red[threadIdx.x / W] = v;
     }
     const int s1 = (lz + RZ) * S1X * S1Y + (ly + RY) * S1X + (lx + RX);
     if constexpr (ALIAS) {
@@ -1099,6 +1106,7 @@ __device__ __forceinline__ void fused_body(const KArgs &a, double *lds)
     }
 #pragma unroll
     for (int j = 0; j < SPT; ++j) {
+        if (!own) continue;
         const int c = s1 + j * S1X;
         L1[c] = m1[j].x;
         L1[T1 + c] = m1[j].y;
@@ -1118,7 +1126,7 @@ __device__ __forceinline__ void fused_body(const KArgs &a, double *lds)
 
     // stage 2 at the own sites from S1
     __builtin_amdgcn_sched_barrier(0);
-    {
+    if (own) {
         v3 s[SPT];
         fused_sums<1, F>(a, L1, s1, s);
 #pragma unroll
@@ -1141,7 +1149,7 @@ __device__ __forceinline__ void fused_body(const KArgs &a, double *lds)
             for (int i = threadIdx.x; i < a.n_ered; i += NB) v += a.ered_in[i];
 #pragma unroll
         for (int o = 32; o > 0; o >>= 1) v = v + __shfl_xor(v, o, 64);
-        if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
+        if ((threadIdx.x & 63) == 0 && threadIdx.x < NB) red[threadIdx.x >> 6] = v;
         __syncthreads();
         if (threadIdx.x == 0) {
             double r = red[0];

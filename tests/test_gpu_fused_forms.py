@@ -1,5 +1,5 @@
-"""The forms of the fused step (single tiles, double tiles, double tiles with two
-sites per thread) against the two stage kernels, bit for bit, where they can go
+"""The forms of the fused step (single tiles, with the ring's own wavefronts or
+without, double tiles, double tiles with two sites per thread) against the two stage kernels, bit for bit, where they can go
 wrong: lattices smaller than a tile and its halo, one site past whole tiles, one
 row short of them, open edges, odd rows (no paired loads), several planes, a
 per-site field, every reach of the stencil from 1 to 3."""
@@ -26,7 +26,7 @@ CASES = {
 def _run(c, env, integ, T, n):
     from matjes_amd import llg
     env = dict({"MJ_FUSE": "1", "MJ_JIT": "1"}, **env)
-    old = {k: os.environ.get(k) for k in ("MJ_FUSE", "MJ_JIT", "MJ_FUSE_SPT", "MJ_FUSE_SUB")}
+    old = {k: os.environ.get(k) for k in ("MJ_FUSE", "MJ_JIT", "MJ_FUSE_SPT", "MJ_FUSE_SUB", "MJ_FUSE_WIDE")}
     for k in old:
         os.environ.pop(k, None)
     os.environ.update(env)
@@ -54,7 +54,8 @@ def test_forms_equal_the_stage_kernels(name, integ, T):
             "film": dict(workloads.FILM_DIP, dipolar=False)}[s.pop("w")]
     c = workloads.build_case(dict(base, seed=11, **s))
     ref = _run(c, {"MJ_FUSE": "0"}, integ, T, 5)
-    for env in ({"MJ_FUSE_SPT": "1"}, {"MJ_FUSE_SUB": "2"}, {"MJ_FUSE_SPT": "2"}):
+    for env in ({"MJ_FUSE_SPT": "1", "MJ_FUSE_WIDE": "0"}, {"MJ_FUSE_SPT": "1", "MJ_FUSE_WIDE": "1"},
+                {"MJ_FUSE_SUB": "2"}, {"MJ_FUSE_SPT": "2"}):
         got = _run(c, env, integ, T, 5)
         for a, b in zip(ref, got):
             assert np.array_equal(a, b), (name, env)
