@@ -25,6 +25,7 @@
 
 #include <algorithm>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 #include "mj_internal.h"
@@ -38,7 +39,7 @@ struct DipolarFFT {
     double *grid_in = nullptr;  // M on the N_rep grid (3 * nk): zero outside the lattice from set-up on, the
                                 // lattice's sites rewritten per call; none where the state is the input itself
     double2 *spec = nullptr;    // M_F / H_F (3 * nc)
-    double2 *kf = nullptr;      // K_F: 6 or 9 components (nc each)
+    double2 *kf = nullptr;      // K_F: 6 or 9 components (nc each; doubles where `half`)
     void *work = nullptr;
     size_t work_size = 0;
     rocfft_plan fwd = nullptr, inv = nullptr;
@@ -51,6 +52,7 @@ struct DipolarFFT {
     int kpb = 0;                // in-plane k points per workgroup of the layer kernel
     int nzt = 0;                // layer offsets stored per component: nzr, or lz when K2_F has a z-parity
     int odd = 0;                // z-parity form: bit q set where K(q)(-dz) = -K(q)(dz) (else +K(q)(dz))
+    int half = 0;               // the dipolar form's K2_F as one real number each (real, or imaginary for xz and yz)
 };
 
 static int rf_check(rocfft_status s, const char *what)
@@ -107,6 +109,18 @@ __device__ __forceinline__ void cmac(double2 &h, double2 k, double2 m)
     h.x = fma(-k.y, m.y, h.x);
     h.y = fma(k.x, m.y, h.y);
     h.y = fma(k.y, m.x, h.y);
+}
+
+// h += k m and h += i k m, k real
+__device__ __forceinline__ void rmac(double2 &h, double k, double2 m)
+{
+    h.x = fma(k, m.x, h.x);
+    h.y = fma(k, m.y, h.y);
+}
+__device__ __forceinline__ void imac(double2 &h, double k, double2 m)
+{
+    h.x = fma(-k, m.y, h.x);
+    h.y = fma(k, m.x, h.y);
 }
 
 // H_F(i) = sum_a K_F(a,i) M_F(a), in place over the spectrum (one thread per k)
@@ -213,19 +227,27 @@ __global__ void k_layer_mix(const double2 *__restrict__ mf, const double2 *__res
 // rows are both staged in LDS, and the next block's are fetched into
 // registers while the current one is mixed; a negative offset costs two sign
 // flips per source layer instead of a test per component.
-template <int LZ>
+// HALF: K_n is even under in-plane inversion (xz and yz: odd) bit for bit, as
+// open directions have it, so its transform is real (imaginary): one number per
+// value, k2b a stream of doubles.
+// Memory bounds it: 256x256x16 moves 100 MB in 26.6 us (3.8 TB/s, a copy of that
+// size 4.5); two or four layers per thread, with a quarter of the LDS reads,
+// took the same or longer (26.8, 33.5).  HALF: 128x128x16 open 26.6 -> 19.2 us.
+template <int LZ, bool HALF>
 __global__ void __launch_bounds__(8 * LZ) k_layer_mix_dip(const double2 *__restrict__ mf,
-                                                          const double2 *__restrict__ k2b, double2 *__restrict__ hf,
+                                                          const void *__restrict__ k2b, double2 *__restrict__ hf,
                                                           int64_t nc2, int nblk)
 {
+    typedef typename std::conditional<HALF, double, double2>::type K;
     constexpr int KPB = 8, NC = 6, NT = KPB * LZ;
     extern __shared__ double2 sh[];
-    double2 *Ks = sh;                    // [NC][LZ][KPB]
-    double2 *Ms = sh + NC * LZ * KPB;    // [3 LZ][KPB]
-    double2 rk0, rk1, rk2, rk3, rk4, rk5, rm0, rm1, rm2;   // the next block's share of this thread
+    double2 *Ms = sh;                      // [3 LZ][KPB]
+    K *Ks = (K *)(sh + 3 * LZ * KPB);      // [NC][LZ][KPB]
+    K rk0, rk1, rk2, rk3, rk4, rk5;        // the next block's share of this thread
+    double2 rm0, rm1, rm2;
 #define MJ_MIX_FETCH(B)                                                                            \
     do {                                                                                           \
-        const double2 *kt_ = k2b + (int64_t)(B) * NC * LZ * KPB + threadIdx.x;                     \
+        const K *kt_ = (const K *)k2b + (int64_t)(B) * NC * LZ * KPB + threadIdx.x;                \
         rk0 = kt_[0 * NT], rk1 = kt_[1 * NT], rk2 = kt_[2 * NT];                                   \
         rk3 = kt_[3 * NT], rk4 = kt_[4 * NT], rk5 = kt_[5 * NT];                                   \
         const int64_t kk_ = (int64_t)(B) * KPB + threadIdx.x % KPB;                                \
@@ -253,18 +275,28 @@ __global__ void __launch_bounds__(8 * LZ) k_layer_mix_dip(const double2 *__restr
             const int dz = neg ? zp - z : z - zp;
             const double2 m0 = Ms[(0 * LZ + zp) * KPB + kl], m1 = Ms[(1 * LZ + zp) * KPB + kl],
                           m2 = Ms[(2 * LZ + zp) * KPB + kl];
-            const double2 kxx = Ks[(0 * LZ + dz) * KPB + kl], kxy = Ks[(1 * LZ + dz) * KPB + kl];
-            double2 kxz = Ks[(2 * LZ + dz) * KPB + kl];
-            const double2 kyy = Ks[(3 * LZ + dz) * KPB + kl];
-            double2 kyz = Ks[(4 * LZ + dz) * KPB + kl];
-            const double2 kzz = Ks[(5 * LZ + dz) * KPB + kl];
+            const K kxx = Ks[(0 * LZ + dz) * KPB + kl], kxy = Ks[(1 * LZ + dz) * KPB + kl];
+            K kxz = Ks[(2 * LZ + dz) * KPB + kl];
+            const K kyy = Ks[(3 * LZ + dz) * KPB + kl];
+            K kyz = Ks[(4 * LZ + dz) * KPB + kl];
+            const K kzz = Ks[(5 * LZ + dz) * KPB + kl];
             if (neg) {
-                kxz.x = -kxz.x, kxz.y = -kxz.y;
-                kyz.x = -kyz.x, kyz.y = -kyz.y;
+                if constexpr (HALF) {
+                    kxz = -kxz, kyz = -kyz;
+                } else {
+                    kxz.x = -kxz.x, kxz.y = -kxz.y;
+                    kyz.x = -kyz.x, kyz.y = -kyz.y;
+                }
             }
-            cmac(h0, kxx, m0), cmac(h0, kxy, m1), cmac(h0, kxz, m2);
-            cmac(h1, kxy, m0), cmac(h1, kyy, m1), cmac(h1, kyz, m2);
-            cmac(h2, kxz, m0), cmac(h2, kyz, m1), cmac(h2, kzz, m2);
+            if constexpr (HALF) {
+                rmac(h0, kxx, m0), rmac(h0, kxy, m1), imac(h0, kxz, m2);
+                rmac(h1, kxy, m0), rmac(h1, kyy, m1), imac(h1, kyz, m2);
+                imac(h2, kxz, m0), imac(h2, kyz, m1), rmac(h2, kzz, m2);
+            } else {
+                cmac(h0, kxx, m0), cmac(h0, kxy, m1), cmac(h0, kxz, m2);
+                cmac(h1, kxy, m0), cmac(h1, kyy, m1), cmac(h1, kyz, m2);
+                cmac(h2, kxz, m0), cmac(h2, kyz, m1), cmac(h2, kzz, m2);
+            }
         }
         const int64_t k = (int64_t)b * KPB + kl;
         if (k < nc2) {
@@ -277,20 +309,19 @@ __global__ void __launch_bounds__(8 * LZ) k_layer_mix_dip(const double2 *__restr
 }
 
 // launches k_layer_mix_dip for the film's layer count (2 .. 32)
-template <int LZ>
+template <int LZ, bool HALF>
 static bool launch_layer_mix_dip(int lz, unsigned nb, hipStream_t st, const double2 *mf, const double2 *k2b,
                                  double2 *hf, int64_t nc2)
 {
     if constexpr (LZ > 32) {
         return false;
     } else {
-        if (lz != LZ) return launch_layer_mix_dip<LZ + 1>(lz, nb, st, mf, k2b, hf, nc2);
-        const size_t shm = sizeof(double2) * 9 * LZ * 8;
+        if (lz != LZ) return launch_layer_mix_dip<LZ + 1, HALF>(lz, nb, st, mf, k2b, hf, nc2);
+        constexpr size_t shm = (sizeof(double2) * 3 + (HALF ? sizeof(double) : sizeof(double2)) * 6) * LZ * 8;
         // as many workgroups as are resident at once, at most one per k block
         static const int per_cu = [] {
             int n = 0;
-            if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k_layer_mix_dip<LZ>, 8 * LZ,
-                                                             sizeof(double2) * 9 * LZ * 8) != hipSuccess)
+            if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k_layer_mix_dip<LZ, HALF>, 8 * LZ, shm) != hipSuccess)
                 n = 1;
             return n > 0 ? n : 1;
         }();
@@ -299,9 +330,24 @@ static bool launch_layer_mix_dip(int lz, unsigned nb, hipStream_t st, const doub
             hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
             cus = 256;
         const unsigned grid = std::min<unsigned>(nb, (unsigned)(per_cu * cus));
-        hipLaunchKernelGGL(k_layer_mix_dip<LZ>, dim3(grid), dim3(8 * LZ), shm, st, mf, k2b, hf, nc2, (int)nb);
+        hipLaunchKernelGGL((k_layer_mix_dip<LZ, HALF>), dim3(grid), dim3(8 * LZ), shm, st, mf, (const void *)k2b, hf, nc2, (int)nb);
         return true;
     }
+}
+
+// the dipolar tensor's form: symmetric, xz and yz odd in dz, 8 k points a block
+static bool dipolar_form(const DipolarFFT *d)
+{
+    return d->lz > 1 && d->sym && d->nzt != d->nzr && d->odd == ((1 << 2) | (1 << 4)) && d->kpb == 8;
+}
+
+// the tiles of K2_F (q = (t / (nzt kpb)) % 6) as one number each: real, imaginary for q = 2 and 4
+__global__ void k_layer_half(const double2 *__restrict__ k2b, double *__restrict__ kh, int per_q, int64_t total)
+{
+    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= total) return;
+    const int q = (int)(t / per_q % 6);
+    kh[t] = q == 2 || q == 4 ? k2b[t].y : k2b[t].x;
 }
 
 // K2_F, [q][dz][k] with k fastest (nzs offsets per component), into tiles of
@@ -341,6 +387,16 @@ __global__ void k_scale(double2 *x, int64_t n, double s)
     if (i >= n) return;
     x[i].x *= s;
     x[i].y *= s;
+}
+
+// a symmetric tensor's components (per_q points each) as real numbers, xz and yz as imaginary ones
+__global__ void k_one_part(double2 *x, int64_t per_q, int64_t n)
+{
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    const int64_t q = i / per_q;
+    if (q == 2 || q == 4) x[i].x = 0.0;
+    else x[i].y = 0.0;
 }
 
 static int make_plan(rocfft_plan *p, rocfft_transform_type t, const int nrep[3], size_t batch, int dims = 3)
@@ -438,6 +494,22 @@ static int dip_create_layers(mj_ctx *c, DipolarFFT *d, const double *K_n, int nc
     hipLaunchKernelGGL(k_scale, dim3((unsigned)((tot + 255) / 256)), dim3(256), 0, c->stream, d->kf, tot,
                        1.0 / (double)np2);
     rocfft_plan_destroy(pk);
+    // in-plane inversion: K(q)(-x, -y, dz) = K(q)(x, y, dz), its negative for xz
+    // and yz, bit for bit: the transform's other part is zero but for rounding
+    const char *henv = getenv("MJ_DIP_HALF");   // "0": as transformed (tests)
+    bool inv = d->sym && !(henv && henv[0] == '0');
+    for (int q = 0; q < 6 && inv; ++q)
+        for (int dz = 0; dz < nzr && inv; ++dz) {
+            const double *p = &kr[((size_t)q * nzr + dz) * np2];
+            const double sg = q == 2 || q == 4 ? -1.0 : 1.0;
+            for (int y = 0; y < d->nrep[1] && inv; ++y) {
+                const double *a = p + (int64_t)y * d->nrep[0], *b = p + (int64_t)((d->nrep[1] - y) % d->nrep[1]) * d->nrep[0];
+                for (int x = 0; x < d->nrep[0]; ++x) inv = inv && a[x] == sg * b[(d->nrep[0] - x) % d->nrep[0]];
+            }
+        }
+    if (inv)
+        hipLaunchKernelGGL(k_one_part, dim3((unsigned)((tot + 255) / 256)), dim3(256), 0, c->stream, d->kf,
+                           (int64_t)nzr * nc2, tot);
     // z-parity: K(q)(-dz) = +-K(q)(dz) exactly for every component (the
     // dipolar tensor: xz, yz odd), checked on K_n and again on K2_F (the
     // in-plane transform of a negated layer is the negated transform, if the
@@ -497,6 +569,19 @@ static int dip_create_layers(mj_ctx *c, DipolarFFT *d, const double *K_n, int nc
     hipFree(d->kf);
     d->kf = kb;
     hipFree(kdev);
+    if (inv && dipolar_form(d)) {
+        double *kh = nullptr;
+        if (hipMalloc(&kh, sizeof(double) * tiles) != hipSuccess) {
+            mj_set_error("mj_set_fft_operator: device allocation failed");
+            return MJ_ENOMEM;
+        }
+        hipLaunchKernelGGL(k_layer_half, dim3((unsigned)((tiles + 255) / 256)), dim3(256), 0, c->stream, d->kf, kh,
+                           nzt * d->kpb, tiles);
+        MJ_HIP_CHECK(hipStreamSynchronize(c->stream));
+        hipFree(d->kf);
+        d->kf = (double2 *)kh;
+        d->half = 1;
+    }
     return MJ_OK;
 }
 
@@ -611,11 +696,12 @@ int dip_clone(mj_ctx *dst, const mj_ctx *src)
     d->kpb = s->kpb;
     d->nzt = s->nzt;
     d->odd = s->odd;
+    d->half = s->half;
     const int ncomp = d->sym ? 6 : 9;
     size_t kbytes;
     if (d->layer) {
         const int64_t nblk = (d->nc2 + d->kpb - 1) / d->kpb;
-        kbytes = sizeof(double2) * (size_t)(nblk * ncomp * d->nzt * d->kpb);
+        kbytes = (d->half ? sizeof(double) : sizeof(double2)) * (size_t)(nblk * ncomp * d->nzt * d->kpb);
         MJ_HIP_CHECK(hipMalloc(&d->grid, sizeof(double) * 3 * d->lz * d->np2));
         if (int rc_ = alloc_grid_in(dst, d, false)) return rc_;
         MJ_HIP_CHECK(hipMalloc(&d->spec, sizeof(double2) * 3 * d->lz * d->nc2));
@@ -675,9 +761,8 @@ static int dip_apply_layers(mj_ctx *c, DipolarFFT *d, const double *m, KArgs *ka
     const size_t shm = sizeof(double2) * (size_t)(ncomp * d->nzt) * d->kpb;
     const bool par = d->nzt != d->nzr;
     const dim3 g(nb), t(d->kpb * d->lz);
-    // the dipolar tensor's parity (xz and yz odd): the kernel of that form
-    const bool dipf = d->sym && par && d->odd == ((1 << 2) | (1 << 4)) && d->kpb == 8;
-    const bool done = dipf && launch_layer_mix_dip<2>(d->lz, nb, c->stream, d->spec, d->kf, d->spec_h, d->nc2);
+    const bool done = dipolar_form(d) && (d->half ? launch_layer_mix_dip<2, true> : launch_layer_mix_dip<2, false>)(
+                                             d->lz, nb, c->stream, d->spec, d->kf, d->spec_h, d->nc2);
     if (done)
         ;   // launched above
     else if (d->sym && par)
