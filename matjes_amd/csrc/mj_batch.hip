@@ -1,11 +1,11 @@
 // Batched LLG: independent systems of uneven sizes and parallel-tempering
 // replicas advanced together, one launch per integrator stage (integration 2:
-// one fused launch per step) for the whole batch, the steps between replica
+// one fused launch per step, compiled per stencil) for the whole batch, the steps between replica
 // exchanges captured in one hipGraph; integration 2 can also run each such
 // segment as one persistent launch with grid barriers.
 //
 // Every system keeps the single-system path's arithmetic: its translation-
-// invariant stencil (classified iso | dm | gen by mj_finalize), Zeeman term,
+// invariant stencil (in mj_finalize's order of summation), Zeeman term,
 // damping and Philox stream (seed, step, site) are copied from a finalized
 // mj_ctx, and the stage kernel runs the same body (mj_stage_body.h) with a
 // geometry policy that reads the system of each workgroup from a table.  A
@@ -274,7 +274,8 @@ __device__ __forceinline__ void batch_fused_tile(const KArgs &a, const int *ofs0
     }
 }
 
-// one step of every system: base.src -> base.dst; compiled for at least 6
+// one step of every system of a batch without a compiled step (batch_groups):
+// base.src -> base.dst; compiled for at least 6
 // waves per SIMD (Heun) or 4 (SIB and Depondt, whose ring also draws the
 // thermal field: they spill at 5)
 template <int INTEG>
