@@ -231,17 +231,25 @@ __device__ __forceinline__ void adj_reduce(const AdjArgs &a, double *red, const 
         return;
     }
     const int nw = nthr >> 6;
-    double w[G::kMaxVals];
+    if constexpr (G::kConst) {   // the values' butterflies side by side
+        double w[G::kMaxVals];
 #pragma unroll
-    for (int q = 0; q < G::kMaxVals; ++q) w[q] = vals[q];
+        for (int q = 0; q < G::kMaxVals; ++q) w[q] = vals[q];
 #pragma unroll
-    for (int o = 32; o > 0; o >>= 1)
+        for (int o = 32; o > 0; o >>= 1)
+#pragma unroll
+            for (int q = 0; q < G::kMaxVals; ++q) w[q] = w[q] + __shfl_xor(w[q], o, 64);
 #pragma unroll
         for (int q = 0; q < G::kMaxVals; ++q)
-            if (q < nv) w[q] = w[q] + __shfl_xor(w[q], o, 64);
+            if ((threadIdx.x & 63) == 0) red[q * nw + (threadIdx.x >> 6)] = w[q];
+    } else {
+        for (int q = 0; q < nv; ++q) {
+            double v = vals[q];
 #pragma unroll
-    for (int q = 0; q < G::kMaxVals; ++q)
-        if (q < nv && (threadIdx.x & 63) == 0) red[q * nw + (threadIdx.x >> 6)] = w[q];
+            for (int o = 32; o > 0; o >>= 1) v = v + __shfl_xor(v, o, 64);
+            if ((threadIdx.x & 63) == 0) red[q * nw + (threadIdx.x >> 6)] = v;
+        }
+    }
     __syncthreads();
     if ((int)threadIdx.x < nv) {
         const int q = threadIdx.x;

@@ -32,43 +32,43 @@
 
 #define MJ_ADJ_MAXP kAdjMaxParam
 
-__global__ void k_adj_sib1(const AdjArgs a)
+__global__ void __launch_bounds__(256) k_adj_sib1(const AdjArgs a)
 {
     extern __shared__ double L[];
     adj_sib1_body<AdjRt>(a, L);
 }
 
-__global__ void k_adj_sib2(const AdjArgs a)
+__global__ void __launch_bounds__(256) k_adj_sib2(const AdjArgs a)
 {
     extern __shared__ double L[];
     adj_sib2_body<AdjRt>(a, L);
 }
 
-__global__ void k_adj_sibf(const AdjArgs a)
+__global__ void __launch_bounds__(256) k_adj_sibf(const AdjArgs a)
 {
     extern __shared__ double L[];
     adj_sibf_body<AdjRt>(a, L);
 }
 
-__global__ void k_adj_r1(const AdjArgs a)
+__global__ void __launch_bounds__(256) k_adj_r1(const AdjArgs a)
 {
     extern __shared__ double L[];
     adj_r1_body<AdjRt>(a, L);
 }
 
-__global__ void k_adj_r3r1(const AdjArgs a)
+__global__ void __launch_bounds__(256) k_adj_r3r1(const AdjArgs a)
 {
     extern __shared__ double L[];
     adj_r3r1_body<AdjRt>(a, L);
 }
 
-__global__ void k_adj_r2(const AdjArgs a)
+__global__ void __launch_bounds__(256) k_adj_r2(const AdjArgs a)
 {
     extern __shared__ double L[];
     adj_r2_body<AdjRt>(a, L);
 }
 
-__global__ void k_adj_r3(const AdjArgs a)
+__global__ void __launch_bounds__(256) k_adj_r3(const AdjArgs a)
 {
     extern __shared__ double L[];
     adj_r3_body<AdjRt>(a, L);

@@ -396,7 +396,7 @@ int mj_stage_alloc(MjHostStage &h, int64_t n3)
     const int64_t cap = 3 * 21824;   // 512 KiB
     h.half = std::min<int64_t>(std::max<int64_t>(n3, 192), cap);
     h.chunks = n3 > cap ? 2 : 1;
-    hipError_t e = hipHostMalloc(&h.buf, sizeof(double) * (size_t)(h.half * h.chunks), hipHostMallocDefault);
+    hipError_t e = hipHostMalloc(&h.buf, sizeof(double) * (size_t)(h.half * h.chunks), hipHostMallocCoherent);
     for (int k = 0; k < 2 && e == hipSuccess; ++k) e = hipEventCreateWithFlags(&h.ev[k], hipEventDisableTiming);
     if (e == hipSuccess) return MJ_OK;
     mj_stage_free(h);
