@@ -378,7 +378,8 @@ int mj_jit_batch_fused(const std::vector<int> &ofs3, const std::vector<int> &cls
     bool alias = false;
     const int s0x = bx + 4 * rx, s0y = by + 4 * ry, s1x = bx + 2 * rx, s1y = by + 2 * ry;
     g << "struct BatchFused {\n";
-    *shm = emit_fused_tile(g, bx, by, 1, rx, ry, rz, bx * by, 1, 1, bx * by, 0, true, T0, alias);
+    const bool dma = bx % 2 == 0;   // 16-byte pairs along x: no pair spans two rows of the region
+    *shm = emit_fused_tile(g, bx, by, 1, rx, ry, rz, bx * by, 1, 1, bx * by, 0, dma, T0, alias);
     if (*shm > 65536) {
         *fn = nullptr;
         return MJ_OK;
@@ -389,7 +390,7 @@ int mj_jit_batch_fused(const std::vector<int> &ofs3, const std::vector<int> &cls
     };
     arg("nx", "int", "a.nx"), arg("ny", "int", "a.ny"), arg("nz", "int", "a.nz");
     arg("ntx", "int", "a.ntx"), arg("nty", "int", "a.nty"), arg("nty_base", "int", "a.nty");
-    arg("bmode", "int", "a.bmode"), arg("dma", "bool", "((a.nx | a.np) & 1) == 0"), arg("block", "int", "a.vbid");
+    arg("bmode", "int", "a.bmode"), arg("dma", "bool", dma ? "((a.nx | a.np) & 1) == 0" : "false"), arg("block", "int", "a.vbid");
     auto cf = [&](int ent, int q) -> std::string {
         const int k = cls[9 * ent + q];
         return k == 0 ? std::string() : std::string(k < 0 ? "-" : "") + "a.cf[" + std::to_string(abs(k) - 1) + "]";

@@ -2,6 +2,7 @@
 for bit, where it can go wrong: one group of systems and several (a launch
 each), more groups than it takes (the ahead-of-time kernel runs), coefficients
 that differ, change sign or vanish between systems, odd rows (no paired loads),
+tiles from one site a row (rows of the region that do not pair up) to one row, inside the lattice,
 lattices smaller than a tile and its halo, open edges, a per-site field."""
 import os
 
@@ -22,6 +23,7 @@ BATCHES = {
     "reach3": [("sq", dict(size=[64, 66, 1], J=[1e-3, -0.2e-3, 0.1e-3, 0.05e-3, -0.04e-3, 0.03e-3]))] * 2,
     "five_stencils": [("sq", dict(size=[32, 32, 1], J=[1e-3, 0.2e-3, 0.1e-3, 0.05e-3, 0.04e-3][:k])) for k in range(1, 5)]
     + [("tri", dict(size=[24, 24, 1]))],
+    "long": [("sq", dict(size=[8, 1030, 1])), ("sq", dict(size=[1030, 8, 1], D=0.1e-3))],
     "vanishing": [("sq", dict(size=[48, 40, 1], J=[0.0], B=[0.0, 0.0, 0.0])), ("sq", SQ[0])],
 }
 
@@ -51,8 +53,9 @@ def _run(specs, jit, integ, tiles):
             os.environ["MJ_JIT"] = old
 
 
-@pytest.mark.parametrize("integ,tiles", [(2, None), (2, (16, 16)), (5, None), (6, None)])
-@pytest.mark.parametrize("name", sorted(BATCHES))
+@pytest.mark.parametrize("name,integ,tiles", [(n, i, t) for n in sorted(BATCHES)
+                                              for i, t in [(2, None), (2, (16, 16)), (5, None), (6, None)]]
+                         + [("long", i, t) for i, t in [(2, (1, 256)), (5, (1, 256)), (2, (2, 128)), (2, (256, 1))]])
 def test_compiled_equals_ahead_of_time(name, integ, tiles):
     ref, e0 = _run(BATCHES[name], "0", integ, tiles)
     got, e1 = _run(BATCHES[name], "1", integ, tiles)
