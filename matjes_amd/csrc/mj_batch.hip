@@ -548,7 +548,7 @@ struct HostSys {
 // systems that share a stencil's offsets and a tile: their fused step's kernels
 // (per integration, compiled on first use), their blocks and coefficient classes
 struct BatchGroup {
-    std::vector<int> ofs3, cls, blocks;
+    std::vector<int> ofs3, cls, blocks, first;   // first: a place of each class
     int bx, by, rx, ry, rz, ncls = 0;
     int *d_list = nullptr;       // their blocks (null: all of the batch's)
     double *d_vals = nullptr;    // the classes' values, ncls per system of the batch
@@ -884,7 +884,7 @@ static int batch_groups(mj_batch *b, const std::vector<BatchSys> &tab, const std
     }
     for (size_t k = 0; k < gr.size(); ++k) {
         BatchGroup &g = gr[k];
-        std::vector<int> first;   // a place of each class
+        std::vector<int> first;
         auto matches = [&](int p, int c, double sign) {
             for (size_t q = 0; q < b->sys.size(); ++q)
                 if (of[q] == (int)k && b->sys[q].cf[p] != sign * b->sys[q].cf[c]) return false;
@@ -911,20 +911,23 @@ static int batch_groups(mj_batch *b, const std::vector<BatchSys> &tab, const std
         }
         if (first.size() > 32) return MJ_OK;
         g.ncls = (int)std::max<size_t>(first.size(), 1);
+        g.first = first;
+    }
+    // every group fits: from here the batch owns them (free_dev)
+    for (size_t q = 0; q < blk2sys.size(); ++q) gr[of[blk2sys[q]]].blocks.push_back((int)q);
+    b->groups = std::move(gr);
+    for (size_t k = 0; k < b->groups.size(); ++k) {
+        BatchGroup &g = b->groups[k];
         std::vector<double> v(g.ncls * b->sys.size(), 0.0);
         for (size_t q = 0; q < b->sys.size(); ++q)
             if (of[q] == (int)k)
-                for (size_t c = 0; c < first.size(); ++c) v[q * g.ncls + c] = b->sys[q].cf[first[c]];
+                for (size_t c = 0; c < g.first.size(); ++c) v[q * g.ncls + c] = b->sys[q].cf[g.first[c]];
         if (hipMalloc(&g.d_vals, sizeof(double) * v.size()) != hipSuccess) BFAIL(MJ_ENOMEM, "mj_batch: device allocation failed");
-        b->groups.push_back(g);   // owned from here (free_dev)
         MJ_HIP_CHECK(hipMemcpy(g.d_vals, v.data(), sizeof(double) * v.size(), hipMemcpyHostToDevice));
+        if (b->groups.size() == 1) continue;
+        if (hipMalloc(&g.d_list, sizeof(int) * g.blocks.size()) != hipSuccess) BFAIL(MJ_ENOMEM, "mj_batch: device allocation failed");
+        MJ_HIP_CHECK(hipMemcpy(g.d_list, g.blocks.data(), sizeof(int) * g.blocks.size(), hipMemcpyHostToDevice));
     }
-    for (size_t q = 0; q < blk2sys.size(); ++q) b->groups[of[blk2sys[q]]].blocks.push_back((int)q);
-    if (b->groups.size() > 1)
-        for (auto &g : b->groups) {
-            MJ_HIP_CHECK(hipMalloc(&g.d_list, sizeof(int) * g.blocks.size()));
-            MJ_HIP_CHECK(hipMemcpy(g.d_list, g.blocks.data(), sizeof(int) * g.blocks.size(), hipMemcpyHostToDevice));
-        }
     return MJ_OK;
 }
 

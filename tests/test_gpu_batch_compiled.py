@@ -1,6 +1,7 @@
 """The fused batch step compiled per stencil against the ahead-of-time one, bit
 for bit, where it can go wrong: one group of systems and several (a launch
-each), more groups than it takes (the ahead-of-time kernel runs), coefficients
+each), more groups than it takes or a later group of too many coefficients (the
+ahead-of-time kernel runs), coefficients
 that differ, change sign or vanish between systems, odd rows (no paired loads),
 tiles from one site a row (rows of the region that do not pair up) to one row, inside the lattice,
 lattices smaller than a tile and its halo, open edges, a per-site field."""
@@ -24,6 +25,8 @@ BATCHES = {
     "five_stencils": [("sq", dict(size=[32, 32, 1], J=[1e-3, 0.2e-3, 0.1e-3, 0.05e-3, 0.04e-3][:k])) for k in range(1, 5)]
     + [("tri", dict(size=[24, 24, 1]))],
     "long": [("sq", dict(size=[8, 1030, 1])), ("sq", dict(size=[1030, 8, 1], D=0.1e-3))],
+    # the second stencil has more coefficients than the compiled step takes
+    "second_too_rich": [("sq", SQ[0]), ("sq", dict(size=[40, 36, 1], rich=True)), ("sq", SQ[1])],
     "vanishing": [("sq", dict(size=[48, 40, 1], J=[0.0], B=[0.0, 0.0, 0.0])), ("sq", SQ[0])],
 }
 
@@ -37,7 +40,12 @@ def _run(specs, jit, integ, tiles):
     try:
         with batch.Batch() as b:
             for k, (w, s) in enumerate(specs):
+                s = dict(s)
+                rich = s.pop("rich", False)
                 h = llg.from_case(workloads.build_case(dict(base[w], seed=5 + k, **s)), form="stencil")
+                if rich:   # 36 values more: a block of its own for each of four further neighbours
+                    rng = np.random.default_rng(1)
+                    h.add_stencil({o: 1e-4 * rng.normal(size=(3, 3)) for o in [(1, 1, 0), (2, 0, 0), (0, 2, 0), (2, 1, 0)]})
                 b.add(h, 0.05 + 0.1 * (k % 2), kT=(4.0 * k) * lattice.K_B, seed=40 + k)
                 hs.append(h)
             if tiles:
