@@ -667,7 +667,6 @@ static int mc_prepare(mj_ctx *c, const char *who)
     }
     if (ne > mc->csh_cap) {
         if (mc->d_csh) hipFree(mc->d_csh);
-    if (mc->d_cf9) hipFree(mc->d_cf9);
         mc->d_csh = nullptr;
         mc->csh_cap = ne;
         MJ_HIP_CHECK(hipMalloc(&mc->d_csh, sizeof(int) * ne));
@@ -895,6 +894,7 @@ void mj_mc_destroy(mj_ctx *c)
     if (mc->d_part) hipFree(mc->d_part);
     if (mc->d_samples) hipFree(mc->d_samples);
     if (mc->d_csh) hipFree(mc->d_csh);
+    if (mc->d_cf9) hipFree(mc->d_cf9);
     if (mc->d_cm) hipFree(mc->d_cm);
     if (mc->d_tab) hipFree(mc->d_tab);
     void *pt[] = {mc->d_rcm, mc->d_rst, mc->d_rkT, mc->d_ladder, mc->d_image, mc->d_swaps, mc->d_E4, mc->d_rpart,

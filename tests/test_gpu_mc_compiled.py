@@ -56,3 +56,29 @@ def test_compiled_equals_ahead_of_time(name, sampler, kT, reps):
     c = workloads.build_case(dict(base, seed=11, **s))
     for a, b in zip(_run(c, "0", sampler, kT, reps), _run(c, "1", sampler, kT, reps)):
         assert np.array_equal(a, b), name
+
+
+@pytest.mark.parametrize("jit", ["0", "1"])
+def test_stencil_that_grows_between_sweeps(jit, monkeypatch):
+    """A term that enlarges the stencil of a context that has already swept, against
+    a context that had it from the start."""
+    from matjes_amd import llg, workloads
+    monkeypatch.setenv("MJ_JIT", jit)
+    c = workloads.build_case(dict(workloads.SQUARE_JDKB, size=[64, 64, 1], seed=4))
+    blk = -0.1e-3 * np.eye(3)
+    more = {(2, 0, 0): blk, (-2, 0, 0): blk, (0, 2, 0): blk, (0, -2, 0): blk, (1, 1, 0): 2.0 * blk, (-1, -1, 0): 2.0 * blk}
+    out = []
+    for early in (False, True):
+        with llg.Hamiltonian(c["lat"].dim_lat, c["lat"].periodic) as h:
+            h.load_terms(c["H"], form="stencil")
+            if early:
+                h.add_stencil(more)
+            else:
+                h.set_state(c["m0"])
+                h.mc_sweeps(2, 0, 1e-3, seed=8)
+                h.add_stencil(more)
+            h.set_state(c["m0"])
+            h.mc_set_cone(0.4)
+            h.mc_sweeps(4, 1, 1e-3, seed=9)
+            out.append(h.get_state())
+    assert np.array_equal(out[0], out[1])
