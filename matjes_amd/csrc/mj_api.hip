@@ -1378,7 +1378,7 @@ static int run_steps(mj_ctx *c, int nsteps, int integ, double timestep, double a
         const double key_arr[] = {(double)integ, energies ? 1.0 : 0.0, noisy ? 1.0 : 0.0, timestep, alpha, kT,
                                   (double)(seed >> 32), (double)(seed & 0xffffffffu), (double)(uintptr_t)c->A,
                                   (double)(uintptr_t)c->Bb, (double)(uintptr_t)c->epart, (double)c->use_jit,
-                                  fused ? 1.0 : 0.0};
+                                  fused ? 1.0 : 0.0, (double)nl};   // nl: the order of integration 4
         std::vector<double> key(key_arr, key_arr + sizeof key_arr / sizeof key_arr[0]);
         if (key != c->gkey) drop_graph(c);
         if (!c->d_step) MJ_HIP_CHECK(hipMalloc(&c->d_step, sizeof(uint64_t)));

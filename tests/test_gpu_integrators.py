@@ -68,3 +68,19 @@ def test_paramagnet_equilibrium_on_device(integ, c):
             h.steps(200, integ, dt, alpha, kT=kT, seed=11, step0=2000 + 200 * k)
             acc.append(h.get_state()[:, 2].mean())
     assert abs(np.mean(acc) - _langevin(c * x)) < 0.01, (np.mean(acc), _langevin(c * x))
+
+
+def test_order_of_integration_4_between_calls():
+    """The same call of integration 4 after another order was set (both calls long
+    enough to replay a captured chunk of steps), against a context of that order."""
+    from matjes_amd import llg, workloads
+    c = workloads.build_case(dict(workloads.SQUARE_JDKB, size=[24, 20, 1], seed=6))
+    out = []
+    for orders in ((4, 2), (2,)):
+        with llg.from_case(c) as h:
+            for n in orders:
+                h.set_rk_order(n)
+                h.set_state(c["m0"])
+                E = h.steps(70, 4, 2.0, 0.2, energies=True)
+            out.append((h.get_state(), E))
+    assert np.array_equal(out[0][0], out[1][0]) and np.array_equal(out[0][1], out[1][1])
