@@ -395,7 +395,7 @@ static int pow2ceil(int v)
 // under a second once per Hamiltonian and process.
 constexpr int64_t kJitSites = 1024;
 
-static void tile_shape(const mj_ctx *c, int rz, int &bx, int &by, int &bz)
+static void tile_shape(const mj_ctx *c, int &bx, int &by, int &bz)
 {
     if (c->bx && c->by && c->bz) {
         bx = c->bx;
@@ -414,17 +414,27 @@ static void tile_shape(const mj_ctx *c, int rz, int &bx, int &by, int &bz)
     // 64x64x16 6.4 against 10.8, 96x96x2 5.8 against 10.1; 32x4x2 and 32x2x4 do not
     // fit either).  With a dipolar term, a launch per stage: 256x256x16 2153 us
     // for 8 steps against 2276.
-    if (c->n >= kJitSites && rz > 0) {
+    // A tile whose region (with the padding of its direct fill) passes the 160 KiB
+    // of LDS a workgroup can have gives way to smaller ones: reach 6 across the
+    // planes needs 168 KiB at 16x4x4 and 122 at 8x8x1.
+    auto fits = [&]() {
+        const int64_t region = (int64_t)(bx + 2 * c->rx) * (by + 2 * c->ry) * (bz + 2 * c->rz);
+        return 24 * (region + 2 * bx * by * bz) <= 163840;
+    };
+    if (c->n >= kJitSites && c->rz > 0) {
         bx = std::min(pow2ceil(c->dim[0]), 16);
         bz = std::min(pow2ceil(c->dim[2]), 4);
         by = std::min(pow2ceil(c->dim[1]), 256 / (bx * bz));
-        if (bx * by * bz >= 64) return;
+        if (bx * by * bz >= 64 && fits()) return;
     }
     int nthr = 256;
     while (c->n < kJitSites && nthr > 64 && c->n / nthr < 512) nthr >>= 1;
-    bx = std::min(pow2ceil(c->dim[0]), std::max(8, nthr / 8));
-    by = std::min(pow2ceil(c->dim[1]), std::max(1, nthr / bx));
-    bz = std::min(pow2ceil(c->dim[2]), std::max(1, nthr / (bx * by)));
+    for (;; nthr >>= 1) {
+        bx = std::min(pow2ceil(c->dim[0]), std::max(8, nthr / 8));
+        by = std::min(pow2ceil(c->dim[1]), std::max(1, nthr / bx));
+        bz = std::min(pow2ceil(c->dim[2]), std::max(1, nthr / (bx * by)));
+        if (nthr <= 64 || fits()) break;
+    }
     while (bx * by * bz < 64 && (bx * by * bz) < c->n) {
         // keep at least one full wavefront per tile when the lattice allows it
         if (by < pow2ceil(c->dim[1])) by <<= 1;
@@ -554,7 +564,7 @@ int mj_finalize(mj_ctx *c)
             c->ry = std::max(c->ry, std::abs(o[1]));
             c->rz = std::max(c->rz, std::abs(o[2]));
         }
-        tile_shape(c, c->rz, bx, by, bz);
+        tile_shape(c, bx, by, bz);
         const int sx = bx + 2 * c->rx, sy = by + 2 * c->ry;
         std::vector<double> cf_iso, cf_dm, cf_gen;
         std::vector<int> o3_iso, o3_dm, o3_gen;
@@ -642,7 +652,7 @@ int mj_finalize(mj_ctx *c)
     }
     // energy partial buffers
     int bx, by, bz;
-    tile_shape(c, c->rz, bx, by, bz);
+    tile_shape(c, bx, by, bz);
     int nb = ((c->dim[0] + bx - 1) / bx) * ((c->dim[1] + by - 1) / by) * ((c->dim[2] + bz - 1) / bz);
     if (c->epart_cap < nb) {
         if (c->epart) hipFree(c->epart);
@@ -664,7 +674,7 @@ static void base_args(const mj_ctx *c, KArgs &a)
     a.px = c->periodic[0];
     a.py = c->periodic[1];
     a.pz = c->periodic[2];
-    tile_shape(c, c->rz, a.bx, a.by, a.bz);
+    tile_shape(c, a.bx, a.by, a.bz);
     a.rx = c->rx;
     a.ry = c->ry;
     a.rz = c->rz;

@@ -45,3 +45,26 @@ def test_default_tile_equals_the_stage_kernels(name, integ, T):
     from matjes_amd import workloads
     c = workloads.build_case(dict(workloads.FILM_DIP, dipolar=False, D=0.3e-3, mediator_dz=-0.5, seed=2, **CASES[name]))
     assert np.array_equal(_run(c, None, "1", integ, T), _run(c, (32, 8, 1), "0", integ, T))
+
+
+@pytest.mark.parametrize("size,reach", [([16, 16, 16], 6), ([16, 16, 8], 4), ([64, 64, 1], 31), ([70, 66, 1], 33)])
+@pytest.mark.parametrize("jit", ["0", "1"])
+def test_long_reach_fits_the_lds(size, reach, jit, monkeypatch):
+    """Bonds so long that the usual tile's region passes the LDS: the field of
+    -J m_(i +- reach) along every axis, each value a sum of at most six products
+    and their doubling."""
+    from matjes_amd import llg, workloads
+    monkeypatch.setenv("MJ_JIT", jit)
+    axes = [a for a in range(3) if size[a] > 1]
+    ofs = [tuple(s * reach * (a == b) for b in range(3)) for a in axes for s in (1, -1)
+           if not (s < 0 and 2 * reach == size[a])]
+    m = workloads.random_sphere(int(np.prod(size)), 9)
+    with llg.Hamiltonian(size, [True, True, size[2] > 1]) as h:
+        h.add_stencil({o: -1e-3 * np.eye(3) for o in ofs})
+        h.set_state(m)
+        B = h.get_eff_field()
+        h.steps(2, 2, 0.1, 0.1)
+    g = m.reshape(size[2], size[1], size[0], 3)
+    want = sum(2e-3 * 0.5 * (np.roll(g, (-o[2], -o[1], -o[0]), (0, 1, 2)) + np.roll(g, (o[2], o[1], o[0]), (0, 1, 2)))
+               for o in ofs).reshape(-1, 3)
+    assert np.max(np.abs(B - want)) <= 8 * 2.0 ** -53 * 1e-3 * 2 * len(ofs)
