@@ -261,8 +261,7 @@ static int adj_launch(const AdjState *s, int kind, const AdjArgs &a, int ntiles,
     hipLaunchKernelGGL(aot[kind], dim3(a.nblocks), dim3(nthr), shm, st, a);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) {
-        mj_set_error(std::string("adjoint kernel launch: ") + hipGetErrorString(e));
-        return MJ_EHIP;
+        return mj_hip_fail(MJ_EHIP, std::string("adjoint kernel launch: ") + hipGetErrorString(e));
     }
     return MJ_OK;
 }
@@ -278,8 +277,7 @@ static int adj_alloc(double **p, size_t n)
     if (*p) hipFree(*p);
     *p = nullptr;
     if (hipMalloc(p, sizeof(double) * std::max<size_t>(n, 1)) != hipSuccess) {
-        mj_set_error("adjoint: device allocation failed");
-        return MJ_ENOMEM;
+        return mj_hip_fail(MJ_ENOMEM, "adjoint: device allocation failed");
     }
     return MJ_OK;
 }
@@ -380,15 +378,13 @@ static int adj_segment_fwd(mj_ctx *c, AdjState *s, int len)
         if (rc != MJ_OK || e != hipSuccess) {
             if (g) (void)hipGraphDestroy(g);
             if (rc != MJ_OK) return rc;
-            mj_set_error(std::string("adjoint forward capture: ") + hipGetErrorString(e));
-            return MJ_EHIP;
+            return mj_hip_fail(MJ_EHIP, std::string("adjoint forward capture: ") + hipGetErrorString(e));
         }
         e = hipGraphInstantiate(&s->g_fwd, g, nullptr, nullptr, 0);
         (void)hipGraphDestroy(g);
         if (e != hipSuccess) {
             s->g_fwd = nullptr;
-            mj_set_error(std::string("adjoint forward graph: ") + hipGetErrorString(e));
-            return MJ_EHIP;
+            return mj_hip_fail(MJ_EHIP, std::string("adjoint forward graph: ") + hipGetErrorString(e));
         }
     }
     MJ_HIP_CHECK(hipGraphLaunch(s->g_fwd, c->stream));
@@ -586,15 +582,13 @@ static int adj_segment_rev(mj_ctx *c, AdjState *s, int len)
         if (rc != MJ_OK || e != hipSuccess) {
             if (g) (void)hipGraphDestroy(g);
             if (rc != MJ_OK) return rc;
-            mj_set_error(std::string("adjoint reverse capture: ") + hipGetErrorString(e));
-            return MJ_EHIP;
+            return mj_hip_fail(MJ_EHIP, std::string("adjoint reverse capture: ") + hipGetErrorString(e));
         }
         e = hipGraphInstantiate(&s->g_rev, g, nullptr, nullptr, 0);
         (void)hipGraphDestroy(g);
         if (e != hipSuccess) {
             s->g_rev = nullptr;
-            mj_set_error(std::string("adjoint reverse graph: ") + hipGetErrorString(e));
-            return MJ_EHIP;
+            return mj_hip_fail(MJ_EHIP, std::string("adjoint reverse graph: ") + hipGetErrorString(e));
         }
     }
     MJ_HIP_CHECK(hipGraphLaunch(s->g_rev, c->stream));

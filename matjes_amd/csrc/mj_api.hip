@@ -37,10 +37,11 @@ static int launch(mj_ctx *c, int mode, bool noise, const KArgs &a);
 static thread_local std::string g_err;
 void mj_set_error(const std::string &msg) { g_err = msg; }
 
-#define MJ_FAIL(code, msg)        \
-    do {                          \
-        mj_set_error(msg);        \
-        return (code);            \
+#define MJ_FAIL(code, msg)                                                            \
+    do {                                                                              \
+        if ((code) == MJ_EHIP || (code) == MJ_ENOMEM) return mj_hip_fail(code, msg);  \
+        mj_set_error(msg);                                                            \
+        return (code);                                                                \
     } while (0)
 #define MJ_TRY(x)               \
     do {                        \
@@ -996,14 +997,12 @@ extern "C" int mj_math_probe(mj_ctx *c, int fn, int64_t n, const double *x, doub
     MJ_HIP_CHECK(hipMalloc(&d, sizeof(double) * 2 * (size_t)n));
     int rc = MJ_OK;
     if (hipMemcpy(d, x, sizeof(double) * n, hipMemcpyHostToDevice) != hipSuccess) {
-        mj_set_error("mj_math_probe: copy in");
-        rc = MJ_EHIP;
+        rc = mj_hip_fail(MJ_EHIP, "mj_math_probe: copy in");
     }
     if (rc == MJ_OK) rc = mj_launch_math_probe(fn, n, d, d + n, c->stream);
     if (rc == MJ_OK && (hipMemcpyAsync(y, d + n, sizeof(double) * n, hipMemcpyDeviceToHost, c->stream) != hipSuccess ||
                         hipStreamSynchronize(c->stream) != hipSuccess)) {
-        mj_set_error("mj_math_probe: copy out");
-        rc = MJ_EHIP;
+        rc = mj_hip_fail(MJ_EHIP, "mj_math_probe: copy out");
     }
     hipFree(d);
     return rc;

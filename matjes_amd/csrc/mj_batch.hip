@@ -603,10 +603,11 @@ struct mj_batch {
     std::vector<uint64_t> k_acc, k_att;
 };
 
-#define BFAIL(code, msg)    \
-    do {                    \
-        mj_set_error(msg);  \
-        return (code);      \
+#define BFAIL(code, msg)                                                              \
+    do {                                                                              \
+        if ((code) == MJ_EHIP || (code) == MJ_ENOMEM) return mj_hip_fail(code, msg);  \
+        mj_set_error(msg);                                                            \
+        return (code);                                                                \
     } while (0)
 #define BTRY(x)                     \
     do {                            \

@@ -58,8 +58,7 @@ struct DipolarFFT {
 static int rf_check(rocfft_status s, const char *what)
 {
     if (s != rocfft_status_success) {
-        mj_set_error(std::string("rocFFT ") + what + " failed (status " + std::to_string((int)s) + ")");
-        return MJ_EHIP;
+        return mj_hip_fail(MJ_EHIP, std::string("rocFFT ") + what + " failed (status " + std::to_string((int)s) + ")");
     }
     return MJ_OK;
 }
@@ -560,8 +559,7 @@ static int dip_create_layers(mj_ctx *c, DipolarFFT *d, const double *K_n, int nc
     double2 *kb = nullptr;
     if (hipMalloc(&kb, sizeof(double2) * tiles) != hipSuccess) {
         hipFree(kdev);
-        mj_set_error("mj_set_fft_operator: device allocation failed");
-        return MJ_ENOMEM;
+        return mj_hip_fail(MJ_ENOMEM, "mj_set_fft_operator: device allocation failed");
     }
     hipLaunchKernelGGL(k_layer_tiles, dim3((unsigned)((tiles + 255) / 256)), dim3(256), 0, c->stream, d->kf, kb, nc2,
                        ncomp, nzr, nzt, d->kpb, tiles);
@@ -572,8 +570,7 @@ static int dip_create_layers(mj_ctx *c, DipolarFFT *d, const double *K_n, int nc
     if (inv && dipolar_form(d)) {
         double *kh = nullptr;
         if (hipMalloc(&kh, sizeof(double) * tiles) != hipSuccess) {
-            mj_set_error("mj_set_fft_operator: device allocation failed");
-            return MJ_ENOMEM;
+            return mj_hip_fail(MJ_ENOMEM, "mj_set_fft_operator: device allocation failed");
         }
         hipLaunchKernelGGL(k_layer_half, dim3((unsigned)((tiles + 255) / 256)), dim3(256), 0, c->stream, d->kf, kh,
                            nzt * d->kpb, tiles);
@@ -782,8 +779,7 @@ static int dip_apply_layers(mj_ctx *c, DipolarFFT *d, const double *m, KArgs *ka
     RF_TRY(rocfft_execute(d->inv, in2, out2, d->info), "execute inverse (2D)");
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) {
-        mj_set_error(std::string("dipolar kernels: ") + hipGetErrorString(e));
-        return MJ_EHIP;
+        return mj_hip_fail(MJ_EHIP, std::string("dipolar kernels: ") + hipGetErrorString(e));
     }
     ka->hdip = d->grid;
     ka->dnx = d->nrep[0];
@@ -812,8 +808,7 @@ int dip_apply(mj_ctx *c, const double *m, KArgs *ka)
     RF_TRY(rocfft_execute(d->inv, in2, out2, d->info), "execute inverse");
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) {
-        mj_set_error(std::string("dipolar kernels: ") + hipGetErrorString(e));
-        return MJ_EHIP;
+        return mj_hip_fail(MJ_EHIP, std::string("dipolar kernels: ") + hipGetErrorString(e));
     }
     ka->hdip = d->grid;
     ka->dnx = d->nrep[0];

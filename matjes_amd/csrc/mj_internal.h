@@ -10,13 +10,19 @@
 
 void mj_set_error(const std::string &msg);
 
-#define MJ_HIP_CHECK(call)                                                                       \
-    do {                                                                                         \
-        hipError_t e_ = (call);                                                                  \
-        if (e_ != hipSuccess) {                                                                  \
-            mj_set_error(std::string(#call) + ": " + hipGetErrorString(e_));                     \
-            return MJ_EHIP;                                                                      \
-        }                                                                                        \
+// a HIP call failed: the message, and the error taken off the runtime's record,
+// where the next launch's check would find it again
+inline int mj_hip_fail(int code, const std::string &msg)
+{
+    (void)hipGetLastError();
+    mj_set_error(msg);
+    return code;
+}
+
+#define MJ_HIP_CHECK(call)                                                                                    \
+    do {                                                                                                      \
+        hipError_t e_ = (call);                                                                               \
+        if (e_ != hipSuccess) return mj_hip_fail(MJ_EHIP, std::string(#call) + ": " + hipGetErrorString(e_)); \
     } while (0)
 
 #include "mj_kargs.h"

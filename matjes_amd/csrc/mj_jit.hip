@@ -342,10 +342,7 @@ static int compile_source(const std::string &src, hipModule_t *out)
     hiprtcDestroyProgram(&prog);
     hipModule_t mod;
     hipError_t e = hipModuleLoadData(&mod, code.data());
-    if (e != hipSuccess) {
-        mj_set_error(std::string("hipModuleLoadData: ") + hipGetErrorString(e));
-        return MJ_EHIP;
-    }
+    if (e != hipSuccess) return mj_hip_fail(MJ_EHIP, std::string("hipModuleLoadData: ") + hipGetErrorString(e));
     g_mod_cache[src] = mod;
     *out = mod;
     return MJ_OK;
@@ -411,10 +408,7 @@ int mj_jit_batch_fused(const std::vector<int> &ofs3, const std::vector<int> &cls
     const int rc = compile_source(s.str(), &mod);
     if (rc != MJ_OK) return rc;
     const hipError_t e = hipModuleGetFunction(fn, mod, "mj_batch_fused");
-    if (e != hipSuccess) {
-        mj_set_error(std::string("hipModuleGetFunction mj_batch_fused: ") + hipGetErrorString(e));
-        return MJ_EHIP;
-    }
+    if (e != hipSuccess) return mj_hip_fail(MJ_EHIP, std::string("hipModuleGetFunction mj_batch_fused: ") + hipGetErrorString(e));
     return MJ_OK;
 }
 
@@ -498,10 +492,7 @@ int mj_jit_adjoint(const mj_ctx *c, const AdjStencil &st, const int b[3], const 
     for (int k = 0; k < MJ_ADJ_KERNELS; ++k) {
         if (!want(k)) continue;
         const hipError_t e = hipModuleGetFunction(&fn[k], mod, (std::string("mj_adj_") + names[k]).c_str());
-        if (e != hipSuccess) {
-            mj_set_error(std::string("hipModuleGetFunction: ") + hipGetErrorString(e));
-            return MJ_EHIP;
-        }
+        if (e != hipSuccess) return mj_hip_fail(MJ_EHIP, std::string("hipModuleGetFunction: ") + hipGetErrorString(e));
     }
     return MJ_OK;
 }
@@ -609,10 +600,7 @@ int mj_jit_mc(const mj_ctx *c, const std::vector<int> &o3, const std::vector<dou
     if (rc != MJ_OK) return rc;
     hipError_t e = hipModuleGetFunction(pass, mod, "mj_mc_pass");
     if (e == hipSuccess) e = hipModuleGetFunction(energy, mod, "mj_mc_energy");
-    if (e != hipSuccess) {
-        mj_set_error(std::string("hipModuleGetFunction: ") + hipGetErrorString(e));
-        return MJ_EHIP;
-    }
+    if (e != hipSuccess) return mj_hip_fail(MJ_EHIP, std::string("hipModuleGetFunction: ") + hipGetErrorString(e));
     return MJ_OK;
 }
 
@@ -669,10 +657,7 @@ static int jit_resolve(mj_ctx *c, int mode, bool noise, hipFunction_t *out)
         char name[64];
         snprintf(name, sizeof name, "mj_stage_%d_%d", mode, noise ? 1 : 0);
         hipError_t e = hipModuleGetFunction(&f, mod, name);
-        if (e != hipSuccess) {
-            mj_set_error(std::string("hipModuleGetFunction ") + name + ": " + hipGetErrorString(e));
-            return MJ_EHIP;
-        }
+        if (e != hipSuccess) return mj_hip_fail(MJ_EHIP, std::string("hipModuleGetFunction ") + name + ": " + hipGetErrorString(e));
         j->fn[mode][noise ? 1 : 0] = f;
     }
     *out = f;
@@ -709,15 +694,11 @@ static int jit_resolve_persistent(mj_ctx *c, int mode, hipFunction_t *out, int *
         snprintf(name, sizeof name, "mj_pstage_%d", mode);
         hipFunction_t f;
         hipError_t e = hipModuleGetFunction(&f, mod, name);
-        if (e != hipSuccess) {
-            mj_set_error(std::string("hipModuleGetFunction ") + name + ": " + hipGetErrorString(e));
-            return MJ_EHIP;
-        }
+        if (e != hipSuccess) return mj_hip_fail(MJ_EHIP, std::string("hipModuleGetFunction ") + name + ": " + hipGetErrorString(e));
         int per_cu = 0, ncu = 0;
         if (hipModuleOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, f, j->nthr, j->pers_shm) != hipSuccess ||
             hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, c->device) != hipSuccess) {
-            mj_set_error("persistent stage kernel: occupancy query failed");
-            return MJ_EHIP;
+            return mj_hip_fail(MJ_EHIP, "persistent stage kernel: occupancy query failed");
         }
         int g = std::max(1, per_cu) * std::max(1, ncu);
         g = std::min(g, j->nblocks);
@@ -748,10 +729,7 @@ int mj_jit_launch(mj_ctx *c, int mode, bool noise, const KArgs &a, hipStream_t s
         void *params[] = {&arg};
         hipError_t e = hipModuleLaunchKernel(fp, (unsigned)grid, 1, 1, (unsigned)j->nthr, 1, 1, (unsigned)j->pers_shm, s,
                                              params, nullptr);
-        if (e != hipSuccess) {
-            mj_set_error(std::string("hipModuleLaunchKernel (persistent): ") + hipGetErrorString(e));
-            return MJ_EHIP;
-        }
+        if (e != hipSuccess) return mj_hip_fail(MJ_EHIP, std::string("hipModuleLaunchKernel (persistent): ") + hipGetErrorString(e));
         return MJ_OK;
     }
     hipFunction_t f;
@@ -763,9 +741,6 @@ int mj_jit_launch(mj_ctx *c, int mode, bool noise, const KArgs &a, hipStream_t s
     hipError_t e = hipModuleLaunchKernel(f, (unsigned)(fused ? j->fuse_nblocks : a.nblocks), 1, 1,
                                          (unsigned)(fused ? j->fuse_nthr : j->nthr), 1, 1,
                                          (unsigned)(fused ? j->fuse_shm : j->shm), s, params, nullptr);
-    if (e != hipSuccess) {
-        mj_set_error(std::string("hipModuleLaunchKernel: ") + hipGetErrorString(e));
-        return MJ_EHIP;
-    }
+    if (e != hipSuccess) return mj_hip_fail(MJ_EHIP, std::string("hipModuleLaunchKernel: ") + hipGetErrorString(e));
     return MJ_OK;
 }

@@ -44,15 +44,18 @@ __global__ void k_math_probe(int fn, int64_t n, const double *x, double *y)
     y[i] = r;
 }
 
+static int launched(const char *what)
+{
+    const hipError_t e = hipGetLastError();
+    if (e == hipSuccess) return MJ_OK;
+    mj_set_error(std::string(what) + ": " + hipGetErrorString(e));
+    return MJ_EHIP;
+}
+
 int mj_launch_math_probe(int fn, int64_t n, const double *x, double *y, hipStream_t s)
 {
     hipLaunchKernelGGL(k_math_probe, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, fn, n, x, y);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) {
-        mj_set_error(std::string("math probe launch: ") + hipGetErrorString(e));
-        return MJ_EHIP;
-    }
-    return MJ_OK;
+    return launched("math probe launch");
 }
 
 // energy partials -> E with the fold of a stage kernel's block 0 (blockDim =
@@ -290,23 +293,13 @@ __global__ void __launch_bounds__(256) k_term_mult(const TermArgs t)
 int mj_launch_term_mult(const TermArgs &t, int64_t n, hipStream_t s)
 {
     hipLaunchKernelGGL(k_term_mult, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, t);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) {
-        mj_set_error(std::string("term product launch: ") + hipGetErrorString(e));
-        return MJ_EHIP;
-    }
-    return MJ_OK;
+    return launched("term product launch");
 }
 
 int mj_launch_term_energy(const TermArgs &t, int nblocks, hipStream_t s)
 {
     hipLaunchKernelGGL(k_term_energy, dim3(nblocks), dim3(256), 0, s, t);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) {
-        mj_set_error(std::string("term energy launch: ") + hipGetErrorString(e));
-        return MJ_EHIP;
-    }
-    return MJ_OK;
+    return launched("term energy launch");
 }
 
 int mj_launch_stage(int mode, bool noise, const KArgs &args, hipStream_t s)
@@ -322,51 +315,31 @@ int mj_launch_stage(int mode, bool noise, const KArgs &args, hipStream_t s)
     size_t need = (size_t)nthr * sizeof(double);
     if (shm < need) shm = need;  // block reduction scratch
     hipLaunchKernelGGL(f, dim3(a.nblocks), dim3(nthr), shm, s, a);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) {
-        mj_set_error(std::string("stage kernel launch: ") + hipGetErrorString(e));
-        return MJ_EHIP;
-    }
-    return MJ_OK;
+    return launched("stage kernel launch");
 }
 
 int mj_launch_reduce(const double *part, int n, double *out, double scale, hipStream_t s)
 {
     hipLaunchKernelGGL(k_reduce, dim3(1), dim3(1024), 0, s, part, n, out, scale);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) {
-        mj_set_error(std::string("reduce launch: ") + hipGetErrorString(e));
-        return MJ_EHIP;
-    }
-    return MJ_OK;
+    return launched("reduce launch");
 }
 
 int mj_launch_fold(const double *part, int n, double *out, double scale, int nthr, hipStream_t s)
 {
     hipLaunchKernelGGL(k_fold, dim3(1), dim3(nthr), sizeof(double) * nthr, s, part, n, out, scale);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) {
-        mj_set_error(std::string("fold launch: ") + hipGetErrorString(e));
-        return MJ_EHIP;
-    }
-    return MJ_OK;
+    return launched("fold launch");
 }
 
 int mj_launch_reduce_max(const double *part, int n, double *out, hipStream_t s)
 {
     hipLaunchKernelGGL(k_reduce_max, dim3(1), dim3(1024), 0, s, part, n, out);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) {
-        mj_set_error(std::string("reduce launch: ") + hipGetErrorString(e));
-        return MJ_EHIP;
-    }
-    return MJ_OK;
+    return launched("reduce launch");
 }
 
 int mj_launch_step_counter(uint64_t *p, uint64_t v, int add, hipStream_t s)
 {
     hipLaunchKernelGGL(k_step_counter, dim3(1), dim3(64), 0, s, p, v, add);
-    return hipGetLastError() == hipSuccess ? MJ_OK : MJ_EHIP;
+    return launched("step counter launch");
 }
 
 int mj_launch_spmv(const mj_ctx *c, const double *m, double *out, hipStream_t s)
@@ -374,19 +347,19 @@ int mj_launch_spmv(const mj_ctx *c, const double *m, double *out, hipStream_t s)
     int64_t n3 = 3 * c->n;
     hipLaunchKernelGGL(k_spmv_sym, dim3((unsigned)((n3 + 255) / 256)), dim3(256), 0, s, n3, c->d_rp, c->d_ci,
                        c->d_v, m, c->np, out);
-    return hipGetLastError() == hipSuccess ? MJ_OK : MJ_EHIP;
+    return launched("operator product launch");
 }
 
 int mj_launch_aos2soa(const double *in, double *out, int64_t n, int64_t np, hipStream_t s)
 {
     hipLaunchKernelGGL(k_aos2soa, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, in, out, n, np);
-    return hipGetLastError() == hipSuccess ? MJ_OK : MJ_EHIP;
+    return launched("layout launch");
 }
 
 int mj_launch_soa2aos(const double *in, double *out, int64_t n, int64_t np, double eps, hipStream_t s)
 {
     hipLaunchKernelGGL(k_soa2aos, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, in, out, n, np, eps);
-    return hipGetLastError() == hipSuccess ? MJ_OK : MJ_EHIP;
+    return launched("layout launch");
 }
 
 int mj_stage_alloc(MjHostStage &h, int64_t n3)
@@ -400,8 +373,7 @@ int mj_stage_alloc(MjHostStage &h, int64_t n3)
     for (int k = 0; k < 2 && e == hipSuccess; ++k) e = hipEventCreateWithFlags(&h.ev[k], hipEventDisableTiming);
     if (e == hipSuccess) return MJ_OK;
     mj_stage_free(h);
-    mj_set_error(std::string("pinned staging memory: ") + hipGetErrorString(e));
-    return MJ_ENOMEM;
+    return mj_hip_fail(MJ_ENOMEM, std::string("pinned staging memory: ") + hipGetErrorString(e));
 }
 
 void mj_stage_free(MjHostStage &h)
@@ -427,7 +399,7 @@ static int download(MjHostStage &h, const double *dev, int64_t total, int64_t np
             const int m = (int)std::min(step, total - k * step);
             hipLaunchKernelGGL(k_to_host<SITES>, dim3((m + 255) / 256), dim3(256), 0, s, dev,
                                h.buf + (h.chunks == 2 ? k % 2 : 0) * step, SITES ? k * step / 3 : k * step, m, np, eps);
-            if (hipGetLastError() != hipSuccess) return MJ_EHIP;
+            if (int rc = launched("copy to the host")) return rc;
             MJ_HIP_CHECK(hipEventRecord(h.ev[k % 2], s));
         }
         const int64_t q = h.chunks == 2 ? k - 1 : k;   // one buffer: its chunk at once
@@ -456,7 +428,7 @@ int mj_upload(MjHostStage &h, const double *host, double *soa, int64_t n, int64_
     const int m = (int)(3 * n);
     memcpy(h.buf, host, sizeof(double) * (size_t)m);
     hipLaunchKernelGGL(k_from_host, dim3((m + 255) / 256), dim3(256), 0, s, h.buf, soa, m, np);
-    if (hipGetLastError() != hipSuccess) return MJ_EHIP;
+    if (int rc = launched("copy from the host")) return rc;
     MJ_HIP_CHECK(hipStreamSynchronize(s));
     return MJ_OK;
 }
@@ -464,5 +436,5 @@ int mj_upload(MjHostStage &h, const double *host, double *soa, int64_t n, int64_
 int mj_launch_normals(uint64_t seed, uint64_t step, int64_t n, double *out, hipStream_t s)
 {
     hipLaunchKernelGGL(k_normals, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, seed, step, n, out);
-    return hipGetLastError() == hipSuccess ? MJ_OK : MJ_EHIP;
+    return launched("thermal field launch");
 }

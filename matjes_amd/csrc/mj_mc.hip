@@ -35,10 +35,11 @@
 #include "mj_stage_body.h"
 #include "mj_mc_body.h"
 
-#define MJ_FAIL(code, msg)        \
-    do {                          \
-        mj_set_error(msg);        \
-        return (code);            \
+#define MJ_FAIL(code, msg)                                                            \
+    do {                                                                              \
+        if ((code) == MJ_EHIP || (code) == MJ_ENOMEM) return mj_hip_fail(code, msg);  \
+        mj_set_error(msg);                                                            \
+        return (code);                                                                \
     } while (0)
 #define MJ_TRY(x)                   \
     do {                            \
@@ -923,13 +924,11 @@ extern "C" int mj_energy_single(mj_ctx *c, int64_t n, const int64_t *sites1, con
     int rc = MJ_OK;
     if (hipMalloc(&d_sites, sizeof(int64_t) * n) != hipSuccess || hipMalloc(&d_e, sizeof(double) * n) != hipSuccess ||
         (spins && hipMalloc(&d_spins, sizeof(double) * 3 * n) != hipSuccess)) {
-        mj_set_error("mj_energy_single: device allocation failed");
-        rc = MJ_ENOMEM;
+        rc = mj_hip_fail(MJ_ENOMEM, "mj_energy_single: device allocation failed");
     }
     if (rc == MJ_OK && (hipMemcpy(d_sites, s0.data(), sizeof(int64_t) * n, hipMemcpyHostToDevice) != hipSuccess ||
                         (spins && hipMemcpy(d_spins, spins, sizeof(double) * 3 * n, hipMemcpyHostToDevice) != hipSuccess))) {
-        mj_set_error("mj_energy_single: copy to the device failed");
-        rc = MJ_EHIP;
+        rc = mj_hip_fail(MJ_EHIP, "mj_energy_single: copy to the device failed");
     }
     if (rc == MJ_OK) {
         McArgs a;
@@ -943,8 +942,7 @@ extern "C" int mj_energy_single(mj_ctx *c, int64_t n, const int64_t *sites1, con
         rc = launch_check("energy_single launch");
         if (rc == MJ_OK && (hipMemcpyAsync(E, d_e, sizeof(double) * n, hipMemcpyDeviceToHost, c->stream) != hipSuccess ||
                             hipStreamSynchronize(c->stream) != hipSuccess)) {
-            mj_set_error("mj_energy_single: copy back failed");
-            rc = MJ_EHIP;
+            rc = mj_hip_fail(MJ_EHIP, "mj_energy_single: copy back failed");
         }
     }
     if (d_sites) hipFree(d_sites);

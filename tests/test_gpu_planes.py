@@ -68,3 +68,20 @@ def test_long_reach_fits_the_lds(size, reach, jit, monkeypatch):
     want = sum(2e-3 * 0.5 * (np.roll(g, (-o[2], -o[1], -o[0]), (0, 1, 2)) + np.roll(g, (o[2], o[1], o[0]), (0, 1, 2)))
                for o in ofs).reshape(-1, 3)
     assert np.max(np.abs(B - want)) <= 8 * 2.0 ** -53 * 1e-3 * 2 * len(ofs)
+
+
+@pytest.mark.parametrize("jit", ["0", "1"])
+def test_refused_launch_stays_with_its_call(jit, monkeypatch):
+    """A reach for which no tile fits (nothing is launched): the call that asks for it
+    fails, and the next one, of another context, does not."""
+    from matjes_amd import _lib, llg, workloads
+    monkeypatch.setenv("MJ_JIT", jit)
+    m = workloads.random_sphere(20 ** 3, 9)
+    with llg.Hamiltonian([20, 20, 20], [True, True, True]) as bad, llg.Hamiltonian([20, 20, 20], [True] * 3) as good:
+        bad.add_stencil({(9, 0, 0): np.eye(3), (0, 9, 0): np.eye(3), (0, 0, 9): np.eye(3)})
+        good.add_stencil({(1, 0, 0): np.eye(3)})
+        bad.set_state(m)
+        with pytest.raises(_lib.MatjesError, match="invalid argument"):
+            bad.get_eff_field()
+        good.set_state(m)
+        assert np.array_equal(good.get_state(), m)
