@@ -940,7 +940,7 @@ static int batch_resolve(mj_batch *b)
     for (auto &g : b->groups) {
         hipFunction_t &fn = g.fn[fused_slot(b->integ)];
         const int mode = b->integ == MJ_SIB ? MODE_SIBF : b->integ == MJ_DEPONDT ? MODE_DEPF : MODE_HEUNF;
-        if (!fn) BTRY(mj_jit_batch_fused(g.ofs3, g.cls, g.ncls, g.bx, g.by, g.rx, g.ry, g.rz, mode, &fn, &g.shm));
+        if (!fn) BTRY(mj_jit_batch_fused(b->device, g.ofs3, g.cls, g.ncls, g.bx, g.by, g.rx, g.ry, g.rz, mode, &fn, &g.shm));
     }
     return MJ_OK;
 }

@@ -149,8 +149,8 @@ int mj_jit_adjoint(const mj_ctx *c, const AdjStencil &st, const int b[3], const 
 int mj_jit_mc(const mj_ctx *c, const std::vector<int> &o3, const std::vector<double> &cf9, const std::vector<int> &csh,
               int p, int ca, int cb, hipFunction_t *pass, hipFunction_t *energy);
 // the fused step of a batch's systems of one stencil and tile (fn null: its tile does not fit in LDS)
-int mj_jit_batch_fused(const std::vector<int> &ofs3, const std::vector<int> &cls, int ncls, int bx, int by, int rx,
-                       int ry, int rz, int mode, hipFunction_t *fn, size_t *shm);
+int mj_jit_batch_fused(int device, const std::vector<int> &ofs3, const std::vector<int> &cls, int ncls, int bx, int by,
+                       int rx, int ry, int rz, int mode, hipFunction_t *fn, size_t *shm);
 
 void mj_adj_destroy(mj_ctx *c);   // mj_adjoint.hip
 void mj_mc_destroy(mj_ctx *c);    // mj_mc.hip

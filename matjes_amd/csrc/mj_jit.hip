@@ -17,12 +17,12 @@
 #include <algorithm>
 #include <array>
 #include <map>
-#include <mutex>
 #include <sstream>
 #include <string>
 #include <vector>
 
 #include "mj_internal.h"
+#include "mj_modcache.h"
 #include "_jit_embed.h"   // kJitRngH, kJitDeviceH, kJitKargsH, kJitBodyH (generated by matjes_amd/build.py)
 
 struct JitState {
@@ -46,9 +46,6 @@ static bool persistent_mode(int mode)
 {
     return mode == MODE_HEUN1 || mode == MODE_EULER || mode == MODE_SIB1 || mode == MODE_DEP1;
 }
-
-static std::mutex g_jit_mu;
-static std::map<std::string, hipModule_t> g_mod_cache;   // full source -> module
 
 static void hexd(std::ostringstream &o, double v)
 {
@@ -309,15 +306,9 @@ std::string mj_jit_source(const mj_ctx *c, int fam)
     return c->jit ? family_source((const JitState *)c->jit, fam) : std::string();
 }
 
-// the module of a source text: compiled once per process
-static int compile_source(const std::string &src, hipModule_t *out)
+// compiles a source and loads it on the current device
+static int compile_module(const std::string &src, hipModule_t *out)
 {
-    std::lock_guard<std::mutex> lk(g_jit_mu);
-    auto it = g_mod_cache.find(src);
-    if (it != g_mod_cache.end()) {
-        *out = it->second;
-        return MJ_OK;
-    }
     hiprtcProgram prog;
     if (hiprtcCreateProgram(&prog, src.c_str(), "mj_stage_jit.hip", 0, nullptr, nullptr) != HIPRTC_SUCCESS) {
         mj_set_error("hiprtcCreateProgram failed");
@@ -343,12 +334,21 @@ static int compile_source(const std::string &src, hipModule_t *out)
     hipModule_t mod;
     hipError_t e = hipModuleLoadData(&mod, code.data());
     if (e != hipSuccess) return mj_hip_fail(MJ_EHIP, std::string("hipModuleLoadData: ") + hipGetErrorString(e));
-    g_mod_cache[src] = mod;
     *out = mod;
     return MJ_OK;
 }
 
-static int compile_family(JitState *j, int fam, hipModule_t *out) { return compile_source(family_source(j, fam), out); }
+// the module of a source text on a device (the caller's current one)
+static int compile_source(int device, const std::string &src, hipModule_t *out)
+{
+    static ModCache<hipModule_t> *cache = new ModCache<hipModule_t>();   // to the process's end
+    return cache->get(device, src, out, [&](hipModule_t *m) { return compile_module(src, m); });
+}
+
+static int compile_family(const mj_ctx *c, JitState *j, int fam, hipModule_t *out)
+{
+    return compile_source(c->device, family_source(j, fam), out);
+}
 
 static std::string device_headers()
 {
@@ -367,8 +367,8 @@ static std::string device_headers()
 // (18 neighbours, T > 0) and 12 more lattices of 32 to 400 a side, 2.2 M sites:
 // 50 us a step, the ahead-of-time kernel (k_batch_fused: offsets and full 3x3
 // blocks read in a loop, wrapped coordinates per staged site) 81 us.
-int mj_jit_batch_fused(const std::vector<int> &ofs3, const std::vector<int> &cls, int ncls, int bx, int by, int rx,
-                       int ry, int rz, int mode, hipFunction_t *fn, size_t *shm)
+int mj_jit_batch_fused(int device, const std::vector<int> &ofs3, const std::vector<int> &cls, int ncls, int bx, int by,
+                       int rx, int ry, int rz, int mode, hipFunction_t *fn, size_t *shm)
 {
     std::ostringstream g;
     int T0 = 0;
@@ -405,7 +405,7 @@ int mj_jit_batch_fused(const std::vector<int> &ofs3, const std::vector<int> &cls
          "  const int s = blk2sys[gb];\n  KArgs a = sys_args(base, sys[s], gb, sigma[s], *stepp + base.step);\n"
          "  a.cf = vals + (int64_t)s * " << ncls << ";\n  fused_body<" << mode << ", true, BatchFused>(a, lds);\n}\n";
     hipModule_t mod;
-    const int rc = compile_source(s.str(), &mod);
+    const int rc = compile_source(device, s.str(), &mod);
     if (rc != MJ_OK) return rc;
     const hipError_t e = hipModuleGetFunction(fn, mod, "mj_batch_fused");
     if (e != hipSuccess) return mj_hip_fail(MJ_EHIP, std::string("hipModuleGetFunction mj_batch_fused: ") + hipGetErrorString(e));
@@ -487,7 +487,7 @@ int mj_jit_adjoint(const mj_ctx *c, const AdjStencil &st, const int b[3], const 
             s << "extern \"C\" __global__ void __launch_bounds__(" << nthr << ") mj_adj_" << names[k]
               << "(const AdjArgs a) { extern __shared__ double lds[]; adj_" << names[k] << "_body<AdjJit>(a, lds); }\n";
     hipModule_t mod;
-    const int rc = compile_source(s.str(), &mod);
+    const int rc = compile_source(c->device, s.str(), &mod);
     if (rc != MJ_OK) return rc;
     for (int k = 0; k < MJ_ADJ_KERNELS; ++k) {
         if (!want(k)) continue;
@@ -596,7 +596,7 @@ int mj_jit_mc(const mj_ctx *c, const std::vector<int> &o3, const std::vector<dou
     s << "extern \"C\" __global__ void __launch_bounds__(kMcThreads) mj_mc_energy(const McArgs a, double *part) { "
          "mc_energy_body<McGeom>(a, part); }\n";
     hipModule_t mod;
-    const int rc = compile_source(s.str(), &mod);
+    const int rc = compile_source(c->device, s.str(), &mod);
     if (rc != MJ_OK) return rc;
     hipError_t e = hipModuleGetFunction(pass, mod, "mj_mc_pass");
     if (e == hipSuccess) e = hipModuleGetFunction(energy, mod, "mj_mc_energy");
@@ -648,7 +648,7 @@ static int jit_resolve(mj_ctx *c, int mode, bool noise, hipFunction_t *out)
         auto it = j->mods.find(fam);
         hipModule_t mod;
         if (it == j->mods.end()) {
-            int rc = compile_family(j, fam, &mod);
+            int rc = compile_family(c, j, fam, &mod);
             if (rc) return rc;
             j->mods[fam] = mod;
         } else {
