@@ -113,6 +113,7 @@ struct AdjState {
     int nsteps = 0, ckpt_every = 0, ncp = 0;
     double alpha = 0.0, dt = 0.0;
     std::vector<double> theta;
+    int ready = 0;                   // a forward pass has run to its end with the buffers and sizes held here
     int last_valid = 0;              // segm/segp hold the last segment of the forward pass
     // graphs of one full segment (ckpt_every steps): forward recompute, reverse sweep
     hipGraphExec_t g_fwd = nullptr, g_rev = nullptr;
@@ -402,6 +403,8 @@ extern "C" int mj_adjoint_forward(mj_ctx *c, const double *theta, const double *
     }
     MJ_HIP_CHECK(hipSetDevice(c->device));
     AdjState *s = ADJ(c);
+    s->ready = 0;
+    adj_drop_graphs(s);   // their launches hold the buffers and kernels replaced below
     s->theta.assign(theta, theta + s->nparam);
     s->nsteps = nsteps;
     s->ckpt_every = ckpt_every;
@@ -500,7 +503,6 @@ extern "C" int mj_adjoint_forward(mj_ctx *c, const double *theta, const double *
     const unsigned nb = (unsigned)((c->n + 255) / 256);
     hipLaunchKernelGGL(k_adj_bmap, dim3(nb), dim3(256), 0, c->stream, s->d_bext, hmap_dev, s->d_bmap, c->n, c->np);
     // forward with checkpoints: segment by segment, states kept as in the recompute
-    adj_drop_graphs(s);
     s->last_valid = 0;
     hipLaunchKernelGGL(k_adj_aos_soa, dim3(nb), dim3(256), 0, c->stream, m0_dev, s->segm, c->n, c->np, 1);
     int len = 0;
@@ -517,6 +519,7 @@ extern "C" int mj_adjoint_forward(mj_ctx *c, const double *theta, const double *
     hipLaunchKernelGGL(k_adj_aos_soa, dim3(nb), dim3(256), 0, c->stream, s->segm + n3 * len, mfinal_dev, c->n, c->np,
                        0);
     MJ_HIP_CHECK(hipStreamSynchronize(c->stream));
+    s->ready = 1;
     return MJ_OK;
 }
 
@@ -603,7 +606,7 @@ extern "C" int mj_adjoint_backward(mj_ctx *c, const double *gfinal_dev, double *
         return MJ_EINVAL;
     }
     AdjState *s = ADJ(c);
-    if (s->nsteps < 1 || !s->ckpt) {
+    if (!s->ready) {
         mj_set_error("mj_adjoint_backward: call mj_adjoint_forward first");
         return MJ_ESTATE;
     }
@@ -613,12 +616,12 @@ extern "C" int mj_adjoint_backward(mj_ctx *c, const double *gfinal_dev, double *
     adj_args(c, s, a0);
     const int nv = s->nparam + 3;
     if (!s->g) {   // kept until the next mj_adjoint_setup (sizes fixed per context and parameter set)
-        ATRY(adj_alloc(&s->g, n3));
         ATRY(adj_alloc(&s->gB, 2 * n3));
         ATRY(adj_alloc(&s->gacc, n3));
         ATRY(adj_alloc(&s->gpd, n3));
         ATRY(adj_alloc(&s->ghmap, n3));
         ATRY(adj_alloc(&s->ppart, (size_t)a0.nblocks * nv));
+        ATRY(adj_alloc(&s->g, n3));   // last: there only when all are
     }
     MJ_HIP_CHECK(hipMemsetAsync(s->ghmap, 0, sizeof(double) * n3, c->stream));
     MJ_HIP_CHECK(hipMemsetAsync(s->ppart, 0, sizeof(double) * a0.nblocks * nv, c->stream));

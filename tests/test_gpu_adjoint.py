@@ -247,3 +247,28 @@ def test_bad_arguments():
         assert rc == _lib.MJ_ESTATE          # no Zeeman term registered
         rc = L_.mj_adjoint_backward(d.ctx, None, None, None, None, None)
         assert rc == _lib.MJ_EINVAL
+
+
+def test_backward_after_a_failed_forward_is_refused():
+    """A forward pass whose buffers cannot be had (2^30 states a segment) after one
+    that ran: there is nothing to go back over, until a forward pass runs again."""
+    import torch
+    from matjes_amd import _lib, adjoint
+    lat = _lat((8, 6, 1))
+    _, _, hd, m0d = _inputs(lat)
+    r = adjoint.SIBRunner(lat, NAMES, nsteps=6, timestep=1.0, damping=0.2, ckpt_every=3)
+    try:
+        out, g, gh, gm = torch.empty_like(m0d), torch.ones_like(m0d), torch.empty_like(m0d), torch.empty_like(m0d)
+        r.forward(THETA, [0.1, -0.2, 0.5], hd, m0d, out)
+        want = r.backward(g, gh, gm)
+        r.ckpt_every = 2 ** 30
+        with pytest.raises(_lib.MatjesError, match="allocation"):
+            r.forward(THETA, [0.1, -0.2, 0.5], hd, m0d, out)
+        with pytest.raises(_lib.MatjesError, match="forward first"):
+            r.backward(g, gh, gm)
+        r.ckpt_every = 3
+        r.forward(THETA, [0.1, -0.2, 0.5], hd, m0d, out)
+        got = r.backward(g, gh, gm)
+        assert all(np.array_equal(a, b) for a, b in zip(want, got))
+    finally:
+        r.close()
