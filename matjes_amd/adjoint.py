@@ -65,7 +65,7 @@ class SIBRunner:
         _lib.check(self._L.mj_adjoint_setup(self.h.ctx, len(blocks), ctypes.c_void_p(nofs.ctypes.data),
                                             ctypes.c_void_p(ofs.ctypes.data), ctypes.c_void_p(blk.ctypes.data)),
                    "mj_adjoint_setup")
-        self._last = None   # id of the inputs of the last forward
+        self._passes = 0    # forward passes so far; the last one's number is the trajectory in the buffers
 
     def forward(self, theta, b_ext, hmap, m0, out):
         import torch
@@ -77,12 +77,12 @@ class SIBRunner:
             if not (t.is_cuda and t.dtype == torch.float64 and t.is_contiguous() and t.shape == (self.n, 3)):
                 raise ValueError("m0, hmap and the output must be contiguous float64 (N,3) GPU tensors")
         torch.cuda.current_stream().synchronize()
+        self._passes += 1
         _lib.check(self._L.mj_adjoint_forward(self.h.ctx, ctypes.c_void_p(th.ctypes.data),
                                               ctypes.c_void_p(be.ctypes.data),
                                               None if hmap is None else _tp(hmap), _tp(m0), self.nsteps,
                                               self.timestep, self.damping, self.ckpt_every, _tp(out)),
                    "mj_adjoint_forward")
-        self._last = (th.tobytes(), be.tobytes(), None if hmap is None else hmap.data_ptr(), m0.data_ptr())
         return out
 
     def backward(self, gfinal, ghmap, gm0):
@@ -120,12 +120,13 @@ def _make_function():
             out = torch.empty_like(m0c)
             runner.forward(_np(theta), _np(b_ext), hc, m0c, out)
             ctx.runner = runner
-            ctx.key = runner._last
+            ctx.key = runner._passes
             # the tensor inputs go through save_for_backward: autograd then
             # refuses a backward after an in-place change of m0 or hmap (the
             # runner's checkpoints would belong to the old values)
             ctx.save_for_backward(hmap, m0)
-            ctx.params = (_np(theta), _np(b_ext))
+            # copies: an optimizer changes theta and b_ext in place between this and backward
+            ctx.params = (_np(theta).copy(), _np(b_ext).copy())
             ctx.meta = (theta, b_ext)
             return out
 
@@ -136,7 +137,7 @@ def _make_function():
             th, be = ctx.params
             m0c = m0.detach().contiguous()
             hc = None if hmap is None else hmap.detach().contiguous()
-            if runner._last != ctx.key:      # another forward ran since: recompute this one
+            if runner._passes != ctx.key:    # another forward ran since: recompute this one
                 runner.forward(th, be, hc, m0c, torch.empty_like(m0c))
             g = g.detach().contiguous()
             ghm = torch.empty_like(m0c) if ctx.needs_input_grad[2] else None

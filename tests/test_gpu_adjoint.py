@@ -272,3 +272,36 @@ def test_backward_after_a_failed_forward_is_refused():
         assert all(np.array_equal(a, b) for a, b in zip(want, got))
     finally:
         r.close()
+
+
+@pytest.mark.parametrize("between", ["start_of_another_layout", "theta_in_place"])
+def test_backward_of_an_earlier_forward(between):
+    """Two forward passes, then the first one's backward: its gradient is the one it
+    has by itself, bit for bit, also where the starts reach the runner as copies
+    (rows of another layout) and where theta has changed in place since."""
+    import torch
+    from matjes_amd import adjoint
+    lat = _lat((8, 6, 1))
+    _, _, hd, m0d = _inputs(lat)
+    r = adjoint.SIBRunner(lat, NAMES, nsteps=20, timestep=1.0, damping=0.2, ckpt_every=10)
+
+    def start(x):
+        x = x.t().contiguous().t() if between == "start_of_another_layout" else x.clone()
+        return x.requires_grad_(True)
+    try:
+        grads = []
+        for alone in (True, False):
+            theta = torch.tensor(THETA, dtype=torch.float64, requires_grad=True)
+            a, b = start(m0d), start(m0d.flip(0))
+            out = adjoint.sib_trajectory(theta, [0.1, -0.2, 0.5], hd, a, r)
+            if not alone:
+                adjoint.sib_trajectory(theta, [0.1, -0.2, 0.5], hd, b, r)
+                if between == "theta_in_place":
+                    with torch.no_grad():
+                        theta.mul_(1.5)
+            (out * out.detach().roll(1, 1)).sum().backward()
+            grads.append((theta.grad.numpy().copy(), a.grad.cpu().numpy()))
+        for x, y in zip(*grads):
+            assert np.array_equal(x, y)
+    finally:
+        r.close()
