@@ -222,6 +222,11 @@ int mj_profile_steps(mj_ctx *ctx, int nsteps, int integrator, double timestep, d
  * 3 1.0 / x. */
 int mj_math_probe(mj_ctx *ctx, int fn, int64_t n, const double *x, double *y);
 
+/* Modules of kernels compiled at run time (tests; no counterpart in the
+ * reference): how many this process has compiled, and how many it keeps beside
+ * those its objects hold.  Either pointer may be null. */
+int mj_jit_stats(int64_t *compiled, int64_t *kept);
+
 /* Thermal normals of one step (for inspection/tests): out (AoS 3N) = N(0,1) draws. */
 int mj_thermal_normals(mj_ctx *ctx, uint64_t seed, uint64_t step, double *out, int64_t n3);
 

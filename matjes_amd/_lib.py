@@ -27,7 +27,7 @@ EXPORTS = [
     "mj_batch_info", "mj_energy_single", "mj_mc_sweeps", "mj_mc_set_cone", "mj_mc_stats", "mj_term_mult",
     "mj_mc_pt_setup", "mj_mc_pt_sweeps", "mj_mc_pt_state", "mj_mc_pt_get_state", "mj_set_bfield_maps",
     "mj_steps_driven", "mj_energy_noalloc", "mj_set_rk_order", "mj_math_probe", "mj_keep_last_field",
-    "mj_last_field", "mj_steps_temperature",
+    "mj_last_field", "mj_steps_temperature", "mj_jit_stats",
 ]
 
 _lib = None
@@ -74,6 +74,7 @@ def _sig(L):
     L.mj_set_tile.argtypes = [vp, c_int, c_int, c_int]
     L.mj_set_rk_order.argtypes = [vp, c_int]
     L.mj_math_probe.argtypes = [vp, c_int, c_i64, vp, vp]
+    L.mj_jit_stats.argtypes = [vp, vp]
     L.mj_adjoint_setup.argtypes = [vp, c_int, vp, vp, vp]
     L.mj_adjoint_forward.argtypes = [vp, vp, vp, vp, vp, c_int, c_dbl, c_dbl, c_int, vp]
     L.mj_adjoint_backward.argtypes = [vp, vp, vp, vp, vp, vp]

@@ -105,6 +105,7 @@ struct AdjState {
     double *d_cf = nullptr, *d_pcf = nullptr;
     double *d_cls = nullptr;         // compiled kernels: the total stencil's distinct values
     hipFunction_t fn[MJ_ADJ_KERNELS] = {};   // (null: ahead-of-time)
+    JitRef mod;                              // their module
     double *d_bext = nullptr, *d_bmap = nullptr;
     double *ckpt = nullptr;          // ncp * 3np
     double *segm = nullptr, *segp = nullptr;   // (ckpt + 1) * 3np and ckpt * 3np
@@ -339,7 +340,7 @@ static int adj_compile(mj_ctx *c, AdjState *s, const std::vector<std::array<int,
     ATRY(adj_alloc(&s->d_cls, vals.size()));
     if (!vals.empty())
         MJ_HIP_CHECK(hipMemcpy(s->d_cls, vals.data(), sizeof(double) * vals.size(), hipMemcpyHostToDevice));
-    return mj_jit_adjoint(c, st, b, r, s->d_ofs0 != nullptr, s->fn);
+    return mj_jit_adjoint(c, st, b, r, s->d_ofs0 != nullptr, &s->mod, s->fn);
 }
 
 // one forward SIB step from x_in to x_out (SoA), storing the midpoint in pbuf:

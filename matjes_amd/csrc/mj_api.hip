@@ -110,11 +110,11 @@ extern "C" int mj_destroy(mj_ctx **pc)
     mj_ctx *c = *pc;
     hipSetDevice(c->device);
     if (c->stream) hipStreamSynchronize(c->stream);
+    drop_graph(c);   // its launches hold the kernels of c->jit
     if (c->dip) dip_destroy(c);
     if (c->jit) mj_jit_destroy(c);
     if (c->adj) mj_adj_destroy(c);
     if (c->mc) mj_mc_destroy(c);
-    drop_graph(c);
     if (c->d_step) hipFree(c->d_step);
     if (c->estage) hipFree(c->estage);
     mj_stage_free(c->host);

@@ -553,6 +553,7 @@ struct BatchGroup {
     int *d_list = nullptr;       // their blocks (null: all of the batch's)
     double *d_vals = nullptr;    // the classes' values, ncls per system of the batch
     hipFunction_t fn[3] = {};    // Heun, SIB, Depondt
+    JitRef mod[3];               // their modules
     size_t shm = 0;
 };
 
@@ -940,7 +941,8 @@ static int batch_resolve(mj_batch *b)
     for (auto &g : b->groups) {
         hipFunction_t &fn = g.fn[fused_slot(b->integ)];
         const int mode = b->integ == MJ_SIB ? MODE_SIBF : b->integ == MJ_DEPONDT ? MODE_DEPF : MODE_HEUNF;
-        if (!fn) BTRY(mj_jit_batch_fused(b->device, g.ofs3, g.cls, g.ncls, g.bx, g.by, g.rx, g.ry, g.rz, mode, &fn, &g.shm));
+        if (!fn) BTRY(mj_jit_batch_fused(b->device, g.ofs3, g.cls, g.ncls, g.bx, g.by, g.rx, g.ry, g.rz, mode, &g.mod[fused_slot(b->integ)], &fn,
+                                             &g.shm));
     }
     return MJ_OK;
 }

@@ -3,6 +3,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <memory>
 #include <string>
 #include <vector>
 
@@ -128,6 +129,14 @@ struct mj_ctx {
 
 int mj_finalize(mj_ctx *c);   // build device-side Hamiltonian if dirty
 
+// a compiled module on its device, unloaded with its last holder
+struct JitModule {
+    int device = 0;
+    hipModule_t mod = nullptr;
+    ~JitModule();
+};
+using JitRef = std::shared_ptr<JitModule>;
+
 // per-Hamiltonian stage kernels (mj_jit.hip)
 int mj_jit_prepare(mj_ctx *c, int bx, int by, int bz, int nblocks, int ntx, int nty);
 int mj_jit_launch(mj_ctx *c, int mode, bool noise, const KArgs &a, hipStream_t s);
@@ -143,14 +152,14 @@ struct AdjStencil {
     std::vector<std::vector<double>> pblk;
 };
 int mj_jit_adjoint(const mj_ctx *c, const AdjStencil &st, const int b[3], const int r[3], bool fused,
-                   hipFunction_t fn[MJ_ADJ_KERNELS]);
+                   JitRef *mod, hipFunction_t fn[MJ_ADJ_KERNELS]);
 // Monte Carlo kernels of a stencil without its on-site entry (offsets o3, full blocks cf9, class shifts csh) on the
 // context's lattice coloured (x + ca y + cb z) mod p
 int mj_jit_mc(const mj_ctx *c, const std::vector<int> &o3, const std::vector<double> &cf9, const std::vector<int> &csh,
-              int p, int ca, int cb, hipFunction_t *pass, hipFunction_t *energy);
+              int p, int ca, int cb, JitRef *mod, hipFunction_t *pass, hipFunction_t *energy);
 // the fused step of a batch's systems of one stencil and tile (fn null: its tile does not fit in LDS)
 int mj_jit_batch_fused(int device, const std::vector<int> &ofs3, const std::vector<int> &cls, int ncls, int bx, int by,
-                       int rx, int ry, int rz, int mode, hipFunction_t *fn, size_t *shm);
+                       int rx, int ry, int rz, int mode, JitRef *mod, hipFunction_t *fn, size_t *shm);
 
 void mj_adj_destroy(mj_ctx *c);   // mj_adjoint.hip
 void mj_mc_destroy(mj_ctx *c);    // mj_mc.hip

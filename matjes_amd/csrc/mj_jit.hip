@@ -7,8 +7,8 @@
 // sum is fully unrolled with immediate LDS offsets and the block coefficients
 // as exact literals.  The kernel body is the same source as the
 // ahead-of-time kernel (mj_stage_body.h) with the same summation order, so
-// the two give identical results; modules are cached per source text and
-// compiled per integrator family on first use.
+// the two give identical results; modules are found by their source text
+// (mj_modcache.h) and compiled per integrator family on first use.
 #include <hip/hiprtc.h>
 #include <stdio.h>
 #include <stdlib.h>
@@ -27,7 +27,7 @@
 
 struct JitState {
     std::string geom;              // generated geometry + stencil source
-    std::map<int, hipModule_t> mods;  // family -> module
+    std::map<int, JitRef> mods;    // family -> module
     hipFunction_t fn[12][2] = {};     // resolved kernels per (mode, noise)
     int nthr = 0;
     size_t shm = 0;
@@ -294,7 +294,7 @@ int mj_jit_prepare(mj_ctx *c, int bx, int by, int bz, int nblocks, int ntx, int 
 
 void mj_jit_destroy(mj_ctx *c)
 {
-    delete (JitState *)c->jit;   // modules stay cached for the process
+    delete (JitState *)c->jit;
     c->jit = nullptr;
 }
 
@@ -306,8 +306,18 @@ std::string mj_jit_source(const mj_ctx *c, int fam)
     return c->jit ? family_source((const JitState *)c->jit, fam) : std::string();
 }
 
-// compiles a source and loads it on the current device
-static int compile_module(const std::string &src, hipModule_t *out)
+JitModule::~JitModule()
+{
+    int cur = 0;
+    (void)hipGetDevice(&cur);
+    (void)hipSetDevice(device);
+    (void)hipDeviceSynchronize();   // its kernels are done
+    (void)hipModuleUnload(mod);
+    (void)hipSetDevice(cur);
+}
+
+// compiles a source and loads it on `device` (the current one)
+static int compile_module(int device, const std::string &src, JitRef *out)
 {
     hiprtcProgram prog;
     if (hiprtcCreateProgram(&prog, src.c_str(), "mj_stage_jit.hip", 0, nullptr, nullptr) != HIPRTC_SUCCESS) {
@@ -334,18 +344,35 @@ static int compile_module(const std::string &src, hipModule_t *out)
     hipModule_t mod;
     hipError_t e = hipModuleLoadData(&mod, code.data());
     if (e != hipSuccess) return mj_hip_fail(MJ_EHIP, std::string("hipModuleLoadData: ") + hipGetErrorString(e));
-    *out = mod;
+    *out = std::make_shared<JitModule>();
+    (*out)->device = device;
+    (*out)->mod = mod;
     return MJ_OK;
 }
 
-// the module of a source text on a device (the caller's current one)
-static int compile_source(int device, const std::string &src, hipModule_t *out)
+// the modules of the process: 64 (some 0.1 MB each) beside those in use
+static ModCache<JitModule> &modules()
 {
-    static ModCache<hipModule_t> *cache = new ModCache<hipModule_t>();   // to the process's end
-    return cache->get(device, src, out, [&](hipModule_t *m) { return compile_module(src, m); });
+    static auto *cache = new ModCache<JitModule>(64);   // never destroyed: the runtime ends first
+    return *cache;
 }
 
-static int compile_family(const mj_ctx *c, JitState *j, int fam, hipModule_t *out)
+// the module of a source text on a device (the caller's current one)
+static int compile_source(int device, const std::string &src, JitRef *out)
+{
+    return modules().get(device, src, out, [&](JitRef *m) { return compile_module(device, src, m); });
+}
+
+extern "C" int mj_jit_stats(int64_t *compiled, int64_t *kept)
+{
+    long long a = 0, b = 0;
+    modules().stats(&a, &b);
+    if (compiled) *compiled = a;
+    if (kept) *kept = b;
+    return MJ_OK;
+}
+
+static int compile_family(const mj_ctx *c, JitState *j, int fam, JitRef *out)
 {
     return compile_source(c->device, family_source(j, fam), out);
 }
@@ -368,7 +395,7 @@ static std::string device_headers()
 // 50 us a step, the ahead-of-time kernel (k_batch_fused: offsets and full 3x3
 // blocks read in a loop, wrapped coordinates per staged site) 81 us.
 int mj_jit_batch_fused(int device, const std::vector<int> &ofs3, const std::vector<int> &cls, int ncls, int bx, int by,
-                       int rx, int ry, int rz, int mode, hipFunction_t *fn, size_t *shm)
+                       int rx, int ry, int rz, int mode, JitRef *mod, hipFunction_t *fn, size_t *shm)
 {
     std::ostringstream g;
     int T0 = 0;
@@ -404,10 +431,9 @@ int mj_jit_batch_fused(int device, const std::vector<int> &ofs3, const std::vect
          "  const int b = mj_xcd_remap(blockIdx.x, nlist);\n  const int gb = list ? list[b] : b;\n"
          "  const int s = blk2sys[gb];\n  KArgs a = sys_args(base, sys[s], gb, sigma[s], *stepp + base.step);\n"
          "  a.cf = vals + (int64_t)s * " << ncls << ";\n  fused_body<" << mode << ", true, BatchFused>(a, lds);\n}\n";
-    hipModule_t mod;
-    const int rc = compile_source(device, s.str(), &mod);
+    const int rc = compile_source(device, s.str(), mod);
     if (rc != MJ_OK) return rc;
-    const hipError_t e = hipModuleGetFunction(fn, mod, "mj_batch_fused");
+    const hipError_t e = hipModuleGetFunction(fn, (*mod)->mod, "mj_batch_fused");
     if (e != hipSuccess) return mj_hip_fail(MJ_EHIP, std::string("hipModuleGetFunction mj_batch_fused: ") + hipGetErrorString(e));
     return MJ_OK;
 }
@@ -421,7 +447,7 @@ int mj_jit_batch_fused(int device, const std::vector<int> &ofs3, const std::vect
 // neighbours, 3 parameters: forward step 7.9 -> 4.2 us, R2 11.1 -> 4.8, R3 with
 // R1 11.2 -> 4.9.
 int mj_jit_adjoint(const mj_ctx *c, const AdjStencil &st, const int b[3], const int r[3], bool fused,
-                   hipFunction_t fn[MJ_ADJ_KERNELS])
+                   JitRef *mod, hipFunction_t fn[MJ_ADJ_KERNELS])
 {
     std::ostringstream g;
     const int nthr = b[0] * b[1] * b[2];
@@ -486,12 +512,11 @@ int mj_jit_adjoint(const mj_ctx *c, const AdjStencil &st, const int b[3], const 
         if (want(k))
             s << "extern \"C\" __global__ void __launch_bounds__(" << nthr << ") mj_adj_" << names[k]
               << "(const AdjArgs a) { extern __shared__ double lds[]; adj_" << names[k] << "_body<AdjJit>(a, lds); }\n";
-    hipModule_t mod;
-    const int rc = compile_source(c->device, s.str(), &mod);
+    const int rc = compile_source(c->device, s.str(), mod);
     if (rc != MJ_OK) return rc;
     for (int k = 0; k < MJ_ADJ_KERNELS; ++k) {
         if (!want(k)) continue;
-        const hipError_t e = hipModuleGetFunction(&fn[k], mod, (std::string("mj_adj_") + names[k]).c_str());
+        const hipError_t e = hipModuleGetFunction(&fn[k], (*mod)->mod, (std::string("mj_adj_") + names[k]).c_str());
         if (e != hipSuccess) return mj_hip_fail(MJ_EHIP, std::string("hipModuleGetFunction: ") + hipGetErrorString(e));
     }
     return MJ_OK;
@@ -507,7 +532,7 @@ int mj_jit_adjoint(const mj_ctx *c, const AdjStencil &st, const int b[3], const 
 // constants 8.1 and 6.6; replica energies 34.6 -> 22.  Blocks of 64 and 128
 // threads: 8 and 2 % slower at 1024^2, equal at 256^2.
 int mj_jit_mc(const mj_ctx *c, const std::vector<int> &o3, const std::vector<double> &cf9, const std::vector<int> &csh,
-              int p, int ca, int cb, hipFunction_t *pass, hipFunction_t *energy)
+              int p, int ca, int cb, JitRef *mod, hipFunction_t *pass, hipFunction_t *energy)
 {
     constexpr int kGroup = 18;
     const int nx = c->dim[0], ny = c->dim[1], nz = c->dim[2], W = (nx + p - 1) / p, ne = (int)csh.size();
@@ -595,11 +620,10 @@ int mj_jit_mc(const mj_ctx *c, const std::vector<int> &o3, const std::vector<dou
          "mc_pass_body<McGeom>(a); }\n";
     s << "extern \"C\" __global__ void __launch_bounds__(kMcThreads) mj_mc_energy(const McArgs a, double *part) { "
          "mc_energy_body<McGeom>(a, part); }\n";
-    hipModule_t mod;
-    const int rc = compile_source(c->device, s.str(), &mod);
+    const int rc = compile_source(c->device, s.str(), mod);
     if (rc != MJ_OK) return rc;
-    hipError_t e = hipModuleGetFunction(pass, mod, "mj_mc_pass");
-    if (e == hipSuccess) e = hipModuleGetFunction(energy, mod, "mj_mc_energy");
+    hipError_t e = hipModuleGetFunction(pass, (*mod)->mod, "mj_mc_pass");
+    if (e == hipSuccess) e = hipModuleGetFunction(energy, (*mod)->mod, "mj_mc_energy");
     if (e != hipSuccess) return mj_hip_fail(MJ_EHIP, std::string("hipModuleGetFunction: ") + hipGetErrorString(e));
     return MJ_OK;
 }
@@ -646,7 +670,7 @@ static int jit_resolve(mj_ctx *c, int mode, bool noise, hipFunction_t *out)
     if (!f) {
         int fam = family_of(mode);
         auto it = j->mods.find(fam);
-        hipModule_t mod;
+        JitRef mod;
         if (it == j->mods.end()) {
             int rc = compile_family(c, j, fam, &mod);
             if (rc) return rc;
@@ -656,7 +680,7 @@ static int jit_resolve(mj_ctx *c, int mode, bool noise, hipFunction_t *out)
         }
         char name[64];
         snprintf(name, sizeof name, "mj_stage_%d_%d", mode, noise ? 1 : 0);
-        hipError_t e = hipModuleGetFunction(&f, mod, name);
+        hipError_t e = hipModuleGetFunction(&f, mod->mod, name);
         if (e != hipSuccess) return mj_hip_fail(MJ_EHIP, std::string("hipModuleGetFunction ") + name + ": " + hipGetErrorString(e));
         j->fn[mode][noise ? 1 : 0] = f;
     }
@@ -689,7 +713,7 @@ static int jit_resolve_persistent(mj_ctx *c, int mode, hipFunction_t *out, int *
         hipFunction_t f0;
         int rc = jit_resolve(c, mode, false, &f0);   // compiles the family
         if (rc != MJ_OK) return rc;
-        hipModule_t mod = j->mods[family_of(mode)];
+        hipModule_t mod = j->mods[family_of(mode)]->mod;
         char name[64];
         snprintf(name, sizeof name, "mj_pstage_%d", mode);
         hipFunction_t f;

@@ -469,6 +469,7 @@ static_assert(kMcIsing == MJ_MC_ISING, "sampler codes");
 
 struct McCtx {
     hipFunction_t fn_pass = nullptr, fn_energy = nullptr;   // compiled for this stencil and lattice (null: ahead-of-time)
+    JitRef mod;
     int resolved = 0;
     // stencil without the on-site entry, and the colouring it admits
     std::vector<int> o3;
@@ -763,7 +764,8 @@ static int mc_resolve(mj_ctx *c, McCtx *mc, int64_t sites)
         return MJ_OK;
     }
     if (mc->resolved) return MJ_OK;
-    MJ_TRY(mj_jit_mc(c, mc->o3, mc->cf9, mc->csh, mc->p, mc->ca, mc->cb, &mc->fn_pass, &mc->fn_energy));
+    MJ_TRY(mj_jit_mc(c, mc->o3, mc->cf9, mc->csh, mc->p, mc->ca, mc->cb, &mc->mod, &mc->fn_pass,
+                     &mc->fn_energy));
     mc->resolved = 1;
     return MJ_OK;
 }

@@ -177,3 +177,29 @@ def test_persistent_stage_kernels_equal_one_tile_per_workgroup(which, integ, T):
         b = _run_env(c, {"MJ_PERSIST": "1"}, integ, n, kT)
         assert np.array_equal(a[1], b[1]), (which, integ, n)
         assert np.array_equal(a[0], b[0]), (which, integ, n)
+
+
+def _stats():
+    import ctypes
+    from matjes_amd import _lib
+    v = (ctypes.c_int64 * 2)()
+    _lib.check(_lib.load().mj_jit_stats(ctypes.addressof(v), ctypes.addressof(v) + 8), "mj_jit_stats")
+    return list(v)
+
+
+def test_more_hamiltonians_than_modules_are_kept():
+    """A scan over a coupling, an object each: what is kept stays bounded, and an
+    object that lives through the scan still runs the kernels it has."""
+    from matjes_amd import llg, workloads
+    c = workloads.build_case(dict(workloads.SQUARE_JDKB, size=[64, 64, 1], seed=4))
+    with llg.from_case(c) as first:
+        B, made = first.get_eff_field(), _stats()[0]
+        for k in range(70):
+            with llg.Hamiltonian(c["lat"].dim_lat, c["lat"].periodic) as h:
+                h.add_stencil({(1, 0, 0): -1e-3 * (1.0 + k / 70.0) * np.eye(3)})
+                h.set_state(c["m0"])
+                h.get_eff_field()
+        assert _stats()[0] - made == 70 and _stats()[1] <= 64
+        assert np.array_equal(first.get_eff_field(), B)
+    with llg.from_case(c) as again:
+        assert np.array_equal(again.get_eff_field(), B)
