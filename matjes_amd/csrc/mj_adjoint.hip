@@ -284,8 +284,8 @@ static int adj_alloc(double **p, size_t n)
     return MJ_OK;
 }
 
-// The kernels compiled for the parameter set (mj_jit_adjoint), from the size at
-// which a lattice gets compiled kernels (MJ_JIT=0 never, 1 always).  The values
+// The kernels compiled for the parameter set (mj_jit_adjoint), from kJitSites
+// sites on (MJ_JIT=0 never, 1 always).  The values
 // of the total stencil change with theta, its structure does not: places with
 // the same unit coefficients in every parameter (up to one sign) hold the same
 // value, places with none hold zero.  More than 64 values, or places whose sums
@@ -297,7 +297,7 @@ static int adj_compile(mj_ctx *c, AdjState *s, const std::vector<std::array<int,
 {
     for (auto &f : s->fn) f = nullptr;
     const char *env = getenv("MJ_JIT");
-    if ((env && env[0] == '0') || (!(env && env[0] == '1') && c->n < 4096)) return MJ_OK;
+    if ((env && env[0] == '0') || (!(env && env[0] == '1') && c->n < kJitSites)) return MJ_OK;
     AdjStencil st;
     std::vector<std::vector<double>> keys;
     std::vector<double> vals;

@@ -390,12 +390,6 @@ static int pow2ceil(int v)
 }
 
 // effective tile for the current lattice
-// Lattices of at least this many sites get kernels compiled for their Hamiltonian
-// (MJ_JIT=0 never, 1 always).  40 steps of 56x59, triangular at 10 K, ahead of time ->
-// compiled: Heun 640 -> 240 us, SIB 660 -> 250, Depondt 685 -> 257; compiling takes
-// under a second once per Hamiltonian and process.
-constexpr int64_t kJitSites = 1024;
-
 static void tile_shape(const mj_ctx *c, int &bx, int &by, int &bz)
 {
     if (c->bx && c->by && c->bz) {
@@ -404,8 +398,8 @@ static void tile_shape(const mj_ctx *c, int &bx, int &by, int &bz)
         bz = c->bz;
         return;
     }
-    // 256-site tiles (32x8); below the lattices that get compiled kernels
-    // (mj_finalize) smaller ones, down to one wavefront, while there would be
+    // 256-site tiles (32x8); below the lattices that can get compiled kernels
+    // (kJitSmall) smaller ones, down to one wavefront, while there would be
     // fewer than 512 workgroups.  The fused step is the faster for its smaller
     // ring (64x64, Heun at 10 K: triangular 5.4 us per step against 6.2 with 8x8
     // tiles, square 4.4 against 4.65; 256x256: 5.9 against 6.5 with 16x8)
@@ -422,14 +416,14 @@ static void tile_shape(const mj_ctx *c, int &bx, int &by, int &bz)
         const int64_t region = (int64_t)(bx + 2 * c->rx) * (by + 2 * c->ry) * (bz + 2 * c->rz);
         return 24 * (region + 2 * bx * by * bz) <= 163840;
     };
-    if (c->n >= kJitSites && c->rz > 0) {
+    if (c->n >= kJitSmall && c->rz > 0) {
         bx = std::min(pow2ceil(c->dim[0]), 16);
         bz = std::min(pow2ceil(c->dim[2]), 4);
         by = std::min(pow2ceil(c->dim[1]), 256 / (bx * bz));
         if (bx * by * bz >= 64 && fits()) return;
     }
     int nthr = 256;
-    while (c->n < kJitSites && nthr > 64 && c->n / nthr < 512) nthr >>= 1;
+    while (c->n < kJitSmall && nthr > 64 && c->n / nthr < 512) nthr >>= 1;
     for (;; nthr >>= 1) {
         bx = std::min(pow2ceil(c->dim[0]), std::max(8, nthr / 8));
         by = std::min(pow2ceil(c->dim[1]), std::max(1, nthr / bx));
@@ -443,6 +437,27 @@ static void tile_shape(const mj_ctx *c, int &bx, int &by, int &bz)
         else if (bx < pow2ceil(c->dim[0])) bx <<= 1;
         else break;
     }
+}
+
+// the compiled kernels' geometry and sums (compiled on first use)
+static int prepare_jit(mj_ctx *c)
+{
+    int bx, by, bz;
+    tile_shape(c, bx, by, bz);
+    const int ntx = (c->dim[0] + bx - 1) / bx, nty = (c->dim[1] + by - 1) / by, ntz = (c->dim[2] + bz - 1) / bz;
+    MJ_TRY(mj_jit_prepare(c, bx, by, bz, ntx * nty * ntz, ntx, nty));
+    c->use_jit = 1;
+    c->jit_later = 0;
+    return MJ_OK;
+}
+
+// `launches` stage kernels are about to run: from kJitSmall sites on, kernels are
+// compiled once the context has run so many that compiling pays
+static int expect_launches(mj_ctx *c, int64_t launches)
+{
+    if (!c->jit_later) return MJ_OK;
+    c->aot_launches += launches;
+    return c->aot_launches < kJitPays ? MJ_OK : prepare_jit(c);
 }
 
 int mj_finalize(mj_ctx *c)
@@ -535,7 +550,7 @@ int mj_finalize(mj_ctx *c)
         c->h_ord.clear();
         c->h_blk.clear();
         c->rx = c->ry = c->rz = 0;
-        c->use_jit = 0;
+        c->use_jit = c->jit_later = 0;
     } else {
         // stencil: C_d = A_d + A_{-d}^T
         std::vector<std::array<int, 3>> offs;
@@ -643,13 +658,12 @@ int mj_finalize(mj_ctx *c)
             MJ_HIP_CHECK(hipMemcpy(c->d_ofs, ofs.data(), sizeof(int) * ofs.size(), hipMemcpyHostToDevice));
             MJ_HIP_CHECK(hipMemcpy(c->d_cf, c->h_blk.data(), sizeof(double) * c->h_blk.size(), hipMemcpyHostToDevice));
         }
-        // per-Hamiltonian compiled kernels: MJ_JIT=0 off, 1 on, otherwise for lattices >= 64x64 sites
+        // per-Hamiltonian compiled kernels: MJ_JIT=0 off, 1 on, otherwise by the lattice's size
         const char *env = getenv("MJ_JIT");
-        c->use_jit = env && env[0] == '0' ? 0 : (env && env[0] == '1') ? 1 : (c->n >= kJitSites ? 1 : 0);
-        if (c->use_jit) {
-            int ntx = (c->dim[0] + bx - 1) / bx, nty = (c->dim[1] + by - 1) / by, ntz = (c->dim[2] + bz - 1) / bz;
-            MJ_TRY(mj_jit_prepare(c, bx, by, bz, ntx * nty * ntz, ntx, nty));
-        }
+        const bool off = env && env[0] == '0', on = (env && env[0] == '1') || c->n >= kJitSites;
+        c->use_jit = 0;
+        c->jit_later = !off && c->n >= kJitSmall;
+        if (!off && on) MJ_TRY(prepare_jit(c));
     }
     // energy partial buffers
     int bx, by, bz;
@@ -779,6 +793,7 @@ extern "C" int mj_eff_field(mj_ctx *c, double *B, int64_t n3)
     if (!c->state_set) MJ_FAIL(MJ_ESTATE, "mj_eff_field: no state set");
     MJ_TRY(set_dev(c));
     MJ_TRY(mj_finalize(c));
+    MJ_TRY(expect_launches(c, 1));
     KArgs a;
     base_args(c, a);
     a.src = c->A;
@@ -825,6 +840,7 @@ extern "C" int mj_energy(mj_ctx *c, double *E)
     if (!c->state_set) MJ_FAIL(MJ_ESTATE, "mj_energy: no state set");
     MJ_TRY(set_dev(c));
     MJ_TRY(mj_finalize(c));
+    MJ_TRY(expect_launches(c, 1));
     MJ_TRY(energy_async(c, c->host.buf, 1.0));   // reduced straight into pinned memory
     MJ_HIP_CHECK(hipStreamSynchronize(c->stream));
     *E = c->host.buf[0];
@@ -1200,6 +1216,7 @@ static int run_steps(mj_ctx *c, int nsteps, int integ, double timestep, double a
     if (nsteps == 0) return MJ_OK;
     const bool noisy = kT * alpha > 1.0e-10;
     const int nl = (integ == MJ_EULER) ? 1 : (integ == MJ_RK) ? c->rk_order : 2;
+    if (!prof) MJ_TRY(expect_launches(c, (int64_t)nsteps * nl));
     double rkT[9][9];
     if (integ == MJ_RK) {
         rk_butcher(c->rk_order, rkT);
@@ -1585,6 +1602,7 @@ extern "C" int mj_profile_steps(mj_ctx *c, int nsteps, int integrator, double ti
     if (!c || !total_ms || !kind_ms || !kind_count) MJ_FAIL(MJ_EINVAL, "mj_profile_steps: null argument");
     MJ_TRY(set_dev(c));
     MJ_TRY(mj_finalize(c));
+    MJ_TRY(expect_launches(c, 2 * (int64_t)std::max(nsteps, 0)));
     Prof p;
     // one kernel per step: the fused kernel of integration 2, SIB or Depondt
     // (as run_steps picks it) or Euler on the stencil path

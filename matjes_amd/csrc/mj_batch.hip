@@ -858,14 +858,14 @@ static int blaunch_err(const char *what)
 
 // Groups of systems for the compiled fused step.  A batch of more than 4
 // groups (one launch each per step), or of coefficients in more than 32
-// classes, keeps the ahead-of-time kernel; so does a batch below the size from
-// which a lattice gets compiled kernels (MJ_JIT=0 never, 1 always).
+// classes, keeps the ahead-of-time kernel; so does a batch of fewer than
+// kJitSites sites in all (MJ_JIT=0 never, 1 always).
 static int batch_groups(mj_batch *b, const std::vector<BatchSys> &tab, const std::vector<int> &blk2sys)
 {
     const char *env = getenv("MJ_JIT");
     int64_t sites = 0;
     for (auto &s : b->sys) sites += s.n;
-    if ((env && env[0] == '0') || b->has_dip || !b->fused_ok || (!(env && env[0] == '1') && sites < 4096)) return MJ_OK;
+    if ((env && env[0] == '0') || b->has_dip || !b->fused_ok || (!(env && env[0] == '1') && sites < kJitSites)) return MJ_OK;
     std::vector<BatchGroup> gr;
     std::vector<int> of(b->sys.size());
     for (size_t q = 0; q < b->sys.size(); ++q) {

@@ -107,7 +107,9 @@ struct mj_ctx {
 
     DipolarFFT *dip = nullptr;
     void *jit = nullptr;               // per-Hamiltonian compiled stage kernels (mj_jit.hip)
-    int use_jit = 0;
+    int use_jit = 0;                   // they run now; jit_later: once aot_launches reach kJitPays
+    int jit_later = 0;
+    int64_t aot_launches = 0;          // stage kernels this context has run ahead of time
     void *adj = nullptr;               // differentiable SIB trajectory (mj_adjoint.hip)
     void *mc = nullptr;                // Metropolis Monte Carlo state (mj_mc.hip)
     // graph of a chunk of steps (small lattices: one replay instead of 2 launches per step)
@@ -128,6 +130,18 @@ struct mj_ctx {
 };
 
 int mj_finalize(mj_ctx *c);   // build device-side Hamiltonian if dirty
+
+// Objects of at least kJitSites sites run kernels compiled for their Hamiltonian
+// from their first call on (stage kernels, Monte Carlo passes, the adjoint, a
+// batch's fused step by the sites of all its systems); compiling takes 0.2 s for
+// the field, 0.5 to 0.7 s for an integrator.  A lattice of at least kJitSmall does
+// so once it has run kJitPays stage kernels ahead of time: compiled, a launch of
+// 32x32 to 56x59 sites is shorter by 1.5 to 2.5 us for the field and by 3 to 4.5
+// for a stage of an integrator, so that by then about the time of compiling has
+// gone into them; a Hamiltonian of fewer (a field, 40 steps of Heun in 0.4 to 0.5
+// ms) would wait 500 times its own time.  The kernels give the same bits.
+// MJ_JIT=0: none compiled, 1: all.
+constexpr int64_t kJitSites = 4096, kJitSmall = 1024, kJitPays = 100000;
 
 // a compiled module on its device, unloaded with its last holder
 struct JitModule {

@@ -749,14 +749,14 @@ static int launch_check(const char *what)
     return MJ_OK;
 }
 
-// The compiled kernels of passes over `sites` sites: from the size at which a
-// lattice gets compiled kernels (MJ_JIT=0 never, 1 always), where a class's
+// The compiled kernels of passes over `sites` sites (all replicas'): from kJitSites
+// on (MJ_JIT=0 never, 1 always), where a class's
 // offsets and the slots fit 31 bits
 static int mc_resolve(mj_ctx *c, McCtx *mc, int64_t sites)
 {
     const char *env = getenv("MJ_JIT");
     const int64_t W = ceil_div(c->dim[0], mc->p), cs = (int64_t)mc->p * c->dim[1] * c->dim[2] * W;
-    const bool want = !(env && env[0] == '0') && ((env && env[0] == '1') || sites >= 4096) && cs < (1 << 28) &&
+    const bool want = !(env && env[0] == '0') && ((env && env[0] == '1') || sites >= kJitSites) && cs < (1 << 28) &&
                       (!c->periodic[0] || c->dim[0] % mc->p == 0);
     if (!want) {
         mc->fn_pass = mc->fn_energy = nullptr;

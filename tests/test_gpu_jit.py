@@ -203,3 +203,28 @@ def test_more_hamiltonians_than_modules_are_kept():
         assert np.array_equal(first.get_eff_field(), B)
     with llg.from_case(c) as again:
         assert np.array_equal(again.get_eff_field(), B)
+
+
+@pytest.mark.parametrize("w", ["sq", "tri"])
+def test_small_lattices_compile_when_it_pays(w, monkeypatch):
+    """A lattice of 1024 sites: fields, energies and a short trajectory compile
+    nothing, a trajectory of more than 100,000 stages does at its start; both give
+    the bits of the ahead-of-time kernels."""
+    from matjes_amd import llg, workloads
+    monkeypatch.delenv("MJ_JIT", raising=False)
+    base = {"sq": workloads.SQUARE_JDKB, "tri": workloads.TRIANGULAR_J3DKB}[w]
+    c = workloads.build_case(dict(base, size=[32, 32, 1], seed=4))
+
+    def run(h):
+        out = [h.get_eff_field(), h.energy(), h.steps(50, 2, 0.5, 0.1, energies=True), h.get_state()]
+        made = _stats()[0]
+        return out, made, [h.steps(50010, 2, 0.1, 0.1, energies=True), h.get_state(), h.get_eff_field()]
+    with llg.from_case(c) as h:
+        m0 = _stats()[0]
+        a, m1, b = run(h)
+        assert m1 == m0 and _stats()[0] > m1
+    monkeypatch.setenv("MJ_JIT", "0")
+    with llg.from_case(c) as h:
+        a0, _, b0 = run(h)
+    for x, y in zip(a + b, a0 + b0):
+        assert np.array_equal(x, y)
