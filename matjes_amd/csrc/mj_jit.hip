@@ -26,7 +26,7 @@
 #include "_jit_embed.h"   // kJitRngH, kJitDeviceH, kJitKargsH, kJitBodyH (generated by matjes_amd/build.py)
 
 struct JitState {
-    std::string geom;              // generated geometry + stencil source
+    std::string geom;              // generated geometry + stencil source of the stage kernels
     std::map<int, JitRef> mods;    // family -> module
     hipFunction_t fn[12][2] = {};     // resolved kernels per (mode, noise)
     int nthr = 0;
@@ -34,6 +34,8 @@ struct JitState {
     // both stages of integration 2, SIB or Depondt (MODE_HEUNF, _SIBF, _DEPF) in one kernel, when the tile fits
     int fuse_ok = 0, fuse_nthr = 0, fuse_nblocks = 0;
     size_t fuse_shm = 0;
+    std::string fuse_tile;         // its constants; its sums are written when a family that has it is asked for
+    int fuse_spt = 1, fuse_T0 = 0, fuse_s0x = 0, fuse_s0y = 0, fuse_s1x = 0, fuse_s1y = 0, fuse_s1z = 0;
     // persistent stage-1 kernels (stage_body_persistent): direct fill, whole XCD bands
     int pers_ok = 0, nblocks = 0;
     size_t pers_shm = 0;
@@ -183,8 +185,7 @@ static size_t emit_fused_tile(std::ostringstream &g, int BX, int BY, int BZ, int
 // 8.03 but Depondt 9.2 -> 10.2, square 6.2 -> 6.4, 128x128x16 11.8 -> 12.2).
 // MJ_FUSE_SPT=1 or 2 asks for single tiles or pairs, MJ_FUSE_SUB=2 for double
 // tiles, MJ_FUSE_WIDE=0 or 1 against or for the ring's own wavefronts.
-static void prepare_fused(mj_ctx *c, JitState *j, std::ostringstream &g, int bx, int by, int bz, int ntx, int nty,
-                          int ntz)
+static void prepare_fused(const mj_ctx *c, JitState *j, int bx, int by, int bz, int ntx, int nty, int ntz)
 {
     j->fuse_ok = 0;
     const int nb = bx * by * bz;
@@ -202,7 +203,6 @@ static void prepare_fused(mj_ctx *c, JitState *j, std::ostringstream &g, int bx,
     for (; form >= 0; --form) {
         const int spt = form == 2 ? 2 : 1, nsub = form ? 2 : 1;
         const int BX = bx, BY = by * nsub, BZ = bz, nthr = BX * BY * BZ / spt;
-        const int s0x = BX + 4 * rx, s0y = BY + 4 * ry, s1x = BX + 2 * rx, s1y = BY + 2 * ry;
         const bool dma = bx % 2 == 0 && c->dim[0] % 2 == 0 && nthr % 64 == 0;
         std::ostringstream t;
         int T0 = 0;
@@ -214,30 +214,42 @@ static void prepare_fused(mj_ctx *c, JitState *j, std::ostringstream &g, int bx,
         const size_t shm = emit_fused_tile(t, BX, BY, BZ, rx, ry, rz, nthr, spt, nsub, nb, wide, dma, T0, alias);
         if (shm > 65536 || nthr + wide > 1024) continue;
         const int ntyf = (c->dim[1] + BY - 1) / BY, ntzf = (c->dim[2] + BZ - 1) / BZ;
-        g << "struct JitFused {\n" << t.str();
-        g << "  static constexpr bool kEnergy = true;\n";
+        t << "  static constexpr bool kEnergy = true;\n";
         auto cst = [&](const char *n, const char *ty, long v) {
-            g << "  static __device__ __forceinline__ constexpr " << ty << " " << n << "(const KArgs &) { return " << v
+            t << "  static __device__ __forceinline__ constexpr " << ty << " " << n << "(const KArgs &) { return " << v
               << "; }\n";
         };
         cst("nx", "int", c->dim[0]), cst("ny", "int", c->dim[1]), cst("nz", "int", c->dim[2]);
         cst("ntx", "int", ntx), cst("nty", "int", ntyf), cst("nty_base", "int", nty);
         cst("bmode", "int", c->bmode), cst("dma", "bool", dma);   // bmode: 0 no Zeeman, 1 uniform, 2 per site
-        g << "  static __device__ __forceinline__ int block(const KArgs &) { return mj_xcd_remap(blockIdx.x, "
+        t << "  static __device__ __forceinline__ int block(const KArgs &) { return mj_xcd_remap(blockIdx.x, "
           << ntx * ntyf * ntzf << "); }\n";
-        const auto ofs3 = sum_offsets(c);
-        const auto cf = literal_coef(c);
-        const int t1 = s1x * s1y * (BZ + 2 * rz);
-        emit_sum(g, ofs3, "stencil0", 1, s0x, s0x * s0y, T0, cf);
-        emit_sum(g, ofs3, spt == 2 ? "pair1" : "stencil1", spt, s1x, s1x * s1y, t1, cf);
-        if (spt == 2) emit_sum(g, ofs3, "pair0", 2, s0x, s0x * s0y, T0, cf);
-        g << "};\n";
+        j->fuse_tile = t.str();
+        j->fuse_spt = spt;
+        j->fuse_T0 = T0;
+        j->fuse_s0x = BX + 4 * rx;
+        j->fuse_s0y = BY + 4 * ry;
+        j->fuse_s1x = BX + 2 * rx;
+        j->fuse_s1y = BY + 2 * ry;
+        j->fuse_s1z = BZ + 2 * rz;
         j->fuse_ok = 1;
         j->fuse_nthr = nthr + wide;
         j->fuse_nblocks = ntx * ntyf * ntzf;
         j->fuse_shm = shm;
         return;
     }
+}
+
+static void emit_fused(std::ostringstream &g, const mj_ctx *c, const JitState *j)
+{
+    g << "struct JitFused {\n" << j->fuse_tile;
+    const auto ofs3 = sum_offsets(c);
+    const auto cf = literal_coef(c);
+    const int xy0 = j->fuse_s0x * j->fuse_s0y, xy1 = j->fuse_s1x * j->fuse_s1y, t1 = xy1 * j->fuse_s1z;
+    emit_sum(g, ofs3, "stencil0", 1, j->fuse_s0x, xy0, j->fuse_T0, cf);
+    emit_sum(g, ofs3, j->fuse_spt == 2 ? "pair1" : "stencil1", j->fuse_spt, j->fuse_s1x, xy1, t1, cf);
+    if (j->fuse_spt == 2) emit_sum(g, ofs3, "pair0", 2, j->fuse_s0x, xy0, j->fuse_T0, cf);
+    g << "};\n";
 }
 
 int mj_jit_fused_ok(const mj_ctx *c) { return c->jit && ((const JitState *)c->jit)->fuse_ok; }
@@ -287,7 +299,7 @@ int mj_jit_prepare(mj_ctx *c, int bx, int by, int bz, int nblocks, int ntx, int 
     j->pers_shm = (size_t)6 * TS * sizeof(double);
     for (auto &f : j->fnp) f = nullptr;
     for (auto &g2 : j->pers_grid) g2 = 0;
-    prepare_fused(c, j, g, bx, by, bz, ntx, nty, ntx == 0 ? 0 : nblocks / (ntx * nty));
+    prepare_fused(c, j, bx, by, bz, ntx, nty, ntx == 0 ? 0 : nblocks / (ntx * nty));
     j->geom = g.str();
     return MJ_OK;
 }
@@ -298,12 +310,13 @@ void mj_jit_destroy(mj_ctx *c)
     c->jit = nullptr;
 }
 
-static std::string family_source(const JitState *j, int fam);
+static std::string family_source(const mj_ctx *c, const JitState *j, int fam);
+static std::string device_headers();
 
 // the source of the kernels of one integrator family (for offline inspection)
 std::string mj_jit_source(const mj_ctx *c, int fam)
 {
-    return c->jit ? family_source((const JitState *)c->jit, fam) : std::string();
+    return c->jit ? device_headers() + family_source(c, (const JitState *)c->jit, fam) : std::string();
 }
 
 JitModule::~JitModule()
@@ -357,10 +370,14 @@ static ModCache<JitModule> &modules()
     return *cache;
 }
 
-// the module of a source text on a device (the caller's current one)
-static int compile_source(int device, const std::string &src, JitRef *out)
+// The module of a source on a device (the caller's current one): the device
+// headers, `extra` ones, and `src`, which alone says which module it is.  With
+// the 80 KB of headers in the text to be built and found, the first field of a
+// new object took 30 to 70 us more (64x64 and 128x128, triangular).
+static int compile_source(int device, const std::string &src, const char *extra, JitRef *out)
 {
-    return modules().get(device, src, out, [&](JitRef *m) { return compile_module(device, src, m); });
+    return modules().get(device, src, out,
+                         [&](JitRef *m) { return compile_module(device, device_headers() + extra + "\n" + src, m); });
 }
 
 extern "C" int mj_jit_stats(int64_t *compiled, int64_t *kept)
@@ -374,7 +391,7 @@ extern "C" int mj_jit_stats(int64_t *compiled, int64_t *kept)
 
 static int compile_family(const mj_ctx *c, JitState *j, int fam, JitRef *out)
 {
-    return compile_source(c->device, family_source(j, fam), out);
+    return compile_source(c->device, family_source(c, j, fam), "", out);
 }
 
 static std::string device_headers()
@@ -423,7 +440,7 @@ int mj_jit_batch_fused(int device, const std::vector<int> &ofs3, const std::vect
     emit_sum(g, ofs3, "stencil1", 1, s1x, s1x * s1y, s1x * s1y * (1 + 2 * rz), cf);
     g << "};\n";
     std::ostringstream s;
-    s << device_headers() << kJitBatchH << "\n" << g.str();
+    s << g.str();
     s << "extern \"C\" __global__ void __launch_bounds__(" << bx * by
       << ") mj_batch_fused(const KArgs base, const BatchSys *__restrict__ sys, const int *__restrict__ blk2sys, "
          "const double *__restrict__ sigma, const uint64_t *__restrict__ stepp, const int *__restrict__ list, int nlist, "
@@ -431,7 +448,7 @@ int mj_jit_batch_fused(int device, const std::vector<int> &ofs3, const std::vect
          "  const int b = mj_xcd_remap(blockIdx.x, nlist);\n  const int gb = list ? list[b] : b;\n"
          "  const int s = blk2sys[gb];\n  KArgs a = sys_args(base, sys[s], gb, sigma[s], *stepp + base.step);\n"
          "  a.cf = vals + (int64_t)s * " << ncls << ";\n  fused_body<" << mode << ", true, BatchFused>(a, lds);\n}\n";
-    const int rc = compile_source(device, s.str(), mod);
+    const int rc = compile_source(device, s.str(), kJitBatchH, mod);
     if (rc != MJ_OK) return rc;
     const hipError_t e = hipModuleGetFunction(fn, (*mod)->mod, "mj_batch_fused");
     if (e != hipSuccess) return mj_hip_fail(MJ_EHIP, std::string("hipModuleGetFunction mj_batch_fused: ") + hipGetErrorString(e));
@@ -505,14 +522,14 @@ int mj_jit_adjoint(const mj_ctx *c, const AdjStencil &st, const int b[3], const 
     }
     g << "  }\n};\n";
     std::ostringstream s;
-    s << device_headers() << kJitAdjH << "\n" << g.str();
+    s << g.str();
     static const char *names[MJ_ADJ_KERNELS] = {"sib1", "sib2", "sibf", "r1", "r2", "r3r1", "r3"};
     auto want = [&](int k) { return k == MJ_ADJ_SIBF ? fused : k == MJ_ADJ_SIB1 || k == MJ_ADJ_SIB2 ? !fused : true; };
     for (int k = 0; k < MJ_ADJ_KERNELS; ++k)
         if (want(k))
             s << "extern \"C\" __global__ void __launch_bounds__(" << nthr << ") mj_adj_" << names[k]
               << "(const AdjArgs a) { extern __shared__ double lds[]; adj_" << names[k] << "_body<AdjJit>(a, lds); }\n";
-    const int rc = compile_source(c->device, s.str(), mod);
+    const int rc = compile_source(c->device, s.str(), kJitAdjH, mod);
     if (rc != MJ_OK) return rc;
     for (int k = 0; k < MJ_ADJ_KERNELS; ++k) {
         if (!want(k)) continue;
@@ -615,12 +632,12 @@ int mj_jit_mc(const mj_ctx *c, const std::vector<int> &o3, const std::vector<dou
     if (ne == 0) g << "    mid();\n";
     g << "    return mk3(ax, ay, az);\n  }\n};\n";
     std::ostringstream s;
-    s << device_headers() << kJitMcH << "\n" << g.str();
+    s << g.str();
     s << "extern \"C\" __global__ void __launch_bounds__(kMcThreads) mj_mc_pass(const McArgs a) { "
          "mc_pass_body<McGeom>(a); }\n";
     s << "extern \"C\" __global__ void __launch_bounds__(kMcThreads) mj_mc_energy(const McArgs a, double *part) { "
          "mc_energy_body<McGeom>(a, part); }\n";
-    const int rc = compile_source(c->device, s.str(), mod);
+    const int rc = compile_source(c->device, s.str(), kJitMcH, mod);
     if (rc != MJ_OK) return rc;
     hipError_t e = hipModuleGetFunction(pass, (*mod)->mod, "mj_mc_pass");
     if (e == hipSuccess) e = hipModuleGetFunction(energy, (*mod)->mod, "mj_mc_energy");
@@ -628,10 +645,11 @@ int mj_jit_mc(const mj_ctx *c, const std::vector<int> &o3, const std::vector<dou
     return MJ_OK;
 }
 
-static std::string family_source(const JitState *j, int fam)
+static std::string family_source(const mj_ctx *c, const JitState *j, int fam)
 {
     std::ostringstream s;
-    s << device_headers() << j->geom << "\n";
+    s << j->geom << "\n";
+    if (j->fuse_ok && fam >= 2 && fam <= 4) emit_fused(s, c, j);
     static const int fam_modes[6][3] = {{MODE_FIELD, -1, -1}, {MODE_EULER, -1, -1}, {MODE_HEUN1, MODE_HEUN2, MODE_HEUNF},
                                         {MODE_SIB1, MODE_SIB2, MODE_SIBF}, {MODE_DEP1, MODE_DEP2, MODE_DEPF},
                                         {MODE_RKS, -1, -1}};
