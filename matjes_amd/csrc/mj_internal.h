@@ -164,6 +164,10 @@ struct AdjStencil {
     std::vector<int> o3, cls;
     std::vector<std::vector<int>> po3;
     std::vector<std::vector<double>> pblk;
+    bool operator==(const AdjStencil &o) const
+    {
+        return o3 == o.o3 && cls == o.cls && po3 == o.po3 && pblk == o.pblk;
+    }
 };
 int mj_jit_adjoint(const mj_ctx *c, const AdjStencil &st, const int b[3], const int r[3], bool fused,
                    JitRef *mod, hipFunction_t fn[MJ_ADJ_KERNELS]);

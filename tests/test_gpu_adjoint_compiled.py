@@ -24,7 +24,7 @@ CASES = {
 }
 
 
-def _run(c, jit):
+def _run(c, jit, before=()):
     import torch
     from matjes_amd import adjoint, workloads
     env = dict({"MJ_JIT": jit}, **c.get("env", {}))
@@ -42,6 +42,8 @@ def _run(c, jit):
         r = adjoint.SIBRunner(lat, c.get("names", ["J1", "D", "K"]), nsteps=13, timestep=1.0, damping=0.2, ckpt_every=5)
         try:
             out, gh, gm = torch.empty_like(m0), torch.empty_like(m0), torch.empty_like(m0)
+            for th in before:
+                r.forward(np.array(th), np.array([0.0, 0.1, 0.5]), h, m0, out)
             r.forward(np.array(c.get("theta", [1e-3, 0.3e-3, -0.05e-3])), np.array([0.0, 0.1, 0.5]), h, m0, out)
             gt, gb = r.backward((2 * (out - tgt)).contiguous(), gh, gm)
             torch.cuda.synchronize()
@@ -61,3 +63,12 @@ def test_compiled_equals_ahead_of_time(name):
     ref, got = _run(CASES[name], "0"), _run(CASES[name], "1")
     for a, b in zip(ref, got):
         assert np.isfinite(a).all() and np.array_equal(a, b), name
+
+
+def test_other_parameters_in_the_same_runner():
+    """Passes with other values, zero and of the other sign, before the one compared
+    (the kernels stay, their values change; sums that round apart leave them)."""
+    c = CASES["reach2"]
+    before = ([2e-3, -0.1e-3, 0.0, 0.05e-3], [1e-3, 0.0, 0.0, 0.0], [-1e-3, 0.3e-3, 0.1e-3, 0.0])
+    for a, b in zip(_run(c, "0"), _run(c, "1", before)):
+        assert np.array_equal(a, b)
