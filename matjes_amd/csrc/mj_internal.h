@@ -172,9 +172,12 @@ struct AdjStencil {
 int mj_jit_adjoint(const mj_ctx *c, const AdjStencil &st, const int b[3], const int r[3], bool fused,
                    JitRef *mod, hipFunction_t fn[MJ_ADJ_KERNELS]);
 // Monte Carlo kernels of a stencil without its on-site entry (offsets o3, full blocks cf9, class shifts csh) on the
-// context's lattice coloured (x + ca y + cb z) mod p
+// context's lattice coloured (x + ca y + cb z) mod p; vals: the distinct coefficients, for McArgs::vals (more than
+// kMcMaxVals are literals, and none returned)
+constexpr int kMcMaxVals = 32;
 int mj_jit_mc(const mj_ctx *c, const std::vector<int> &o3, const std::vector<double> &cf9, const std::vector<int> &csh,
-              int p, int ca, int cb, JitRef *mod, hipFunction_t *pass, hipFunction_t *energy);
+              int p, int ca, int cb, JitRef *mod, hipFunction_t *pass, hipFunction_t *energy,
+              std::vector<double> *vals);
 // the fused step of a batch's systems of one stencil and tile (fn null: its tile does not fit in LDS)
 int mj_jit_batch_fused(int device, const std::vector<int> &ofs3, const std::vector<int> &cls, int ncls, int bx, int by,
                        int rx, int ry, int rz, int mode, JitRef *mod, hipFunction_t *fn, size_t *shm);

@@ -541,15 +541,18 @@ int mj_jit_adjoint(const mj_ctx *c, const AdjStencil &st, const int b[3], const 
 
 // Monte Carlo passes and replica energies: the neighbours' slots from the
 // lattice's constants, the spins of 18 neighbours in flight together (the
-// proposal is computed under the first ones), coefficients as literals, terms
+// proposal is computed under the first ones), coefficients as operands, terms
 // in the order and with the operations of mc_pair_field_cm (zero ones left out).
 // Latency bounds a pass (two wavefronts per SIMD at 131072 sites): 18 neighbours
 // in three trips through a table of slots took 18.2 us per class of 1024^2 (8
 // classes) and 13.9 us for 8 replicas of 256^2, one trip with the addresses from
-// constants 8.1 and 6.6; replica energies 34.6 -> 22.  Blocks of 64 and 128
+// constants 8.1 and 6.6; replica energies 34.6 -> 22.  The distinct coefficients
+// (up to sign) are read into scalar registers, so that a scan over couplings
+// compiles once per structure; more than 32 are literals.  Blocks of 64 and 128
 // threads: 8 and 2 % slower at 1024^2, equal at 256^2.
 int mj_jit_mc(const mj_ctx *c, const std::vector<int> &o3, const std::vector<double> &cf9, const std::vector<int> &csh,
-              int p, int ca, int cb, JitRef *mod, hipFunction_t *pass, hipFunction_t *energy)
+              int p, int ca, int cb, JitRef *mod, hipFunction_t *pass, hipFunction_t *energy,
+              std::vector<double> *vals)
 {
     constexpr int kGroup = 18;
     const int nx = c->dim[0], ny = c->dim[1], nz = c->dim[2], W = (nx + p - 1) / p, ne = (int)csh.size();
@@ -593,6 +596,22 @@ int mj_jit_mc(const mj_ctx *c, const std::vector<int> &o3, const std::vector<dou
         g << "    const int r" << i << " = (y" << i << " + " << ny << " * z" << i << ") * " << W << "; const bool cr" << i
           << " = cy" << i << " && cz" << i << ";\n";
     }
+    vals->clear();
+    auto place = [&](double v) {   // of +-v among them
+        return std::find_if(vals->begin(), vals->end(), [&](double w) { return w == v || w == -v; }) - vals->begin();
+    };
+    for (double v : cf9)
+        if (v != 0.0 && place(v) == (ptrdiff_t)vals->size()) vals->push_back(v);
+    const bool literal = vals->size() > kMcMaxVals;
+    if (literal) vals->clear();
+    auto coef = [&](double v) {
+        if (literal) {
+            hexd(g, v);
+        } else {
+            const auto k = place(v);
+            g << ((*vals)[k] == v ? "" : "-") << "a.vals[" << k << "]";
+        }
+    };
     auto has = [&](int e, int col) { return cf9[9 * e + col] != 0.0 || cf9[9 * e + 3 + col] != 0.0 || cf9[9 * e + 6 + col] != 0.0; };
     static const char *mm[3] = {"mx", "my", "mz"}, *acc[3] = {"ax", "ay", "az"};
     for (int e0 = 0; e0 < ne; e0 += kGroup) {
@@ -624,7 +643,7 @@ int mj_jit_mc(const mj_ctx *c, const std::vector<int> &o3, const std::vector<dou
                     const double v = cf9[9 * e + 3 * r + d];
                     if (v == 0.0) continue;
                     g << "    " << acc[r] << " = fma(";
-                    hexd(g, v);
+                    coef(v);
                     g << ", " << mm[d] << e << ", " << acc[r] << ");\n";
                 }
         }

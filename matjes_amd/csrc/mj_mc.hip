@@ -466,10 +466,12 @@ __global__ void __launch_bounds__(kMcThreads) k_mc_msum_final(const double *part
 // host side
 // ---------------------------------------------------------------------------
 static_assert(kMcIsing == MJ_MC_ISING, "sampler codes");
+static_assert(kMcVals == kMcMaxVals, "places for the values");
 
 struct McCtx {
     hipFunction_t fn_pass = nullptr, fn_energy = nullptr;   // compiled for this stencil and lattice (null: ahead-of-time)
     JitRef mod;
+    std::vector<double> vals;          // their coefficients' values
     int resolved = 0;
     // stencil without the on-site entry, and the colouring it admits
     std::vector<int> o3;
@@ -757,15 +759,16 @@ static int mc_resolve(mj_ctx *c, McCtx *mc, int64_t sites)
     const char *env = getenv("MJ_JIT");
     const int64_t W = ceil_div(c->dim[0], mc->p), cs = (int64_t)mc->p * c->dim[1] * c->dim[2] * W;
     const bool want = !(env && env[0] == '0') && ((env && env[0] == '1') || sites >= kJitSites) && cs < (1 << 28) &&
-                      (!c->periodic[0] || c->dim[0] % mc->p == 0);
+                      (!c->periodic[0] || c->dim[0] % mc->p == 0) &&
+                      std::all_of(mc->cf9.begin(), mc->cf9.end(), [](double v) { return std::isfinite(v); });
     if (!want) {
         mc->fn_pass = mc->fn_energy = nullptr;
         mc->resolved = 0;
         return MJ_OK;
     }
     if (mc->resolved) return MJ_OK;
-    MJ_TRY(mj_jit_mc(c, mc->o3, mc->cf9, mc->csh, mc->p, mc->ca, mc->cb, &mc->mod, &mc->fn_pass,
-                     &mc->fn_energy));
+    MJ_TRY(mj_jit_mc(c, mc->o3, mc->cf9, mc->csh, mc->p, mc->ca, mc->cb, &mc->mod, &mc->fn_pass, &mc->fn_energy,
+                     &mc->vals));
     mc->resolved = 1;
     return MJ_OK;
 }
@@ -865,6 +868,7 @@ static void mc_args(const mj_ctx *c, const McCtx *mc, McArgs &a)
     a.cs = (int64_t)mc->p * c->dim[1] * c->dim[2] * a.W;
     a.csh = mc->d_csh;
     a.cf9 = mc->d_cf9;
+    std::copy(mc->vals.begin(), mc->vals.end(), a.vals);
     a.fast = mc->fast;
     a.ne = (int)(mc->o3.size() / 3);
     a.ylo = mc->ylo;

@@ -5,6 +5,7 @@
 constexpr uint32_t kMcStream = 0x4D430000u;   // counter word 3 of the Monte Carlo draws
 constexpr int kMcIsing = 1;            // MJ_MC_ISING
 constexpr int kMcThreads = 256;
+constexpr int kMcVals = 32;
 
 struct McState {
     double cone, cos_cone, acc, nb, rate;
@@ -59,6 +60,7 @@ struct McArgs {
     const int64_t *sites;
     const double *spins;    // AoS 3 per site, or null for the current spin
     double *e_out;
+    double vals[kMcVals];   // compiled kernels: the stencil's distinct values
 };
 
 __device__ __forceinline__ v3 mc_zeeman(const McArgs &a, const double *bmap, int64_t stride, int64_t i)

@@ -82,3 +82,31 @@ def test_stencil_that_grows_between_sweeps(jit, monkeypatch):
             h.mc_sweeps(4, 1, 1e-3, seed=9)
             out.append(h.get_state())
     assert np.array_equal(out[0], out[1])
+
+
+def test_scan_over_a_coupling_compiles_once(monkeypatch):
+    """Sweeps of Hamiltonians that differ in their couplings' values: one module for
+    all, each with its own values (against the ahead-of-time passes)."""
+    import ctypes
+    from matjes_amd import _lib, llg, workloads
+
+    def made():
+        v = ctypes.c_int64()
+        _lib.check(_lib.load().mj_jit_stats(ctypes.addressof(v), None), "mj_jit_stats")
+        return v.value
+
+    def sweep(c, jit):
+        monkeypatch.delenv("MJ_JIT", raising=False)
+        if jit is not None:
+            monkeypatch.setenv("MJ_JIT", jit)
+        with llg.from_case(c, form="stencil") as h:
+            n = made()
+            h.mc_set_cone(0.4)
+            h.mc_sweeps(4, 0, 1e-3, seed=9)
+            return h.get_state(), made() - n
+    base = workloads.TRIANGULAR_J3DKB
+    for k, scale in enumerate((1.0, 0.7, -1.3)):
+        c = workloads.build_case(dict(base, size=[136, 64, 1], seed=11, J=[scale * j for j in base["J"]],
+                                      D=scale * base["D"]))
+        (ref, _), (got, n) = sweep(c, "0"), sweep(c, None)
+        assert np.array_equal(ref, got) and n == (1 if k == 0 else 0)
