@@ -398,9 +398,11 @@ static void tile_shape(const mj_ctx *c, int &bx, int &by, int &bz)
         bz = c->bz;
         return;
     }
-    // 256-site tiles (32x8); below the lattices that can get compiled kernels
-    // (kJitSmall) smaller ones, down to one wavefront, while there would be
-    // fewer than 512 workgroups.  The fused step is the faster for its smaller
+    // 256-site tiles (32x8); below the lattices that run compiled kernels from
+    // their first call on smaller ones, down to one wavefront, while there would be
+    // fewer than 512 workgroups: ahead of time a launch is the latency of a tile
+    // (40x40, 100 steps, square, 32x8 -> 8x8: Heun 1165 -> 1063 us, SIB 1138 -> 1046;
+    // triangular Heun 1493 -> 1460).  The fused step is the faster for its smaller
     // ring (64x64, Heun at 10 K: triangular 5.4 us per step against 6.2 with 8x8
     // tiles, square 4.4 against 4.65; 256x256: 5.9 against 6.5 with 16x8)
     // Bonds across the planes: 16x4x4 (two planes: 16x8x2), whose ring is half of
@@ -423,7 +425,7 @@ static void tile_shape(const mj_ctx *c, int &bx, int &by, int &bz)
         if (bx * by * bz >= 64 && fits()) return;
     }
     int nthr = 256;
-    while (c->n < kJitSmall && nthr > 64 && c->n / nthr < 512) nthr >>= 1;
+    while (c->n < kJitSites && nthr > 64 && c->n / nthr < 512) nthr >>= 1;
     for (;; nthr >>= 1) {
         bx = std::min(pow2ceil(c->dim[0]), std::max(8, nthr / 8));
         by = std::min(pow2ceil(c->dim[1]), std::max(1, nthr / bx));
