@@ -271,7 +271,7 @@ int mj_jit_prepare(mj_ctx *c, int bx, int by, int bz, int nblocks, int ntx, int 
     const int TS = dma ? 2 * nthr * ((T / 2 + nthr - 1) / nthr) : T;   // LDS component stride
     g << "struct JitGeom {\n";
     g << "  static constexpr int kNit = " << (T + bx * by * bz - 1) / (bx * by * bz) << ";\n";
-    g << "  static constexpr bool kDma = " << (dma ? "true" : "false") << ", kCfLds = false;\n";
+    g << "  static constexpr bool kDma = " << (dma ? "true" : "false") << ", kCfLds = false;\n  static constexpr int kTrips = 1;\n";
     g << "  static constexpr int kT = " << TS << ";\n";
     g << "  static __device__ __forceinline__ int tstride(const KArgs &, int) { return " << TS << "; }\n";
     g << "  static constexpr int kBx = " << bx << ", kBy = " << by << ", kBz = " << bz << ", kRx = " << c->rx

@@ -310,7 +310,7 @@ int mj_launch_stage(int mode, bool noise, const KArgs &args, hipStream_t s)
     size_t T = (size_t)a.sx * a.sy * a.sz;
     size_t shm = a.use_stencil ? 3 * T * sizeof(double) : 0;
     const size_t blocks = (size_t)9 * a.n_ent * sizeof(double);
-    a.cf_lds = a.use_stencil && blocks <= 8192 && shm + blocks <= 65536;
+    a.cf_lds = a.use_stencil && a.n_ent > 0 && blocks <= 8192 && shm + blocks <= 65536;
     if (a.cf_lds) shm += blocks;
     size_t need = (size_t)nthr * sizeof(double);
     if (shm < need) shm = need;  // block reduction scratch

@@ -98,7 +98,8 @@ __device__ __forceinline__ double mj_block_max(double v, double *red, int nthr)
 struct RtGeom {
     static constexpr int kNit = 0;         // trips of the tile fill: known only at run time
     static constexpr bool kDma = false;    // direct global -> LDS fill (compile-time geometry only)
-    static constexpr bool kCfLds = false;  // the stencil's blocks staged in LDS behind the tile
+    static constexpr bool kCfLds = false;  // the stencil's blocks staged in LDS behind the tile,
+    static constexpr int kTrips = 1;       // so many values a thread at once
     // LDS stride between the x, y, z components of the tile (the tile size here)
     static __device__ __forceinline__ int tstride(const KArgs &, int T) { return T; }
     static __device__ __forceinline__ int bx(const KArgs &a) { return a.bx; }
@@ -152,20 +153,35 @@ struct RtGeom {
 // few tiles, where a launch is the latency of one tile, and the blocks' way
 // through a cold scalar cache came after the tile's instead of with it (32x32,
 // Heun, us per step: square 11.5 -> 11.2, triangular 15.1 -> 15.3, integration 4
-// 26.5 -> 25.3 and 34.6 -> 33.6)
+// 26.5 -> 25.3 and 34.6 -> 33.6).  A tile of one wavefront copies three values a
+// thread: all in flight before the tile's loads, stored after them (24x24, 100
+// steps, copied one after the other -> so: triangular Heun 1465 -> 1372 us, SIB
+// 1448 -> 1364, square 1055 -> 1045).
 struct AotGeom : RtGeom {
     static constexpr bool kCfLds = true;
+    static constexpr int kTrips = 3;
     static __device__ __forceinline__ void stencil(const KArgs &a, const double *L, int T, int c, double &ax,
                                                    double &ay, double &az)
     {
         if (a.cf_lds) sum(a.n_ent, a.ofs, L + 3 * T, L, T, c, ax, ay, az);
         else sum(a.n_ent, a.ofs, a.cf, L, T, c, ax, ay, az);
     }
-    // issued before the tile's loads
-    static __device__ __forceinline__ void stage(const KArgs &a, double *L, int T)
+    // the blocks, a few values a thread, in flight before the tile's loads ...
+    static __device__ __forceinline__ void load(const KArgs &a, double v[kTrips])
     {
-        if (a.cf_lds)
-            for (int t = threadIdx.x; t < 9 * a.n_ent; t += blockDim.x) L[3 * T + t] = a.cf[t];
+        if (!a.cf_lds) return;
+#pragma unroll
+        for (int i = 0; i < kTrips; ++i) v[i] = a.cf[min((int)(threadIdx.x + i * blockDim.x), 9 * a.n_ent - 1)];
+    }
+    // ... and stored after them
+    static __device__ __forceinline__ void store(const KArgs &a, double *L, int T, const double v[kTrips])
+    {
+        if (!a.cf_lds) return;
+        int t = threadIdx.x;
+#pragma unroll
+        for (int i = 0; i < kTrips; ++i, t += blockDim.x)
+            if (t < 9 * a.n_ent) L[3 * T + t] = v[i];
+        for (; t < 9 * a.n_ent; t += blockDim.x) L[3 * T + t] = a.cf[t];
     }
 };
 
@@ -610,10 +626,8 @@ __device__ __forceinline__ void stage_body(const KArgs &a, double *lds)
                                 (int64_t)(x0 - RX) + (int64_t)NX * ((int64_t)(y0 - RY) + (int64_t)NY * (z0 - RZ)));
     }
     SiteCtx st = site_begin<MODE, NOISE, G>(a, x0, y0, z0, nstep);
-    if constexpr (G::kCfLds) {
-        if (a.use_stencil)
-            G::stage(a, lds, (G::bx(a) + 2 * G::rx(a)) * (G::by(a) + 2 * G::ry(a)) * (G::bz(a) + 2 * G::rz(a)));
-    }
+    [[maybe_unused]] double cf[G::kTrips];
+    if constexpr (G::kCfLds) G::load(a, cf);
     if (direct) {
         site_thermal<MODE, NOISE>(a, st);
         __builtin_amdgcn_s_waitcnt(0);   // this wave's tile loads are in LDS
@@ -626,6 +640,8 @@ __device__ __forceinline__ void stage_body(const KArgs &a, double *lds)
     // loaded after it (fewer registers live across it)
     constexpr bool kAux = MODE == MODE_HEUN2 || MODE == MODE_DEP2;
     if constexpr (kAux && NOISE && G::kNit > 0) st.pre_aux = mk3(a.aux[st.gi], a.aux[st.gi + a.np], a.aux[st.gi + 2 * a.np]);
+    if constexpr (G::kCfLds)
+        G::store(a, lds, (G::bx(a) + 2 * G::rx(a)) * (G::by(a) + 2 * G::ry(a)) * (G::bz(a) + 2 * G::rz(a)), cf);
     if (a.use_stencil) __syncthreads();
     site_end<MODE, NOISE, G>(a, lds, st, G::part(a), blockIdx.x == 0);
 }

@@ -84,3 +84,17 @@ def test_order_of_integration_4_between_calls():
                 E = h.steps(70, 4, 2.0, 0.2, energies=True)
             out.append((h.get_state(), E))
     assert np.array_equal(out[0][0], out[1][0]) and np.array_equal(out[0][1], out[1][1])
+
+
+@pytest.mark.parametrize("n", [5, 8, 24])
+def test_a_field_without_bonds(n):
+    """No entry in the stencil, on lattices below the compiled kernels: the effective
+    field is the external one, and two calls agree."""
+    from matjes_amd import llg
+    m0 = np.tile([0.6, 0.0, 0.8], (n * n, 1))
+    c = _paramagnet_case(n, [0.0, 0.0, 2.5], m0)
+    with llg.from_case(c) as h:
+        B = h.get_eff_field()
+        h.steps(3, 2, 1.0, 0.1)
+        assert np.max(np.abs(B - np.array([0.0, 0.0, L.MU_B * 2.5]))) <= 4 * 2.0 ** -53 * L.MU_B * 2.5
+        assert np.array_equal(h.get_eff_field(), B)
