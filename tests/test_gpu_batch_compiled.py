@@ -4,7 +4,8 @@ each), more groups than it takes or a later group of too many coefficients (the
 ahead-of-time kernel runs), coefficients
 that differ, change sign or vanish between systems, odd rows (no paired loads),
 tiles from one site a row (rows of the region that do not pair up) to one row, inside the lattice,
-lattices smaller than a tile and its halo, open edges, a per-site field."""
+lattices smaller than a tile and its halo, open edges, several planes, a
+per-site field."""
 import os
 
 import numpy as np
@@ -27,13 +28,15 @@ BATCHES = {
     "long": [("sq", dict(size=[8, 1030, 1])), ("sq", dict(size=[1030, 8, 1], D=0.1e-3))],
     # the second stencil has more coefficients than the compiled step takes
     "second_too_rich": [("sq", SQ[0]), ("sq", dict(size=[40, 36, 1], rich=True)), ("sq", SQ[1])],
+    "planes": [("film", dict(size=[20, 17, 4])), ("film", dict(size=[34, 12, 3], periodic=[False, False, False]))],
     "vanishing": [("sq", dict(size=[48, 40, 1], J=[0.0], B=[0.0, 0.0, 0.0])), ("sq", SQ[0])],
 }
 
 
 def _run(specs, jit, integ, tiles):
     from matjes_amd import batch, lattice, llg, workloads
-    base = {"sq": workloads.SQUARE_JDKB, "tri": workloads.TRIANGULAR_J3DKB}
+    base = {"sq": workloads.SQUARE_JDKB, "tri": workloads.TRIANGULAR_J3DKB,
+            "film": dict(workloads.FILM_DIP, dipolar=False)}
     old = os.environ.get("MJ_JIT")
     os.environ["MJ_JIT"] = jit
     hs = []
