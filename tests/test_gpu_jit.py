@@ -228,3 +228,37 @@ def test_small_lattices_compile_when_it_pays(w, monkeypatch):
         a0, _, b0 = run(h)
     for x, y in zip(a + b, a0 + b0):
         assert np.array_equal(x, y)
+
+
+def test_threads_share_the_modules():
+    """Four threads, an object at a time each, over six Hamiltonians (each compiled by
+    whichever thread comes first): the results are those of one thread."""
+    import threading
+    from matjes_amd import llg, workloads
+    cases = [workloads.build_case(dict(workloads.SQUARE_JDKB, size=[66, 64, 1], seed=4, J=[(1.0 + 0.03 * k) * 1e-3]))
+             for k in range(6)]
+
+    def run(c):
+        with llg.from_case(c, form="stencil") as h:
+            E = h.steps(6, 2, 0.5, 0.1, kT=1e-3, seed=3, energies=True)
+            h.mc_sweeps(1, 0, 1e-3, seed=5)
+            return E, h.get_state(), h.get_eff_field()
+    got, errors = {}, []
+
+    def work(t):
+        try:
+            for i in range(len(cases)):
+                k = (i + t) % len(cases)
+                got[t, k] = run(cases[k])
+        except Exception as e:   # shown by the assertion below
+            errors.append(e)
+    threads = [threading.Thread(target=work, args=(t,)) for t in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not errors
+    for k, c in enumerate(cases):
+        want = run(c)
+        for t in range(4):
+            assert all(np.array_equal(a, b) for a, b in zip(got[t, k], want)), (t, k)
