@@ -1,4 +1,4 @@
-// Per-Hamiltonian stage kernels compiled at set-up with hipRTC.
+// Per-Hamiltonian stage kernels compiled with hipRTC on first use.
 //
 // The stencil of a translation-invariant Hamiltonian is known once the
 // Hamiltonian is registered, so the stage kernel is specialised for it: the
@@ -407,7 +407,7 @@ static std::string device_headers()
 // cls[9 entry + q]: 0 a coefficient that is zero in every such system, +-k the
 // k-th value of a system's `ncls` (or its negative): the values stay in scalar
 // registers, an operand of the fused products.
-// FP64 issue bounds it, as the single lattice's step.  24 replicas of 256^2
+// Instruction issue bounds it, as the single lattice's step.  24 replicas of 256^2
 // (18 neighbours, T > 0) and 12 more lattices of 32 to 400 a side, 2.2 M sites:
 // 50 us a step, the ahead-of-time kernel (k_batch_fused: offsets and full 3x3
 // blocks read in a loop, wrapped coordinates per staged site) 81 us.

@@ -11,8 +11,9 @@
 //
 // The thermal normals use the word forms below (mj_ln_u32, mj_sincos2pi_u32,
 // mj_cos2pi_u32, mj_radius): the uniform is taken from its 32-bit word by
-// integer operations, which issue at twice the rate of FP64 ones (octant,
-// fraction and signs of the angle, exponent and mantissa of the logarithm),
+// integer operations (octant, fraction and signs of the angle, exponent and
+// mantissa of the logarithm: fewer instructions than the FP64 ones they replace;
+// each takes the same issue slot),
 // the polynomials are the interpolants at Chebyshev nodes of the ranges they
 // cover (within 5e-18 to 3e-17, two terms shorter than the series), the
 // logarithm's quotient and the square root start from the hardware reciprocal
@@ -36,7 +37,7 @@
 
 // a b + c for a constant c.  On the device c comes from scalar registers: left
 // to itself the compiler copies such a constant into vector registers before
-// every fma that accumulates onto it, one more FP64 issue slot per term of a
+// every fma that accumulates onto it, one more issue slot per term of a
 // polynomial.  a and b must not be results of v_rcp/v_rsq taken directly (the
 // compiler does not insert the wait state those need before inline assembly).
 MJ_HD double mj_fma_k(double a, double b, double c)
