@@ -136,10 +136,11 @@ int mj_finalize(mj_ctx *c);   // build device-side Hamiltonian if dirty
 // batch's fused step by the sites of all its systems); compiling takes 0.2 s for
 // the field, 0.5 to 0.7 s for an integrator.  A lattice of at least kJitSmall does
 // so once it has run kJitPays stage kernels ahead of time: compiled, a launch of
-// 32x32 to 56x59 sites is shorter by 1.5 to 2.5 us for the field and by 3 to 4.5
-// for a stage of an integrator, so that by then about the time of compiling has
-// gone into them; a Hamiltonian of fewer (a field, 40 steps of Heun in 0.4 to 0.5
-// ms) would wait 500 times its own time.  The kernels give the same bits.
+// 32x32 to 56x59 sites is shorter by 1.4 to 2.9 us for the field, 1.3 to 2.1 for
+// Euler and 2.8 to 3.7 for a stage of Heun, SIB or Depondt (8.7 us a step -> 3.1 on
+// the square lattice, 11.9 -> 4.5 on the triangular one), so that by then about the
+// time of compiling would have been saved; a Hamiltonian of fewer (a field, 40 steps
+// of Heun in 0.4 to 0.5 ms) would wait 500 times its own time.  The kernels give the same bits.
 // MJ_JIT=0: none compiled, 1: all.
 constexpr int64_t kJitSites = 4096, kJitSmall = 1024, kJitPays = 100000;
 
