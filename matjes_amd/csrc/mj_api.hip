@@ -475,9 +475,9 @@ int mj_finalize(mj_ctx *c)
         if (c->bvec.empty()) MJ_FAIL(MJ_ESTATE, "Zeeman term registered but no B order parameter set");
         bool uniform = true;
         if (c->bvec.size() != 3) {
+            const double *v = c->bvec.data(), x = v[0], y = v[1], z = v[2];
             for (int64_t i = 1; i < c->n && uniform; ++i)
-                for (int a = 0; a < 3; ++a)
-                    if (c->bvec[3 * i + a] != c->bvec[a]) uniform = false;
+                uniform = !((v[3 * i] != x) | (v[3 * i + 1] != y) | (v[3 * i + 2] != z));
         }
         if (uniform) {
             c->bmode = 1;
